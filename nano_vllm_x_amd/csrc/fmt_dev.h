@@ -51,6 +51,14 @@ template <int LPR> __device__ __forceinline__ float group_sum(float v) {      //
     return v;
 }
 
+// block256_sum for a `red` that nothing else of the kernel uses: one barrier, and the sums of a wave in the vector ALU
+__device__ __forceinline__ float block256_sum_once(float v, float* red) {
+    v = group_sum<64>(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3];
+}
+
 // A step's table of rotations: row t holds cos of token t's angles and, sin_off entries further on, their sin (float32).  `cos` points at
 // the first angle of the rotation in question (several rotations share a row).
 struct TurnRows { const float* cos; int64_t stride; int64_t sin_off; };

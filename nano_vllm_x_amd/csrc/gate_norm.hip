@@ -105,6 +105,74 @@ __global__ __launch_bounds__(256) void postnorm_residual_kernel(const A* __restr
     }
 }
 
+// The same for rows that stand on borders of four elements in every operand (width a multiple of four, at most 1024 * NC): a row passes
+// through the workgroup's registers, so every operand is read once, all loads are asked for together and the two sums are all that a row
+// waits for.  The kernel above reads its rows two elements at a time and some of them three times.  Bound: HBM on long steps (14 bytes an
+// element with one 16-bit result), one trip to memory and two sums on short ones.  4096 rows of 1024: 17.1 -> 11.0 us; 16 rows of 2048:
+// 9.3 -> 5.0 us.
+template <typename A, int NC>
+__global__ __launch_bounds__(256) void postnorm_residual_wide_kernel(const A* __restrict__ y, int64_t y_stride, const A* __restrict__ y2,
+                                                                    int64_t y2_stride, float a, float b, const float* __restrict__ w_post,
+                                                                    int w_post_n, float* __restrict__ x, const float* __restrict__ w_next,
+                                                                    int w_next_n, float eps, A* __restrict__ h_out, int width) {
+    typedef A veca __attribute__((ext_vector_type(4)));
+    __shared__ float red[2][4];
+    const int64_t t = blockIdx.x;
+    float* xr = x + t * (int64_t)width;
+    nvx_f32x4 v[NC], r[NC], wp[NC], wn[NC];
+    const float wp1 = y && w_post_n == 1 ? w_post[0] : 0.f, wn1 = w_next && w_next_n == 1 ? w_next[0] : 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        v[i] = r[i] = wp[i] = wn[i] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+        if (c < width) {
+            v[i] = *reinterpret_cast<const nvx_f32x4*>(xr + c);
+            if (y) {
+                const veca u = *reinterpret_cast<const veca*>(y + t * y_stride + c);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) r[i][k] = a * (float)u[k];
+                wp[i] = w_post_n == 1 ? nvx_f32x4{wp1, wp1, wp1, wp1} : *reinterpret_cast<const nvx_f32x4*>(w_post + c);
+            }
+            if (y2) {
+                const veca u = *reinterpret_cast<const veca*>(y2 + t * y2_stride + c);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) r[i][k] += b * (float)u[k];
+            }
+            if (w_next) wn[i] = w_next_n == 1 ? nvx_f32x4{wn1, wn1, wn1, wn1} : *reinterpret_cast<const nvx_f32x4*>(w_next + c);
+        }
+    }
+    if (y) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) ss += r[i][0] * r[i][0] + r[i][1] * r[i][1] + r[i][2] * r[i][2] + r[i][3] * r[i][3];
+        const float rn = 1.0f / sqrtf(block256_sum_once(ss, red[0]) / (float)width + eps);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int c = (threadIdx.x + i * 256) * 4;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[i][k] += r[i][k] * rn * wp[i][k];
+            if (c < width) *reinterpret_cast<nvx_f32x4*>(xr + c) = v[i];
+        }
+    }
+    if (!h_out) return;
+    float rx = 1.0f;
+    if (w_next) {
+        float sx = 0.f;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) sx += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+        rx = 1.0f / sqrtf(block256_sum_once(sx, red[1]) / (float)width + eps);
+    }
+    A* hr = h_out + t * (int64_t)width;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        veca o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = (A)(w_next ? v[i][k] * rx * wn[i][k] : v[i][k]);
+        if (c < width) *reinterpret_cast<veca*>(hr + c) = o;
+    }
+}
+
 // Several residual streams per token (x: (tokens, streams, width) float32) and the sublayer boundary between them.  Per token t:
 //   with a result y:   r = y[t] * scale (scale: one number per channel, or none);
 //                      every stream at once from the old ones:  x_j' = sum_s mix[s][j] x_s + w_out[j] r      (mix indexed [from][to])
@@ -350,6 +418,55 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
 }
 
 
+// The same by four elements a thread (rows on borders of four elements in every operand), a head's values in registers: LPR lanes a head
+// of 4 * LPR values, or (LPR = 256) a workgroup a head of at most 1024 * NC values -- a read-out whose heads are normed together.  One wave
+// that walks such a head alone, 64 values a trip, took 36 us over 16 rows of 2048 where this takes 5.0; 4096 rows of 1024: 28.5 -> 10.3 us.
+// Heads of 128, 3847 x 16: 32.3 -> 15.7 us.  Bound: HBM (12 bytes a value in 16-bit formats).
+template <typename A, int LPR, int NC>
+__global__ __launch_bounds__(256) void head_norm_gate_vec_kernel(const float* __restrict__ o, const float* __restrict__ w, int w_shared,
+                                                                const A* __restrict__ gate, int64_t gate_stride, int kind, float eps, float mul,
+                                                                A* __restrict__ out, int64_t out_stride, int64_t n_rows, int heads, int vdim) {
+    typedef A veca __attribute__((ext_vector_type(4)));
+    __shared__ float red[4];
+    const int64_t idx = LPR == 256 ? blockIdx.x : ((int64_t)blockIdx.x * 256 + threadIdx.x) / LPR;
+    const bool in = idx < n_rows;                  // (lanes past the last head take part in the sums of their own group only)
+    const int64_t t = (in ? idx : 0) / heads;
+    const int hd = (int)((in ? idx : 0) % heads), l = threadIdx.x % LPR;
+    const float* row = o + t * (int64_t)heads * vdim + (int64_t)hd * vdim;
+    const A* gr = kind ? gate + t * gate_stride + (int64_t)hd * vdim : nullptr;
+    const float* wr = w ? w + (w_shared ? 0 : hd * vdim) : nullptr;
+    nvx_f32x4 v[NC], wv[NC];
+    veca z[NC];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int e = (l + i * LPR) * 4;
+        v[i] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+        wv[i] = nvx_f32x4{1.f, 1.f, 1.f, 1.f};
+        if (e < vdim) {
+            v[i] = *reinterpret_cast<const nvx_f32x4*>(row + e);
+            if (wr) wv[i] = *reinterpret_cast<const nvx_f32x4*>(wr + e);
+            if (kind) z[i] = *reinterpret_cast<const veca*>(gr + e);
+        }
+        ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+    }
+    const float total = LPR == 256 ? block256_sum_once(ss, red) : group_sum<LPR == 256 ? 64 : LPR>(ss);
+    const float rn = mul / sqrtf(total / (float)vdim + eps);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int e = (l + i * LPR) * 4;
+        if (!in || e >= vdim) continue;
+        veca r;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float u = v[i][k] * rn * wv[i][k];
+            if (kind) { const float g = (float)z[i][k]; u *= kind == 1 ? sigmoid_f(g) : g * sigmoid_f(g); }
+            r[k] = (A)u;
+        }
+        *reinterpret_cast<veca*>(out + t * out_stride + (int64_t)hd * vdim + e) = r;
+    }
+}
+
 // Projections onto FEW outputs or from FEW inputs, in float32: gate and router logits (outputs = heads or experts), the two
 // halves of a low-rank decay.  out[t][n] = g(sum_k W[n][k] * f(x[t][k]) + bias[n]), f = identity or tanh, g = identity or
 // sigmoid(.)^power (formed as exp(power * logsigmoid(.))); W float32 (n_out, k_in), bias float32 or null.  A
@@ -534,6 +651,26 @@ extern "C" int nvx_head_norm_gate(const float* o, const float* w, int w_shared, 
                 "nvx_head_norm_gate: null pointer or row stride");
     const int64_t rows = n_tok * heads;
     NVX_REQUIRE((rows + 3) / 4 < (1ll << 31), NVX_EINVAL, "nvx_head_norm_gate: too many rows");
+    // four elements a thread where every operand's rows stand on such borders: groups of lanes for heads that fill them, a workgroup for
+    // heads from 512 values on (a wave alone takes as many trips as there are 64s in the head); other head sizes keep the wave
+    const size_t item = fmt == 2 ? 4 : 2;
+    const auto ok4 = [&](const void* p, size_t size) { return (reinterpret_cast<uintptr_t>(p) & (4 * size - 1)) == 0; };
+    if (vdim % 4 == 0 && ok4(o, 4) && ok4(w, 4) && ok4(out, item) && out_stride % 4 == 0 && (kind == 0 || (ok4(gate, item) && gate_stride % 4 == 0))) {
+#define NVX_HEAD_NORM(LPR, NC)                                                                                                                       \
+    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((head_norm_gate_vec_kernel<A_, LPR, NC>), dim3((unsigned)(LPR == 256 ? rows : (rows + 256 / LPR - 1) / (256 / LPR))), \
+                                         dim3(256), 0, (hipStream_t)stream, o, w, w_shared, (const A_*)gate, gate_stride, kind, eps, mul, (A_*)out, out_stride,  \
+                                         rows, (int)heads, (int)vdim))
+        bool done = true;
+        if (vdim == 64) NVX_HEAD_NORM(16, 1);
+        else if (vdim == 128) NVX_HEAD_NORM(32, 1);
+        else if (vdim == 256) NVX_HEAD_NORM(64, 1);
+        else if (vdim >= 512 && vdim <= 1024) NVX_HEAD_NORM(256, 1);
+        else if (vdim > 1024 && vdim <= 2048) NVX_HEAD_NORM(256, 2);
+        else if (vdim > 2048 && vdim <= 4096) NVX_HEAD_NORM(256, 4);
+        else done = false;
+#undef NVX_HEAD_NORM
+        if (done) return nvx_check_launch("nvx_head_norm_gate");
+    }
     NVX_FMT_CALL(fmt, hipLaunchKernelGGL(head_norm_gate_kernel<A_>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, (hipStream_t)stream, o, w,
                                          w_shared, (const A_*)gate, gate_stride, kind, eps, mul, (A_*)out, out_stride, rows, (int)heads, (int)vdim));
     return nvx_check_launch("nvx_head_norm_gate");
@@ -550,6 +687,22 @@ extern "C" int nvx_postnorm_residual(const void* y, int64_t y_stride, const void
                 "nvx_postnorm_residual: a result needs its norm weight (one number or one per channel)");
     NVX_REQUIRE(!y2 || (y && y2_stride >= width), NVX_EINVAL, "nvx_postnorm_residual: a second result needs a first");
     NVX_REQUIRE(!w_next || (h_out && (w_next_n == 1 || w_next_n == width)), NVX_EINVAL, "nvx_postnorm_residual: the closing norm needs an output");
+    const size_t item = fmt == 2 ? 4 : 2;
+    const auto ok4 = [&](const void* p, size_t size) { return (reinterpret_cast<uintptr_t>(p) & (4 * size - 1)) == 0; };
+    // rows of up to 4096 elements on borders of four in every operand: a thread's share stays in registers.  One weight for the whole row
+    // may stand anywhere.
+    if (width % 4 == 0 && width <= 4096 && ok4(x, 4) && ok4(y, item) && ok4(y2, item) && ok4(h_out, item) && (!y || y_stride % 4 == 0) &&
+        (!y2 || y2_stride % 4 == 0) && (!y || w_post_n == 1 || ok4(w_post, 4)) && (w_next_n == 1 || ok4(w_next, 4))) {
+#define NVX_POSTNORM(NC)                                                                                                                        \
+    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((postnorm_residual_wide_kernel<A_, NC>), dim3((unsigned)n_tok), dim3(256), 0, (hipStream_t)stream, (const A_*)y, \
+                                         y_stride, (const A_*)y2, y2_stride, a, b, w_post, (int)w_post_n, x, w_next, (int)w_next_n, eps, (A_*)h_out,  \
+                                         (int)width))
+        if (width <= 1024) NVX_POSTNORM(1);
+        else if (width <= 2048) NVX_POSTNORM(2);
+        else NVX_POSTNORM(4);
+#undef NVX_POSTNORM
+        return nvx_check_launch("nvx_postnorm_residual");
+    }
     NVX_FMT_CALL(fmt, hipLaunchKernelGGL(postnorm_residual_kernel<A_>, dim3((unsigned)n_tok), dim3(256), 0, (hipStream_t)stream, (const A_*)y,
                                          y_stride, (const A_*)y2, y2_stride, a, b, w_post, (int)w_post_n, x, w_next, (int)w_next_n, eps, (A_*)h_out,
                                          (int)width));
