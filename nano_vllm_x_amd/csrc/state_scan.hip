@@ -15,8 +15,9 @@
 // share a column and add their partial read-outs by lane exchange.  The tokens' keys, queries and values are staged
 // through LDS TB tokens at a time (converted to float32, unit-normed where the design asks for it), so the sequential
 // loop touches no global memory but its output.  Memory, normaliser, maximum, gates and decays are float32.
+// Portions of several tokens with keys of up to 128 go to the matrix cores instead where the recurrence has a block form (scan_mfma.hip).
 // A batch is ragged (see seq_mix.hip): qo_indptr / pos0 / state_slot; a sequence at position 0 takes zeros for its state.
-#include "fmt_dev.h"
+#include "scan_dev.h"
 
 namespace NVX_NS {
 
@@ -845,6 +846,12 @@ static bool scan_launch(int64_t dim, int64_t vdim, ScanLaunch* g) {      // (a t
     return true;
 }
 
+// Whether a launch of decay, gla or mlstm goes to the matrix cores: keys that its staging rows hold, and portions that fill a block of 16
+// tokens on average or are cut into chunks (a single token costs there what 16 do).
+static bool scan_on_matrix_cores(const int32_t* qo_indptr, int64_t n_tok, int64_t n_seq, int64_t dim, int64_t chunk) {
+    return dim <= 128 && qo_indptr && (chunk || n_tok >= 16 * n_seq);
+}
+
 }  // namespace NVX_NS
 
 using namespace NVX_NS;
@@ -910,7 +917,8 @@ extern "C" int nvx_token_shift_mix(const void* h, int64_t h_stride, int fmt, con
 extern "C" int64_t nvx_scan_column_blocks(int64_t dim, int64_t vdim) {
     ScanLaunch g;
     if (dim <= 0 || vdim <= 0 || !scan_launch(dim, vdim, &g)) return 0;
-    return (vdim + g.cb - 1) / g.cb;
+    const int64_t cb = dim <= 128 && nvx_scan_mfma_columns() < g.cb ? nvx_scan_mfma_columns() : g.cb;      // (the narrower of the two kernels' blocks)
+    return (vdim + cb - 1) / cb;
 }
 
 extern "C" int nvx_mlstm_scan(const void* x, int64_t x_stride, int fmt, int64_t q_off, int64_t k_off, int64_t v_off, const float* gates,
@@ -931,7 +939,8 @@ extern "C" int nvx_mlstm_scan(const void* x, int64_t x_stride, int fmt, int64_t 
     NVX_REQUIRE(chunk == 0 || (chunk > 0 && chunk < (1 << 30) && n_chunk_max > 0 && n_seq * n_chunk_max <= 65535 && ws && qo_indptr), NVX_EINVAL,
                 "nvx_mlstm_scan: chunks need a ragged step, their workspace, and at most 65535 of them");
     const dim3 grid((unsigned)((vdim + g.cb - 1) / g.cb), (unsigned)heads, (unsigned)(chunk ? n_seq * n_chunk_max : n_seq));
-    NVX_REQUIRE(chunk || grid.x == 1 || (N_in != N && M_in != M), NVX_EINVAL,
+    const bool mfma = scan_on_matrix_cores(qo_indptr, n_tok, n_seq, dim, chunk);
+    NVX_REQUIRE(chunk || (mfma ? vdim <= nvx_scan_mfma_columns() : grid.x == 1) || (N_in != N && M_in != M), NVX_EINVAL,
                 "nvx_mlstm_scan: a head with several column blocks reads its normaliser and maximum from copies");
     // the workspace: memories, normalisers, maxima, forget sums / keep factors, put factors of all chunks
     const int64_t n_ws = chunk ? n_seq * n_chunk_max * heads : 0;
@@ -942,17 +951,25 @@ extern "C" int nvx_mlstm_scan(const void* x, int64_t x_stride, int fmt, int64_t 
     NVX_FMT_CALL(fmt, hipLaunchKernelGGL((mlstm_scan_kernel<A_, PHASE>), grid, dim3(g.threads), lds, st, (const A_*)x, x_stride, (int)q_off, (int)k_off, \
                                          (int)v_off, gates, gate_bias, cap, S, N_in, M_in, N, M, qo_indptr, pos0, state_slot, out, (int)heads, (int)dim, \
                                          (int)vdim, g.p_lanes, tb, (int)stage_vec_ok<A_>(x, x_stride, q_off, k_off, v_off, dim, vdim, g.cb), ck))
+    ScanArgs sa = {};
+    sa.x = x; sa.x_stride = x_stride; sa.q_off = (int)q_off; sa.k_off = (int)k_off; sa.v_off = (int)v_off; sa.heads = (int)heads; sa.dim = (int)dim;
+    sa.vdim = (int)vdim; sa.chunk = (int)chunk; sa.n_chunk_max = (int)n_chunk_max; sa.q_mul = 1.0f / sqrtf((float)dim); sa.k_mul = 1.0f; sa.cap = cap;
+    sa.gates = gates; sa.gate_bias = gate_bias; sa.S = S; sa.ws = ck.S; sa.N_in = N_in; sa.M_in = M_in; sa.N = N; sa.M = M; sa.N_ws = ck.N; sa.M_ws = ck.M;
+    sa.F_ws = ck.F; sa.qo_indptr = qo_indptr; sa.pos0 = pos0; sa.state_slot = state_slot; sa.out = out;
     if (!chunk) {
-        NVX_MLSTM_SCAN(0);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_MLSTM, 0, n_seq, st);
+        else NVX_MLSTM_SCAN(0);
     } else {
-        NVX_MLSTM_SCAN(1);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_MLSTM, 1, n_seq, st);
+        else NVX_MLSTM_SCAN(1);
         hipLaunchKernelGGL(mlstm_chunk_scalars_kernel, dim3((unsigned)((n_seq * heads + 63) / 64)), dim3(64), 0, st, M, ck.M, ck.F, put, qo_indptr, pos0,
                            state_slot, (int)heads, (int)chunk, (int)n_chunk_max, (int)n_seq);
         hipLaunchKernelGGL(chunk_carry_kernel, dim3((unsigned)((heads * dim * vdim + 255) / 256), (unsigned)n_seq), dim3(256), 0, st, S, ck.S,
                            (const float*)ck.F, 0, (const float*)put, qo_indptr, pos0, state_slot, (int)heads, (int)dim, (int)vdim, (int)chunk, (int)n_chunk_max);
         hipLaunchKernelGGL(chunk_carry_kernel, dim3((unsigned)((heads * dim + 255) / 256), (unsigned)n_seq), dim3(256), 0, st, N, ck.N,
                            (const float*)ck.F, 0, (const float*)put, qo_indptr, pos0, state_slot, (int)heads, (int)dim, 1, (int)chunk, (int)n_chunk_max);
-        NVX_MLSTM_SCAN(3);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_MLSTM, 3, n_seq, st);
+        else NVX_MLSTM_SCAN(3);
     }
 #undef NVX_MLSTM_SCAN
     return nvx_check_launch("nvx_mlstm_scan");
@@ -1023,15 +1040,23 @@ extern "C" int nvx_decay_scan(const void* x, int64_t x_stride, int fmt, int64_t 
                                          (int)q_off, (int)k_off, (int)v_off, act, decay, S, qo_indptr, pos0, state_slot, out, (int)heads, (int)dim,  \
                                          (int)vdim, g.p_lanes, tb, (int)stage_vec_ok<A_>(x, x_stride, q_off, k_off, v_off, dim, vdim, g.cb * nc), (int)chunk, (int)n_chunk_max, ws, tr, \
                                          rot_dims / 2, k_mul))
+    const bool mfma = scan_on_matrix_cores(qo_indptr, n_tok, n_seq, dim, chunk);
+    ScanArgs sa = {};
+    sa.x = x; sa.x_stride = x_stride; sa.q_off = (int)q_off; sa.k_off = (int)k_off; sa.v_off = (int)v_off; sa.act = act; sa.heads = (int)heads; sa.dim = (int)dim;
+    sa.vdim = (int)vdim; sa.chunk = (int)chunk; sa.n_chunk_max = (int)n_chunk_max; sa.half = rot_dims / 2; sa.q_mul = 1.0f; sa.k_mul = k_mul; sa.decay = decay;
+    sa.S = S; sa.ws = ws; sa.qo_indptr = qo_indptr; sa.pos0 = pos0; sa.state_slot = state_slot; sa.out = out; sa.turn = tr;
     if (!chunk) {
-        NVX_DECAY_SCAN(0, 1);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_DECAY, 0, n_seq, (hipStream_t)stream);
+        else NVX_DECAY_SCAN(0, 1);
     } else {
-        if (nc == 2) NVX_DECAY_SCAN(1, 2);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_DECAY, 1, n_seq, (hipStream_t)stream);
+        else if (nc == 2) NVX_DECAY_SCAN(1, 2);
         else NVX_DECAY_SCAN(1, 1);
         hipLaunchKernelGGL(decay_chunk_carry_kernel, dim3((unsigned)((heads * dim * vdim + 255) / 256), (unsigned)n_seq), dim3(256), 0,
                            (hipStream_t)stream, decay, S, ws, qo_indptr, pos0, state_slot, (int)heads, (int)dim, (int)vdim, (int)chunk,
                            (int)n_chunk_max);
-        if (nc == 2) NVX_DECAY_SCAN(3, 2);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_DECAY, 3, n_seq, (hipStream_t)stream);
+        else if (nc == 2) NVX_DECAY_SCAN(3, 2);
         else NVX_DECAY_SCAN(3, 1);
     }
 #undef NVX_DECAY_SCAN
@@ -1093,15 +1118,23 @@ extern "C" int nvx_gla_scan(const void* x, int64_t x_stride, int fmt, int64_t q_
     NVX_FMT_CALL(fmt, hipLaunchKernelGGL((gla_scan_kernel<A_, PHASE, NC>), grid, dim3(g.threads), lds, st, (const A_*)x, x_stride, (int)q_off, (int)k_off, \
                                          (int)v_off, q_mul, alpha, S, qo_indptr, pos0, state_slot, out, (int)heads, (int)dim, (int)vdim, g.p_lanes, \
                                          tb, (int)(stage_vec_ok<A_>(x, x_stride, q_off, k_off, v_off, dim, vdim, g.cb * nc) && nvx_aligned16(alpha)), (int)chunk, (int)n_chunk_max, ws, keep))
+    const bool mfma = scan_on_matrix_cores(qo_indptr, n_tok, n_seq, dim, chunk);
+    ScanArgs sa = {};
+    sa.x = x; sa.x_stride = x_stride; sa.q_off = (int)q_off; sa.k_off = (int)k_off; sa.v_off = (int)v_off; sa.heads = (int)heads; sa.dim = (int)dim;
+    sa.vdim = (int)vdim; sa.chunk = (int)chunk; sa.n_chunk_max = (int)n_chunk_max; sa.q_mul = q_mul; sa.k_mul = 1.0f; sa.alpha = alpha; sa.S = S; sa.ws = ws;
+    sa.keep_ws = keep; sa.qo_indptr = qo_indptr; sa.pos0 = pos0; sa.state_slot = state_slot; sa.out = out;
     if (!chunk) {
-        NVX_GLA_SCAN(0, 1);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_GLA, 0, n_seq, st);
+        else NVX_GLA_SCAN(0, 1);
     } else {
-        if (nc == 2) NVX_GLA_SCAN(1, 2);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_GLA, 1, n_seq, st);
+        else if (nc == 2) NVX_GLA_SCAN(1, 2);
         else NVX_GLA_SCAN(1, 1);
         hipLaunchKernelGGL(chunk_carry_kernel, dim3((unsigned)((heads * dim * vdim + 255) / 256), (unsigned)n_seq), dim3(256), 0, st, S, ws,
                            (const float*)keep, 1, (const float*)nullptr, qo_indptr, pos0, state_slot, (int)heads, (int)dim, (int)vdim, (int)chunk,
                            (int)n_chunk_max);
-        if (nc == 2) NVX_GLA_SCAN(3, 2);
+        if (mfma) nvx_launch_scan_mfma(sa, fmt, SCAN_GLA, 3, n_seq, st);
+        else if (nc == 2) NVX_GLA_SCAN(3, 2);
         else NVX_GLA_SCAN(3, 1);
     }
 #undef NVX_GLA_SCAN

@@ -978,22 +978,22 @@ def token_shift_mix(h, mu, state, layout: StepLayout):
     return out
 
 
-SCAN_CHUNK_FROM = 256       # portions from this length on are cut into chunks that run side by side
-SCAN_CHUNKS = ((49152, 32), (98304, 64), (None, 128))      # (tokens x heads of a step up to ..., tokens of a chunk): short chunks while
-# the step is too small to fill the chip with long ones, long chunks (fewer carried states) from there on (4 x 1 024 tokens: 8 heads 97 us
-# at 32, 151 at 64, 267 at 128; 16 heads 238, 164, 287; 32 heads 400, 418, 302)
-GLA_SCAN_CHUNKS = ((32768, 32), (None, 64))       # (4 x 1 024 tokens: 8 heads 116 us at 32, 164 at 64; 16 heads 222 and 178)
-MLSTM_SCAN_CHUNKS = ((None, 64),)                 # (the same: 191 and 167; 312 and 291; one walk per portion: 1 420)
+SCAN_CHUNK_FROM = 129       # portions of more than two stages are cut into chunks that run side by side (8 heads, 130 tokens: gla 32 -> 25 us;
+# decay 30 -> 28; mlstm 31 -> 33; 256 tokens: 46 -> 25, 43 -> 27, 47 -> 33)
 SCAN_WS_BYTES = 1 << 30     # the chunks' states may take this much; longer chunks otherwise
+SCAN_WORKGROUPS = 512       # what a step's chunks should come to: two workgroups a compute unit
 
 
-def _scan_chunks(layout: StepLayout, heads: int, per_chunk: int, chunk: Optional[int], table=SCAN_CHUNKS):
+def _scan_chunks(layout: StepLayout, heads: int, per_chunk: int, chunk: Optional[int], vdim: int):
     """(chunk, chunks of the longest portion) a recurrence over a matrix per head cuts a step's portions into (0, 0: not at all).
-    `per_chunk`: floats of workspace a chunk of one sequence takes; `chunk` None: by the step's shape, from `table`."""
+    `per_chunk`: floats of workspace a chunk of one sequence takes; `chunk` None: by the step's shape, as many tokens as give the chip
+    SCAN_WORKGROUPS workgroups, in the 64 tokens that a workgroup stages together (16 heads 64 x 128, us for decay / gla / mlstm
+    at 32, 64, 128, 256 tokens a chunk: 3 847 tokens 121 / 112 / 149, 93 / 89 / 112, 105 / 87 / 103, 147 / 116 / 126; 8 heads, 16 384
+    tokens: 218 / 219 / 330, 155 / 160 / 215, 141 / 141 / 171, 137 / 125 / 146)."""
     if chunk is None:
         chunk = 0
         if layout.qo_indptr is not None and layout.max_q >= SCAN_CHUNK_FROM:
-            chunk = next(c for upto, c in table if upto is None or layout.n_tok * heads <= upto)
+            chunk = 64 * max(1, layout.n_tok * heads * -(-vdim // 128) // (64 * SCAN_WORKGROUPS))
     if not chunk or layout.qo_indptr is None:
         return 0, 0
     while layout.n_seq * -(-layout.max_q // chunk) * per_chunk * 4 > SCAN_WS_BYTES or layout.n_seq * -(-layout.max_q // chunk) > 65535:
@@ -1021,7 +1021,7 @@ def mlstm_scan(x, offsets, gates, gate_bias, cap: float, mem, norm, peak, layout
     # a head whose value columns take several workgroups: all of them read the normaliser and the maximum, the first writes them
     # back, so they read from copies (a workgroup that starts late must not see the new values)
     per_chunk = heads * (dim * (vdim + 1) + 3)
-    chunk, n_chunks = _scan_chunks(layout, heads, per_chunk, chunk, MLSTM_SCAN_CHUNKS)
+    chunk, n_chunks = _scan_chunks(layout, heads, per_chunk, chunk, vdim)
     ws = torch.empty((layout.n_seq * n_chunks * per_chunk,), dtype=F32, device=x.device) if chunk else None
     several = not chunk and lib.nvx_scan_column_blocks(dim, vdim) != 1
     norm_in, peak_in = (norm.clone(), peak.clone()) if several else (norm, peak)
@@ -1316,7 +1316,7 @@ def decay_scan(x, offsets, decay, mem, layout: StepLayout, heads: int, dim: int,
     _need(decay.numel() == heads and mem.shape == (n_slots, heads, dim, vdim), "decay_scan: shapes")
     t = x.shape[0]
     out = torch.empty((t, heads, vdim), dtype=F32, device=x.device)
-    chunk, n_chunks = _scan_chunks(layout, heads, heads * dim * vdim, chunk)
+    chunk, n_chunks = _scan_chunks(layout, heads, heads * dim * vdim, chunk, vdim)
     ws = torch.empty((layout.n_seq * n_chunks, heads, dim, vdim), dtype=F32, device=x.device) if chunk else None
     lib = _lib.load()
     _lib.check(lib.nvx_decay_scan(_ptr(x), x.stride(0), _fmt(x), offsets[0], offsets[1], offsets[2], {"none": 0, "silu": 1}[act], _ptr(decay),
@@ -1733,7 +1733,7 @@ def gla_scan(x, offsets, alpha, mem, layout: StepLayout, heads: int, dim: int, v
     _need(alpha.shape == (t, heads * dim) and mem.shape == (n_slots, heads, dim, vdim), "gla_scan: shapes")
     out = torch.empty((t, heads, vdim), dtype=F32, device=x.device)
     per_chunk = heads * dim * (vdim + 1)
-    chunk, n_chunks = _scan_chunks(layout, heads, per_chunk, chunk, GLA_SCAN_CHUNKS)
+    chunk, n_chunks = _scan_chunks(layout, heads, per_chunk, chunk, vdim)
     ws = torch.empty((layout.n_seq * n_chunks * per_chunk,), dtype=F32, device=x.device) if chunk else None
     lib = _lib.load()
     _lib.check(lib.nvx_gla_scan(_ptr(x), x.stride(0), _fmt(x), offsets[0], offsets[1], offsets[2], float(q_mul), _ptr(alpha), _ptr(mem), n_slots,
