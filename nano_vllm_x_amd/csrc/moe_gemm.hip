@@ -1,0 +1,232 @@
+// The experts of steps of many tokens: two grouped matrix products over the (token, choice) pairs in expert order, without the pairs' numbers
+// ever reaching the host.
+//   up    y[r] = act(s W_gate x, s W_up x)   for row r of the expert order, x read from the token's own row (no copy into expert order), the
+//         choice's weight s (where it scales the input) and the activation applied to the float32 sums;
+//   down  out[r] = W_down y[r], float32.
+// A workgroup of four waves takes a tile of 128 pairs of one expert and 128 rows of its weights (up: 64 gate rows and the 64 up rows beside
+// them, so that a wave holds both halves of an output); which expert and tile it is comes from the experts' counts, so one launch serves
+// whatever the router chose.  64 columns of both operands at a time travel memory -> LDS without registers into one of two buffers while the
+// other is multiplied (v_mfma_f32_32x32x16, one barrier a step; 16-byte pieces XOR-swizzled on the global side, operand reads free of
+// conflicts); 64 KB a workgroup, two a CU.  Results turn around in LDS and leave as whole rows.  Tiles are dealt so that an XCD works on
+// neighbouring tiles (8 row tiles by as many weight tiles share its L2).  Bound: the CU's 64 bytes a clock from L2, at which two workgroups
+// of this tile keep the matrix cores busy for at most as long as they wait.  One library product per expert and direction, with a copy into
+// expert order ahead of them and the activation between, needed 16 + 3 launches and the counts on the host.
+// 8192 pairs over 8 experts of 1536 x 1024: up 93 us (560 TFLOP/s), down 54 (480), the weighted sum 8.6; the library's products with copy,
+// activation and sum took 270 for a layer, and its counts a wait of the host.
+#include "moe_dev.h"
+
+namespace NVX_NS {
+
+constexpr int GT = 128;                // pairs, and weight rows, of a tile
+constexpr int GK = 64;                 // columns of a step
+constexpr int G_ROWS = 8;              // row tiles whose workgroups are neighbours
+
+__device__ __forceinline__ nvx_f32x16 mfma32(nvx_u32x4 a, nvx_u32x4 b, nvx_f32x16 c, __bf16) {
+    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ nvx_f32x16 mfma32(nvx_u32x4 a, nvx_u32x4 b, nvx_f32x16 c, _Float16) {
+    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+}
+
+// 64 lanes x 16 bytes from the lanes' addresses to 1 KB of LDS from a wave-uniform address on.  From inline assembly: the compiler would hold
+// every LDS read back until the copy has landed (it cannot tell the two buffers apart), so the wait ahead of the barrier is explicit too.
+__device__ __forceinline__ void copy_to_lds(const void* g, unsigned lds) {
+    const unsigned uni = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(uni) : "memory");
+}
+__device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
+
+// x: the pairs' inputs, row src[r] / src_div (src null: row r), scale[src[r]] (or null) a factor of the sums; w: (experts, rows of UP ? 2 * n_out :
+// n_out, k) row-major; out: (pairs, n_out), of type A (UP) or float32.  k is a multiple of 64, n_out of 64 (UP) or 128; n_exp <= 64.
+template <typename A, bool UP>
+__global__ __launch_bounds__(256, 2) void moe_group_gemm_kernel(const A* __restrict__ x, int64_t x_stride, const int32_t* __restrict__ src, int src_div,
+                                                               const float* __restrict__ scale, const int32_t* __restrict__ counts, int n_exp,
+                                                               const A* __restrict__ w, int k_in, int n_out, float limit, float alpha, float shift,
+                                                               void* __restrict__ out) {
+    __shared__ __align__(16) unsigned char smem[2 * 2 * GT * GK * 2];      // two buffers of [pairs | weight rows]
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int tiles_n = n_out / (UP ? GT / 2 : GT);
+    // which tile: every lane an expert
+    const int cnt = lane < n_exp ? counts[lane] : 0;
+    int rows_to = cnt, tiles_to = (cnt + GT - 1) / GT;                     // (running sums, this expert's included)
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+        const int a = __shfl_up(rows_to, s, 64), b = __shfl_up(tiles_to, s, 64);
+        if (lane >= s) { rows_to += a; tiles_to += b; }
+    }
+    const int total = __shfl(tiles_to, 63, 64) * tiles_n, per = (total + 7) / 8;
+    const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || t >= total) return;
+    const int e = __popcll(__ballot(tiles_to * tiles_n <= t));
+    const int before = e ? __shfl(tiles_to, e - 1, 64) : 0, row0 = e ? __shfl(rows_to, e - 1, 64) : 0, n_rows = __shfl(cnt, e, 64);
+    const int m_tiles = (n_rows + GT - 1) / GT, tl = t - before * tiles_n;
+    const int group = tl / (G_ROWS * tiles_n), gm = min(G_ROWS, m_tiles - group * G_ROWS), in = tl - group * G_ROWS * tiles_n;
+    const int m0 = (group * G_ROWS + in % gm) * GT, tn = in / gm, n0 = tn * (UP ? GT / 2 : GT);
+    const A* we = w + (int64_t)e * (UP ? 2 : 1) * n_out * k_in;
+
+    // this lane's sources: rows 8 * (4 * wave + i) + lane / 8 of either operand; the piece that belongs at place lane % 8
+    const int piece = (lane & 7) ^ (lane >> 3);
+    const A* pa[4];
+    const A* pb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = (4 * wave + i) * 8 + (lane >> 3);
+        const int m = row0 + min(m0 + r, n_rows - 1);                      // (rows past the expert's last repeat it and are not stored)
+        pa[i] = x + (int64_t)(src ? src[m] / src_div : m) * x_stride + piece * 8;
+        // up: weight rows in the order [32 gate | 32 up] for the first and for the second 32 outputs
+        const int wr = UP ? ((r >> 5) & 1) * n_out + n0 + (r >> 6) * 32 + (r & 31) : n0 + r;
+        pb[i] = we + (int64_t)wr * k_in + piece * 8;
+    }
+    const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)smem;
+    auto ask = [&](int step) {
+        const unsigned buf = lds0 + (step & 1) * (2 * GT * GK * 2) + wave * 4096;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            copy_to_lds(pa[i] + step * GK, buf + i * 1024);
+            copy_to_lds(pb[i] + step * GK, buf + GT * GK * 2 + i * 1024);
+        }
+    };
+    const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, hi = lane >> 5;
+    nvx_f32x16 acc[2][2];                                                  // [weight rows][pairs]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    typedef __attribute__((address_space(3))) const nvx_u32x4 lds_u4;
+    const int steps = k_in / GK;
+    ask(0);
+    for (int s = 0; s < steps; ++s) {
+        wait_copies();
+        __syncthreads();                                                   // step s is there, and nobody reads the other buffer any more
+        if (s + 1 < steps) ask(s + 1);
+        const unsigned xb = lds0 + (s & 1) * (2 * GT * GK * 2) + (wm * 64 + l32) * 128, wb = lds0 + (s & 1) * (2 * GT * GK * 2) + GT * GK * 2 + (wn * 64 + l32) * 128;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const unsigned off = (unsigned)((2 * kk + hi) ^ (lane & 7)) * 16;
+            nvx_u32x4 fx[2], fw[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                fx[i] = *reinterpret_cast<lds_u4*>((uintptr_t)(xb + i * 4096 + off));
+                fw[i] = *reinterpret_cast<lds_u4*>((uintptr_t)(wb + i * 4096 + off));
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(fw[i], fx[j], acc[i][j], A{});
+        }
+    }
+    // a lane has pair wm * 64 + 32 j + l32 and of every block of 32 weight rows those 8 q + 4 hi + 0..3: four neighbouring outputs at a time
+    if constexpr (UP) {
+        constexpr int NC = GT / 2, LO = NC + 8;                            // outputs of the tile; elements of a row of it in LDS
+        typedef A vec4 __attribute__((ext_vector_type(4)));
+        A* so = reinterpret_cast<A*>(smem);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int m = m0 + wm * 64 + 32 * j + l32;
+            const float f = scale ? scale[src[row0 + min(m, n_rows - 1)]] : 1.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                vec4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float g = fminf(f * acc[0][j][4 * q + r], limit), u = fminf(fmaxf(f * acc[1][j][4 * q + r], -limit), limit);
+                    v[r] = (A)(g * sigmoid_f(alpha * g) * (u + shift));
+                }
+                *reinterpret_cast<vec4*>(so + (wm * 64 + 32 * j + l32) * LO + wn * 32 + 8 * q + 4 * hi) = v;
+            }
+        }
+        __syncthreads();
+        for (int p = threadIdx.x; p < GT * NC / 8; p += 256) {
+            const int r = p / (NC / 8), c = p % (NC / 8) * 8;
+            if (m0 + r < n_rows)
+                *reinterpret_cast<nvx_u32x4*>((A*)out + (int64_t)(row0 + m0 + r) * n_out + n0 + c) = *reinterpret_cast<const nvx_u32x4*>(so + r * LO + c);
+        }
+    } else {
+        constexpr int LO = GT + 4;
+        float* so = reinterpret_cast<float*>(smem);                        // (64 pairs at a time)
+        for (int h = 0; h < 2; ++h) {
+            __syncthreads();
+            if (wm == h) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const nvx_f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                            *reinterpret_cast<nvx_f32x4*>(so + (32 * j + l32) * LO + wn * 64 + 32 * i + 8 * q + 4 * hi) = v;
+                        }
+            }
+            __syncthreads();
+            for (int p = threadIdx.x; p < 64 * GT / 4; p += 256) {
+                const int r = p / (GT / 4), c = p % (GT / 4) * 4, m = m0 + 64 * h + r;
+                if (m < n_rows) *reinterpret_cast<nvx_f32x4*>((float*)out + (int64_t)(row0 + m) * n_out + n0 + c) = *reinterpret_cast<const nvx_f32x4*>(so + r * LO + c);
+            }
+        }
+    }
+}
+
+// out[t] = sum_k wts[t * top + k] * o[dst[t * top + k]]   (wts == null: ones), four columns a thread
+template <typename A>
+__global__ __launch_bounds__(256) void moe_pair_gather_kernel(const float* __restrict__ o, const int64_t* __restrict__ dst, const float* __restrict__ wts,
+                                                             int top, A* __restrict__ out, int64_t n, int width4) {
+    typedef A vec4 __attribute__((ext_vector_type(4)));
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int64_t t = i / width4;
+    const int c = (int)(i % width4) * 4;
+    nvx_f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < top; ++k) {
+        const float f = wts ? wts[t * top + k] : 1.0f;
+        const nvx_f32x4 v = *reinterpret_cast<const nvx_f32x4*>(o + dst[t * top + k] * (int64_t)width4 * 4 + c);
+        for (int r = 0; r < 4; ++r) sum[r] += f * v[r];
+    }
+    *reinterpret_cast<vec4*>(out + t * (int64_t)width4 * 4 + c) = vec4{(A)sum[0], (A)sum[1], (A)sum[2], (A)sum[3]};
+}
+
+}  // namespace NVX_NS
+
+using namespace NVX_NS;
+
+bool nvx_moe_grouped_fits(int fmt, int64_t n_exp, int64_t width, int64_t ff) {
+    return fmt < 2 && n_exp <= 63 && width % GT == 0 && ff % 64 == 0;
+}
+
+// The whole mixture (see nvx_moe_expert_rows) for a step of many tokens; ws as there.  The pairs' order is made here too.
+int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
+                    int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
+                    hipStream_t st) {
+    const int64_t pairs = n_tok * top;
+    // ws: n_tok * top * (width + ff) floats = the pairs' results (float32), their hidden rows (16 bits), then the order: its counts, source and
+    // place of every pair (12 bytes a pair and 256: they fit in the half of the hidden rows that 16 bits leave, 2 * ff >= 128 bytes a pair)
+    float* o = ws;
+    char* y = reinterpret_cast<char*>(ws + pairs * width);
+    int64_t* dst = reinterpret_cast<int64_t*>(y + pairs * ff * 2);
+    int32_t* src = reinterpret_cast<int32_t*>(dst + pairs);
+    int32_t* counts = src + pairs;
+    if (const int rc = nvx_moe_order_pairs(idx, pairs, n_exp, dst, src, counts, st)) return rc;
+    // as many workgroups as the counts can ask for: an expert's last tile may hold one pair
+    const int64_t m_tiles = pairs / GT + (n_exp < pairs ? n_exp : pairs);
+    const int64_t up = (m_tiles * (ff / (GT / 2)) + 7) / 8 * 8, down = (m_tiles * (width / GT) + 7) / 8 * 8;
+    NVX_REQUIRE(up < (1ll << 31) && down < (1ll << 31), NVX_EINVAL, "nvx_moe_expert_rows: too many tiles");
+#define NVX_GROUPED(A_)                                                                                                                            \
+    do {                                                                                                                                           \
+        hipLaunchKernelGGL((moe_group_gemm_kernel<A_, true>), dim3((unsigned)up), dim3(256), 0, st, (const A_*)h, h_stride, (const int32_t*)src,   \
+                           (int)top, weight_out ? (const float*)nullptr : wts, (const int32_t*)counts, (int)n_exp, (const A_*)w_gu, (int)width,    \
+                           (int)ff, limit, alpha, shift, (void*)y);                                                                                \
+        hipLaunchKernelGGL((moe_group_gemm_kernel<A_, false>), dim3((unsigned)down), dim3(256), 0, st, (const A_*)y, ff, (const int32_t*)nullptr,  \
+                           1, (const float*)nullptr, (const int32_t*)counts, (int)n_exp, (const A_*)w_d, (int)ff, (int)width, limit, alpha, shift,  \
+                           (void*)o);                                                                                                              \
+        hipLaunchKernelGGL(moe_pair_gather_kernel<A_>, dim3((unsigned)((n_tok * (width / 4) + 255) / 256)), dim3(256), 0, st, (const float*)o,     \
+                           (const int64_t*)dst, weight_out ? wts : (const float*)nullptr, (int)top, (A_*)out, n_tok * (width / 4), (int)(width / 4)); \
+    } while (0)
+    if (fmt == 0) NVX_GROUPED(__bf16);
+    else NVX_GROUPED(_Float16);
+#undef NVX_GROUPED
+    return nvx_check_launch("nvx_moe_expert_rows");
+}

@@ -43,8 +43,9 @@ class ExpertBank(nn.Module):
     which scale the experts' inputs, or their outputs if `weight_out`.
 
     Steps of few tokens (decode steps, which a hipGraph replays: no host decision may depend on the choices) evaluate each
-    token's experts in one launch, streaming the chosen experts' rows.  Steps of many tokens put the inputs into expert order
-    (ops.moe_order: a counting sort, which also gives the per-expert counts) and run one pair of matrix products per expert
+    token's experts in one launch, streaming the chosen experts' rows.  Steps of many tokens in 16-bit formats are grouped products over
+    the pairs in expert order behind the same call (ops.moe_expert_rows): the experts' counts stay on the device.  Where the sizes do
+    not fit those (GROUPED_WIDTH, GROUPED_FF, float32), steps of many tokens put the inputs into expert order (ops.moe_order: a counting sort, which also gives the per-expert counts) and run one pair of matrix products per expert
     that received tokens; the counts are the one host read of that path.  An expert's product runs over its row count rounded up
     to a multiple of ROW_STEP: the rows past its own are the next experts', whose products come later on the same stream and
     write them anew (the buffers end in ROW_STEP spare rows), so every row ends as its own expert's.  The library then sees a
@@ -52,6 +53,8 @@ class ExpertBank(nn.Module):
 
     ROWS_PATH_TOKENS = 32           # ... 64 in 16-bit formats, where an expert's rows serve up to 16 pairs at a time
     ROW_STEP = 64
+    GROUPED_WIDTH, GROUPED_FF = 128, 64      # the grouped products' tiles divide the width and the hidden size
+    MAX_ROWS_TOKENS = 65535                  # of a step through ops.moe_expert_rows
 
     def __init__(self, width: int, experts: int, top: int, ff: int, limit: float, alpha: float, shift: float):
         super().__init__()
@@ -81,13 +84,15 @@ class ExpertBank(nn.Module):
         return dst, read
 
     def by_rows(self, t: int, decode_step: bool) -> bool:
-        """Whether a step of t tokens streams the chosen experts' rows (else: per-expert products over the expert order)."""
+        """Whether a step of t tokens is one call of ops.moe_expert_rows (else: per-expert products over the expert order)."""
         if self._rows_fit is None:
             self._rows_fit = ops.moe_expert_rows_fits(self.width, self.ff)
             self._order_fit = ops.moe_order_fits(self.experts)      # more experts than the ordering kernel holds: pair by pair
             if not (self._rows_fit or self._order_fit):
                 raise NotImplementedError(f"{self.experts} experts of {self.ff} x {self.width}: neither expert path is built for these sizes")
-        return self._rows_fit and (decode_step or t <= (1 if self.w_gu.dtype == torch.float32 else 2) * self.ROWS_PATH_TOKENS or not self._order_fit)
+        grouped = self._order_fit and self.w_gu.dtype != torch.float32 and self.width % self.GROUPED_WIDTH == 0 and self.ff % self.GROUPED_FF == 0 \
+            and t <= self.MAX_ROWS_TOKENS
+        return self._rows_fit and (decode_step or grouped or t <= (1 if self.w_gu.dtype == torch.float32 else 2) * self.ROWS_PATH_TOKENS or not self._order_fit)
 
     def run(self, h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, decode_step: bool, weight_out: bool, order=None) -> torch.Tensor:
         """`order` = (dst, counts as a list, or a function that gives them): the expert order of idx where the caller has it already
