@@ -12,7 +12,7 @@
 //     that are cached as projected and normed as they are scored (tied keys and values: one row per token serves as both), a sink (one more term in the softmax's sum, with a score of its
 //     own -- one number, or one per head -- and no value), the first tokens of a sequence kept visible behind the window, the read-out turned back by the query's position (the counterpart of rotated values) and multiplied by
 //     a sigmoid gate (one per element, or one per head).
-#include "fmt_dev.h"
+#include "cap_attn_dev.h"
 
 namespace NVX_NS {
 
@@ -341,11 +341,6 @@ __global__ __launch_bounds__(256) void tied_prep_store_vec_kernel(const A* __res
 }
 
 // What limits the keys a token at `pos` sees from below: a window of `window` keys, chunks of `chunk` positions counted from 0 (neither: 0)
-__device__ __forceinline__ int first_seen(int pos, int window, int chunk) {
-    if (window > 0) return pos - window + 1 > 0 ? pos - window + 1 : 0;
-    return chunk > 0 ? pos - pos % chunk : 0;
-}
-
 // The end of an attention read-out for one (token, head): `so` holds its vdim values in LDS (every thread of the workgroup has
 // passed a barrier since they were written).  With `turn` (the query token's cos | sin row, vdim / 2 each, as nvx_attn_prep_store
 // hands it out) the pairs are turned BACK by those angles (values were cached turned by their own positions, so the weighted sum
@@ -688,13 +683,6 @@ template <typename A> __device__ __forceinline__ nvx_f32x4 ca_mfma32(nvx_u32x4 a
     else
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ca_f16x8, a), __builtin_bit_cast(ca_f16x8, b), c, 0, 0, 0);
 }
-template <typename A> __device__ __forceinline__ uint32_t ca_pack2(float lo, float hi) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    typedef A a2 __attribute__((ext_vector_type(2)));
-    const f2 v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, a2));
-}
-
 constexpr int TILE_Q = 64;       // query tokens per workgroup
 constexpr int TILE_K = 32;       // keys per step
 constexpr int VT_ROW = 40;       // elements per row of the V^T tile in LDS: 32 keys and a pad that spreads the rows over the banks
@@ -878,9 +866,9 @@ __global__ __launch_bounds__(256) void softcap_attn_tile_kernel(const A* __restr
             l_run += p[e];
             ph[e] = (float)(A)p[e];
         }
-        const nvx_u32x4 p_hi = {ca_pack2<A>(ph[0], ph[1]), ca_pack2<A>(ph[2], ph[3]), ca_pack2<A>(ph[4], ph[5]), ca_pack2<A>(ph[6], ph[7])};
-        const nvx_u32x4 p_lo = {ca_pack2<A>(p[0] - ph[0], p[1] - ph[1]), ca_pack2<A>(p[2] - ph[2], p[3] - ph[3]),
-                                ca_pack2<A>(p[4] - ph[4], p[5] - ph[5]), ca_pack2<A>(p[6] - ph[6], p[7] - ph[7])};
+        const nvx_u32x4 p_hi = {cap_pack2<A>(ph[0], ph[1]), cap_pack2<A>(ph[2], ph[3]), cap_pack2<A>(ph[4], ph[5]), cap_pack2<A>(ph[6], ph[7])};
+        const nvx_u32x4 p_lo = {cap_pack2<A>(p[0] - ph[0], p[1] - ph[1]), cap_pack2<A>(p[2] - ph[2], p[3] - ph[3]),
+                                cap_pack2<A>(p[4] - ph[4], p[5] - ph[5]), cap_pack2<A>(p[6] - ph[6], p[7] - ph[7])};
         if (__any(alpha != 1.0f)) {
 #pragma unroll
             for (int t = 0; t < VT; ++t) acc[t] *= alpha;
@@ -949,7 +937,7 @@ __global__ __launch_bounds__(256) void softcap_attn_tile_kernel(const A* __restr
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[r] *= sigmoid_f((float)gv[r]);
         }
-        *reinterpret_cast<uint2*>(orow + t * 16) = make_uint2(ca_pack2<A>(o[0], o[1]), ca_pack2<A>(o[2], o[3]));
+        *reinterpret_cast<uint2*>(orow + t * 16) = make_uint2(cap_pack2<A>(o[0], o[1]), cap_pack2<A>(o[2], o[3]));
     }
 }
 
@@ -1123,7 +1111,20 @@ extern "C" int nvx_softcap_attn(const void* q, const void* k_cache, const void* 
     sink = sink || sinks;
     NVX_REQUIRE(!vcs || (vdim % 2 == 0 && nvx_aligned16(vcs)), NVX_EINVAL, "nvx_softcap_attn: a read-out that is turned back has an even size");
     NVX_REQUIRE(!gate || gate_stride >= (gate_per_head ? heads : heads * vdim), NVX_EINVAL, "nvx_softcap_attn: row stride of the gate");
-    // steps of many tokens in a 16-bit format, sizes the tile kernel is built for, 8-byte rows of the gate: the matrix cores
+    // Steps of many tokens in a 16-bit format go to the matrix cores.  Heads of 128 whose operands stand on 16-byte borders: the kernel that
+    // shares a tile of keys and values between four waves (16 / 8 heads, 1 024 tokens a sequence: about half the time of the other at every
+    // length); the other sizes the tile kernel is built for, or 8-byte rows of the output and the gate: that one.
+    if (matrix_cores && fmt < 2 && dim == 128 && vdim == 128 && qo_indptr && n_split == 1 && n_seq > 0 && (!k_rn || k_cache == v_cache) && nvx_aligned16(q) &&
+        nvx_aligned16(k_cache) && nvx_aligned16(v_cache) && nvx_aligned16(out) && out_stride % 8 == 0 &&
+        (!gate || gate_per_head || (nvx_aligned16(gate) && gate_stride % 8 == 0))) {
+        CapAttnArgs a = {};
+        a.q = q; a.k_cache = k_cache; a.v_cache = v_cache; a.kv_indices = kv_indices; a.kv_start = kv_start; a.kv_len = kv_len; a.qo_indptr = qo_indptr;
+        a.n_seq = (int)n_seq; a.heads = (int)heads; a.kv_heads = (int)kv_heads; a.window = (int)window; a.chunk = (int)chunk; a.keep = (int)keep_first;
+        a.v_inter = v_interleaved; a.gate_one = gate_per_head; a.sink = sink; a.scale = scale; a.cap = cap; a.sink_score = sink_score; a.out_mul = out_mul;
+        a.r1 = r1; a.r2 = r2; a.slopes = slopes; a.k_rn = k_rn; a.vcs = vcs; a.sinks = sinks; a.gate = gate; a.gate_stride = gate_stride;
+        a.out_stride = out_stride; a.out = out;
+        return nvx_softcap_attn_rows32(a, fmt, n_tok, (hipStream_t)stream);
+    }
     if (matrix_cores && nvx_softcap_attn_tile_fits(fmt, dim, vdim, vcs != nullptr && !v_interleaved) && qo_indptr && n_split == 1 && n_seq > 0 &&
         nvx_aligned16(q) && nvx_aligned16(k_cache) && nvx_aligned16(v_cache) && (reinterpret_cast<uintptr_t>(out) & 7u) == 0 && out_stride % 4 == 0 &&
         (!gate || gate_per_head || ((reinterpret_cast<uintptr_t>(gate) & 7u) == 0 && gate_stride % 4 == 0))) {
