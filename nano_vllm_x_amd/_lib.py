@@ -173,6 +173,17 @@ for _name in F16_ENTRY_POINTS:
     SIGNATURES[_name + "_f16"] = SIGNATURES[_name]
 
 
+class PrefillStep(ctypes.Structure):
+    """NvxPrefillStep of csrc/prefill_step.hip, field by field."""
+    _fields_ = [("layers", _c_vp)] + [(n, _c_i64) for n in ("n_layers", "n_tok", "batch", "hidden", "hq", "hkv", "inter", "rope_rows", "n_slots")] \
+        + [(n, _c_vp) for n in ("x", "final_norm", "positions", "slots", "rope", "qo_indptr", "kv_indptr", "kv_indices", "plan", "h", "sum", "res0", "res1", "qkv",
+                                "q", "attn", "act", "out")] + [("eps", ctypes.c_double), ("scale", ctypes.c_double)]
+
+
+# What the host of this package calls beside the C ABI (sequences of its entry points queued natively); not declared in include/nvx.h
+INTERNAL = {name: (_c_i32, [ctypes.POINTER(PrefillStep), _c_vp]) for name in ("nvx_internal_prefill_step", "nvx_internal_prefill_step_f16")}
+
+
 class _SubsetLibrary:
     """The subset library behind the same attribute access: an entry point it was not built with raises by name."""
 
@@ -213,6 +224,9 @@ def load():
             raise NvxLibraryError(f"{LIB_PATH} does not export {name}") from e
         fn.restype = res
         fn.argtypes = args
+    for name, (res, args) in INTERNAL.items() if not subset else ():
+        fn = getattr(lib, name)
+        fn.restype, fn.argtypes = res, args
     if subset:
         lib = _SubsetLibrary(lib, path)
     want, got = header_abi_version(), lib.nvx_abi_version()

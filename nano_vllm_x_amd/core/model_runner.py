@@ -32,6 +32,7 @@ from ..registry import load_config, model_class_of
 from .common import ForwardBatch, ForwardMode
 from .hip_graph import HIPGraph, decode_batch_ladder
 from .kv_cache import KVCachePool
+from .upload import upload
 
 # Largest step whose LM head + draw go through ops.lmhead_sample: it holds 64 rows per compute unit, takes 65..128 rows as two
 # row groups on paired workgroups in one launch (a tile fetched from HBM by one is found in L2 by the other), and more rows as
@@ -132,6 +133,7 @@ class ModelRunner:
             else:
                 self.model.init_random(self.seed)
         self.model.pack_decode_weights()
+        self.model.attention_modules = [m for m in self.model.modules() if hasattr(m, "set_attention_metadata")]
         self.sampler = Sampler(seed=self.seed)
         # Decode-sized steps whose rows have no sampling filter take the LM head and the draw in ONE pass over the weight
         # (ops.lmhead_sample): the tiled copy of this rank's LM-head rows it streams is made here, once.  NVX_LMHEAD_FUSED=0
@@ -217,8 +219,7 @@ class ModelRunner:
     def prepare_input(self, batch: ForwardBatch):
         ids = [t for s in batch.seqs for t in s.token_ids[s.cached_kv_len:]]
         pos = np.concatenate([np.arange(s.cached_kv_len, len(s.token_ids), dtype=np.int64) for s in batch.seqs])
-        ids_t = torch.from_numpy(np.asarray(ids, dtype=np.int64)).to(self.device, non_blocking=True)
-        return ids_t, torch.from_numpy(pos).to(self.device, non_blocking=True)
+        return tuple(upload((np.asarray(ids, dtype=np.int64), pos), self.device))
 
     def prepare_sampling_params(self, batch: ForwardBatch):
         """One (4, B) fp32 upload: temperature, min_p, top_p, top_k (-1 -> vocabulary size,
@@ -239,18 +240,18 @@ class ModelRunner:
         # no row with a filter (greedy rows, temperature <= 0, ignore theirs): tensor-parallel ranks can then draw from
         # their own shards of the vocabulary and exchange 8 bytes per row instead of the logits
         self._sp_unfiltered = bool(np.all((host[0] <= 0) | ((host[3] >= v) & (host[2] >= 1.0) & (host[1] <= 0.0))))
-        dev = torch.from_numpy(host).to(self.device, non_blocking=True)
+        dev, = upload((host,), self.device)
         self._sp_key, self._sp_dev = key, (dev[0], dev[1], dev[2], dev[3].to(torch.int64))
         return self._sp_dev
 
     @staticmethod
     def prepare_last_hidden_states(batch: ForwardBatch, hidden_states: torch.Tensor) -> torch.Tensor:
         if batch.want_rows is not None:     # the caller names the rows (any tokens of the step, in any number)
-            return hidden_states[torch.tensor(batch.want_rows, dtype=torch.int64).to(hidden_states.device)]
+            return hidden_states[upload((np.asarray(batch.want_rows, dtype=np.int64),), hidden_states.device)[0]]
         last = np.cumsum([len(s.token_ids) - s.cached_kv_len for s in batch.seqs]) - 1
         if len(last) == hidden_states.shape[0]:
             return hidden_states   # decode: every row is a last row
-        return hidden_states[torch.from_numpy(last).to(hidden_states.device)]
+        return hidden_states[upload((last,), hidden_states.device)[0]]
 
     # -- execution -----------------------------------------------------------------------------------
     @torch.inference_mode()

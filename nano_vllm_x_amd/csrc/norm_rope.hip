@@ -436,7 +436,6 @@ extern "C" int NVX_ENTRY(nvx_qknorm_rope_store)(const void* qkv, int64_t qkv_row
 // ---------------------------------------------------------------------------------------------
 // SiluAndMul
 // ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ float silu_h16(float x) { return round_h16(x / (1.0f + __expf(-x))); }
 
 // IDX: the type the element index is counted in.  A 64-bit division per element costs about a hundred instructions;
 // every decode batch and most prefill batches fit 32 bits.

@@ -72,6 +72,7 @@ __device__ __forceinline__ uint32_t pack_h16x2(float lo, float hi) {
 }
 // value of f after a round trip through the 16-bit format (what eager arithmetic in that format keeps of every result)
 __device__ __forceinline__ float round_h16(float f) { return h16bits_to_f32(f32_to_h16bits(f)); }
+__device__ __forceinline__ float silu_h16(float x) { return round_h16(x / (1.0f + __expf(-x))); }
 
 // c + a.x * b.x + a.y * b.y on packed pairs, fp32 accumulate (v_dot2c_f32_bf16 / v_dot2_f32_f16)
 __device__ __forceinline__ float dot2_h16(uint32_t a, uint32_t b, float c) {

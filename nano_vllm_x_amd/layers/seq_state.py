@@ -15,6 +15,7 @@ import torch
 from .. import ops
 from ..core.common import ForwardBatch, ForwardMode
 from ..core.kv_cache import LatentCachePool, RecurrentStatePool
+from ..core.upload import upload
 
 
 class SeqStateCache:
@@ -49,9 +50,6 @@ class SeqStateBackend:
     def __init__(self, cache: SeqStateCache, device: torch.device):
         self.cache, self.device = cache, device
 
-    def _up(self, a: np.ndarray) -> torch.Tensor:
-        return torch.from_numpy(a).to(self.device, non_blocking=True)
-
     def build_metadata(self, batch: ForwardBatch) -> SeqStateMetadata:
         seqs = batch.seqs
         n = len(seqs)
@@ -69,15 +67,15 @@ class SeqStateBackend:
         flat = np.concatenate([np.asarray(s.kv_indices[:len(s.token_ids)], dtype=np.int32) for s in seqs])
         out_slots = np.concatenate([np.asarray(s.kv_indices[s.cached_kv_len:len(s.token_ids)], dtype=np.int64) for s in seqs])
         t = int(q_lens.sum())
-        if batch.forward_mode == ForwardMode.DECODE and t == n:
-            layout = ops.StepLayout(t, n, self._up(pos0), self._up(slot))
-        else:
-            qo = np.zeros(n + 1, dtype=np.int32)
-            np.cumsum(q_lens, out=qo[1:])
-            tok_seq = np.repeat(np.arange(n, dtype=np.int32), q_lens)
-            layout = ops.StepLayout(t, n, self._up(pos0), self._up(slot), self._up(qo), self._up(tok_seq), max_q=int(q_lens.max()))
         kv_indptr = np.zeros(n + 1, dtype=np.int32)
         np.cumsum(kv_lens, out=kv_indptr[1:])
-        return SeqStateMetadata(forward_mode=batch.forward_mode, cache=self.cache, layout=layout, kv_indices=self._up(flat),
-                                kv_start=self._up(kv_start), kv_len=self._up(kv_lens), out_slots=self._up(out_slots),
-                                kv_indptr=self._up(kv_indptr))
+        arrays = [pos0, slot, flat, kv_start, kv_lens, out_slots, kv_indptr]
+        per_token = batch.forward_mode != ForwardMode.DECODE or t != n
+        if per_token:
+            qo = np.zeros(n + 1, dtype=np.int32)
+            np.cumsum(q_lens, out=qo[1:])
+            arrays += [qo, np.repeat(np.arange(n, dtype=np.int32), q_lens)]
+        pos0, slot, flat, kv_start, kv_lens, out_slots, kv_indptr, *ragged = upload(arrays, self.device)
+        layout = ops.StepLayout(t, n, pos0, slot, *ragged, max_q=int(q_lens.max())) if per_token else ops.StepLayout(t, n, pos0, slot)
+        return SeqStateMetadata(forward_mode=batch.forward_mode, cache=self.cache, layout=layout, kv_indices=flat, kv_start=kv_start,
+                                kv_len=kv_lens, out_slots=out_slots, kv_indptr=kv_indptr)

@@ -8,6 +8,7 @@ capturable into a hipGraph.  `nano_vllm_x_amd.torch_ops` registers the stateless
 """
 from __future__ import annotations
 
+import ctypes as _ctypes
 from typing import Optional
 
 import torch
@@ -25,7 +26,8 @@ def _fn(lib, name: str, dtype):
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle alone: building a torch.cuda.Stream around it costs 3 us a launch
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need(cond: bool, msg: str):
@@ -132,6 +134,48 @@ def qknorm_rope_store(qkv, positions, cos_sin_cache, q_norm_weight, k_norm_weigh
                                          _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], t, n_q_heads, n_kv_heads, _stream()),
                "nvx_qknorm_rope_store")
     return q_out
+
+
+def prefill_step(layers, x, positions, cos_sin_cache, slots, qo_indptr, kv_indptr, kv_indices, plan_ws, final_norm, n_q_heads, n_kv_heads, eps, sm_scale):
+    """All layers of a Qwen3 prefill step of few tokens and the final norm, queued by one native call.
+    `layers`: per layer (input norm, qkv, q norm, k norm, o, post-attention norm, gate | up, down, k rows, v rows); x (T, hidden) the embedding
+    rows.  The sizes must be ones that prefill_step_fits accepts.  Returns the final-normed hidden states (T, hidden)."""
+    t, hidden = x.shape
+    inter, b = layers[0][7].shape[1], qo_indptr.numel() - 1
+    flat = [w for layer in layers for w in layer]
+    _dev(x, positions, cos_sin_cache, slots, qo_indptr, kv_indptr, kv_indices, plan_ws, final_norm, *flat)
+    dt, qw, aw = x.dtype, (n_q_heads + 2 * n_kv_heads) * 128, n_q_heads * 128
+    shapes = ((hidden,), (qw, hidden), (128,), (128,), (hidden, aw), (hidden,), (2 * inter, hidden), (hidden, inter))
+    n_slots = layers[0][8].shape[0]
+    for layer in layers:
+        for w, s in zip(layer, shapes):
+            _need(w.shape == s and w.dtype == dt and w.is_contiguous(), "prefill_step: weights")
+        for c in layer[8:]:
+            _need(c.shape == (n_slots, n_kv_heads, 128) and c.dtype == dt and c.is_contiguous(), "prefill_step: cache layout")
+    _need(dt in H16 and x.is_contiguous() and final_norm.shape == (hidden,) and final_norm.dtype == dt, "prefill_step: rows")
+    _need(positions.dtype == torch.int64 and positions.is_contiguous() and positions.numel() == t and slots.dtype == torch.int64 and slots.is_contiguous() and
+          slots.numel() == t, "prefill_step: positions and slots must be int64 (T)")
+    _need(cos_sin_cache.dtype == torch.float32 and cos_sin_cache.shape[-1] == 128 and cos_sin_cache.is_contiguous(), "prefill_step: table")
+    for a in (qo_indptr, kv_indptr, kv_indices, plan_ws):
+        _need(a.dtype == torch.int32 and a.is_contiguous(), "prefill_step: the block table must be contiguous int32")
+    _need(kv_indptr.numel() == b + 1, "prefill_step: indptr lengths differ")
+    out = torch.empty((t, hidden), dtype=dt, device=x.device)
+    ws = torch.empty((t * (4 * hidden + qw + 2 * aw + inter),), dtype=dt, device=x.device)
+    size, at, p = ws.element_size(), [], ws.data_ptr()
+    for n in (hidden, hidden, hidden, hidden, qw, aw, aw, inter):
+        at.append(p)
+        p += t * n * size
+    table = (_ctypes.c_int64 * len(flat))(*[w.data_ptr() for w in flat])
+    step = _lib.PrefillStep(_ctypes.addressof(table), len(layers), t, b, hidden, n_q_heads, n_kv_heads, inter, cos_sin_cache.shape[0], n_slots, _ptr(x),
+                            _ptr(final_norm), _ptr(positions), _ptr(slots), _ptr(cos_sin_cache), _ptr(qo_indptr), _ptr(kv_indptr), _ptr(kv_indices),
+                            _ptr(plan_ws), *at, _ptr(out), float(eps), float(sm_scale))
+    _lib.check(_fn(_lib.load(), "nvx_internal_prefill_step", dt)(step, _stream()), "prefill_step")
+    return out
+
+
+def prefill_step_fits(hidden: int, n_q_heads: int, n_kv_heads: int, inter: int) -> bool:
+    """Whether a model's projections are all ones that csrc/prefill_gemm.hip takes: rows of W in 128s, columns in 256s."""
+    return hidden % 256 == 0 and inter % 256 == 0 and n_q_heads % 2 == 0 and n_q_heads % n_kv_heads == 0 and n_q_heads // n_kv_heads in (1, 2, 4, 8)
 
 
 def linear_decode_splits(n: int, k: int) -> int:

@@ -23,7 +23,7 @@ from . import distributed as tpd
 from . import ops
 from .layers.activation import SiluAndMul
 from .core.common import ForwardMode
-from .layers.attention import Attention
+from .layers.attention import Attention, PagedPrefillWrapper
 from .layers.layernorm import RMSNorm
 from .layers.rotary_embedding import RotaryEmbedding, build_cos_sin_cache
 
@@ -92,6 +92,11 @@ DECODE_LINEAR_MAX_ROWS = {"qkv": 256, "o": 256, "gate_up": 256, "down": 256}
 # which the library GEMM sustains better (Qwen3-8B o_proj, 33 MB: 28 us here vs ~12 us of streaming).
 DECODE_LINEAR_MAX_WEIGHT_BYTES = 16 << 20
 
+
+# Multiply-adds of a layer's projections up to which a prefill step is queued by one native call with the products of csrc/prefill_gemm.hip
+# (ops.prefill_step): 1526 tokens of Qwen3-0.6B (a step of 1536 takes 4250 us that way and 4600 from Python, one of 2048 5190 and 4870), 477 of Qwen3-1.7B,
+# 125 of Qwen3-8B (a layer's products at 64 rows: 115 us and the library's 120, at 216 rows 184 and 169).
+PREFILL_STEP_MAX_WORK = int(24e9)
 
 # NVX_FP32_LINEAR=1 (read when a model is built): every dense projection, the LM head included, multiplies in fp32 and
 # rounds its result to the model's 16-bit format once (the LM head's logits stay fp32).  Not a serving mode: it takes
@@ -337,11 +342,74 @@ class Qwen3Model(nn.Module):
         return self.layers[self.start_layer:self.end_layer]
 
     def forward(self, input_ids, positions, fused: bool = True):
+        if fused and self._plain_prefill():
+            return self._prefill(input_ids, positions)
         hidden_states, residual = self.embed_tokens(input_ids), None
         for layer in self.layers:
             hidden_states, residual = layer(positions, hidden_states, residual, fused)
         hidden_states, _ = self.norm(hidden_states, residual)
         return hidden_states
+
+    def _plain_prefill(self) -> bool:
+        """Whether this step is a prefill that _prefill may queue: one rank, the package's own attention wrapper, 16-bit projections, and no
+        hook on any module of the stack (a hook wants the modules called)."""
+        if len(self.layers) == 0 or FP32_LINEAR or torch.is_grad_enabled() or tpd.collectives_active() or tpd.pp_size() > 1:
+            return False
+        md = self.layers[0].self_attn.attn.attention_metadata
+        if md is None or md.forward_mode != ForwardMode.PREFILL or type(md.wrapper) is not PagedPrefillWrapper:
+            return False
+        m = torch.nn.modules.module
+        if m._global_forward_hooks or m._global_forward_pre_hooks:
+            return False
+        return not any(x._forward_hooks or x._forward_pre_hooks for x in self.modules_of_a_step())
+
+    def modules_of_a_step(self):
+        yield self.embed_tokens
+        yield self.norm
+        for layer in self.layers:
+            a, mlp = layer.self_attn, layer.mlp
+            yield from (layer, a, mlp, a.qkv_proj, a.o_proj, a.attn, mlp.gate_up_proj, mlp.down_proj, mlp.act_fn, layer.input_layernorm, layer.post_attention_layernorm)
+
+    def _prefill(self, input_ids, positions):
+        """What the module graph computes for a prefill step, queued without calling the modules: a module call costs the host 3-5 us and a
+        layer has eleven.  Steps of few tokens go out in one native call (ops.prefill_step)."""
+        cfg, first = self.config, self.layers[0].self_attn
+        md = first.attn.attention_metadata
+        wrapper, cache, slots = md.wrapper, md.kv_cache, md.output_kv_indices
+        hidden_states, residual, t = self.embed_tokens(input_ids), None, input_ids.shape[0]
+        hq, hkv, eps = first.num_heads, first.num_kv_heads, cfg.rms_norm_eps
+        norm = lambda m: m._parameters["weight"]
+        lin = lambda m, n: m._modules[n]._parameters["weight"]
+        work = t * (cfg.hidden_size * (2 * hq + 2 * hkv) * 128 + 3 * cfg.hidden_size * cfg.intermediate_size)
+        if work <= PREFILL_STEP_MAX_WORK and ops.prefill_step_fits(cfg.hidden_size, hq, hkv, cfg.intermediate_size) \
+                and positions.numel() == t == slots.numel() and positions.is_contiguous():
+            qo_indptr, kv_indptr, kv_indices, n_q, n_kv = wrapper._planned
+            layers = []
+            for layer in self.layers:
+                a, mlp = layer._modules["self_attn"], layer._modules["mlp"]
+                layers.append((lin(layer, "input_layernorm"), lin(a, "qkv_proj"), lin(a, "q_norm"), lin(a, "k_norm"), lin(a, "o_proj"),
+                               lin(layer, "post_attention_layernorm"), lin(mlp, "gate_up_proj"), lin(mlp, "down_proj"), *cache.get_kv_cache(a.attn.layer_id)))
+            # (weights as they are loaded; a caller's own, strided or of another type, take the products below)
+            if all(w.is_contiguous() and w.dtype == hidden_states.dtype for layer in layers + [(norm(self.norm),)] for w in layer):
+                return ops.prefill_step(layers, hidden_states, positions, self.rope_table, slots, qo_indptr, kv_indptr, kv_indices, wrapper._plan_ws, norm(self.norm),
+                                        hq, hkv, eps, first.attn.scaling)
+        q = torch.empty((t, hq * 128), dtype=hidden_states.dtype, device=hidden_states.device)
+        read_out = torch.empty_like(q)
+        for layer in self.layers:
+            a, mlp = layer._modules["self_attn"], layer._modules["mlp"]
+            w = lin(layer, "input_layernorm")
+            if residual is None:
+                h, residual = ops.rmsnorm(hidden_states, w, eps), hidden_states
+            else:
+                h, residual = ops.rmsnorm(hidden_states, w, eps, residual)
+            k_cache, v_cache = cache.get_kv_cache(a.attn.layer_id)
+            ops.qknorm_rope_store(F.linear(h, lin(a, "qkv_proj")), positions, self.rope_table, lin(a, "q_norm"), lin(a, "k_norm"), eps, slots, k_cache, v_cache, hq,
+                                  hkv, q_out=q)
+            wrapper._sm_scale = a.attn.scaling
+            wrapper.run(q, (k_cache, v_cache), out=read_out)
+            h, residual = ops.rmsnorm(F.linear(read_out, lin(a, "o_proj")), lin(layer, "post_attention_layernorm"), eps, residual)
+            hidden_states = F.linear(ops.silu_mul(F.linear(h, lin(mlp, "gate_up_proj"))), lin(mlp, "down_proj"))
+        return ops.rmsnorm(hidden_states, norm(self.norm), eps, residual)[0]
 
     def forward_stage(self, input_ids, positions, hidden_states, residual, fused: bool = True):
         """One pipeline stage.  The first stage embeds `input_ids` (hidden_states/residual are None), the
