@@ -180,8 +180,9 @@ class PrefillStep(ctypes.Structure):
                                 "q", "attn", "act", "out")] + [("eps", ctypes.c_double), ("scale", ctypes.c_double)]
 
 
-# What the host of this package calls beside the C ABI (sequences of its entry points queued natively); not declared in include/nvx.h
+# What the host of this package calls beside the C ABI; not declared in include/nvx.h
 INTERNAL = {name: (_c_i32, [ctypes.POINTER(PrefillStep), _c_vp]) for name in ("nvx_internal_prefill_step", "nvx_internal_prefill_step_f16")}
+INTERNAL["nvx_internal_few_rows"] = (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_vp, _c_i32, _c_i32, _c_i64, _c_i64, _c_i64, _c_vp])
 
 
 class _SubsetLibrary:
@@ -215,7 +216,7 @@ def load():
             f"{LIB_PATH} not found: build it with `make -C nano_vllm_x_amd/csrc` "
             "(or `python -c 'import __graft_entry__ as g; g.build()'`). There is no fallback path.")
     lib = ctypes.CDLL(path)
-    for name, (res, args) in SIGNATURES.items():
+    for name, (res, args) in (*SIGNATURES.items(), *INTERNAL.items()):
         try:
             fn = getattr(lib, name)
         except AttributeError as e:
@@ -224,9 +225,6 @@ def load():
             raise NvxLibraryError(f"{LIB_PATH} does not export {name}") from e
         fn.restype = res
         fn.argtypes = args
-    for name, (res, args) in INTERNAL.items() if not subset else ():
-        fn = getattr(lib, name)
-        fn.restype, fn.argtypes = res, args
     if subset:
         lib = _SubsetLibrary(lib, path)
     want, got = header_abi_version(), lib.nvx_abi_version()

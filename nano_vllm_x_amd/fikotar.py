@@ -24,6 +24,7 @@ from torch import nn
 from . import distributed as tpd
 from . import ops
 from .layers.cap_attention import ConvAttention
+from .layers.linear import Linear
 from .layers.moe import GatedSharedExpert, GroupedSoftmaxMoE
 from .layers.recurrent import Retention
 from .layers.rotary_embedding import TurnTables
@@ -130,8 +131,8 @@ class FikotarLayer(nn.Module):
         for b in blocks:
             self.in_at.append(self.in_at[-1] + b.proj_rows)
             self.out_at.append(self.out_at[-1] + b.out_cols)
-        self.in_proj = nn.Linear(w, self.in_at[-1], bias=False)
-        self.out_proj = nn.Linear(self.out_at[-1], w, bias=False)
+        self.in_proj = Linear(w, self.in_at[-1], bias=False)
+        self.out_proj = Linear(self.out_at[-1], w, bias=False)
         self.norm1, self.norm1_b = _f32(w), _f32(w)
 
     def forward(self, h: torch.Tensor, turns: TurnTables, table, md, decode_step: bool):

@@ -25,12 +25,12 @@ from dataclasses import dataclass, field
 from typing import Iterable
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import distributed as tpd
 from . import ops
 from .layers.cap_attention import NormedAttention
+from .layers.linear import Linear, linear
 from .layers.moe import DenseGLU, TableMoE
 from .layers.recurrent import DecayLinearAttention
 
@@ -150,7 +150,7 @@ class ParallelMixer(nn.Module):
                                     qk_norm="head", rot=a["rot"], rotate_values=a["rot"] is not None, softcap=a["softcap"], window=a["window"],
                                     out_gate=True, bias=True, own_proj=False)
         self.right = DecayLinearAttention(width, r["heads"], r["dim"], r["vdim"], r["decay"], eps, state_name=(i, "mix"), own_proj=False)
-        self.in_proj = nn.Linear(width, self.left.proj_rows + self.right.proj_rows, bias=True)
+        self.in_proj = Linear(width, self.left.proj_rows + self.right.proj_rows, bias=True)
         nn.init.zeros_(self.in_proj.bias)      # it stays zero where the design has no bias (the gates, the right branch)
         self.left_scale, self.right_scale = m["left_scale"], m["right_scale"]
 
@@ -252,7 +252,7 @@ class GibavikForCausalLM(nn.Module):
 
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """float32 logits, through cap * tanh(. / cap) where the model has a cap."""
-        return ops.tanh_cap(F.linear(hidden_states, self.head), self.config.logit_softcap)
+        return ops.tanh_cap(linear(hidden_states, self.head), self.config.logit_softcap)
 
     # -- weights ----------------------------------------------------------------------------------------
     @torch.no_grad()

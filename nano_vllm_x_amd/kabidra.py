@@ -27,6 +27,7 @@ from torch import nn
 from . import distributed as tpd
 from . import ops
 from .layers.latent_attention import LatentAttention
+from .layers.linear import Linear, linear
 from .layers.recurrent import MinGRU
 
 MIXERS = ("mingru", "latent_attention")
@@ -82,8 +83,8 @@ def _f32(*shape):
 class SquaredReLUMLP(nn.Module):
     def __init__(self, width: int, ff: int):
         super().__init__()
-        self.up_proj = nn.Linear(width, ff, bias=False)
-        self.down_proj = nn.Linear(ff, width, bias=False)
+        self.up_proj = Linear(width, ff, bias=False)
+        self.down_proj = Linear(ff, width, bias=False)
 
     def forward(self, h):
         return self.down_proj(ops.relu2(self.up_proj(h)))
@@ -191,7 +192,7 @@ class KabidraForCausalLM(nn.Module):
             x, h = self._boundary(y, post, x, md, dtype, nxt.norm1, nxt.canon1, (i + 1, "canon1"), hist=hist, hist_slot=i + 1, mix=layer.dwa)
 
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_states, self.head)
+        return linear(hidden_states, self.head)
 
     # -- weights ----------------------------------------------------------------------------------------
     @torch.no_grad()

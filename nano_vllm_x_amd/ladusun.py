@@ -26,13 +26,13 @@ from dataclasses import dataclass, field
 from typing import Iterable
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from . import distributed as tpd
 from . import ops
 from .layers.cap_attention import NormedAttention
 from .layers.latent_attention import RotaryLatentAttention
+from .layers.linear import Linear, linear
 from .layers.moe import GroupedSoftmaxMoE
 from .layers.recurrent import RGLRU
 
@@ -149,8 +149,8 @@ class DenseRelu2(nn.Module):
     def __init__(self, width: int, ff: int):
         super().__init__()
         self.ff = ff
-        self.up = nn.Linear(width, ff, bias=True)
-        self.down = nn.Linear(ff, width, bias=True)
+        self.up = Linear(width, ff, bias=True)
+        self.down = Linear(ff, width, bias=True)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         return self.down(ops.relu2(self.up(h)))
@@ -286,7 +286,7 @@ class LadusunForCausalLM(nn.Module):
 
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """float32 logits against the embedding table itself."""
-        return F.linear(hidden_states, self.embed).float()
+        return linear(hidden_states, self.embed).float()
 
     # -- weights ----------------------------------------------------------------------------------------
     @torch.no_grad()

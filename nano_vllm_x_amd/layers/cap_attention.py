@@ -9,6 +9,7 @@ import torch
 from torch import nn
 
 from .. import ops
+from .linear import Linear
 from .rotary_embedding import rotary_frequencies
 
 
@@ -33,8 +34,8 @@ class SoftcapAttention(nn.Module):
             self.register_buffer("freq", freq.to(torch.float64), persistent=False)
         else:
             self.freq, self.mag = None, 1.0
-        self.qkv_proj = nn.Linear(width, heads * dim + kv_heads * (dim + vdim), bias=False)     # rows: q | k | v
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.qkv_proj = Linear(width, heads * dim + kv_heads * (dim + vdim), bias=False)     # rows: q | k | v
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     def cache_rows(self) -> dict:
         return {self.k_name: self.kv_heads * self.dim, self.v_name: self.kv_heads * self.vdim}
@@ -112,10 +113,10 @@ class NormedAttention(nn.Module):
         self.proj_rows = self.q_cols + self.k_cols + self.v_cols + self.g_cols
         self.has_bias = bias
         if own_proj:
-            self.in_proj = nn.Linear(width, self.proj_rows, bias=bias)
+            self.in_proj = Linear(width, self.proj_rows, bias=bias)
             if bias:
                 nn.init.zeros_(self.in_proj.bias)      # the gate's rows have no bias: theirs stays zero
-        self.o_proj = nn.Linear(heads * vdim, width, bias=o_bias)
+        self.o_proj = Linear(heads * vdim, width, bias=o_bias)
 
     def cache_rows(self) -> dict:
         return {} if self.borrows else {self.k_name: self.kv_heads * self.dim, self.v_name: self.kv_heads * self.vdim}
@@ -164,13 +165,13 @@ class TiedAttention(nn.Module):
         self.heads, self.kv_heads, self.dim, self.vdim = heads, kv_heads, dim, dim
         self.scale, self.eps, self.window, self.chunk, self.cache_name = float(scale), eps, int(window or 0), int(chunk or 0), cache_name
         self.q_cols, self.k_cols = heads * dim, kv_heads * dim
-        self.in_proj = nn.Linear(width, self.q_cols + self.k_cols, bias=bias)      # rows: q | k
+        self.in_proj = Linear(width, self.q_cols + self.k_cols, bias=bias)      # rows: q | k
         self.q_norm = nn.Parameter(torch.zeros(dim, dtype=torch.float32))
         self.k_norm = nn.Parameter(torch.zeros(dim, dtype=torch.float32))
         if slopes is not None and len(slopes) != heads:
             raise ValueError(f"{heads} heads need {heads} slopes, got {len(slopes)}")
         self.register_buffer("slopes", torch.tensor([float(s) for s in slopes], dtype=torch.float32) if slopes is not None else None, persistent=False)
-        self.o_proj = nn.Linear(heads * dim, width, bias=o_bias)
+        self.o_proj = Linear(heads * dim, width, bias=o_bias)
 
     def cache_rows(self, at=None) -> dict:
         n = self.cache_name if at is None else at

@@ -2,10 +2,10 @@
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
+from .linear import Linear
 from .rotary_embedding import rotary_frequencies
 
 
@@ -22,13 +22,13 @@ class LatentAttention(nn.Module):
         super().__init__()
         self.heads, self.dim, self.vdim, self.q_rank, self.kv_rank = heads, dim, vdim, q_rank, kv_rank
         self.scale, self.eps, self.layer_id = scale, eps, layer_id
-        self.down_proj = nn.Linear(width, q_rank + kv_rank + heads, bias=False)     # rows: dq | dkv | g
+        self.down_proj = Linear(width, q_rank + kv_rank + heads, bias=False)     # rows: dq | dkv | g
         self.q_norm = nn.Parameter(torch.ones(q_rank, dtype=torch.float32))
         self.kv_norm = nn.Parameter(torch.ones(kv_rank, dtype=torch.float32))
-        self.uq_proj = nn.Linear(q_rank, heads * dim, bias=False)
+        self.uq_proj = Linear(q_rank, heads * dim, bias=False)
         self.uk = nn.Parameter(torch.empty(heads, dim, kv_rank))       # W_uk, head by head
         self.uv = nn.Parameter(torch.empty(heads, vdim, kv_rank))      # W_uv, head by head
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     def forward(self, h: torch.Tensor, md) -> torch.Tensor:
         t = h.shape[0]
@@ -67,12 +67,12 @@ class RotaryLatentAttention(nn.Module):
         self.row = self.padded_row(kv_rank + rot_dim)
         hd = dim + rot_dim
         self.q_cols, self.kv_cols = heads * hd, kv_rank + rot_dim
-        self.in_proj = nn.Linear(width, self.q_cols + self.kv_cols + heads, bias=False)      # rows: q | dkv | g
+        self.in_proj = Linear(width, self.q_cols + self.kv_cols + heads, bias=False)      # rows: q | dkv | g
         self.kv_norm = nn.Parameter(torch.ones(kv_rank, dtype=torch.float32))
         # W_uk and W_uv head by head, widened to the cache row: the rotated columns pass through the key fold and drop out of the values
         self.uk = nn.Parameter(torch.zeros(heads, hd, self.row))
         self.uv = nn.Parameter(torch.zeros(heads, self.row, vdim))
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     @staticmethod
     def padded_row(n: int) -> int:

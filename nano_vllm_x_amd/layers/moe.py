@@ -4,10 +4,10 @@ enters the choice only, or chosen by a table of token ids with fixed weights on 
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
+from .linear import Linear
 
 
 class DenseGLU(nn.Module):
@@ -16,8 +16,8 @@ class DenseGLU(nn.Module):
     def __init__(self, width: int, ff: int, limit: float, alpha: float):
         super().__init__()
         self.ff, self.limit, self.alpha = ff, float(limit), float(alpha)
-        self.gu_proj = nn.Linear(width, 2 * ff, bias=False)      # rows: gate | up
-        self.down = nn.Linear(ff, width, bias=False)
+        self.gu_proj = Linear(width, 2 * ff, bias=False)      # rows: gate | up
+        self.down = Linear(ff, width, bias=False)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         return self.down(ops.moe_glu(self.gu_proj(h), self.limit, self.alpha, 1.0))
@@ -29,8 +29,8 @@ class GeluGLU(nn.Module):
     def __init__(self, width: int, ff: int):
         super().__init__()
         self.ff = ff
-        self.gu_proj = nn.Linear(width, 2 * ff, bias=False)      # rows: gate | up
-        self.down = nn.Linear(ff, width, bias=False)
+        self.gu_proj = Linear(width, 2 * ff, bias=False)      # rows: gate | up
+        self.down = Linear(ff, width, bias=False)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         return self.down(ops.gelu_glu(self.gu_proj(h)))

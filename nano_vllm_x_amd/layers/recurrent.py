@@ -6,6 +6,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
+from .linear import Linear
 
 
 class MinGRU(nn.Module):
@@ -17,8 +18,8 @@ class MinGRU(nn.Module):
     def __init__(self, width: int, inner: int, state_name):
         super().__init__()
         self.width, self.inner, self.state_name = width, inner, state_name
-        self.zxg_proj = nn.Linear(width, 3 * inner, bias=True)     # rows: z | x | g (the gate g has no bias: zeros)
-        self.o_proj = nn.Linear(inner, width, bias=False)
+        self.zxg_proj = Linear(width, 3 * inner, bias=True)     # rows: z | x | g (the gate g has no bias: zeros)
+        self.o_proj = Linear(inner, width, bias=False)
 
     def state_shapes(self) -> dict:
         return {self.state_name: (self.inner,)}
@@ -45,10 +46,10 @@ class MLSTM(nn.Module):
     def __init__(self, width: int, heads: int, dim: int, vdim: int, gate_cap: float, eps: float, state_name):
         super().__init__()
         self.heads, self.dim, self.vdim, self.gate_cap, self.eps, self.state_name = heads, dim, vdim, float(gate_cap), eps, state_name
-        self.qkvg_proj = nn.Linear(width, 2 * heads * dim + 2 * heads * vdim, bias=False)     # rows: q | k | v | g
+        self.qkvg_proj = Linear(width, 2 * heads * dim + 2 * heads * vdim, bias=False)     # rows: q | k | v | g
         self.gate_w, self.gate_b = _f32(2 * heads, width), _f32(2 * heads)                   # rows: input | forget
         self.norm = _f32(heads * vdim)
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     def state_shapes(self, at=None) -> dict:
         n = self.state_name if at is None else at
@@ -77,12 +78,12 @@ class GatedDelta(nn.Module):
             raise ValueError("heads must be a multiple of kv_heads")
         self.heads, self.kv_heads, self.dim, self.vdim, self.taps, self.eps, self.state_name = heads, kv_heads, dim, vdim, taps, eps, state_name
         self.conv_ch = 2 * kv_heads * dim + heads * vdim
-        self.qkvg_proj = nn.Linear(width, self.conv_ch + heads * vdim, bias=False)            # rows: q | k | v | g
+        self.qkvg_proj = Linear(width, self.conv_ch + heads * vdim, bias=False)            # rows: q | k | v | g
         self.conv_w = _f32(taps, self.conv_ch)                                                # row j: the tap taps - 1 - j tokens back
         self.ab_w = _f32(2 * heads, width)                                                    # rows: decay | write strength
         self.a_log, self.dt_bias = _f32(heads), _f32(heads)
         self.norm = _f32(vdim)
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     def state_shapes(self) -> dict:
         shapes = {(self.state_name, "S"): (self.heads, self.dim, self.vdim)}
@@ -120,7 +121,7 @@ class TimeMix(nn.Module):
         self.w1, self.w2, self.w0 = _f32(decay_rank, width), _f32(hd, decay_rank), _f32(hd)
         self.bonus = _f32(heads, dim)
         self.norm = _f32(hd)
-        self.o_proj = nn.Linear(hd, width, bias=False)
+        self.o_proj = Linear(hd, width, bias=False)
 
     def state_shapes(self) -> dict:
         return {(self.state_name, "S"): (self.heads, self.dim, self.dim), (self.state_name, "prev"): (self.width,)}
@@ -151,9 +152,9 @@ class DecayLinearAttention(nn.Module):
         self.register_buffer("decay", torch.tensor(decay, dtype=torch.float32), persistent=False)
         self.proj_rows = 2 * heads * dim + 2 * heads * vdim
         if own_proj:
-            self.in_proj = nn.Linear(width, self.proj_rows, bias=False)
+            self.in_proj = Linear(width, self.proj_rows, bias=False)
         self.norm = _f32(heads * vdim)
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     def state_shapes(self) -> dict:
         return {(self.state_name, "S"): (self.heads, self.dim, self.vdim)}
@@ -186,14 +187,14 @@ class RGLRU(nn.Module):
             raise ValueError("the channels must divide into the blocks")
         self.width, self.inner, self.blocks, self.taps, self.decay_scale, self.state_name = width, inner, blocks, taps, float(decay_scale), state_name
         bw = inner // blocks
-        self.in_proj = nn.Linear(width, 2 * inner, bias=True)              # rows: y | x
+        self.in_proj = Linear(width, 2 * inner, bias=True)              # rows: y | x
         self.conv_w = _f32(taps, inner)                                    # row j: the tap taps - 1 - j tokens back
         self.conv_b = _f32(inner)
         self.gate_w = nn.Parameter(torch.empty(blocks, bw, 2 * bw))        # per block: input channel -> recurrence gate | input gate
         self.gate_b = _f32(2, inner)                                       # rows: recurrence gate | input gate
         self.lam = _f32(inner)
         self.register_buffer("rate", torch.zeros(inner, dtype=torch.float32), persistent=False)
-        self.o_proj = nn.Linear(inner, width, bias=False)
+        self.o_proj = Linear(inner, width, bias=False)
 
     def finalize(self):
         """After the weights are loaded: the constant factor of every channel's decay exponent."""
@@ -225,10 +226,10 @@ class GatedLinearAttention(nn.Module):
     def __init__(self, width: int, heads: int, dim: int, vdim: int, tau: float, rank: int, eps: float, state_name):
         super().__init__()
         self.heads, self.dim, self.vdim, self.tau, self.eps, self.state_name = heads, dim, vdim, float(tau), eps, state_name
-        self.qkvg_proj = nn.Linear(width, 2 * heads * dim + 2 * heads * vdim, bias=False)     # rows: q | k | v | g
+        self.qkvg_proj = Linear(width, 2 * heads * dim + 2 * heads * vdim, bias=False)     # rows: q | k | v | g
         self.a1, self.a2, self.a2_b = _f32(rank, width), _f32(heads * dim, rank), _f32(heads * dim)
         self.norm = _f32(vdim)
-        self.o_proj = nn.Linear(heads * vdim, width, bias=False)
+        self.o_proj = Linear(heads * vdim, width, bias=False)
 
     def state_shapes(self, at=None) -> dict:
         return {(self.state_name if at is None else at, "S"): (self.heads, self.dim, self.vdim)}

@@ -27,6 +27,7 @@ from torch import nn
 from . import distributed as tpd
 from . import ops
 from .layers.cap_attention import SoftcapAttention
+from .layers.linear import Linear, linear
 from .layers.moe import SigmoidInputMoE
 from .layers.recurrent import MLSTM, GatedDelta, TimeMix
 
@@ -123,13 +124,13 @@ class MeronexLayer(nn.Module):
         else:
             self.mixer = ParallelMixer(w, m, cfg.eps, i)
         self.norm1 = _f32(w)
-        self.rg1, self.rg1_b = nn.Linear(w, w, bias=False), _f32(w)
+        self.rg1, self.rg1_b = Linear(w, w, bias=False), _f32(w)
         self.mlp = None
         if spec["mlp"] is not None:
             e, r = spec["mlp"]["expert"], spec["mlp"]["router"]
             self.mlp = SigmoidInputMoE(w, r["experts"], r["top"], e["ff"], e["limit"], EXPERT_SIGMOID_SLOPE)
             self.norm2 = _f32(w)
-            self.rg2, self.rg2_b = nn.Linear(w, w, bias=False), _f32(w)
+            self.rg2, self.rg2_b = Linear(w, w, bias=False), _f32(w)
 
 
 class MeronexForCausalLM(nn.Module):
@@ -202,7 +203,7 @@ class MeronexForCausalLM(nn.Module):
         return h
 
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_states, self.head)
+        return linear(hidden_states, self.head)
 
     # -- weights ----------------------------------------------------------------------------------------
     @torch.no_grad()

@@ -1813,8 +1813,31 @@ def gelu_glu(gu):
     return y
 
 
+FEW_ROWS = 32       # rows up to which csrc/few_rows.hip beats the library's products at every size measured
+
+
+def few_rows_fits(x, w, bias=None) -> bool:
+    """Whether x W^T (+ bias) is a product few_rows_product takes: up to FEW_ROWS rows of 512s of columns, 16s of outputs."""
+    return (x.dim() == 2 and x.is_cuda and x.dtype in H16 and 0 < x.shape[0] <= FEW_ROWS and w.dtype == x.dtype and w.dim() == 2 and x.shape[1] == w.shape[1]
+            and w.shape[1] % 512 == 0 and w.shape[0] % 16 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]
+            and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and (x.device == w.device)
+            and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous() and bias.device == x.device))
+            and not torch.is_grad_enabled())
+
+
+def few_rows_product(x, w, bias=None, f32: bool = False):
+    """x (T <= FEW_ROWS, k) @ w (n, k).T + bias, in x's format or as the unrounded float32 sums; see few_rows_fits."""
+    _need(few_rows_fits(x, w, bias), "few_rows_product: sizes and layouts of few_rows_fits")
+    t, k, n = x.shape[0], x.shape[1], w.shape[0]
+    y = torch.empty((t, n), dtype=F32 if f32 else x.dtype, device=x.device)
+    _lib.check(_lib.load().nvx_internal_few_rows(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(y), _fmt(x), int(f32), t, n, k, _stream()), "few_rows_product")
+    return y
+
+
 def product_f32(x, w):
-    """x @ w.T as a library product that returns its float32 sums unrounded; x (T, k), w (n, k) in one format."""
+    """x @ w.T as its float32 sums, unrounded; x (T, k), w (n, k) in one format.  A library product except for few rows (few_rows_product)."""
+    if x.dim() == 2 and x.shape[0] <= FEW_ROWS and few_rows_fits(x, w):
+        return few_rows_product(x, w, f32=True)
     if x.dtype == F32:
         return torch.nn.functional.linear(x, w)
     return torch.mm(x, w.t(), out_dtype=F32)
