@@ -529,15 +529,23 @@ __global__ __launch_bounds__(256) void softcap_attn_kernel(const A* __restrict__
 // score to the read-out, for all NH heads: a wave takes U keys per lane group at a time (their loads in flight together), sums the
 // products over the lane group, and adds the weighted rows to what the lane keeps of the read-out.  Every lane group has a running
 // maximum and sum of its own; groups, waves and splits are merged at the end.  TIED: a cached row is key AND value, and k_rn norms its
-// score; otherwise values have rows of their own.
-template <typename A, int NH, int U, int LPR, bool TIED>
+// score; otherwise values have rows of their own.  SCORED: scores are capped, or lessened by the logarithm of the distance; every lane of a
+// group does that for one of its U keys and hands the score to the others (done by all of them for all keys it costs more than the products).
+// 16 sequences of 900-1150 tokens, 16 / 8 heads of 128, three layers with the distance penalty and three with a cap, a window of 512, values
+// turned back and a gate: 17.3 us a launch on average (their rows are 10 us of memory); the kernel above, which reads a row once per head and a
+// key per lane, took 31.7.
+template <typename A, int NH, int U, int LPR, bool TIED, bool SCORED>
 __global__ __launch_bounds__(256) void rows_attn_kernel(const A* __restrict__ q, const A* __restrict__ rows, const A* __restrict__ v_rows,
                                                        const float* __restrict__ k_rn, const int32_t* __restrict__ kv_indices,
                                                        const int64_t* __restrict__ kv_start, const int32_t* __restrict__ kv_len,
                                                        const int32_t* __restrict__ qo_indptr, const int32_t* __restrict__ tok_seq, float scale,
                                                        A* __restrict__ out, int heads, int kv_heads, int dim, int vdim, int n_split,
                                                        float* __restrict__ part, int window, int chunk, const float* __restrict__ slopes, int sink,
-                                                       float sink_score, const float* __restrict__ sinks, int keep, float out_mul, int64_t out_stride) {
+                                                       float sink_score, const float* __restrict__ sinks, int keep, float out_mul, int64_t out_stride,
+                                                       float cap, const float* __restrict__ r1, const float* __restrict__ r2,
+                                                       const float* __restrict__ vcs, int v_inter, const A* __restrict__ gate, int64_t gate_stride,
+                                                       int gate_one) {
+    static_assert(!SCORED || U <= LPR, "a lane of a group has one key");
     extern __shared__ float sm[];
     float* sacc = sm;                       // 4 waves x NH x vdim
     float* sml = sacc + 4 * NH * vdim;      // 4 waves x NH maxima, then as many sums
@@ -556,11 +564,13 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const A* __restrict__ q,
     constexpr int groups = 64 / LPR;
     const bool on = l * 8 < dim, on_v = l * 8 < vdim;
     typedef A vec8 __attribute__((ext_vector_type(8)));
-    float qv[NH][8], acc[NH][8], m[NH], sum[NH], slope[NH];
+    float qv[NH][8], acc[NH][8], m[NH], sum[NH], slope[NH], pen_a[NH], pen_b[NH];
 #pragma unroll
     for (int n = 0; n < NH; ++n) {
         const int h = h0 + (n < n_here ? n : 0);
         slope[n] = slopes ? slopes[h] : 0.f;
+        pen_a[n] = SCORED && r1 ? r1[h] : 0.f;
+        pen_b[n] = SCORED && r1 ? r2[h] : 0.f;
         m[n] = -INFINITY;
         sum[n] = 0.f;
         const vec8 qr = *reinterpret_cast<const vec8*>(q + (t * heads + h) * (int64_t)dim + (on ? l * 8 : 0));
@@ -593,8 +603,27 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const A* __restrict__ q,
                 d = group_sum<LPR>(d);
                 const int i = i0 + u * groups + g, j = i < kept ? i : first + i - kept;
                 if constexpr (TIED) d *= rn[u];
-                s[u] = i < n_keys ? d - slope[n] * (float)(visible - 1 - j) : -INFINITY;
-                mx = fmaxf(mx, s[u]);
+                if constexpr (SCORED) s[u] = d;
+                else {
+                    s[u] = i < n_keys ? d - slope[n] * (float)(visible - 1 - j) : -INFINITY;
+                    mx = fmaxf(mx, s[u]);
+                }
+            }
+            if constexpr (SCORED) {
+                const int mine = l % U, i = i0 + mine * groups + g, j = i < kept ? i : first + i - kept;
+                float d = s[0];
+#pragma unroll
+                for (int u = 1; u < U; ++u) d = mine == u ? s[u] : d;
+                if (cap > 0.f) d = cap * tanhf(d / cap);
+                const float far = (float)(visible - 1 - j);
+                d -= slope[n] * far;
+                if (r1) d -= pen_a[n] * log1pf(pen_b[n] * far);
+                if (i >= n_keys) d = -INFINITY;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    s[u] = __shfl(d, g * LPR + u, 64);
+                    mx = fmaxf(mx, s[u]);
+                }
             }
             const float base = mx == -INFINITY ? 0.f : mx;                  // (nothing seen by this lane group yet)
             const float corr = expf(m[n] - base);
@@ -652,9 +681,17 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(const A* __restrict__ q,
 #pragma unroll
             for (int w = 0; w < 4; ++w) o += sacc[(w * NH + n) * vdim + e] * f[w];
             if (pr) pr[2 + e] = o;
+            else if (vcs || gate) sacc[n * vdim + e] = o / total * out_mul;     // (this thread alone reads column e of the four partial sums)
             else st_f(out, t * out_stride + (int64_t)(h0 + n) * vdim + e, o / total * out_mul);
         }
         if (pr && threadIdx.x == 0) { pr[0] = mm; pr[1] = total; }
+    }
+    if (n_split == 1 && (vcs || gate)) {
+        __syncthreads();
+        for (int n = 0; n < n_here; ++n)
+            attn_readout_end<A>(sacc + n * vdim, vdim, vcs ? vcs + t * (int64_t)vdim : nullptr, v_inter,
+                                gate ? gate + t * gate_stride + (gate_one ? (int64_t)(h0 + n) : (int64_t)(h0 + n) * vdim) : nullptr, gate_one != 0,
+                                out + t * out_stride + (int64_t)(h0 + n) * vdim, 256);
     }
 }
 
@@ -941,7 +978,8 @@ __global__ __launch_bounds__(256) void softcap_attn_tile_kernel(const A* __restr
     }
 }
 
-// out = the n_split partial results of a (token, head) merged: each is (maximum, sum, unnormalised values); one wave each.
+// out = the n_split partial results of a (token, head) merged: each is (maximum, sum, unnormalised values); one wave each.  A chain of memory
+// round trips and little else: maxima and sums by one load of the wave, the splits' columns four at a time (256 of four splits: 7.1 -> 4.9 us).
 template <typename A>
 __global__ __launch_bounds__(64) void softcap_merge_kernel(const float* __restrict__ part, int n_split, A* __restrict__ out, int vdim,
                                                           int heads, const float* __restrict__ vcs, int v_inter,
@@ -951,19 +989,26 @@ __global__ __launch_bounds__(64) void softcap_merge_kernel(const float* __restri
     const int64_t row = blockIdx.x, t = row / heads, hd = row % heads;
     if (sinks) sink_score = sinks[hd];
     const float* pr = part + row * n_split * (vdim + 2);
-    float mm = sink ? sink_score : -INFINITY;
-    for (int s = 0; s < n_split; ++s) mm = fmaxf(mm, pr[s * (vdim + 2)]);
-    float total = sink ? expf(sink_score - mm) : 0.f;
-    for (int s = 0; s < n_split; ++s) {
-        const float m = pr[s * (vdim + 2)];
-        total += m == -INFINITY ? 0.f : pr[s * (vdim + 2) + 1] * expf(m - mm);
-    }
-    for (int e = threadIdx.x; e < vdim; e += 64) {
+    // every lane has a split's maximum and sum; the splits' columns are asked for four at a time
+    const int lane = threadIdx.x;
+    const float m = lane < n_split ? pr[lane * (vdim + 2)] : -INFINITY, l = lane < n_split ? pr[lane * (vdim + 2) + 1] : 0.f;
+    const float mm = fmaxf(wave_max(m), sink ? sink_score : -INFINITY);
+    const float f = m == -INFINITY ? 0.f : expf(m - mm);
+    const float total = wave_sum(l * f) + (sink ? expf(sink_score - mm) : 0.f);
+    for (int e0 = 0; e0 < vdim; e0 += 64) {
+        const int e = min(e0 + lane, vdim - 1);
         float o = 0.f;
-        for (int s = 0; s < n_split; ++s) {
-            const float m = pr[s * (vdim + 2)];
-            if (m != -INFINITY) o += pr[s * (vdim + 2) + 2 + e] * expf(m - mm);
+        for (int s0 = 0; s0 < n_split; s0 += 4) {
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = pr[min(s0 + j, n_split - 1) * (vdim + 2) + 2 + e];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float fs = __shfl(f, min(s0 + j, 63), 64);
+                if (s0 + j < n_split && fs != 0.f) o += v[j] * fs;         // (a split that saw nothing left nothing to read)
+            }
         }
+        if (e0 + lane >= vdim) continue;
         if (vcs || gate) so[e] = o / total * out_mul;
         else st_f(out, t * out_stride + hd * vdim + e, o / total * out_mul);
     }
@@ -1157,20 +1202,26 @@ extern "C" int nvx_softcap_attn(const void* q, const void* k_cache, const void* 
     }
     const size_t lds = (size_t)(dim + 4 * vdim + 8) * sizeof(float);
     NVX_REQUIRE(n_split >= 1 && n_split <= 64 && (n_split == 1 || part), NVX_EINVAL, "nvx_softcap_attn: a key split needs its workspace");
-    // without what the kernel does not do: a row is read once for up to four heads
+    // a row is read once for up to four heads; keys that are values too do not come with caps or distance penalties that way
     const bool tied = k_rn && k_cache == v_cache && dim == vdim;
-    if ((tied || !k_rn) && dim % 8 == 0 && vdim % 8 == 0 && dim <= 512 && cap <= 0.f && !r1 && !vcs && !gate && nvx_aligned16(q) && nvx_aligned16(k_cache) &&
+    if ((tied || !k_rn) && dim % 8 == 0 && vdim % 8 == 0 && dim <= 512 && (!tied || (cap <= 0.f && !r1)) && nvx_aligned16(q) && nvx_aligned16(k_cache) &&
         nvx_aligned16(v_cache)) {
         const int per_kv = (int)(heads / kv_heads), nh = per_kv >= 4 ? 4 : (per_kv >= 2 ? 2 : 1);
         const dim3 tgrid((unsigned)(kv_heads * ((per_kv + nh - 1) / nh)), (unsigned)n_tok, (unsigned)n_split);
         const size_t tlds = (size_t)(4 * nh * vdim + 8 * nh) * sizeof(float);
         const int64_t longest = dim > vdim ? dim : vdim;
-#define NVX_ROWS_ATTN_T(NH, LPR, U, TIED)                                                                                                       \
-    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((rows_attn_kernel<A_, NH, sizeof(A_) == 2 ? U : 4, LPR, TIED>), tgrid, dim3(256), tlds, (hipStream_t)stream, \
+#define NVX_ROWS_ATTN_T(NH, LPR, U, TIED, SC)                                                                                                       \
+    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((rows_attn_kernel<A_, NH, sizeof(A_) == 2 ? U : 4, LPR, TIED, SC>), tgrid, dim3(256), tlds, (hipStream_t)stream, \
                                          (const A_*)q, (const A_*)k_cache, (const A_*)v_cache, k_rn, kv_indices, kv_start, kv_len, qo_indptr, tok_seq, scale, \
                                          (A_*)out, (int)heads, (int)kv_heads, (int)dim, (int)vdim, n_split, part, (int)window, (int)chunk, slopes, sink, \
-                                         sink_score, sinks, (int)keep_first, out_mul, out_stride))
-#define NVX_ROWS_ATTN_L(NH, LPR) do { if (tied) NVX_ROWS_ATTN_T(NH, LPR, 8, true); else NVX_ROWS_ATTN_T(NH, LPR, (NH == 4 ? 4 : 8), false); } while (0)
+                                         sink_score, sinks, (int)keep_first, out_mul, out_stride, cap, r1, r2, vcs, v_interleaved, (const A_*)gate, gate_stride, \
+                                         gate_per_head))
+#define NVX_ROWS_ATTN_L(NH, LPR)                                                          \
+    do {                                                                                  \
+        if (tied) NVX_ROWS_ATTN_T(NH, LPR, 8, true, false);                               \
+        else if (cap > 0.f || r1) NVX_ROWS_ATTN_T(NH, LPR, (NH == 4 ? 4 : 8), false, true); \
+        else NVX_ROWS_ATTN_T(NH, LPR, (NH == 4 ? 4 : 8), false, false);                   \
+    } while (0)
 #define NVX_ROWS_ATTN(NH)                                 \
     do {                                                  \
         if (longest <= 64) NVX_ROWS_ATTN_L(NH, 8);        \
