@@ -180,8 +180,18 @@ class PrefillStep(ctypes.Structure):
                                 "q", "attn", "act", "out")] + [("eps", ctypes.c_double), ("scale", ctypes.c_double)]
 
 
+TABLE_LAYERS = 32
+
+
+class TableChoices(ctypes.Structure):
+    """NvxTableChoices of csrc/moe.hip, field by field."""
+    _fields_ = [("table", _c_vp * TABLE_LAYERS), ("idx", _c_vp * TABLE_LAYERS), ("wts", _c_vp * TABLE_LAYERS), ("vocab", _c_i64 * TABLE_LAYERS),
+                ("top", _c_i32 * TABLE_LAYERS), ("share", ctypes.c_float * TABLE_LAYERS)]
+
+
 # What the host of this package calls beside the C ABI; not declared in include/nvx.h
 INTERNAL = {name: (_c_i32, [ctypes.POINTER(PrefillStep), _c_vp]) for name in ("nvx_internal_prefill_step", "nvx_internal_prefill_step_f16")}
+INTERNAL["nvx_internal_table_choices"] = (_c_i32, [ctypes.POINTER(TableChoices), _c_i32, _c_vp, _c_i64, _c_vp])
 INTERNAL["nvx_internal_few_rows"] = (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_vp, _c_i32, _c_i32, _c_i64, _c_i64, _c_i64, _c_vp])
 
 

@@ -769,3 +769,39 @@ extern "C" int nvx_moe_gather_rows(const void* ys, int fmt, const int64_t* dst, 
                                          wts, (int)top, (A_*)out, (int)width));
     return nvx_check_launch("nvx_moe_gather_rows");
 }
+
+// ---- experts chosen by a table of token ids ---------------------------------------------------------------------------------------
+// The choices of a step's tokens in up to TABLE_LAYERS layers, one launch for all of them: idx[l][t] = table[l][id[t]], wts[l] = share[l].  (A gather and a
+// fill per layer were 11 + 4 us each at 16 tokens: two launches for 32 numbers.)
+constexpr int TABLE_LAYERS = 32;
+struct NvxTableChoices {
+    const int32_t* table[TABLE_LAYERS];    // (vocab, top)
+    int32_t* idx[TABLE_LAYERS];            // (n, top)
+    float* wts[TABLE_LAYERS];              // (n, top)
+    int64_t vocab[TABLE_LAYERS];
+    int32_t top[TABLE_LAYERS];
+    float share[TABLE_LAYERS];
+};
+
+namespace NVX_NS {
+__global__ __launch_bounds__(256) void table_choices_kernel(NvxTableChoices a, const int64_t* __restrict__ ids, int64_t n_tok) {
+    const int l = blockIdx.y, top = a.top[l];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_tok * top) return;
+    const int64_t id = ids[i / top], row = id < 0 ? 0 : (id < a.vocab[l] ? id : a.vocab[l] - 1);      // (no read outside the table)
+    a.idx[l][i] = a.table[l][row * top + i % top];
+    a.wts[l][i] = a.share[l];
+}
+}  // namespace NVX_NS
+
+extern "C" int nvx_internal_table_choices(const NvxTableChoices* a, int n_layers, const int64_t* ids, int64_t n_tok, nvx_stream_t stream) {
+    NVX_REQUIRE(a && ids && n_layers > 0 && n_layers <= TABLE_LAYERS && n_tok >= 0 && n_tok < (1ll << 31), NVX_EINVAL, "nvx_internal_table_choices: sizes");
+    if (n_tok == 0) return NVX_OK;
+    int top = 0;
+    for (int l = 0; l < n_layers; ++l) {
+        NVX_REQUIRE(a->table[l] && a->idx[l] && a->wts[l] && a->vocab[l] > 0 && a->top[l] > 0, NVX_EINVAL, "nvx_internal_table_choices: a layer's table");
+        top = a->top[l] > top ? a->top[l] : top;
+    }
+    hipLaunchKernelGGL(NVX_NS::table_choices_kernel, dim3((unsigned)((n_tok * top + 255) / 256), (unsigned)n_layers), dim3(256), 0, (hipStream_t)stream, *a, ids, n_tok);
+    return nvx_check_launch("nvx_internal_table_choices");
+}

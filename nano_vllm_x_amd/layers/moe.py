@@ -146,12 +146,10 @@ class TableMoE(ExpertBank):
     def __init__(self, width: int, experts: int, top: int, ff: int, vocab: int):
         super().__init__(width, experts, top, ff, float("inf"), 1.0, 0.0)
         self.register_buffer("table", torch.zeros(vocab, top, dtype=torch.int32), persistent=False)
-        self.register_buffer("share", torch.full((1, top), 1.0 / top, dtype=torch.float32), persistent=False)
 
     def choices(self, input_ids: torch.Tensor):
         """(idx, wts) of a step's tokens: they depend on the token ids alone."""
-        idx = self.table.index_select(0, input_ids)
-        return idx, self.share.expand(idx.shape[0], self.top).contiguous()
+        return ops.table_choices([self.table], input_ids)[0]
 
     @staticmethod
     def plan_step(layers, input_ids: torch.Tensor, decode_step: bool) -> list:
@@ -159,11 +157,12 @@ class TableMoE(ExpertBank):
         choices, and for steps of many tokens the expert order with its counts -- ONE host read for all layers instead of one per
         layer in the middle of the step, so the host can queue the whole step without waiting for the device."""
         plans, pending = [], []
+        made = iter(ops.table_choices([moe.table for moe in layers if moe is not None], input_ids))
         for moe in layers:
             if moe is None:
                 plans.append(None)
                 continue
-            idx, wts = moe.choices(input_ids)
+            idx, wts = next(made)
             plan = {"idx": idx, "wts": wts, "order": None}
             if not moe.by_rows(idx.shape[0], decode_step):
                 dst, counts = ops.moe_order(idx, moe.experts)

@@ -1445,6 +1445,29 @@ def _moe_weights(w_gu, w_d, what: str):
     return n_exp, ff2 // 2, width
 
 
+def table_choices(tables, input_ids) -> list:
+    """[(idx (T, top) int32, wts (T, top) float32 of 1 / top)] for every table (vocab, top) int32: idx[t] = table[input_ids[t]], one launch for up to 32."""
+    _dev(input_ids, *tables)
+    _need(input_ids.dtype == torch.int64 and input_ids.is_contiguous() and input_ids.dim() == 1, "table_choices: input_ids must be int64 (T)")
+    out, t = [], input_ids.numel()
+    for first in range(0, len(tables), _lib.TABLE_LAYERS):
+        part = tables[first:first + _lib.TABLE_LAYERS]
+        a, tops = _lib.TableChoices(), [x.shape[1] for x in part]
+        for x in part:
+            _need(x.dtype == torch.int32 and x.dim() == 2 and x.is_contiguous(), "table_choices: tables must be contiguous int32 (vocab, top)")
+        idx = torch.empty((t * sum(tops),), dtype=torch.int32, device=input_ids.device)
+        wts = torch.empty((t * sum(tops),), dtype=F32, device=input_ids.device)
+        at = 0
+        for l, (x, top) in enumerate(zip(part, tops)):
+            i, w = idx[at:at + t * top].view(t, top), wts[at:at + t * top].view(t, top)
+            a.table[l], a.idx[l], a.wts[l], a.vocab[l], a.top[l], a.share[l] = x.data_ptr(), i.data_ptr(), w.data_ptr(), x.shape[0], top, 1.0 / top
+            out.append((i, w))
+            at += t * top
+        if t:
+            _lib.check(_lib.load().nvx_internal_table_choices(a, len(part), _ptr(input_ids), t, _stream()), "table_choices")
+    return out
+
+
 def moe_expert_rows(h, idx, wts, w_gu, w_d, limit: float, alpha: float, shift: float = 1.0, weight_out: bool = False):
     """out[t] = sum over token t's chosen experts of expert(score * h[t]) (or of score * expert(h[t]) if `weight_out`); w_gu
     (experts, 2 * ff, width) = gate | up rows, w_d (experts, width, ff); activation min(g, limit) sigmoid(alpha min(g, limit))
