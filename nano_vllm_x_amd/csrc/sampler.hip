@@ -105,16 +105,42 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_kernel(
     const int lo = slice * per, hi = min(min(vocab, lo + per), tok_end - tok0);
     const float inv_t = greedy ? 1.0f : 1.0f / T;
     float best = -INFINITY; int besti = 0x7fffffff;
-    for (int base = lo + tid * 4; base < hi; base += SMP_THREADS * 4) {
-        uint4 r = make_uint4(0, 0, 0, 0);
-        if (!greedy) r = philox4x32_10(make_uint4((uint32_t)((tok0 + base) >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
-        const uint32_t rr[4] = {r.x, r.y, r.z, r.w};
+    // The loads of U blocks are on their way before the first is used, four tokens a load where the row stands on such a border: with a load per token and
+    // use the pass waited for memory (a block's noise is some 1300 clocks of a wave, which 256 rows of 151 936 tokens wait for: 62 us, 53 with products and logarithms of fewer instructions).
+    constexpr int U = 4;
+    const bool whole = (reinterpret_cast<uintptr_t>(lrow) & (F32 ? 15 : 7)) == 0;
+    for (int b0 = lo + tid * 4; b0 < hi; b0 += U * SMP_THREADS * 4) {
+        float l[U][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int i = base + j;
-            if (i < hi) {
-                const float v = load_logit<F32>(lrow, i) * inv_t + (greedy ? 0.0f : gumbel_from_bits(rr[j]));
-                if (v > best) { best = v; besti = tok0 + i; }
+        for (int u = 0; u < U; ++u) {
+            const int base = b0 + u * SMP_THREADS * 4;
+            if (whole && base + 3 < hi) {
+                if (F32) {
+                    const float4 w = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lrow) + base);
+                    l[u][0] = w.x; l[u][1] = w.y; l[u][2] = w.z; l[u][3] = w.w;
+                } else {
+                    const uint2 w = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(lrow) + base);
+                    l[u][0] = h16lo_to_f32(w.x); l[u][1] = h16hi_to_f32(w.x); l[u][2] = h16lo_to_f32(w.y); l[u][3] = h16hi_to_f32(w.y);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) l[u][j] = base + j < hi ? load_logit<F32>(lrow, base + j) : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int base = b0 + u * SMP_THREADS * 4;
+            if (base >= hi) continue;
+            uint4 r = make_uint4(0, 0, 0, 0);
+            if (!greedy) r = philox4x32_10(make_uint4((uint32_t)((tok0 + base) >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
+            const uint32_t rr[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = base + j;
+                if (i < hi) {
+                    const float v = l[u][j] * inv_t + (greedy ? 0.0f : gumbel_from_bits(rr[j]));
+                    if (v > best) { best = v; besti = tok0 + i; }
+                }
             }
         }
     }
@@ -391,16 +417,10 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_filtered_kernel(
     };
 
     // ---- min-p on softmax of what survived ----
-    float minp_thr = -1.0f, Z2 = 1.0f;
-    if (min_p > 0.0f) {
-        float zl = 0.f;
-        each([&](int i, float l) { if (kept_kp(keyf(l), i)) zl += __expf(l / T - M); });
-        Z2 = block_sum(zl, sc.blk);
-        minp_thr = min_p * (1.0f / Z2);
-    }
+    // (the largest score survives every filter, so the ratio of a token's probability to the largest is e^(x - M), whatever the normaliser)
     auto kept = [&](float l, int i) -> bool {
         if (!kept_kp(keyf(l), i)) return false;
-        if (min_p > 0.0f && (__expf(l / T - M) / Z2) < minp_thr) return false;
+        if (min_p > 0.0f && __expf(l / T - M) < min_p) return false;
         return true;
     };
 
@@ -723,38 +743,40 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     };
 
     // ---- min-p on softmax of what survived ----
-    float minp_thr = -1.0f, Z2 = 1.0f;
+    // The ratio of a token's probability to the largest, which survives every filter, is e^(x - M) whatever the normaliser, and it grows with the
+    // logit: the smallest key that is kept is searched among all keys (every wave for itself, 64 candidates at a time), and the row needs
+    // no pass of exponentials and divisions for it (256 rows with min-p alone: 90 us with two of them, now 33).
+    uint32_t m_key = 0;       // scores with key < m_key are dropped
     if (min_p > 0.0f) {
-        float zl = 0.f;
-        each_pair([&](int i, uint32_t kw) {
-            const uint32_t pr = pair_of_keys(kw);
-            if (kept_kp(kw & 0xffffu, i)) zl += __expf(h16lo_to_f32(pr) / T - M);
-            if (kept_kp(kw >> 16, i + 1)) zl += __expf(h16hi_to_f32(pr) / T - M);
-        });
-        Z2 = block_sum(zl, sc.blk);
-        minp_thr = min_p * (1.0f / Z2);
+        auto dropped = [&](uint32_t ky) -> bool { return ky <= kmax && __expf(logit_of_key(ky) / T - M) < min_p; };
+        if (dropped(kmax)) m_key = 0x10000u;
+        else {
+            uint32_t from = 0x7fu;                                // the key of -infinity
+#pragma unroll
+            for (int step = 1024; step >= 1; step >>= (step == 1024 ? 6 : 4)) {
+                const int c = __popcll(__ballot(dropped(from + (uint32_t)(lane * step))));
+                if (c) from += (uint32_t)(c - 1) * step + 1;       // (candidate c - 1 is dropped, candidate c is not)
+            }
+            m_key = from == 0x7fu ? 0u : from;
+        }
     }
-    auto kept = [&](uint32_t ky, float l, int i) -> bool {
-        if (!kept_kp(ky, i)) return false;
-        if (min_p > 0.0f && (__expf(l / T - M) / Z2) < minp_thr) return false;
-        return true;
-    };
+    auto kept = [&](uint32_t ky, int i) -> bool { return ky >= m_key && kept_kp(ky, i); };
 
     if (PROBS) {
         float zl = 0.f;
         each_pair([&](int i, uint32_t kw) {
             const uint32_t pr = pair_of_keys(kw);
             const float l0 = h16lo_to_f32(pr), l1 = h16hi_to_f32(pr);
-            if (kept(kw & 0xffffu, l0, i)) zl += __expf(l0 / T - M);
-            if (kept(kw >> 16, l1, i + 1)) zl += __expf(l1 / T - M);
+            if (kept(kw & 0xffffu, i)) zl += __expf(l0 / T - M);
+            if (kept(kw >> 16, i + 1)) zl += __expf(l1 / T - M);
         });
         const float Z3 = block_sum(zl, sc.blk);
         float* prow = probs_out + (int64_t)row * vocab;
         each_pair([&](int i, uint32_t kw) {
             const uint32_t pr = pair_of_keys(kw);
             const float l0 = h16lo_to_f32(pr), l1 = h16hi_to_f32(pr);
-            prow[i] = kept(kw & 0xffffu, l0, i) ? __expf(l0 / T - M) / Z3 : 0.0f;
-            prow[i + 1] = kept(kw >> 16, l1, i + 1) ? __expf(l1 / T - M) / Z3 : 0.0f;
+            prow[i] = kept(kw & 0xffffu, i) ? __expf(l0 / T - M) / Z3 : 0.0f;
+            prow[i + 1] = kept(kw >> 16, i + 1) ? __expf(l1 / T - M) / Z3 : 0.0f;
         });
         return;
     }
@@ -766,36 +788,75 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     uint32_t km[5] = {0, 0, 0, 0, 0};
     each_pair([&](int i, uint32_t kw) {
         const int pos = (i / (SMP_THREADS * 8)) * 8 + (i & 7);
-        bool a, b;
-        if (min_p > 0.0f) {
-            const uint32_t pr = pair_of_keys(kw);
-            a = kept(kw & 0xffffu, h16lo_to_f32(pr), i);
-            b = kept(kw >> 16, h16hi_to_f32(pr), i + 1);
-        } else {
-            a = kept_kp(kw & 0xffffu, i);
-            b = kept_kp(kw >> 16, i + 1);
-        }
+        const bool a = kept(kw & 0xffffu, i), b = kept(kw >> 16, i + 1);
         km[pos >> 5] |= ((a ? 1u : 0u) | (b ? 2u : 0u)) << (pos & 31);
     });
     const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
     float best = -INFINITY; int besti = 0x7fffffff;
-    int gbase = -1; uint32_t rr[4] = {0, 0, 0, 0};
+    // Survivors that fit go into one list in LDS (the histogram's memory): a thread then draws its share of them, their logits' loads in flight
+    // together, where a walk over its own takes as many round trips as the thread with the most survivors has (256 rows of 151 936 tokens, some 5000
+    // of each kept: 88 -> 83 us).  Where more survive the walk is the faster one: neighbours share a Philox block.
+    constexpr int LIST = (int)(sizeof(sc.hist) / sizeof(int));
+    int mine = 0;
 #pragma unroll
-    for (int wd = 0; wd < 5; ++wd) {
-        uint32_t m = km[wd];
-        while (m) {
-            const int pos = wd * 32 + __ffs((int)m) - 1;
-            m &= m - 1;
-            const int i = ((pos >> 3) * SMP_THREADS + tid) * 8 + (pos & 7);
-            const float l = h16bits_to_f32(lrow[i]);
-            if ((i & ~3) != gbase) {
-                gbase = i & ~3;
-                const uint4 r = philox4x32_10(make_uint4((uint32_t)(gbase >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
-                rr[0] = r.x; rr[1] = r.y; rr[2] = r.z; rr[3] = r.w;
+    for (int wd = 0; wd < 5; ++wd) mine += __popc(km[wd]);
+    int incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) { const int o = __shfl_up(incl, d, 64); if (lane >= d) incl += o; }
+    __syncthreads();
+    if (lane == 63) sc.wave_cnt[tid >> 6] = incl;
+    __syncthreads();
+    int at = incl - mine, total = 0;
+    for (int w = 0; w < SMP_THREADS / 64; ++w) { if (w < (tid >> 6)) at += sc.wave_cnt[w]; total += sc.wave_cnt[w]; }
+    if (total <= LIST) {
+        int* const list = reinterpret_cast<int*>(sc.hist.h32);
+#pragma unroll
+        for (int wd = 0; wd < 5; ++wd) {
+            uint32_t m = km[wd];
+            while (m) {
+                const int pos = wd * 32 + __ffs((int)m) - 1;
+                m &= m - 1;
+                list[at++] = ((pos >> 3) * SMP_THREADS + tid) * 8 + (pos & 7);
             }
-            const uint32_t bits = (i & 3) == 0 ? rr[0] : (i & 3) == 1 ? rr[1] : (i & 3) == 2 ? rr[2] : rr[3];
-            const float v = l / T + gumbel_from_bits(bits);
-            if (v > best || (v == best && i < besti)) { best = v; besti = i; }
+        }
+        __syncthreads();
+        constexpr int U = 4;
+        for (int n0 = tid; n0 < total; n0 += U * SMP_THREADS) {
+            int id[U]; float l[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                id[u] = list[min(n0 + u * SMP_THREADS, total - 1)];
+                l[u] = h16bits_to_f32(lrow[id[u]]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (n0 + u * SMP_THREADS >= total) continue;
+                const int i = id[u];
+                const uint4 r = philox4x32_10(make_uint4((uint32_t)(i >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
+                const uint32_t bits = (i & 3) == 0 ? r.x : (i & 3) == 1 ? r.y : (i & 3) == 2 ? r.z : r.w;
+                const float v = l[u] / T + gumbel_from_bits(bits);
+                if (v > best || (v == best && i < besti)) { best = v; besti = i; }
+            }
+        }
+    } else {
+        int gbase = -1; uint32_t rr[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int wd = 0; wd < 5; ++wd) {
+            uint32_t m = km[wd];
+            while (m) {
+                const int pos = wd * 32 + __ffs((int)m) - 1;
+                m &= m - 1;
+                const int i = ((pos >> 3) * SMP_THREADS + tid) * 8 + (pos & 7);
+                const float l = h16bits_to_f32(lrow[i]);
+                if ((i & ~3) != gbase) {
+                    gbase = i & ~3;
+                    const uint4 r = philox4x32_10(make_uint4((uint32_t)(gbase >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
+                    rr[0] = r.x; rr[1] = r.y; rr[2] = r.z; rr[3] = r.w;
+                }
+                const uint32_t bits = (i & 3) == 0 ? rr[0] : (i & 3) == 1 ? rr[1] : (i & 3) == 2 ? rr[2] : rr[3];
+                const float v = l / T + gumbel_from_bits(bits);
+                if (v > best || (v == best && i < besti)) { best = v; besti = i; }
+            }
         }
     }
     block_argmax(best, besti, sc.blk);
@@ -868,7 +929,7 @@ extern "C" int nvx_sample(const void* logits, int logits_is_f32, int64_t logits_
     if (batch == 0) return NVX_OK;
     NVX_REQUIRE(out_ids, NVX_EINVAL, "nvx_sample: null pointer");
     NVX_REQUIRE(batch <= 65535, NVX_EUNSUPPORTED, "nvx_sample: more than 65535 rows");
-    // slices per row: enough workgroups for two per compute unit, none without a workspace
+    // slices per row: at least two workgroups per compute unit, none without a workspace
     int n_split = 1;
     if (ws) {
         NVX_REQUIRE((reinterpret_cast<uintptr_t>(ws) & 7u) == 0, NVX_EINVAL, "nvx_sample: workspace must be 8-byte aligned");
@@ -876,6 +937,9 @@ extern "C" int nvx_sample(const void* logits, int logits_is_f32, int64_t logits_
         n_split = n_split < 1 ? 1 : (n_split > SMP_MAX_SPLIT ? SMP_MAX_SPLIT : n_split);
         NVX_REQUIRE(ws_bytes >= batch * n_split * 8, NVX_ENOSPACE, "nvx_sample: workspace too small (%lld < %lld bytes)",
                     (long long)ws_bytes, (long long)(batch * n_split * 8));
+        // more of them where the workspace allows: the rows without a filter may be few among the batch's, and only their slices work
+        const int64_t room = ws_bytes / (batch * 8), want = 2048 / batch < SMP_MAX_SPLIT ? 2048 / batch : SMP_MAX_SPLIT;
+        if (want > n_split) n_split = (int)(want < room ? want : (room > n_split ? room : n_split));
     }
     unsigned long long* winners = (unsigned long long*)ws;
     hipStream_t st = (hipStream_t)stream;
