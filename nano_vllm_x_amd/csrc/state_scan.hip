@@ -738,6 +738,8 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
     float keep = 1.f, put = 1.f, bottom = 1.f;
     if (KIND == SCAN_DECAY) keep = a.decay[hd];
     if (KIND == SCAN_MLSTM) {
+        // the gates are rounded before they meet their maximum: contracted into the exponents' subtractions, the larger one would not weigh exactly 1
+#pragma clang fp contract(off)
         const float* g = a.gates + b * 2 * a.heads;
         const float gi = a.cap * tanhf((g[hd] + a.gate_bias[hd]) / a.cap);
         const float gf = logsigmoid_f(a.cap * tanhf((g[a.heads + hd] + a.gate_bias[a.heads + hd]) / a.cap));
@@ -746,7 +748,7 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
         put = expf(gi - m_new);
         float nq = 0.f;
         for (int d = threadIdx.x; d < dim; d += 256) {          // (its own entries of sq and sk)
-            const float nn = keep * (cont ? a.N_in[at * dim + d] : 0.f) + put * sk[d];
+            const float nn = __builtin_fmaf(keep, cont ? a.N_in[at * dim + d] : 0.f, put * sk[d]);
             a.N[at * dim + d] = nn;
             nq += nn * sq[d];
         }
@@ -777,7 +779,7 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
                 const float kr = put * sk[r], qr = sq[r], kp = KIND == SCAN_GLA ? sa[r] : keep;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    s[u][i] = kp * s[u][i] + kr * val[i];
+                    s[u][i] = __builtin_fmaf(kp, s[u][i], kr * val[i]);      // (k v of 16-bit rows is exact: one rounding)
                     acc[i] += qr * s[u][i];
                 }
                 *reinterpret_cast<nvx_f32x4*>(Sp + (int64_t)r * vdim + e0) = s[u];
