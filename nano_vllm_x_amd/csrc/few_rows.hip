@@ -32,18 +32,20 @@ __device__ __forceinline__ void line_to_lds(const void* g, unsigned lds) {
 }
 
 // MT: tiles of 16 rows of x; DEPTH: pieces of 64 columns a wave has on their way.  k % 512 == 0, n % 16 == 0, rows <= 16 * MT.
-template <typename A, int MT, int NT, int DEPTH>
+template <typename A, int MT, int NT, int DEPTH, int GLU>
 __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __restrict__ x, int64_t x_stride, const A* __restrict__ w,
-                                                                const A* __restrict__ bias, void* __restrict__ y, int f32_out, int rows, int n, int k) {
+                                                                const A* __restrict__ bias, void* __restrict__ y, int f32_out, int rows, int n, int k,
+                                                                float limit, float alpha, float shift) {
+    static_assert(!GLU || NT == 2, "16 gate rows and the 16 up rows beside them");
     constexpr int PIECE = (NT + MT) * 2048, LOADS = 2 * (NT + MT);         // [16 NT rows of w | 16 MT rows of x], 128 bytes each
     static_assert(DEPTH * PIECE >= MT * NT * 1024, "the sums meet in the pieces' memory");
     __shared__ __align__(16) unsigned char smem[FR_WAVES * DEPTH * PIECE];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, n0 = blockIdx.x * 16 * NT;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, n0 = blockIdx.x * 16 * (GLU ? 1 : NT);
     const A* from[LOADS];                                                  // rows 8 i + lane / 8; the piece that belongs at place lane % 8
     const int r8 = lane >> 3, c = wave * 64 + ((lane & 7) ^ r8) * 8;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-        from[i] = i < 2 * NT ? w + (int64_t)(n0 + 8 * i + r8) * k + c : x + (int64_t)min(8 * (i - 2 * NT) + r8, rows - 1) * x_stride + c;   // (rows past the last are not stored)
+        from[i] = i < 2 * NT ? w + (int64_t)(n0 + (GLU && i >= 2 ? n / 2 - 16 : 0) + 8 * i + r8) * k + c : x + (int64_t)min(8 * (i - 2 * NT) + r8, rows - 1) * x_stride + c;   // (rows past the last are not stored)
     const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)smem + wave * DEPTH * PIECE;
     typedef __attribute__((address_space(3))) const nvx_u32x4 lds_u4;
     auto ask = [&](int t) {
@@ -89,7 +91,24 @@ __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __rest
         for (int j = 0; j < MT; ++j) part[wave][i * MT + j][lane] = acc[i][j];
     __syncthreads();
     // a lane of a tile has row l16 and the outputs 4 * quad .. 4 * quad + 3
-    if (wave < NT * MT) {
+    if constexpr (GLU != 0) {            // the projections rounded to the format, as the activation's own kernel reads them
+        if (wave < MT) {
+            nvx_f32x4 g = part[0][wave][lane], u = part[0][MT + wave][lane];
+#pragma unroll
+            for (int i = 1; i < FR_WAVES; ++i) { g += part[i][wave][lane]; u += part[i][MT + wave][lane]; }
+            const int r = 16 * wave + l16;
+            if (r < rows) {
+                typedef A vec4 __attribute__((ext_vector_type(4)));
+                vec4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float gr = (float)(A)g[i], ur = (float)(A)u[i];
+                    o[i] = (A)(GLU == 2 ? gelu_glu_act(gr, ur) : glu_act(gr, ur, limit, alpha, shift));
+                }
+                *reinterpret_cast<vec4*>((A*)y + (int64_t)r * (n / 2) + n0 + 4 * quad) = o;
+            }
+        }
+    } else if (wave < NT * MT) {
         nvx_f32x4 s = part[0][wave][lane];
 #pragma unroll
         for (int i = 1; i < FR_WAVES; ++i) s += part[i][wave][lane];
@@ -109,12 +128,15 @@ __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __rest
 // 16 rows, 16 against 64 rows of w: 9216 x 2048 11.7 / 11.9, 12288 x 2048 14.0 / 13.4, 32000 x 1024 18.2 / 14.6; at 32 rows, 16 against
 // 32: 4096 x 2048 7.4 / 8.1, 6144 x 1024 7.5 / 6.1, 8192 x 4096 21.0 / 18.0.
 template <typename A, int MT>
-static void launch_few_rows(const void* x, int64_t x_stride, const void* w, const void* bias, void* y, int f32_out, int rows, int n, int k, hipStream_t st) {
-#define NVX_FEW(N_, D_) hipLaunchKernelGGL((few_rows_kernel<A, MT, N_, D_>), dim3((unsigned)(n / (16 * N_))), dim3(FR_WAVES * 64), 0, st, (const A*)x, x_stride, \
-                                           (const A*)w, (const A*)bias, y, f32_out, rows, n, k)
-    if (n >= 12288 && n % 64 == 0) NVX_FEW(4, 1);
-    else if (MT == 2 && n > 4096 && n % 32 == 0) NVX_FEW(2, 2);
-    else NVX_FEW(1, 2);
+static void launch_few_rows(const void* x, int64_t x_stride, const void* w, const void* bias, void* y, int f32_out, int rows, int n, int k, int glu,
+                            float limit, float alpha, float shift, hipStream_t st) {
+#define NVX_FEW(N_, D_, G_) hipLaunchKernelGGL((few_rows_kernel<A, MT, N_, D_, G_>), dim3((unsigned)(n / (16 * N_))), dim3(FR_WAVES * 64), 0, st, (const A*)x, x_stride, \
+                                           (const A*)w, (const A*)bias, y, f32_out, rows, n, k, limit, alpha, shift)
+    if (glu == 1) NVX_FEW(2, 2, 1);
+    else if (glu == 2) NVX_FEW(2, 2, 2);
+    else if (n >= 12288 && n % 64 == 0) NVX_FEW(4, 1, 0);
+    else if (MT == 2 && n > 4096 && n % 32 == 0) NVX_FEW(2, 2, 0);
+    else NVX_FEW(1, 2, 0);
 #undef NVX_FEW
 }
 
@@ -123,9 +145,11 @@ static void launch_few_rows(const void* x, int64_t x_stride, const void* w, cons
 using namespace NVX_NS;
 
 // x (rows <= 32, k), rows x_stride elements apart; w (n, k) contiguous; bias (n) in the same format, or null; y (rows, n) contiguous, in the format or
-// float32.  k a multiple of 512, n of 16.
+// float32.  k a multiple of 512, n of 16.  glu 1 / 2: w is [gate | up] and y (rows, n / 2), in the format, is glu_act / gelu_glu_act of the two halves (n a
+// multiple of 32, no bias); what the activation's own launch costs is saved (3 us of 8 for 16 rows of 6144 x 1024).
 extern "C" int nvx_internal_few_rows(const void* x, int64_t x_stride, const void* w, const void* bias, void* y, int fmt, int f32_out, int64_t rows, int64_t n,
-                                     int64_t k, nvx_stream_t stream) {
+                                     int64_t k, int glu, float limit, float alpha, float shift, nvx_stream_t stream) {
+    NVX_REQUIRE(glu >= 0 && glu <= 2 && (glu == 0 || (n % 32 == 0 && !bias && !f32_out)), NVX_EINVAL, "nvx_internal_few_rows: gated products");
     NVX_REQUIRE(x && w && y, NVX_EINVAL, "nvx_internal_few_rows: null pointer");
     NVX_REQUIRE(rows > 0 && rows <= 32 && n > 0 && n % 16 == 0 && n < (1 << 28) && k > 0 && k % 512 == 0 && k < (1 << 28) && (fmt == 0 || fmt == 1), NVX_EUNSUPPORTED,
                 "nvx_internal_few_rows: sizes");
@@ -133,8 +157,8 @@ extern "C" int nvx_internal_few_rows(const void* x, int64_t x_stride, const void
     const hipStream_t st = (hipStream_t)stream;
 #define NVX_FEW_MT(A_)                                                                                                       \
     do {                                                                                                                     \
-        if (rows <= 16) launch_few_rows<A_, 1>(x, x_stride, w, bias, y, f32_out, (int)rows, (int)n, (int)k, st);             \
-        else launch_few_rows<A_, 2>(x, x_stride, w, bias, y, f32_out, (int)rows, (int)n, (int)k, st);        \
+        if (rows <= 16) launch_few_rows<A_, 1>(x, x_stride, w, bias, y, f32_out, (int)rows, (int)n, (int)k, glu, limit, alpha, shift, st); \
+        else launch_few_rows<A_, 2>(x, x_stride, w, bias, y, f32_out, (int)rows, (int)n, (int)k, glu, limit, alpha, shift, st); \
     } while (0)
     if (fmt == 0) NVX_FEW_MT(__bf16);
     else NVX_FEW_MT(_Float16);

@@ -12,6 +12,16 @@ __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 __device__ __forceinline__ float logsigmoid_f(float z) { return fminf(z, 0.0f) - log1pf(expf(-fabsf(z))); }
 
+// gated activations: min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, -limit, limit) + shift), and gelu_tanh(g) u
+__device__ __forceinline__ float glu_act(float g, float u, float limit, float alpha, float shift) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g * sigmoid_f(alpha * g) * (u + shift);
+}
+__device__ __forceinline__ float gelu_glu_act(float g, float u) {
+    return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
+}
+
 // sum over a workgroup of 256 threads; every thread gets the total.  `red` holds 4 floats; safe to call repeatedly.
 __device__ __forceinline__ float block256_sum(float v, float* red) {
     v = wave_sum(v);

@@ -188,12 +188,6 @@ __global__ __launch_bounds__(256) void moe_route_sigmoid_kernel(const float* __r
     }
 }
 
-__device__ __forceinline__ float glu_act(float g, float u, float limit, float alpha, float shift) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return g * sigmoid_f(alpha * g) * (u + shift);
-}
-
 // A token's experts row by row (float32, and sizes that fit no 16-byte loads).  w_gu: (experts, 2 * ff, width) rows [gate | up]; w_d: (experts, width, ff).  Two launches, both
 // with a workgroup per 32 weight rows so that a step of a few tokens still fills the chip: the hidden activations of every
 // (token, choice) pair into a float32 workspace, then the output rows summed over a token's choices.  A wave takes 8 rows; its
@@ -467,11 +461,6 @@ __global__ __launch_bounds__(256) void moe_scatter_rows_kernel(const A* __restri
     const float wt = wts ? wts[r] : 1.0f;
     A* o = xs + dst[r] * (int64_t)width;
     for (int c = threadIdx.x; c < width; c += 256) st_f(o, c, wt * ld_f(h, t * h_stride + c));
-}
-
-// gelu_tanh(g) u
-__device__ __forceinline__ float gelu_glu_act(float g, float u) {
-    return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
 }
 
 // y[r][j] = act(gu[r][j], gu[r][ff + j]) (times sigmoid(row_gate[r]) if given); GELU: gelu_tanh(g) u, the three constants are not read

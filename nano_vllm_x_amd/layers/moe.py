@@ -7,7 +7,7 @@ import torch
 from torch import nn
 
 from .. import ops
-from .linear import Linear
+from .linear import Linear, gated_rows_fit
 
 
 class DenseGLU(nn.Module):
@@ -20,6 +20,8 @@ class DenseGLU(nn.Module):
         self.down = Linear(ff, width, bias=False)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
+        if gated_rows_fit(h, self.gu_proj):
+            return self.down(ops.few_rows_glu(h, self.gu_proj.weight, self.limit, self.alpha, 1.0))
         return self.down(ops.moe_glu(self.gu_proj(h), self.limit, self.alpha, 1.0))
 
 
@@ -33,6 +35,8 @@ class GeluGLU(nn.Module):
         self.down = Linear(ff, width, bias=False)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
+        if gated_rows_fit(h, self.gu_proj):
+            return self.down(ops.few_rows_glu(h, self.gu_proj.weight, gelu=True))
         return self.down(ops.gelu_glu(self.gu_proj(h)))
 
 

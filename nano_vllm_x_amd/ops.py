@@ -1853,7 +1853,17 @@ def few_rows_product(x, w, bias=None, f32: bool = False):
     _need(few_rows_fits(x, w, bias), "few_rows_product: sizes and layouts of few_rows_fits")
     t, k, n = x.shape[0], x.shape[1], w.shape[0]
     y = torch.empty((t, n), dtype=F32 if f32 else x.dtype, device=x.device)
-    _lib.check(_lib.load().nvx_internal_few_rows(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(y), _fmt(x), int(f32), t, n, k, _stream()), "few_rows_product")
+    _lib.check(_lib.load().nvx_internal_few_rows(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(y), _fmt(x), int(f32), t, n, k, 0, 0.0, 0.0, 0.0, _stream()), "few_rows_product")
+    return y
+
+
+def few_rows_glu(x, w, limit: float = 0.0, alpha: float = 0.0, shift: float = 0.0, gelu: bool = False):
+    """moe_glu (or gelu_glu) of few_rows_product(x, w), w (2 ff, k) = gate | up, in one launch; ff a multiple of 16."""
+    _need(few_rows_fits(x, w) and w.shape[0] % 32 == 0, "few_rows_glu: sizes and layouts of few_rows_fits, ff a multiple of 16")
+    t, k, n = x.shape[0], x.shape[1], w.shape[0]
+    y = torch.empty((t, n // 2), dtype=x.dtype, device=x.device)
+    _lib.check(_lib.load().nvx_internal_few_rows(_ptr(x), x.stride(0), _ptr(w), None, _ptr(y), _fmt(x), 0, t, n, k, 2 if gelu else 1, float(limit), float(alpha),
+                                                 float(shift), _stream()), "few_rows_glu")
     return y
 
 

@@ -61,3 +61,17 @@ def test_what_the_kernel_does_not_take_goes_to_the_library():
     y = m(torch.randn(2, 1024, device="cuda").bfloat16().requires_grad_())      # under autograd as torch's own
     y.float().sum().backward()
     assert m.weight.grad is not None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,ff,k", [(1, 16, 512), (16, 3072, 1024), (17, 48, 1536), (32, 6144, 512)])
+def test_gated_product_equals_product_and_activation(rows, ff, k, dtype):
+    """The activation reads the projections rounded to the format either way: the same bits."""
+    from nano_vllm_x_amd import ops
+
+    x, w, _ = _case(rows, 2 * ff, k, dtype, rows + ff)
+    with torch.inference_mode():
+        gu = ops.few_rows_product(x, w)
+        assert torch.equal(ops.few_rows_glu(x, w, gelu=True), ops.gelu_glu(gu))
+        assert torch.equal(ops.few_rows_glu(x, w, 0.7, 1.702, 1.0), ops.moe_glu(gu, 0.7, 1.702, 1.0))
+        assert torch.equal(ops.few_rows_glu(x, w, float("inf"), 1.0, 0.0), ops.moe_glu(gu, float("inf"), 1.0, 0.0))
