@@ -193,6 +193,8 @@ class TableChoices(ctypes.Structure):
 INTERNAL = {name: (_c_i32, [ctypes.POINTER(PrefillStep), _c_vp]) for name in ("nvx_internal_prefill_step", "nvx_internal_prefill_step_f16")}
 INTERNAL["nvx_internal_table_choices"] = (_c_i32, [ctypes.POINTER(TableChoices), _c_i32, _c_vp, _c_i64, _c_vp])
 INTERNAL["nvx_internal_moe_decode"] = SIGNATURES["nvx_moe_expert_rows"]
+INTERNAL["nvx_internal_decode_boundary"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_vp, _c_f32, _c_vp, _c_vp, _c_vp, _c_vp])
+INTERNAL["nvx_internal_linear_decode_scaled"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_vp, _c_f32, _c_vp])
 INTERNAL["nvx_internal_few_rows"] = (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_vp, _c_i32, _c_i32, _c_i64, _c_i64, _c_i64, _c_i32, _c_f32, _c_f32, _c_f32, _c_vp])
 
 

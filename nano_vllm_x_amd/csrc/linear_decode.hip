@@ -18,6 +18,8 @@
 
 #include <stdlib.h>
 
+#include <type_traits>
+
 namespace NVX_NS {
 
 #define LIN_THREADS 512
@@ -29,6 +31,44 @@ __device__ __forceinline__ nvx_f32x4 mfma16(nvx_u32x4 a, nvx_u32x4 b, nvx_f32x4 
 
 // LDS slot (16 bytes each) of the A fragment piece: k-step j, lane quad q (k offset 8q), W row r.
 __device__ __forceinline__ int lin_slot(int j, int q, int r) { return j * 64 + q * 16 + (r ^ ((q << 2) | (j & 3))); }
+
+// 1 / rms of the rows of a workgroup's tiles of X, K unnormed columns, from the squares that the product in front left (decode_boundary.hip), PER columns a
+// sum: a wave reads 1 KB of them as they lie at a time (a lane a row and quarter of it is 64 separate requests an instruction, 0.7 us more of a 9 us
+// product).  The sums of a row meet in a binary tree over its columns, whatever PER.
+template <int K, int PER>
+struct LinScale {
+    static constexpr int SUMS = K / PER, LANES = SUMS / 4, AT_ONCE = 64 / LANES, LOADS = 16 / AT_ONCE;      // lanes of a row; rows of a load; loads of a tile
+    static constexpr int MAX = (PER == 8 ? 2 : 16) * LOADS / LIN_WAVES;                                      // loads of a wave: 8 columns a sum up to 32 rows
+    static_assert(LANES == 16 || LANES == 32, "sums of a row");
+    nvx_f32x4 part[MAX];
+    __device__ __forceinline__ void load(const float* __restrict__ squares, int tiles, int step, int first, int wave, int lane) {   // tiles first, first + step, ...
+#pragma unroll
+        for (int i = 0; i < MAX; ++i) {
+            const int c = wave + LIN_WAVES * i;
+            if (c < tiles * LOADS) part[i] = *reinterpret_cast<const nvx_f32x4*>(squares + (int64_t)(c / LOADS * step + first) * (16 * SUMS) + c % LOADS * 256 + lane * 4);
+        }
+    }
+    __device__ __forceinline__ void store(float* scale, int tiles, float eps, int wave, int lane) const {
+#pragma unroll
+        for (int i = 0; i < MAX; ++i) {
+            const int c = wave + LIN_WAVES * i;
+            if (c < tiles * LOADS) {
+                float t = (part[i][0] + part[i][1]) + (part[i][2] + part[i][3]);
+                t = quarter_sum(t);
+                if constexpr (LANES == 32) t += xor16(t);
+                if (lane % LANES == 0) scale[c / LOADS * 16 + c % LOADS * AT_ONCE + lane / LANES] = 1.0f / sqrtf(t / (float)K + eps);
+            }
+        }
+    }
+};
+// Products over the rms of x's rows sum K as decode_boundary.hip does, so that a row's result does not depend on the number of rows: eight chains, chain c
+// the blocks c, c + 8, ... of 64 columns, added up in order.
+__device__ __forceinline__ nvx_f32x4 lin_chains(const nvx_f32x4 (&acc)[8]) {
+    nvx_f32x4 s = acc[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) s += acc[i];
+    return s;
+}
 
 // MODE 0: y bf16 (M, N).  MODE 1: w rows [0, N/2) are gate rows, [N/2, N) up rows; y bf16 (M, N/2) =
 // bf16(bf16(silu(gate)) * up) on the bf16-rounded projections, as the unfused ops compute it.
@@ -45,11 +85,14 @@ __device__ __forceinline__ int lin_slot(int j, int q, int r) { return j * 64 + q
 // WIDE (modes 0 and 2): the workgroup owns 32 rows of W instead of 16, so half as many workgroups re-read
 // the activations from L2.  gridDim.z > 1 deals the 16-row tiles of X round-robin to that many workgroups
 // per W slice (their ids differ by a multiple of 8, so they share an XCD and its L2 copy of the slice).
-template <int MODE, int KC, bool STAGED, bool WIDE = false>
+// SQUARES (modes 0 and 1): x is unnormed and y the product over the rms of its rows, of whose squares `squares` has that many columns a sum.
+template <int MODE, int KC, bool STAGED, bool WIDE = false, int SQUARES = 0>
 __global__ __launch_bounds__(LIN_THREADS) void linear_decode_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, void* __restrict__ y, int m_rows, int n_rows,
-    int k_total) {
+    int k_total, const float* __restrict__ squares, float eps) {
     static_assert(!(WIDE && MODE == 1), "the gate/up mode already owns 32 rows of W");
+    constexpr bool SCALED = SQUARES > 0;
+    static_assert(!SCALED || MODE != 2, "partial products are summed before they are scaled");
     constexpr int HALVES = (MODE == 1 || WIDE) ? 2 : 1;
     constexpr int STEPS = KC / 32;               // MFMA k-steps per tile
     constexpr int GPT = STAGED ? STEPS / 8 : ((MODE == 1 && KC == 1024) ? 4 : (KC > 1024 ? KC / 512 : 2));   // groups per tile
@@ -95,6 +138,9 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_decode_kernel(
             for (int i = 0; i < GROUP; ++i) dst[i] = *reinterpret_cast<const nvx_u32x4*>(p + (i >> 1) * 64 + (i & 1) * 8);
         }
     };
+    __shared__ float scale[SCALED ? 256 : 1];
+    LinScale<SCALED ? KC : 1024, SCALED ? SQUARES : 16> sq;
+    if constexpr (SCALED) sq.load(squares, tiles, msplit, mz, wave, lane);
     if (n_items > 0) load_b(b_even, 0);
 
     // ---- W slice -> LDS, parked in operand order ---------------------------------------------------
@@ -115,16 +161,23 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_decode_kernel(
             lds[h * STEPS * 64 + lin_slot(2 * (kp >> 3) + (kp & 1), (kp >> 1) & 3, r)] = v[u];   // piece kp -> (k-step, quad)
         }
     }
+    if constexpr (SCALED) sq.store(scale, tiles, eps, wave, lane);
     __syncthreads();
 
     // ---- tiles of X ------------------------------------------------------------------------------
-    nvx_f32x4 acc[HALVES];
+    constexpr int CHAINS = SCALED ? 8 : 1;
+    nvx_f32x4 acc[HALVES], chain[HALVES][CHAINS];
     nvx_u32x4* my_stage = stage + (STAGED ? wave * (16 * 32) : 0);
-    auto compute = [&](const nvx_u32x4 (&bfrag)[GROUP], int item) {
-        const int tile = (wave + LIN_WAVES * (item / GPT)) * msplit + mz, g = item % GPT;
+    // (g, the group within the tile: a constant where chains are chosen by it)
+    auto compute = [&](const nvx_u32x4 (&bfrag)[GROUP], int item, auto g) __attribute__((always_inline)) {
+        const int local = wave + LIN_WAVES * (item / GPT), tile = local * msplit + mz;
         if (g == 0) {
 #pragma unroll
-            for (int h = 0; h < HALVES; ++h) acc[h] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int h = 0; h < HALVES; ++h) {
+                acc[h] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < CHAINS; ++c) chain[h][c] = acc[h];
+            }
         }
 #pragma unroll
         for (int i = 0; i < GROUP; ++i) {
@@ -136,10 +189,18 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_decode_kernel(
                 b = bfrag[i];
             }
 #pragma unroll
-            for (int h = 0; h < HALVES; ++h)
-                acc[h] = mfma16(lds[h * STEPS * 64 + lin_slot(g * GROUP + i, quad, l16)], b, acc[h]);
+            for (int h = 0; h < HALVES; ++h) {
+                const nvx_u32x4 a = lds[h * STEPS * 64 + lin_slot(g * GROUP + i, quad, l16)];
+                if constexpr (SCALED) chain[h][(g * GROUP + i) / 2 % 8] = mfma16(a, b, chain[h][(g * GROUP + i) / 2 % 8]);
+                else acc[h] = mfma16(a, b, acc[h]);
+            }
         }
         if (g != GPT - 1) return;
+        if constexpr (SCALED) {
+            const float inv = scale[local * 16 + l16];
+#pragma unroll
+            for (int h = 0; h < HALVES; ++h) acc[h] = lin_chains(chain[h]) * inv;
+        }
         // C layout: this lane holds X row (tile*16 + l16), W rows n0 + 4*quad + 0..3
         const int row = tile * 16 + l16;
         if (row >= m_rows) return;
@@ -168,26 +229,51 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_decode_kernel(
             }
         }
     };
-    if constexpr (STAGED) {
-        // per item: registers -> this wave's staging area, next item's loads into the freed registers,
-        // fragments back from LDS (a wave's LDS operations complete in order: no barrier needed)
-        for (int item = 0; item < n_items; ++item) {
+    // per item, staged: registers -> this wave's staging area, next item's loads into the freed registers,
+    // fragments back from LDS (a wave's LDS operations complete in order: no barrier needed)
+    auto staged_item = [&](int item, auto g) __attribute__((always_inline)) {
+        if constexpr (STAGED) {
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const int r = 2 * u + (lane >> 5);
                 my_stage[r * 32 + ((lane & 31) ^ r)] = b_even[u];
             }
             if (item + 1 < n_items) load_b(b_even, item + 1);
-            compute(b_even, item);
+            compute(b_even, item, g);
         }
+    };
+    if constexpr (SCALED) {
+        static_assert(GPT == 4, "groups of a tile");
+        for (int item = 0; item < n_items; item += GPT) {
+            auto pair = [&](auto g) __attribute__((always_inline)) {
+                constexpr int G = decltype(g)::value;
+                if constexpr (STAGED) {
+                    staged_item(item + G, g);
+                    __builtin_amdgcn_sched_barrier(0);       // (else the compiler reads all groups' operands first and spills them)
+                    staged_item(item + G + 1, std::integral_constant<int, G + 1>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    load_b(b_odd, item + G + 1);
+                    compute(b_even, item + G, g);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (item + G + 2 < n_items) load_b(b_even, item + G + 2);
+                    compute(b_odd, item + G + 1, std::integral_constant<int, G + 1>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            pair(std::integral_constant<int, 0>{});
+            pair(std::integral_constant<int, 2>{});
+        }
+    } else if constexpr (STAGED) {
+        for (int item = 0; item < n_items; ++item) staged_item(item, item % GPT);
     } else {
         // the next item's loads go in flight before the current item is multiplied
         for (int item = 0; item < n_items; item += 2) {
             if (item + 1 < n_items) load_b(b_odd, item + 1);
-            compute(b_even, item);
+            compute(b_even, item, item % GPT);
             if (item + 1 >= n_items) break;
             if (item + 2 < n_items) load_b(b_even, item + 2);
-            compute(b_odd, item + 1);
+            compute(b_odd, item + 1, (item + 1) % GPT);
         }
     }
 }
@@ -198,10 +284,10 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_decode_kernel(
 // K = 1024 would need 128 KB of LDS beside the 64 KB of staging areas, so W passes through LDS in two
 // halves of K and the accumulators live across them: each wave owns at most ONE tile of X
 // (tiles <= 8 * gridDim.z, checked by the host).
-template <int KC>
+template <int KC, int SQUARES = 0>
 __global__ __launch_bounds__(LIN_THREADS) void linear_gateup_wide_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, uint16_t* __restrict__ y, int m_rows,
-    int n_rows, int k_total) {
+    int n_rows, int k_total, const float* __restrict__ squares, float eps) {
     constexpr int KPH = 2, KP = KC / KPH;        // K phases, k per phase
     constexpr int STEPS = KP / 32, GROUPS = KP / 256;
     constexpr int PIECES_ROW = KP / 8, PIECES_Q = 16 * PIECES_ROW;
@@ -225,10 +311,20 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_gateup_wide_kernel(
             b[u] = *reinterpret_cast<const nvx_u32x4*>(x + (int64_t)row * x_stride + phase * KP + group * 256 + (lane & 31) * 8);
         }
     };
+    constexpr bool SCALED = SQUARES > 0;
+    constexpr int CHAINS = SCALED ? 8 : 1;
+    __shared__ float scale[SCALED ? 256 : 1];
+    LinScale<SCALED ? KC : 1024, SCALED ? SQUARES : 16> sq;
+    const int tiles = ((m_rows + 15) / 16 - (int)blockIdx.z + (int)gridDim.z - 1) / (int)gridDim.z;
+    if constexpr (SCALED) sq.load(squares, tiles, gridDim.z, blockIdx.z, wave, lane);
     if (has) load_x(0, 0);
-    nvx_f32x4 acc[4];
+    nvx_f32x4 acc[4], chain[4][CHAINS];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < 4; ++q) {
+        acc[q] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < CHAINS; ++c) chain[q][c] = acc[q];
+    }
 #pragma unroll
     for (int phase = 0; phase < KPH; ++phase) {
         if (phase) __syncthreads();           // every wave is done with the previous half of W
@@ -249,6 +345,7 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_gateup_wide_kernel(
                 const int r = ph / PIECES_ROW, kp = ph % PIECES_ROW;
                 lds[q * STEPS * 64 + lin_slot(2 * (kp >> 3) + (kp & 1), (kp >> 1) & 3, r)] = v[u];
             }
+            if constexpr (SCALED) if (phase == 0) sq.store(scale, tiles, eps, wave, lane);
         }
         __syncthreads();
         if (has) {
@@ -266,13 +363,21 @@ __global__ __launch_bounds__(LIN_THREADS) void linear_gateup_wide_kernel(
                     const int piece = 8 * (i >> 1) + 2 * quad + (i & 1);
                     const nvx_u32x4 bf = my_stage[l16 * 32 + (piece ^ l16)];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) acc[q] = mfma16(lds[q * STEPS * 64 + lin_slot(g * 8 + i, quad, l16)], bf, acc[q]);
+                    for (int q = 0; q < 4; ++q) {
+                        nvx_f32x4& to = SCALED ? chain[q][(phase * STEPS + g * 8 + i) / 2 % CHAINS] : acc[q];
+                        to = mfma16(lds[q * STEPS * 64 + lin_slot(g * 8 + i, quad, l16)], bf, to);
+                    }
                 }
             }
         }
     }
     const int row = tile * 16 + l16;
     if (!has || row >= m_rows) return;
+    if constexpr (SCALED) {
+        const float inv = scale[wave * 16 + l16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = lin_chains(chain[q]) * inv;
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         float o[4];
@@ -306,7 +411,8 @@ static int lin_wide_min_rows() { static int v = -1; if (v < 0) v = lin_env_int("
 static int lin_msplit() { static int v = -1; if (v < 0) { v = lin_env_int("NVX_LIN_MSPLIT", 2); if (v < 1 || v > 8) v = 2; } return v; }
 
 // rows from which the gate/up mode uses its 64-row kernel: 64 rows 8.2 vs 7.8 us, 123 rows 9.1 vs 9.7,
-// 176 rows 10.7 vs 12.2, 256 rows 12.3 vs 14.9 (two passes of W through LDS cost a barrier pair)
+// 176 rows 10.7 vs 12.2, 256 rows 12.3 vs 14.9 (two passes of W through LDS cost a barrier pair).  Over the rms the eight chains take its registers, and it is
+// used 32 rows later: a layer's four products with it and without, 112 rows 31.1 and 30.3, 160 rows 36.6 and 36.8, 256 rows 40.0 and 41.7.
 static int lin_gateup_wide_min_rows() { static int v = -1; if (v < 0) v = lin_env_int("NVX_LIN_GATEUP_WIDE_MIN", 112); return v; }
 
 static bool lin_chunk_ok(int64_t kc) { return kc == 512 || kc == 768 || kc == 1024; }
@@ -327,8 +433,8 @@ extern "C" int nvx_linear_decode_splits(int64_t n, int64_t k) {
 }
 #endif
 
-extern "C" int NVX_ENTRY(nvx_linear_decode)(const void* x, int64_t x_row_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k,
-                                 int mode, int k_splits, nvx_stream_t stream) {
+static int linear_decode(const void* x, int64_t x_row_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, int mode, int k_splits,
+                         const float* squares, float eps, nvx_stream_t stream) {
     NVX_REQUIRE(x && w && y, NVX_EINVAL, "nvx_linear_decode: null pointer");
     NVX_REQUIRE(m > 0 && m <= 256, NVX_EUNSUPPORTED, "nvx_linear_decode: 1..256 rows (got %lld); larger batches are a library GEMM", (long long)m);
     NVX_REQUIRE(mode >= 0 && mode <= 2, NVX_EINVAL, "nvx_linear_decode: mode must be 0, 1 or 2");
@@ -342,12 +448,13 @@ extern "C" int NVX_ENTRY(nvx_linear_decode)(const void* x, int64_t x_row_stride,
     NVX_REQUIRE(nvx_aligned16(x) && nvx_aligned16(w) && nvx_aligned16(y), NVX_EINVAL, "nvx_linear_decode: pointers must be 16-byte aligned");
     const int kc = (int)(k / k_splits);
     hipStream_t st = (hipStream_t)stream;
-    const bool staged = m > lin_staged_min_rows();
+    const bool staged = m > (squares && mode == 0 ? 32 : lin_staged_min_rows());
     const bool wide = mode != 1 && staged && !whole_k && lin_wide_min_rows() > 0 && m >= lin_wide_min_rows() && n_out % 32 == 0;
     const int msplit = wide && ((n_out / 32) * k_splits) % 8 == 0 ? lin_msplit() : 1;
     const dim3 grid((unsigned)(n_out / (wide ? 32 : 16)), (unsigned)k_splits, (unsigned)msplit);
-#define NVX_LIN(MODE, KC, ST, WD) hipLaunchKernelGGL((linear_decode_kernel<MODE, KC, ST, WD>), grid, dim3(LIN_THREADS), 0, st, (const uint16_t*)x, \
-                                                     x_row_stride, (const uint16_t*)w, y, (int)m, (int)n, (int)k)
+#define NVX_LIN_S(MODE, KC, ST, WD, SQ) hipLaunchKernelGGL((linear_decode_kernel<MODE, KC, ST, WD, SQ>), grid, dim3(LIN_THREADS), 0, st, (const uint16_t*)x, \
+                                                     x_row_stride, (const uint16_t*)w, y, (int)m, (int)n, (int)k, squares, eps)
+#define NVX_LIN(MODE, KC, ST, WD) NVX_LIN_S(MODE, KC, ST, WD, 0)
 #define NVX_LIN_KC(MODE, ST, WD) do { if (kc == 512) NVX_LIN(MODE, 512, ST, WD); else if (kc == 768) NVX_LIN(MODE, 768, ST, WD); else NVX_LIN(MODE, 1024, ST, WD); } while (0)
 #define NVX_LIN_ST(MODE) do { if (staged) NVX_LIN_KC(MODE, true, false); else NVX_LIN_KC(MODE, false, false); } while (0)
     const int64_t tiles = (m + 15) / 16;
@@ -356,18 +463,50 @@ extern "C" int NVX_ENTRY(nvx_linear_decode)(const void* x, int64_t x_row_stride,
         else { if (staged) NVX_LIN(0, 1536, true, false); else NVX_LIN(0, 1536, false, false); }
         return nvx_check_launch("nvx_linear_decode");
     }
-    if (mode == 1 && staged && lin_gateup_wide_min_rows() > 0 && m >= lin_gateup_wide_min_rows() && kc == 1024 && n_out % 32 == 0 &&
+    if (mode == 1 && staged && lin_gateup_wide_min_rows() > 0 && m >= lin_gateup_wide_min_rows() + (squares ? 32 : 0) && kc == 1024 && n_out % 32 == 0 &&
         (n_out / 32) % 8 == 0 && lin_msplit() == 2 && tiles <= 2 * LIN_WAVES) {
-        hipLaunchKernelGGL((linear_gateup_wide_kernel<1024>), dim3((unsigned)(n_out / 32), 1, 2), dim3(LIN_THREADS), 0, st,
-                           (const uint16_t*)x, x_row_stride, (const uint16_t*)w, (uint16_t*)y, (int)m, (int)n, (int)k);
+#define NVX_LIN_GW(SQ) hipLaunchKernelGGL((linear_gateup_wide_kernel<1024, SQ>), dim3((unsigned)(n_out / 32), 1, 2), dim3(LIN_THREADS), 0, st, \
+                           (const uint16_t*)x, x_row_stride, (const uint16_t*)w, (uint16_t*)y, (int)m, (int)n, (int)k, squares, eps)
+#ifndef NVX_F16
+        if (squares) NVX_LIN_GW(16); else
+#endif
+        NVX_LIN_GW(0);
+#undef NVX_LIN_GW
         return nvx_check_launch("nvx_linear_decode");
     }
+#ifndef NVX_F16
+    if (squares) {      // K is 1024, and mode 0 or 1
+        if (m <= 32) NVX_LIN_S(1, 1024, false, false, 8);
+        else if (wide) NVX_LIN_S(0, 1024, true, true, 16);
+        else if (mode == 0) NVX_LIN_S(0, 1024, true, false, 16);
+        else if (staged) NVX_LIN_S(1, 1024, true, false, 16);
+        else NVX_LIN_S(1, 1024, false, false, 16);
+        return nvx_check_launch("nvx_linear_decode");
+    }
+#endif
     if (wide) { if (mode == 0) NVX_LIN_KC(0, true, true); else NVX_LIN_KC(2, true, true); }
     else if (mode == 0) NVX_LIN_ST(0); else if (mode == 1) NVX_LIN_ST(1); else NVX_LIN_ST(2);
 #undef NVX_LIN_ST
 #undef NVX_LIN_KC
 #undef NVX_LIN
+#undef NVX_LIN_S
     return nvx_check_launch("nvx_linear_decode");
 }
+
+extern "C" int NVX_ENTRY(nvx_linear_decode)(const void* x, int64_t x_row_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k,
+                                 int mode, int k_splits, nvx_stream_t stream) {
+    return linear_decode(x, x_row_stride, w, y, m, n, k, mode, k_splits, nullptr, 0.f, stream);
+}
+
+#ifndef NVX_F16
+// mode 1, and from 33 rows on mode 0, over the rms of x's rows, k 1024; squares (rows up to a multiple of 32, k / 8 up to 32 rows, k / 16 from there) as
+// nvx_internal_decode_boundary leaves them
+extern "C" int nvx_internal_linear_decode_scaled(const void* x, const void* w, void* y, int64_t m, int64_t n, int64_t k, int mode, const float* squares,
+                                                 float eps, nvx_stream_t stream) {
+    NVX_REQUIRE(squares && nvx_aligned16(squares) && (mode == 1 || (mode == 0 && m > 32)) && k == 1024, NVX_EINVAL,
+                "nvx_internal_linear_decode_scaled: arguments");
+    return linear_decode(x, k, w, y, m, n, k, mode, 1, squares, eps, stream);
+}
+#endif
 
 }  // namespace NVX_NS

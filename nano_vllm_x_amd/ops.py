@@ -187,10 +187,14 @@ def linear_decode_splits(n: int, k: int) -> int:
     return int(_lib.load().nvx_linear_decode_splits(n, k))
 
 
-def linear_decode(x, w, mode: int = 0, k_splits: int = 1, out=None):
+def linear_decode(x, w, mode: int = 0, k_splits: int = 1, out=None, squares=None, eps: float = 0.0, residual=None, norm_weight=None):
     """x (m <= 256, k) bf16 times w (n, k)^T.  mode 0 -> bf16 (m, n); mode 1 -> SiluAndMul of the
-    [gate; up] projection, bf16 (m, n/2); mode 2 -> fp32 partials (k_splits, m, n) for rmsnorm_splitk."""
+    [gate; up] projection, bf16 (m, n/2); mode 2 -> fp32 partials (k_splits, m, n) for rmsnorm_splitk; mode 3 -> the product + `residual` with the norm
+    behind it left open: (that sum times norm_weight, the sum, the squares of its rows), the first and the last being x and `squares` of a product of mode 0
+    or 1, which then is of the normed rows (sizes: decode_boundary_fits)."""
     _dev(x, w, out)
+    if mode == 3 or squares is not None:
+        return _decode_boundary(x, w, mode, squares, eps, residual, norm_weight)
     _need(x.dim() == 2 and w.dim() == 2 and x.dtype in H16 and w.dtype == x.dtype, "linear_decode: 2-D bfloat16 or float16 operands")
     _need(x.stride(1) == 1 and w.is_contiguous() and x.shape[1] == w.shape[1], "linear_decode: layouts")
     m, k = x.shape
@@ -209,6 +213,37 @@ def linear_decode(x, w, mode: int = 0, k_splits: int = 1, out=None):
     lib = _lib.load()
     _lib.check(_fn(lib, "nvx_linear_decode", x.dtype)(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, mode, k_splits, _stream()), "nvx_linear_decode")
     return out
+
+
+BOUNDARY_ROWS = 256       # largest decode step whose norms ride on its products: what linear_decode takes
+
+
+def decode_boundary_fits(rows: int, hidden: int, attn_width: int, inter: int, dtype) -> bool:
+    """Whether a decode step's products may carry its residual sums and norms (linear_decode's mode 3, and modes 0 and 1 with squares)."""
+    return dtype == torch.bfloat16 and 0 < rows <= BOUNDARY_ROWS and hidden == 1024 and attn_width % 512 == 0 and inter % 512 == 0
+
+
+def _decode_boundary(x, w, mode, squares, eps, residual, norm_weight):
+    (m, k), n = x.shape, w.shape[0]
+    _need(mode in (0, 1, 3) and x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and w.shape[1] == k, "linear_decode: bfloat16, contiguous operands")
+    lib, padded = _lib.load(), (m + 31) // 32 * 32
+    if mode == 3:
+        _dev(x, residual, norm_weight)
+        _need(squares is None and residual.shape == (m, n) and norm_weight.shape == (n,) and all(t.dtype == x.dtype and t.is_contiguous() for t in (residual, norm_weight)),
+              "linear_decode: residual, norm weight")
+        y, new, left = torch.empty_like(residual), torch.empty_like(residual), torch.empty((padded, n // (8 if m <= 32 else 16)), dtype=torch.float32, device=x.device)
+        _lib.check(lib.nvx_internal_decode_boundary(_ptr(x), _ptr(w), _ptr(y), m, n, k, 2, _ptr(left), 0.0, _ptr(residual), _ptr(norm_weight), _ptr(new), _stream()),
+                   "linear_decode")
+        return y, new, left
+    _dev(x, squares)
+    _need(squares.dtype == torch.float32 and squares.is_contiguous() and squares.shape == (padded, k // (8 if m <= 32 else 16)), "linear_decode: squares")
+    y = torch.empty((m, n // 2 if mode else n), dtype=x.dtype, device=x.device)
+    if m <= (16 if mode else 32):
+        rc = lib.nvx_internal_decode_boundary(_ptr(x), _ptr(w), _ptr(y), m, n, k, mode, _ptr(squares), float(eps), None, None, None, _stream())
+    else:
+        rc = lib.nvx_internal_linear_decode_scaled(_ptr(x), _ptr(w), _ptr(y), m, n, k, mode, _ptr(squares), float(eps), _stream())
+    _lib.check(rc, "linear_decode")
+    return y
 
 
 def rmsnorm_splitk(partials, weight, eps, residual=None):

@@ -23,7 +23,7 @@ from . import distributed as tpd
 from . import ops
 from .layers.activation import SiluAndMul
 from .core.common import ForwardMode
-from .layers.attention import Attention, PagedPrefillWrapper
+from .layers.attention import Attention, PagedDecodeWrapper, PagedPrefillWrapper
 from .layers.layernorm import RMSNorm
 from .layers.plain import as_written, bypassable, calls_are_plain, untouched, weight_of
 from .layers.rotary_embedding import RotaryEmbedding, build_cos_sin_cache
@@ -350,13 +350,35 @@ class Qwen3Model(nn.Module):
         if plain:
             return self._prefill(plain, input_ids, positions)
         hidden_states, residual = self.embed_tokens(input_ids), None
+        plain = self._plain_decode(hidden_states) if fused else None
+        if plain:
+            return self._decode(plain, hidden_states, positions)
         for layer in self.layers:
             hidden_states, residual = layer(positions, hidden_states, residual, fused)
         hidden_states, _ = self.norm(hidden_states, residual)
         return hidden_states
 
     def _plain_prefill(self):
-        """For a prefill step that _prefill may queue, the weights of every layer: (input norm, qkv, q norm, k norm, o, post-attention norm, gate | up,
+        return self._plain_layers(ForwardMode.PREFILL, PagedPrefillWrapper, "run")
+
+    def _plain_decode(self, x):
+        """_plain_layers of a decode step (embedding rows x) whose norms may ride on its products (_decode); else None."""
+        c = self.config
+        hidden, aw, inter = c.hidden_size, c.num_attention_heads * 128, c.intermediate_size
+        if not ops.decode_boundary_fits(x.shape[0], hidden, aw, inter, x.dtype) or x.shape[1:] != (hidden,) or not x.is_contiguous():
+            return None
+        plain = self._plain_layers(ForwardMode.DECODE, PagedDecodeWrapper, "run_qkv")
+        if not plain or not self.layers[0].self_attn.attn.attention_metadata.wrapper.qkv_fused:
+            return None
+        shapes = ((hidden,), (aw + 2 * c.num_key_value_heads * 128, hidden), (128,), (128,), (hidden, aw), (hidden,), (2 * inter, hidden), (hidden, inter))
+        for ws in plain:
+            if any(w.shape != shape or w.dtype is not x.dtype or not w.is_contiguous() or w.data_ptr() % 16 or w.numel() * 2 > DECODE_LINEAR_MAX_WEIGHT_BYTES
+                   for w, shape in zip(ws, shapes)):
+                return None
+        return plain
+
+    def _plain_layers(self, mode, wrapper_class, runs):
+        """For a step that _prefill or _decode may queue, the weights of every layer: (input norm, qkv, q norm, k norm, o, post-attention norm, gate | up,
         down).  Else None: one rank, the package's own attention wrapper and 16-bit projections, and every module of the stack as it was built
         (see layers/plain.py), with the numbers that all layers share."""
         layers = self.layers._modules.values()
@@ -379,7 +401,7 @@ class Qwen3Model(nn.Module):
                 return None
             if md is None:
                 md = attn.attention_metadata
-                if md is None or md.forward_mode != ForwardMode.PREFILL or type(md.wrapper) is not PagedPrefillWrapper or "run" in vars(md.wrapper):
+                if md is None or md.forward_mode != mode or type(md.wrapper) is not wrapper_class or runs in vars(md.wrapper):
                     return None
                 common = (a.num_heads, a.num_kv_heads, a.num_heads, attn.scaling, eps, eps, eps)
             if attn.attention_metadata is not md or a.rope_table is not rope \
@@ -428,6 +450,22 @@ class Qwen3Model(nn.Module):
             h, residual = ops.rmsnorm(F.linear(read_out, o), n2, eps, residual)
             hidden_states = F.linear(ops.silu_mul(F.linear(h, gate_up)), down)
         return ops.rmsnorm(hidden_states, final, eps, residual)[0]
+
+    def _decode(self, layers, residual, positions):
+        """What the module graph computes for a decode step (embedding rows `residual`), with the residual sums and norms between two products inside
+        these (csrc/decode_boundary.hip): two launches a layer fewer.  `layers`: as _plain_decode gives them."""
+        eps, attns = self.config.rms_norm_eps, [layer._modules["self_attn"]._modules["attn"] for layer in self.layers]
+        md = attns[0].attention_metadata
+        qkv = decode_linear(ops.rmsnorm(residual, layers[0][0], eps), layers[0][1], "qkv")
+        for i, ((_, _, nq, nk, o, n2, gate_up, down), attn) in enumerate(zip(layers, attns)):
+            md.wrapper._sm_scale = attn.scaling
+            read_out = md.wrapper.run_qkv(qkv, positions, self.rope_table, nq, nk, eps, md.kv_cache.get_kv_cache(attn.layer_id))
+            h, residual, squares = ops.linear_decode(read_out, o, mode=3, residual=residual, norm_weight=n2)
+            act = ops.linear_decode(h, gate_up, mode=1, squares=squares, eps=eps)
+            if i + 1 < len(layers):
+                h, residual, squares = ops.linear_decode(act, down, mode=3, residual=residual, norm_weight=layers[i + 1][0])
+                qkv = ops.linear_decode(h, layers[i + 1][1], mode=0, squares=squares, eps=eps)
+        return self.norm(decode_linear(act, down, "down"), residual)[0]
 
     def forward_stage(self, input_ids, positions, hidden_states, residual, fused: bool = True):
         """One pipeline stage.  The first stage embeds `input_ids` (hidden_states/residual are None), the
