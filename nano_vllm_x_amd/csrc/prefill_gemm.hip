@@ -1,4 +1,5 @@
-// Projections of prefill steps of few hundred tokens: y = x W^T in the 16-bit format, or SiluAndMul of a [gate | up] projection.
+// Projections of prefill steps: y = x W^T in the 16-bit format, SiluAndMul of a [gate | up] projection, or what becomes of a [q | k | v] projection
+// (NvxQkvOut); here the kernel for few hundred tokens and the choice between it and those for many (prefill_wide.hip).
 //
 // Such a product is a few microseconds of matrix work, and what decides its time is how many workgroups the tile leaves to 256 CUs and what a
 // workgroup does between two steps of K.  So the tile follows the size, a workgroup keeps STAGES - 1 steps of both operands on their way (memory
@@ -24,16 +25,17 @@ template <int N>
 __device__ __forceinline__ void wait_for_all_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
 // TM rows of x by TN rows of w a workgroup of four waves (WM of them along the rows of x), KS columns a step.  With SILU the TN rows of w are 16
-// gate and 16 up rows in turn, and the tile gives TN / 2 outputs.  m: rows of x; k % (2 * KS) == 0, n (rows of w) % TN == 0.
-template <int TM, int TN, int KS, int STAGES, int WM, bool SILU>
+// gate and 16 up rows in turn, and the tile gives TN / 2 outputs; with QKV a tile is one head.  m: rows of x; k % (2 * KS) == 0, n (rows of w) % TN == 0.
+template <int TM, int TN, int KS, int STAGES, int WM, int MODE>
 __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w,
-                                                          uint16_t* __restrict__ y, int m, int n, int k) {
+                                                          uint16_t* __restrict__ y, int m, int n, int k, const NvxQkvOut qkv) {
+    constexpr bool SILU = MODE == NVX_PG_SILU;
     constexpr int WN = 4 / WM, FM = TM / WM / 16, FN = TN / WN / 16;       // fragments of a wave
     constexpr int PIECES = KS / 8, AT_ONCE = 64 / PIECES;                  // 16-byte pieces of a row; rows of one copy
     static_assert(PIECES <= 16, "fragments of 16 rows share a swizzle");
     constexpr int ROWS = TM + TN, LOADS = ROWS / AT_ONCE / 4;              // copies of a wave a step
     constexpr int STAGE = ROWS * KS * 2;
-    static_assert(ROWS % (4 * AT_ONCE) == 0 && (!SILU || FN % 2 == 0) && (STAGES - 1) * LOADS < 64, "tile");
+    static_assert(ROWS % (4 * AT_ONCE) == 0 && (!SILU || FN % 2 == 0) && (MODE != NVX_PG_QKV || TN == 128) && (STAGES - 1) * LOADS < 64, "tile");
     constexpr int OUT = SILU ? TN / 2 : TN, LO = OUT + 8;                  // outputs of a row; elements of a row in LDS
     static_assert(TM * LO * 2 <= STAGES * STAGE, "the results turn around in the stages' memory");
     __shared__ __align__(16) unsigned char smem[STAGES * STAGE];
@@ -126,6 +128,13 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
         }
     }
     __syncthreads();
+    if constexpr (MODE == NVX_PG_QKV) {
+        for (int r = threadIdx.x >> 4; r < TM && m0 + r < m; r += 16) {
+            const HalfQuad hq = load_half_quads(so + r * LO, l16);
+            qkv_head_out(hq, quarter_sum(qkv_lane_squares(hq)), l16, tn, m0 + r, qkv);
+        }
+        return;
+    }
     const int cols = SILU ? n / 2 : n;
     for (int p = threadIdx.x; p < TM * OUT / 8; p += 256) {
         const int r = p / (OUT / 8), c = p % (OUT / 8) * 8;
@@ -133,41 +142,79 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
     }
 }
 
-template <int TM, int TN, int KS, int STAGES, int WM, bool SILU>
-static void launch_prefill_gemm(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, hipStream_t st) {
+template <int TM, int TN, int KS, int STAGES, int WM, int MODE>
+static void launch_prefill_gemm(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, const NvxQkvOut* qkv, hipStream_t st) {
     const int64_t tiles = (m + TM - 1) / TM * (n / TN);
-    hipLaunchKernelGGL((prefill_gemm_kernel<TM, TN, KS, STAGES, WM, SILU>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, st, (const uint16_t*)x, x_stride,
-                       (const uint16_t*)w, (uint16_t*)y, (int)m, (int)n, (int)k);
+    hipLaunchKernelGGL((prefill_gemm_kernel<TM, TN, KS, STAGES, WM, MODE>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, st, (const uint16_t*)x, x_stride,
+                       (const uint16_t*)w, (uint16_t*)y, (int)m, (int)n, (int)k, MODE == NVX_PG_QKV ? *qkv : NvxQkvOut{});
 }
 
 }  // namespace NVX_NS
 
 using namespace NVX_NS;
 
-static bool nvx_prefill_gemm_fits(int64_t n, int64_t k) { return n > 0 && k > 0 && n % 128 == 0 && k % 256 == 0; }
+struct PrefillTile { int m, n, slots; float us, us_silu; };
+// Tiles of many rows: workgroups that run at once, us of 1024 columns of K with the chip full of them (SILU: 64 x 128 in two stages, three a CU)
+static const PrefillTile PREFILL_TILES[] = {{256, 256, 256, 26.f, 26.f}, {192, 256, 256, 20.f, 20.f}, {128, 256, 256, 15.5f, 15.5f}, {128, 128, 256, 8.4f, 8.4f}, {64, 128, 512, 10.5f, 13.5f}};
 
-// The smallest tile whose workgroups all run at once (256 CUs; two a CU for 64 x 64 and for the last) is the fastest at every size measured: us at
+// Few rows: the smallest tile whose workgroups all run at once (256 CUs; two a CU for 64 x 64) is the fastest at every size measured: us at
 // 459 rows of 1024 outputs from 2048 columns, 240 workgroups of 32 x 64: 7.9, 480 of 32 x 32: 8.4, 128 of 64 x 64: 9.9; 300 rows of 4096
-// outputs from 1024, 320 of 64 x 64: 8.8, 640 of 32 x 64: 13.6.  Beyond, 64 x 64 in fewer stages (four workgroups a CU) up to 1024 workgroups, then
-// 64 x 128 (700 rows of 6144, SiluAndMul: 18.6, 64 x 64 in two stages 23.5).
-int NVX_ENTRY(nvx_prefill_gemm)(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, bool silu, hipStream_t st) {
-    NVX_REQUIRE(nvx_prefill_gemm_fits(n, k) && m >= 0 && m < (1 << 24) && n < (1 << 24) && k < (1 << 24) && x_stride >= k && x_stride % 8 == 0, NVX_EUNSUPPORTED,
-                "nvx_prefill_gemm: sizes");
-    NVX_REQUIRE(nvx_aligned16(x) && nvx_aligned16(w) && nvx_aligned16(y), NVX_EINVAL, "nvx_prefill_gemm: pointers must be 16-byte aligned");
-    if (m == 0) return NVX_OK;
+// outputs from 1024, 320 of 64 x 64: 8.8, 640 of 32 x 64: 13.6.  With SILU 64 x 64 in two stages (four workgroups a CU) holds on to 800 workgroups (459 rows 12.2,
+// 128 x 128 13.5; 600 rows, 960 workgroups, 14.4 and 13.8).
+// More rows: rounds of a tile's workgroups times what a round costs, by which every tile is chosen somewhere; us of 4096 outputs from 1024 columns, the
+// chosen / 64 x 128: 700 rows 11.8 (128 x 128) / 12.9, 1536 rows 18.7 (128 x 256) / 20.5, 2160 rows 22 (192 x 256) / 30, 4096 rows 32 (256 x 256) / 45; with SILU
+// 6144 from 1024, 1536 rows 24 (192 x 256) / 27, 2160 rows 31 (256 x 256) / 39.
+// QKV: up to 512 rows, where a head's norm and rotation behind the product are less than their own launch (459 rows 12.4, product and launch 14; 1024 rows 17.6
+// and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).
+static int prefill_gemm_rule(int64_t m, int64_t n, bool silu, bool wide) {
     auto tiles = [&](int64_t tm, int64_t tn) { return (m + tm - 1) / tm * (n / tn); };
-    NVX_REQUIRE(tiles(64, 128) < (1ll << 30), NVX_EUNSUPPORTED, "nvx_prefill_gemm: too many tiles");
-    if (silu) {
-        if (tiles(32, 64) <= 256) launch_prefill_gemm<32, 64, 128, 4, 2, true>(x, x_stride, w, y, m, n, k, st);
-        else if (tiles(64, 64) <= 512) launch_prefill_gemm<64, 64, 64, 4, 2, true>(x, x_stride, w, y, m, n, k, st);
-        else if (tiles(64, 64) <= 1024) launch_prefill_gemm<64, 64, 64, 2, 2, true>(x, x_stride, w, y, m, n, k, st);
-        else launch_prefill_gemm<64, 128, 64, 2, 2, true>(x, x_stride, w, y, m, n, k, st);
-    } else {
-        if (tiles(32, 32) <= 256) launch_prefill_gemm<32, 32, 128, 4, 2, false>(x, x_stride, w, y, m, n, k, st);
-        else if (tiles(32, 64) <= 256) launch_prefill_gemm<32, 64, 128, 4, 2, false>(x, x_stride, w, y, m, n, k, st);
-        else if (tiles(64, 64) <= 512) launch_prefill_gemm<64, 64, 64, 4, 2, false>(x, x_stride, w, y, m, n, k, st);
-        else if (tiles(64, 64) <= 1024) launch_prefill_gemm<64, 64, 64, 2, 2, false>(x, x_stride, w, y, m, n, k, st);
-        else launch_prefill_gemm<64, 128, 64, 3, 2, false>(x, x_stride, w, y, m, n, k, st);
+    if (!silu && tiles(32, 32) <= 256) return NVX_PG_32_32;
+    if (tiles(32, 64) <= 256) return NVX_PG_32_64;
+    if (tiles(64, 64) <= 512) return NVX_PG_64_64;
+    if (silu && tiles(64, 64) <= 800) return NVX_PG_64_64_TWO;
+    int best = NVX_PG_64_128;
+    float least = 0.f;
+    for (int i = 4; i >= 0; --i) {
+        const PrefillTile& t = PREFILL_TILES[i];
+        if (n % t.n || (i < 4 && !wide)) continue;
+        const int slots = silu && i == 4 ? 768 : t.slots;
+        const float cost = (float)((tiles(t.m, t.n) + slots - 1) / slots) * (silu ? t.us_silu : t.us);
+        if (i == 4 || cost < least) best = NVX_PG_256_256 + i, least = cost;
     }
+    return best;
+}
+
+// tile: one of NVX_PG_*, or 0 by the rule
+static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, int mode, const NvxQkvOut* qkv, hipStream_t st) {
+    NVX_REQUIRE(mode >= NVX_PG_PLAIN && mode <= NVX_PG_QKV && n > 0 && k > 0 && n % 128 == 0 && k % 256 == 0 && m >= 0 && m < (1 << 24) && n < (1 << 24) && k < (1 << 24) &&
+                x_stride >= k && x_stride % 8 == 0, NVX_EUNSUPPORTED, "nvx_prefill_gemm: sizes");
+    NVX_REQUIRE(mode != NVX_PG_QKV || (qkv && n == (int64_t)(qkv->hq + 2 * qkv->hkv) * 128), NVX_EINVAL, "nvx_prefill_gemm: heads");
+    NVX_REQUIRE(x && w && (y || mode == NVX_PG_QKV) && nvx_aligned16(x) && nvx_aligned16(w) && nvx_aligned16(y), NVX_EINVAL, "nvx_prefill_gemm: pointers must be 16-byte aligned");
+    if (m == 0) return NVX_OK;
+    NVX_REQUIRE((m + 31) / 32 * (n / 32) < (1ll << 30), NVX_EUNSUPPORTED, "nvx_prefill_gemm: too many tiles");
+    const bool silu = mode == NVX_PG_SILU;
+    if (mode == NVX_PG_QKV) tile = NVX_PG_32_128;
+    else if (tile == 0) tile = prefill_gemm_rule(m, n, silu, x_stride < (1 << 21) && n * k < (1ll << 30));       // (what the wide tiles' offsets hold)
+    if (tile >= NVX_PG_256_256 && tile < NVX_PG_64_128)
+        return NVX_ENTRY(nvx_prefill_wide)(x, x_stride, w, y, m, n, k, silu, PREFILL_TILES[tile - NVX_PG_256_256].m, PREFILL_TILES[tile - NVX_PG_256_256].n, st);
+#define NVX_PG(TM, TN, KS, ST, MODE) launch_prefill_gemm<TM, TN, KS, ST, 2, MODE>(x, x_stride, w, y, m, n, k, qkv, st)
+    switch (tile) {
+        case NVX_PG_64_128: if (silu) NVX_PG(64, 128, 64, 2, NVX_PG_SILU); else NVX_PG(64, 128, 64, 3, NVX_PG_PLAIN); break;
+        case NVX_PG_64_64: if (silu) NVX_PG(64, 64, 64, 4, NVX_PG_SILU); else NVX_PG(64, 64, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_32_64: if (silu) NVX_PG(32, 64, 128, 4, NVX_PG_SILU); else NVX_PG(32, 64, 128, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_64_64_TWO: NVX_REQUIRE(silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(64, 64, 64, 2, NVX_PG_SILU); break;
+        case NVX_PG_32_32: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 32, 128, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_32_128: NVX_REQUIRE(mode == NVX_PG_QKV, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 128, 64, 4, NVX_PG_QKV); break;
+        default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);
+    }
+#undef NVX_PG
     return nvx_check_launch("nvx_prefill_gemm");
+}
+int NVX_ENTRY(nvx_prefill_gemm)(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, int mode, const NvxQkvOut* qkv, hipStream_t st) {
+    return prefill_gemm(0, x, x_stride, w, y, m, n, k, mode, qkv, st);
+}
+// one product, PLAIN or SILU, by a tile of the caller's choice (0: the rule's)
+extern "C" int NVX_ENTRY(nvx_internal_prefill_gemm)(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, int silu, int tile,
+                                                    nvx_stream_t stream) {
+    return prefill_gemm(tile, x, x_stride, w, y, m, n, k, silu ? NVX_PG_SILU : NVX_PG_PLAIN, nullptr, (hipStream_t)stream);
 }

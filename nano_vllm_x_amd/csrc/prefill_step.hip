@@ -1,4 +1,4 @@
-// The layers of a Qwen3 prefill step of few tokens, queued by one call.  Host code: it launches the kernels that the module graph launches, in the
+// The layers of a Qwen3 prefill step, queued by one call.  Host code: it launches the kernels that the module graph launches, in the
 // same order, and is not part of the C ABI.
 //
 // Up to some thousand tokens the device needs less than 150 us for a layer and the host, through Python, 160 to queue it (220 where it calls
@@ -32,17 +32,23 @@ extern "C" int NVX_ENTRY(nvx_internal_prefill_step)(const NvxPrefillStep* s, nvx
     int turn = 0;
     for (int64_t l = 0; l < s->n_layers; ++l) {
         const int64_t* w = s->layers + 10 * l;
-        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[1], s->qkv, t, qw, hid, false, st));
-        NVX_STEP(NVX_ENTRY(nvx_qknorm_rope_store)(s->qkv, qw, s->positions, s->rope, s->rope_rows, (const void*)w[2], (const void*)w[3], eps, s->slots, s->q,
-                                                 (void*)w[8], (void*)w[9], s->n_slots, t, (int)s->hq, (int)s->hkv, stream));
+        if (t <= 512) {
+            const NvxQkvOut out = {s->positions, s->slots, s->rope, s->rope_rows, s->n_slots, (const uint16_t*)w[2], (const uint16_t*)w[3], (uint16_t*)s->q,
+                                   (uint16_t*)w[8], (uint16_t*)w[9], (int)s->hq, (int)s->hkv, eps};
+            NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[1], nullptr, t, qw, hid, NVX_PG_QKV, &out, st));
+        } else {
+            NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[1], s->qkv, t, qw, hid, NVX_PG_PLAIN, nullptr, st));
+            NVX_STEP(NVX_ENTRY(nvx_qknorm_rope_store)(s->qkv, qw, s->positions, s->rope, s->rope_rows, (const void*)w[2], (const void*)w[3], eps, s->slots, s->q,
+                                                     (void*)w[8], (void*)w[9], s->n_slots, t, (int)s->hq, (int)s->hkv, stream));
+        }
         NVX_STEP(NVX_ENTRY(nvx_paged_prefill)(s->q, aw, (const void*)w[8], (const void*)w[9], s->n_slots, s->qo_indptr, s->kv_indptr, s->kv_indices, s->plan,
                                              s->attn, t, s->batch, (int)s->hq, (int)s->hkv, (float)s->scale, stream));
-        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->attn, aw, (const void*)w[4], s->sum, t, hid, aw, false, st));
+        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->attn, aw, (const void*)w[4], s->sum, t, hid, aw, NVX_PG_PLAIN, nullptr, st));
         NVX_STEP(NVX_ENTRY(nvx_rmsnorm)(s->sum, hid, residual, (const void*)w[5], 0, s->h, res[turn], t, hid, eps, stream));
         residual = res[turn];
         turn ^= 1;
-        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[6], s->act, t, 2 * s->inter, hid, true, st));
-        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->act, s->inter, (const void*)w[7], s->sum, t, hid, s->inter, false, st));
+        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[6], s->act, t, 2 * s->inter, hid, NVX_PG_SILU, nullptr, st));
+        NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->act, s->inter, (const void*)w[7], s->sum, t, hid, s->inter, NVX_PG_PLAIN, nullptr, st));
         const bool last = l + 1 == s->n_layers;
         NVX_STEP(NVX_ENTRY(nvx_rmsnorm)(s->sum, hid, residual, last ? s->final_norm : (const void*)w[10], 0, last ? s->out : s->h, res[turn], t, hid, eps, stream));
         residual = res[turn];

@@ -138,7 +138,7 @@ def qknorm_rope_store(qkv, positions, cos_sin_cache, q_norm_weight, k_norm_weigh
 
 
 def prefill_step(layers, x, positions, cos_sin_cache, slots, qo_indptr, kv_indptr, kv_indices, plan_ws, final_norm, n_q_heads, n_kv_heads, eps, sm_scale):
-    """All layers of a Qwen3 prefill step of few tokens and the final norm, queued by one native call.
+    """All layers of a Qwen3 prefill step and the final norm, queued by one native call.
     `layers`: per layer (input norm, qkv, q norm, k norm, o, post-attention norm, gate | up, down, k rows, v rows); x (T, hidden) the embedding
     rows.  The sizes must be ones that prefill_step_fits accepts.  Returns the final-normed hidden states (T, hidden), or None for operands
     that the products do not read: weights and caches of other shapes (layers need not be alike) or types, strided, off a 16-byte border."""
@@ -181,6 +181,23 @@ def prefill_step(layers, x, positions, cos_sin_cache, slots, qo_indptr, kv_indpt
 def prefill_step_fits(hidden: int, n_q_heads: int, n_kv_heads: int, inter: int) -> bool:
     """Whether a model's projections are all ones that csrc/prefill_gemm.hip takes: rows of W in 128s, columns in 256s."""
     return hidden % 256 == 0 and inter % 256 == 0 and n_q_heads % 2 == 0 and n_q_heads % n_kv_heads == 0 and n_q_heads // n_kv_heads in (1, 2, 4, 8)
+
+
+def gated_product_fits(x, w) -> bool:
+    """Whether SiluAndMul of x W^T, w = [gate; up], is a product of csrc/prefill_gemm.hip that beats the library's and silu_mul: columns of up to 2048, behind
+    which SiluAndMul is the smaller part and the library's lead in the product (a tenth) the larger.  us, 15754 rows: 6144 x 1024 182, library 159 and 50."""
+    return x.dim() == 2 and w.dim() == 2 and x.dtype in H16 and w.dtype == x.dtype and x.is_cuda and w.device == x.device and 0 < x.shape[0] < 1 << 24 \
+        and x.shape[1] == w.shape[1] <= 2048 and w.shape[1] % 256 == 0 and w.shape[0] % 256 == 0 and x.is_contiguous() and w.is_contiguous() \
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.numel() < 1 << 30
+
+
+def gated_product(x, w):
+    """SiluAndMul of x (T, k) @ w (n, k).T, w = [gate; up], in x's format; see gated_product_fits."""
+    _need(gated_product_fits(x, w), "gated_product: sizes and layouts of gated_product_fits")
+    y = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype, device=x.device)
+    _lib.check(_fn(_lib.load(), "nvx_internal_prefill_gemm", x.dtype)(_ptr(x), x.stride(0), _ptr(w), _ptr(y), x.shape[0], w.shape[0], x.shape[1], 1, 0, _stream()),
+               "gated_product")
+    return y
 
 
 def linear_decode_splits(n: int, k: int) -> int:

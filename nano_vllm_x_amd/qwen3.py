@@ -95,9 +95,11 @@ DECODE_LINEAR_MAX_WEIGHT_BYTES = 16 << 20
 
 
 # Multiply-adds of a layer's projections up to which a prefill step is queued by one native call with the products of csrc/prefill_gemm.hip
-# (ops.prefill_step): 1525 tokens of Qwen3-0.6B (a step of 1536 takes 4250 us that way and 4600 from Python, one of 2048 5190 and 4870), 476 of Qwen3-1.7B,
-# 124 of Qwen3-8B (a layer's products at 64 rows: 115 us and the library's 120, at 216 rows 184 and 169).
-PREFILL_STEP_MAX_WORK = int(24e9)
+# (ops.prefill_step), with layers of up to 2048 and of more: 4450 tokens of Qwen3-0.6B, 1390 of Qwen3-1.7B, 124 of Qwen3-8B.  A layer's products, here and the
+# library's with silu_mul: 0.6B, us, 2160 tokens 96 and 115, 4096 tokens 140 and 149, 8000 tokens 228 and 238, 15754 tokens 437 and 432, with SiluAndMul's
+# product from here and the others the library's 221 and 407; up to some 4000 tokens the host is the slower from Python too.  8B, 64 tokens 115 and 120, 216 tokens
+# 184 and 169.
+PREFILL_STEP_MAX_WORK, PREFILL_STEP_MAX_WORK_WIDE = int(70e9), int(24e9)
 
 # NVX_FP32_LINEAR=1 (read when a model is built): every dense projection, the LM head included, multiplies in fp32 and
 # rounds its result to the model's 16-bit format once (the LM head's logits stay fp32).  Not a serving mode: it takes
@@ -420,7 +422,7 @@ class Qwen3Model(nn.Module):
 
     def _prefill(self, layers, input_ids, positions):
         """What the module graph computes for a prefill step, queued without calling the modules: a module call costs the host 3-5 us and a
-        layer has eleven.  Steps of few tokens go out in one native call (ops.prefill_step).  `layers`: as _plain_prefill gives them."""
+        layer has eleven.  Steps of up to some thousand tokens go out in one native call (ops.prefill_step).  `layers`: as _plain_prefill gives them."""
         cfg, first = self.config, self.layers[0].self_attn
         attns = [layer._modules["self_attn"]._modules["attn"] for layer in self.layers]
         md = attns[0].attention_metadata
@@ -428,7 +430,8 @@ class Qwen3Model(nn.Module):
         hidden_states, residual, t = self.embed_tokens(input_ids), None, input_ids.shape[0]
         hq, hkv, eps, final = first.num_heads, first.num_kv_heads, cfg.rms_norm_eps, weight_of(self.norm)
         work = t * (cfg.hidden_size * (2 * hq + 2 * hkv) * 128 + 3 * cfg.hidden_size * cfg.intermediate_size)
-        if work <= PREFILL_STEP_MAX_WORK and ops.prefill_step_fits(cfg.hidden_size, hq, hkv, cfg.intermediate_size):
+        long = work > (PREFILL_STEP_MAX_WORK if cfg.hidden_size <= 2048 else PREFILL_STEP_MAX_WORK_WIDE)
+        if not long and ops.prefill_step_fits(cfg.hidden_size, hq, hkv, cfg.intermediate_size):
             qo_indptr, kv_indptr, kv_indices, n_q, n_kv = wrapper._planned
             full = [(*ws, *cache.get_kv_cache(attn.layer_id)) for ws, attn in zip(layers, attns)]
             if (n_q, n_kv) == (hq, hkv) and hidden_states.shape == (t, cfg.hidden_size):
@@ -448,7 +451,8 @@ class Qwen3Model(nn.Module):
             wrapper._sm_scale = attn.scaling
             wrapper.run(q, (k_cache, v_cache), out=read_out)
             h, residual = ops.rmsnorm(F.linear(read_out, o), n2, eps, residual)
-            hidden_states = F.linear(ops.silu_mul(F.linear(h, gate_up)), down)
+            act = ops.gated_product(h, gate_up) if long and ops.gated_product_fits(h, gate_up) else ops.silu_mul(F.linear(h, gate_up))
+            hidden_states = F.linear(act, down)
         return ops.rmsnorm(hidden_states, final, eps, residual)[0]
 
     def _decode(self, layers, residual, positions):
