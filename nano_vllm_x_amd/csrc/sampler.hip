@@ -201,6 +201,20 @@ __device__ __forceinline__ unsigned long long shfl_up_u64(unsigned long long v, 
     return ((unsigned long long)hi << 32) | lo;
 }
 
+__device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int m) {
+    const unsigned int lo = __shfl_xor((unsigned int)v, m, 64), hi = __shfl_xor((unsigned int)(v >> 32), m, 64);
+    return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ unsigned long long shfl_quad_u64(unsigned long long v, int j) {      // lane j's of a quad of lanes
+    const unsigned int lo = __shfl((unsigned int)v, j, 4), hi = __shfl((unsigned int)(v >> 32), j, 4);
+    return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += shfl_xor_u64(v, m);
+    return v;
+}
+
 // tot[0..255] -> the first bin d with start + tot[0] + ... + tot[d] > target (255 if none): sel_digit = d,
 // sel_before = start + tot[0..d-1], sel_bucket = tot[d].  With want_total, z_total = sum of all bins and the
 // target is derived from it by `make_target` semantics below (top-p threshold).  Called by wave 0 only.
@@ -522,6 +536,9 @@ __device__ __forceinline__ void reduce_masses(FiltScratch& sc, int tid) {   // h
     if (part == 0) sc.tot[bin] = v;
 }
 
+// what every lane holds alike, in a scalar register
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
 template <bool PROBS>
 __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     const uint16_t* __restrict__ logits, int64_t row_stride, const float* __restrict__ temps, const int64_t* __restrict__ top_ks,
@@ -532,6 +549,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     uint4* const lds_row = reinterpret_cast<uint4*>(smp_dyn + ((sizeof(FiltScratch) + 15) & ~(size_t)15));
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const uint16_t* lrow = logits + row * row_stride;
+    auto alike = [](uint32_t v) { return PROBS ? v : uniform(v); };       // (where the registers are short)
     const float T = temps[row];
     const bool greedy = !(T > 0.0f);
     const int64_t k64 = top_ks[row];
@@ -588,6 +606,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 16; ++i) kmax = max(kmax, (uint32_t)sc.blk.ired[i]);
+    kmax = alike(kmax);
     const float lmax = logit_of_key(kmax);
     if (PROBS && greedy) {   // temperature <= 0: all mass on the first maximum
         int first = 0x7fffffff;
@@ -610,9 +629,127 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     unsigned int* const my32 = sc.hist.h32 + (lane & 31);
     unsigned long long* const my64 = sc.hist.h64 + (lane & 15);
 
-    // ---- top-k: key of the k-th largest score = ascending rank vocab - k ----
-    uint32_t k_key = 0;
-    if (k < vocab) {
+    // ---- both boundaries from one count: how often each of the 2048 largest scores (a row's positive ones, 16 powers of two down from the maximum)
+    // occurs, and each of as many negative ones from minus the maximum up.  Equal scores have equal masses, so count times mass, in integers, is what the
+    // tokens' own masses add up to; the few tokens of neither kind add theirs up in registers.  A boundary that is not among the largest is found in two
+    // passes each, as below.  us, 224 rows of 151 936 tokens, with two passes each and now: top-k 50 41 and 39, top-p 0.9 at temperature
+    // 0.6 81 and 52, at 1.0 107 and 70, both 58 and 44; a token's own mass is an exponential and a 64-bit atomic among ten bins where most meet. ----
+    constexpr int WINDOW = 2048;
+    static_assert(WINDOW == 2 * SMP_THREADS && sizeof(sc.hist) == WINDOW * 16, "a thread has two scores, of four counts each, or two of either kind, of two");
+    const bool k_on = k < vocab, p_on = top_p < 1.0f;
+    bool k_found = !k_on, p_found = !p_on;
+    uint32_t k_key = 0;                          // key of the k-th largest score: ascending rank vocab - k
+    uint32_t p_key = 0;                          // scores with key < p_key are dropped
+    unsigned long long before = 0, thr = 0;      // mass of kept scores strictly below p_key; the mass that may be dropped
+    if (!PROBS && (k_on || p_on)) {      // (beside the pass that writes the probabilities it takes registers that are not there)
+        const bool both = kmax >= 0x8000u + WINDOW;                        // (else no score is positive, and the largest are among the negative ones)
+        const uint32_t base = kmax >= WINDOW ? kmax - (WINDOW - 1) : 0, base_neg = both ? 0xffffu - kmax : base;
+        __syncthreads();
+        zero_hist();
+        __syncthreads();
+        unsigned long long below = 0;
+        if (k_on) {                              // (what lies below the largest is dropped: no count of it, and four counters a score)
+            unsigned int* const mine = sc.hist.h32 + (lane & 3);
+            each_pair([&](int, uint32_t kw) {
+                const uint32_t b0 = (kw & 0xffffu) - base, b1 = (kw >> 16) - base;
+                atomicAdd(mine + (b0 & (WINDOW - 1)) * 4, b0 < WINDOW ? 1u : 0u);
+                atomicAdd(mine + (b1 & (WINDOW - 1)) * 4, b1 < WINDOW ? 1u : 0u);
+            });
+        } else {
+            unsigned int* const mine = sc.hist.h32 + (lane & 1);
+            const uint32_t upper = both ? 0u : (uint32_t)WINDOW;
+            each_pair([&](int, uint32_t kw) {
+                const uint32_t k0 = kw & 0xffffu, k1 = kw >> 16;
+                const uint32_t b0 = k0 - (k0 & 0x8000u ? base : base_neg), b1 = k1 - (k1 & 0x8000u ? base : base_neg);
+                const uint32_t u0 = (k0 >> 4 & (uint32_t)WINDOW) | upper, u1 = (k1 >> 4 & (uint32_t)WINDOW) | upper;
+                atomicAdd(mine + ((b0 & (WINDOW - 1)) + u0) * 2, b0 < WINDOW ? 1u : 0u);
+                atomicAdd(mine + ((b1 & (WINDOW - 1)) + u1) * 2, b1 < WINDOW ? 1u : 0u);
+                if (__any(b0 >= WINDOW || b1 >= WINDOW)) {
+                    const uint32_t pr = pair_of_keys(kw);
+                    below += b0 >= WINDOW ? mass_fixed(h16lo_to_f32(pr), c1, c2m) : 0u;
+                    below += b1 >= WINDOW ? mass_fixed(h16hi_to_f32(pr), c1, c2m) : 0u;
+                }
+            });
+        }
+        __syncthreads();
+        // a thread has two neighbouring scores: how often they occur, or with `masses` what they weigh
+        const uint32_t key0 = base + 2 * (uint32_t)tid;
+        auto count_of = [&](int score) -> unsigned int {             // (from -WINDOW on: the negative ones)
+            if (k_on) return (sc.hist.h32[score * 4] + sc.hist.h32[score * 4 + 1]) + (sc.hist.h32[score * 4 + 2] + sc.hist.h32[score * 4 + 3]);
+            return sc.hist.h32[(WINDOW + score) * 2] + sc.hist.h32[(WINDOW + score) * 2 + 1];
+        };
+        auto mass_of = [&](uint32_t ky, unsigned int n) -> unsigned long long {
+            return n && ky >= k_key ? (unsigned long long)n * mass_fixed(logit_of_key(ky), c1, c2m) : 0ull;
+        };
+        auto of_score = [&](int q, bool masses) -> unsigned long long {
+            const unsigned int n = count_of(2 * tid + q);
+            return masses ? mass_of(key0 + q, n) : n;
+        };
+        auto sum_quads = [&](bool masses) {      // of the scores of four threads -> tot
+            unsigned long long v = of_score(0, masses) + of_score(1, masses);
+            v += shfl_xor_u64(v, 1);
+            v += shfl_xor_u64(v, 2);
+            if ((tid & 3) == 0) sc.tot[tid >> 2] = v;
+            if (tid == 0) { sc.found = -1; sc.z_total = 0; }
+            __syncthreads();
+        };
+        // among the eight scores of the quad that select_bin chose, the first up to which all add up to more than target
+        auto boundary = [&](bool masses, unsigned long long target) {
+            __syncthreads();
+            if ((unsigned)(tid >> 2) == sc.sel_digit) {
+                const unsigned long long v0 = of_score(0, masses), v1 = of_score(1, masses);
+                unsigned long long at = sc.sel_before;
+                for (int j = 0; j < 3; ++j) {
+                    const unsigned long long o = shfl_quad_u64(v0 + v1, j);
+                    if (j < (tid & 3)) at += o;
+                }
+                if (at <= target && at + v0 + v1 > target) {
+                    const bool second = at + v0 <= target;
+                    sc.found = (int)(key0 + (second ? 1 : 0));
+                    sc.sel_bucket = second ? at + v0 : at;
+                }
+            }
+            __syncthreads();
+        };
+        if (k_on) {
+            sum_quads(false);
+            const unsigned long long rank = (unsigned long long)(vocab - k);
+            if (tid < 64) {
+                const unsigned long long in = wave_sum_u64(sc.tot[4 * lane] + sc.tot[4 * lane + 1] + sc.tot[4 * lane + 2] + sc.tot[4 * lane + 3]);
+                select_bin(sc, (unsigned long long)vocab - in, rank, lane);
+            }
+            boundary(false, rank);
+            k_found = (int)alike(sc.found) >= 0;
+            k_key = k_found ? alike(sc.found) : 0;
+            __syncthreads();
+        }
+        if (p_on && k_found) {
+            if (!k_on && both)
+                for (int q = 0; q < 2; ++q) below += mass_of(base_neg + 2 * tid + q, count_of(2 * tid + q - WINDOW));
+            sum_quads(true);
+            below = wave_sum_u64(below);
+            if (lane == 0) atomicAdd(&sc.z_total, below);
+            __syncthreads();
+            if (tid < 64) {
+                const unsigned long long lower = sc.z_total;
+                const unsigned long long z = lower + wave_sum_u64(sc.tot[4 * lane] + sc.tot[4 * lane + 1] + sc.tot[4 * lane + 2] + sc.tot[4 * lane + 3]);
+                const double thr_d = (double)(1.0f - top_p) * (double)z;
+                unsigned long long t = thr_d <= 0.0 ? 0ull : (unsigned long long)thr_d;
+                if (t >= z) t = z > 0 ? z - 1 : 0;   // the largest score always survives
+                if (lane == 0) sc.thr = t;
+                select_bin(sc, lower, t, lane);
+            }
+            __syncthreads();
+            thr = sc.thr;
+            boundary(true, thr);
+            p_found = (int)alike(sc.found) >= 0;
+            p_key = p_found ? alike(sc.found) : 0;
+            before = sc.sel_bucket;
+        }
+    }
+
+    // ---- top-k by two passes of counts: the k-th largest score's high byte, then its low one ----
+    if (!k_found) {
         unsigned long long rank = (unsigned long long)(vocab - k);
         __syncthreads();
         zero_hist();
@@ -626,7 +763,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
         __syncthreads();
         if (tid < 64) select_bin(sc, 0ull, rank, lane);
         __syncthreads();
-        const uint32_t hi = sc.sel_digit;
+        const uint32_t hi = alike(sc.sel_digit);
         rank -= sc.sel_before;
         __syncthreads();
         zero_hist();
@@ -640,14 +777,13 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
         __syncthreads();
         if (tid < 64) select_bin(sc, 0ull, rank, lane);
         __syncthreads();
-        k_key = (hi << 8) | sc.sel_digit;
+        k_key = (hi << 8) | alike(sc.sel_digit);
     }
 
-    // ---- top-p: boundary of cumulative mass in ascending order ----
-    const bool p_on = top_p < 1.0f;
-    uint32_t p_key = 0;       // scores with key < p_key are dropped
-    int p_cut = -1;           // among scores with key == p_key, token ids < p_cut are dropped
-    if (p_on) {
+    // ---- top-p by two passes of masses: boundary of cumulative mass in ascending order ----
+    int p_cut = -1;           // among scores with key == p_key, token ids < p_cut are dropped: n_drop of them
+    int n_drop = 0;
+    if (!p_found) {
         __syncthreads();
         zero_hist();
         __syncthreads();
@@ -675,9 +811,9 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
             select_bin(sc, 0ull, thr, lane);
         }
         __syncthreads();
-        const uint32_t hi = sc.sel_digit;
-        unsigned long long before = sc.sel_before;   // mass of kept scores strictly below the current prefix
-        const unsigned long long thr = sc.thr;
+        const uint32_t hi = alike(sc.sel_digit);
+        before = sc.sel_before;                      // mass of kept scores strictly below the current prefix
+        thr = sc.thr;
         __syncthreads();
         zero_hist();
         __syncthreads();
@@ -697,13 +833,17 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
         __syncthreads();
         if (tid < 64) select_bin(sc, before, thr, lane);
         __syncthreads();
-        p_key = (hi << 8) | sc.sel_digit;
+        p_key = (hi << 8) | alike(sc.sel_digit);
         before = sc.sel_before;
+    }
+    if (p_on) {
         // ties at the boundary score: drop the lowest token ids while the running mass stays <= thr
         const unsigned long long pt = mass_fixed(logit_of_key(p_key), c1, c2m);   // equal scores have equal masses
         const unsigned long long room = thr >= before ? thr - before : 0;
-        const long long n_drop = pt > 0 ? (long long)(room / pt) : 0;
-        if (n_drop > 0) {
+        const long long fit = pt > 0 ? (long long)(room / pt) : 0;
+        n_drop = (int)alike(fit > vocab ? vocab : (int)fit);             // (as many as all of them: none is left)
+    }
+    auto cut_by_passes = [&]() {
             // token id of the tie with ascending-id rank n_drop.  Tokens are ordered (vector row j, thread, element):
             // ties per vector row -> the row holding that rank -> a scan over its threads -> the element.
             __syncthreads();
@@ -728,12 +868,13 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
             unsigned int tie_bits = 0;   // this thread's eight tokens of that row
             {
                 const int i0 = (jstar * SMP_THREADS + tid) * 8;
-                each_pair([&](int i, uint32_t kw) {
-                    if (i >= i0 && i < i0 + 8) {
-                        if ((kw & 0xffffu) == p_key) { tie_bits |= 1u << (i - i0); ++c; }
-                        if ((kw >> 16) == p_key) { tie_bits |= 2u << (i - i0); ++c; }
-                    }
-                });
+                if (i0 < vocab) {
+                    const uint4 v = keys_of_vec(*reinterpret_cast<const uint4*>(lrow + i0));
+                    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if ((w[e >> 1] >> (e & 1 ? 16 : 0) & 0xffffu) == p_key) { tie_bits |= 1u << e; ++c; }
+                }
             }
             int incl = c;
 #pragma unroll
@@ -748,9 +889,9 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
                     if ((tie_bits >> e) & 1u) { if (need == 0) { sc.found = (jstar * SMP_THREADS + tid) * 8 + e; break; } --need; }
             }
             __syncthreads();
-            p_cut = sc.found >= 0 ? sc.found : vocab;
-        }
-    }
+            p_cut = (int)alike(sc.found) >= 0 ? (int)alike(sc.found) : vocab;
+    };
+    if (PROBS && n_drop > 0) cut_by_passes();
 
     auto kept_kp = [&](uint32_t ky, int i) -> bool {
         if (ky < k_key) return false;
@@ -802,17 +943,51 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     // Philox code once and reads their logits back from memory.  Four tokens share one Philox block; its counter
     // depends on the token alone, so skipping the blocks without a survivor changes no draw. ----
     uint32_t km[5] = {0, 0, 0, 0, 0};
-    each_pair([&](int i, uint32_t kw) {
+    // Where some of the ties at top-p's boundary are to be dropped they are all taken down on the way, and the id that parts them is found among the list (in LDS,
+    // the counts' memory), each against all; ties beyond it leave the draw again.  More than a thousand of them are parted by passes over the row.
+    int* const ties = reinterpret_cast<int*>(sc.hist.h32);
+    if (n_drop > 0) {
+        __syncthreads();
+        if (tid == 0) { sc.sel_digit = 0; sc.found = -1; }
+        __syncthreads();
+    }
+    const uint32_t lowest = alike(max(max(k_key, m_key), p_on ? p_key : 0u));       // kept, the boundary's ties among them
+    auto mark = [&](int i, uint32_t kw) __attribute__((always_inline)) {
         const int pos = (i / (SMP_THREADS * 8)) * 8 + (i & 7);
-        const bool a = kept(kw & 0xffffu, i), b = kept(kw >> 16, i + 1);
+        const bool a = (kw & 0xffffu) >= lowest, b = (kw >> 16) >= lowest;
         km[pos >> 5] |= ((a ? 1u : 0u) | (b ? 2u : 0u)) << (pos & 31);
+    };
+    if (n_drop > 0) each_pair([&](int i, uint32_t kw) {
+        mark(i, kw);
+        const bool ta = (kw & 0xffffu) == p_key, tb = (kw >> 16) == p_key;
+        if (ta || tb) {
+            const int first = (int)atomicAdd(&sc.sel_digit, (ta ? 1u : 0u) + (tb ? 1u : 0u));
+            if (first < SMP_THREADS) ties[first] = ta ? i : i + 1;
+            if (ta && tb && first + 1 < SMP_THREADS) ties[first + 1] = i + 1;
+        }
     });
+    else each_pair(mark);
+    if (n_drop > 0) {
+        __syncthreads();
+        const int n_ties = (int)sc.sel_digit;
+        if (n_ties <= SMP_THREADS) {
+            if (tid < n_ties) {
+                const int me = ties[tid];
+                int less = 0;
+                for (int j = 0; j < n_ties; ++j) less += ties[j] < me ? 1 : 0;
+                if (less == n_drop) sc.found = me;              // (ids differ: one thread)
+            }
+            __syncthreads();
+            p_cut = (int)alike(sc.found) >= 0 ? (int)alike(sc.found) : vocab;
+        } else cut_by_passes();
+    }
+    const uint32_t tie_bits = n_drop > 0 ? __float_as_uint(logit_of_key(p_key)) >> 16 : 0x10000u;      // as the row has it
     const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
     float best = -INFINITY; int besti = 0x7fffffff;
-    // Survivors that fit go into one list in LDS (the histogram's memory): a thread then draws its share of them, their logits' loads in flight
+    // Survivors that fit go into one list in LDS (the row's memory: it has been walked for the last time): a thread then draws its share of them, their logits' loads in flight
     // together, where a walk over its own takes as many round trips as the thread with the most survivors has (256 rows of 151 936 tokens, some 5000
-    // of each kept: 88 -> 83 us).  Where more survive the walk is the faster one: neighbours share a Philox block.
-    constexpr int LIST = (int)(sizeof(sc.hist) / sizeof(int));
+    // of each kept: 88 -> 83 us; 224 rows, 17 000 kept: 107 -> 92).  Where more survive the walk is the faster one: neighbours share a Philox block.
+    constexpr int LIST = (SMP_NV - SMP_NV_REG) * SMP_THREADS * 16 / (int)sizeof(int);      // 28 672
     int mine = 0;
 #pragma unroll
     for (int wd = 0; wd < 5; ++wd) mine += __popc(km[wd]);
@@ -825,7 +1000,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     int at = incl - mine, total = 0;
     for (int w = 0; w < SMP_THREADS / 64; ++w) { if (w < (tid >> 6)) at += sc.wave_cnt[w]; total += sc.wave_cnt[w]; }
     if (total <= LIST) {
-        int* const list = reinterpret_cast<int*>(sc.hist.h32);
+        int* const list = reinterpret_cast<int*>(lds_row);
 #pragma unroll
         for (int wd = 0; wd < 5; ++wd) {
             uint32_t m = km[wd];
@@ -838,20 +1013,20 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
         __syncthreads();
         constexpr int U = 4;
         for (int n0 = tid; n0 < total; n0 += U * SMP_THREADS) {
-            int id[U]; float l[U];
+            int id[U]; uint16_t l[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 id[u] = list[min(n0 + u * SMP_THREADS, total - 1)];
-                l[u] = h16bits_to_f32(lrow[id[u]]);
+                l[u] = lrow[id[u]];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (n0 + u * SMP_THREADS >= total) continue;
                 const int i = id[u];
+                if (n0 + u * SMP_THREADS >= total) continue;
                 const uint4 r = philox4x32_10(make_uint4((uint32_t)(i >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
                 const uint32_t bits = (i & 3) == 0 ? r.x : (i & 3) == 1 ? r.y : (i & 3) == 2 ? r.z : r.w;
-                const float v = l[u] / T + gumbel_from_bits(bits);
-                if (v > best || (v == best && i < besti)) { best = v; besti = i; }
+                const float v = h16bits_to_f32(l[u]) / T + gumbel_from_bits(bits);
+                if ((v > best || (v == best && i < besti)) && !(l[u] == tie_bits && i < p_cut)) { best = v; besti = i; }
             }
         }
     } else {
@@ -863,15 +1038,15 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
                 const int pos = wd * 32 + __ffs((int)m) - 1;
                 m &= m - 1;
                 const int i = ((pos >> 3) * SMP_THREADS + tid) * 8 + (pos & 7);
-                const float l = h16bits_to_f32(lrow[i]);
+                const uint16_t l = lrow[i];
                 if ((i & ~3) != gbase) {
                     gbase = i & ~3;
                     const uint4 r = philox4x32_10(make_uint4((uint32_t)(gbase >> 2), (uint32_t)row, (uint32_t)offset, (uint32_t)(offset >> 32)), key);
                     rr[0] = r.x; rr[1] = r.y; rr[2] = r.z; rr[3] = r.w;
                 }
                 const uint32_t bits = (i & 3) == 0 ? rr[0] : (i & 3) == 1 ? rr[1] : (i & 3) == 2 ? rr[2] : rr[3];
-                const float v = l / T + gumbel_from_bits(bits);
-                if (v > best || (v == best && i < besti)) { best = v; besti = i; }
+                const float v = h16bits_to_f32(l) / T + gumbel_from_bits(bits);
+                if ((v > best || (v == best && i < besti)) && !(l == tie_bits && i < p_cut)) { best = v; besti = i; }
             }
         }
     }

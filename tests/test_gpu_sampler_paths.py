@@ -34,6 +34,26 @@ def test_aligned_and_unaligned_rows_draw_the_same(vocab, rows):
         assert torch.equal(_draw(lg, T, k, p, m, 3), _draw(wide[:, :vocab], T, k, p, m, 3))
 
 
+@pytest.mark.parametrize("shape", ["negative", "nearly equal", "wide", "all equal", "few values", "infinite"])
+def test_boundaries_outside_the_largest_scores_draw_the_same(shape):
+    """Boundaries among the 2048 largest scores and below them, masses of neither kind, more than a thousand ties at the boundary, survivors that fill the list:
+    the general kernel's tokens."""
+    rows, vocab = 24, 65536
+    g = torch.Generator(device="cuda").manual_seed(len(shape))
+    x = torch.randn((rows, vocab), generator=g, device="cuda")
+    lg = {"negative": -x.abs() - 1e-4, "nearly equal": 1e-5 * x, "wide": torch.sign(x) * torch.exp(6 * x - 12), "all equal": 0 * x + 1.5, "few values": x.round(),
+          "infinite": torch.where(x > 4, float("inf"), torch.where(x < -2, float("-inf"), x))}[shape].to(torch.bfloat16)
+    wide = torch.empty((rows, vocab + 1), dtype=torch.bfloat16, device="cuda")
+    wide[:, :vocab] = lg
+    T = 0.05 + 0.25 * (torch.arange(rows, device="cuda") % 6).float()
+    off = lambda v, d=torch.float32: torch.full((rows,), v, dtype=d, device="cuda")
+    for k in (vocab, 3, 1000, 30000, vocab - 1):
+        for p in (1.0, 0.999, 0.9, 0.4, 1e-4):
+            for m in (0.0, 0.3):
+                a = (off(k, torch.int64), off(p), off(m))
+                assert torch.equal(_draw(lg, T, *a, 3), _draw(wide[:, :vocab], T, *a, 3)), (k, p, m)
+
+
 def test_min_p_keeps_the_tokens_of_its_ratio():
     """Among logits 0, -1, -2, ... at temperature 1 the ratio of a probability to the largest is e^-i: min_p between e^-3 and e^-2 leaves three tokens."""
     lg = torch.full((64, 1024), -100.0, device="cuda", dtype=torch.bfloat16)
