@@ -14,6 +14,7 @@
 // 8192 pairs over 8 experts of 1536 x 1024: up 93 us (560 TFLOP/s), down 54 (480), the weighted sum 8.6; the library's products with copy,
 // activation and sum took 270 for a layer, and its counts a wait of the host.
 #include "moe_dev.h"
+#include "wide_dev.h"
 
 namespace NVX_NS {
 
@@ -171,6 +172,138 @@ __global__ __launch_bounds__(256, 2) void moe_group_gemm_kernel(const A* __restr
     }
 }
 
+// The same products by tiles of TM pairs and TN rows of weights (up: 16 gate and 16 up rows in turn), with the walk of wide_dev.h.  k is a multiple of 64, of STAGES
+// steps at least, UP ? 2 * n_out : n_out of TN; an expert's weights and all rows of x are under 2 GB.  Up: the rows' numbers are looked up when their
+// tile is placed; down: an expert's rows lie together, and those past the last read zeros.
+// Over 8 experts of 1536 x 1024, us in one trace, the small tile's kernel / here by 256 x 256, 192 x 256, 128 x 128: 8192 pairs, up 86 / 74, 83, 83, down 52 / 50, 44, 46;
+// 5000 pairs 52 / 70, 59, 51 and 34 / 47, 44, 32; 3000 pairs 37 / 35, 31, 37 and 22 / 39, 33, 19; 200 pairs 18 / 33, 26, 16 and 18 / 30, 24, 14.  Of 3072 x 2048, 8192 pairs
+// 280 / 245, 250, 267 and 161 / 168, 159, 148.  (A round costs more than prefill_wide.hip's: the activation in float32 functions.)
+template <typename A>
+struct MoeWideArgs {
+    const A* x;
+    int64_t x_stride;
+    const int32_t* src;
+    int src_div;
+    const float* scale;
+    const int32_t* counts;
+    int n_exp;
+    const A* w;
+    int k, n_out;
+    float limit, alpha, shift;
+    void* out;
+};
+__device__ __forceinline__ nvx_f32x4 mfma16(nvx_u32x4 a, nvx_u32x4 b, nvx_f32x4 c, __bf16) {
+    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ nvx_f32x4 mfma16(nvx_u32x4 a, nvx_u32x4 b, nvx_f32x4 c, _Float16) {
+    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+}
+template <typename A, bool UP, int TM, int TN, int STAGES>
+__global__ __launch_bounds__(512) void moe_wide_kernel(const MoeWideArgs<A> a) {
+    constexpr int WN = 4, GROUP = 4;                                       // waves by the rows of w; tiles of pairs that share rows of w
+    typedef WideTile<TM, TN, STAGES, 2, WN> T;
+    constexpr int FM = T::FM, FN = T::FN, LOADS = T::LOADS;
+    constexpr int OUT = UP ? TN / 2 : TN, WOUT = OUT / WN, P = WOUT / 8, SIDE = UP ? 8 * 16 * WOUT * 2 : 0;
+    static_assert(!UP || (FN % 2 == 0 && (P & (P - 1)) == 0), "tile");
+    __shared__ __align__(16) unsigned char smem[STAGES * T::STAGE + SIDE];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    const int tiles_n = a.n_out / OUT;
+    // every lane an expert: running sums of rows and of tiles, this expert's included
+    const int cnt = lane < a.n_exp ? a.counts[lane] : 0;
+    int rows_to = cnt, tiles_to = (cnt + TM - 1) / TM;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+        const int r = __shfl_up(rows_to, s, 64), q = __shfl_up(tiles_to, s, 64);
+        if (lane >= s) { rows_to += r; tiles_to += q; }
+    }
+    const int total = __builtin_amdgcn_readlane(tiles_to, 63) * tiles_n, per = (total + 7) / 8;
+    const int last = min(((int)(blockIdx.x & 7) + 1) * per, total), stride = (int)(gridDim.x >> 3);
+    int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (t >= last) return;
+
+    const unsigned x_bytes = (unsigned)(2 * a.x_stride), w_bytes = 2u * (unsigned)a.k, l8 = lane >> 3, c8 = ((lane & 7) ^ l8) * 16;
+    int m0, tn, row0, n_rows;              // of the tile: its first pair and outputs, its expert's first pair and their number
+    wide_buffer xb, wb;
+    unsigned off[LOADS];
+    auto of_x = [&](int i) __attribute__((always_inline)) { return (wave * LOADS + (T::MIXED ? i : 0)) * 8 < TM; };
+    auto place = [&]() __attribute__((always_inline)) {
+        const int e = __popcll(__ballot(tiles_to * tiles_n <= t));
+        const int before = e ? __builtin_amdgcn_readlane(tiles_to, e - 1) : 0;
+        row0 = e ? __builtin_amdgcn_readlane(rows_to, e - 1) : 0;
+        n_rows = __builtin_amdgcn_readlane(cnt, e);
+        const int m_tiles = (n_rows + TM - 1) / TM, tl = t - before * tiles_n;
+        const int group = tl / (GROUP * tiles_n), gm = min(GROUP, m_tiles - group * GROUP), in = tl - group * GROUP * tiles_n;
+        m0 = (group * GROUP + in % gm) * TM, tn = in / gm;
+        if constexpr (UP) {
+            xb = wide_buffer_at(a.x, 0x7fffffff);
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                if (of_x(i)) off[i] = (unsigned)(a.src[row0 + min(m0 + (wave * LOADS + i) * 8 + (int)l8, n_rows - 1)] / a.src_div) * x_bytes + c8;
+        } else xb = wide_buffer_at(a.x + (int64_t)(row0 + m0) * a.x_stride, (int64_t)(n_rows - 1 - m0) * x_bytes + 2 * a.k);
+        wb = wide_buffer_at(a.w + ((int64_t)e * (UP ? 2 : 1) * a.n_out + (int64_t)tn * OUT) * a.k, 0x7fffffff);
+    };
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (wave * LOADS + i) * 8, rw = row - TM;
+        off[i] = of_x(i) ? (row + l8) * x_bytes + c8 : ((UP ? (rw >> 4 & 1) * a.n_out + (rw >> 5) * 16 + (rw & 15) : rw) + l8) * w_bytes + c8;
+    }
+    auto ask = [&](int i, int step, unsigned to) __attribute__((always_inline)) { wide_to_lds(of_x(i) ? xb : wb, off[i], (unsigned)step * (T::KS * 2), to); };
+    const int wm = wave / WN, wn = wave % WN;
+    int m_now = 0, tn_now = 0, row_now = 0, rows_now = 0;
+    auto finish = [&](nvx_f32x4 (&acc)[FN][FM]) __attribute__((always_inline)) {
+        const int r0 = m_now + wm * FM * 16;
+        if constexpr (UP) {
+            float f[FM];
+#pragma unroll
+            for (int j = 0; j < FM; ++j) f[j] = a.scale ? a.scale[a.src[row_now + min(r0 + j * 16 + l16, rows_now - 1)]] : 1.0f;
+            typedef A vec4 __attribute__((ext_vector_type(4)));
+            unsigned char* so = smem + STAGES * T::STAGE + wave * 16 * WOUT * 2;       // a wave turns 16 rows around at a time, in memory of its own
+#pragma unroll
+            for (int j = 0; j < FM; ++j) {
+#pragma unroll
+                for (int i = 0; i < FN; i += 2) {
+                    vec4 v;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float g = fminf(f[j] * acc[i][j][r], a.limit), u = fminf(fmaxf(f[j] * acc[i + 1][j][r], -a.limit), a.limit);
+                        v[r] = (A)(g * sigmoid_f(a.alpha * g) * (u + a.shift));
+                    }
+                    *reinterpret_cast<vec4*>(so + l16 * (WOUT * 2) + (((i + (quad >> 1)) ^ (l16 & (P - 1))) * 16) + (quad & 1) * 8) = v;
+                }
+                wide_lds_wait();
+#pragma unroll
+                for (int p = 0; p < (16 * P + 63) / 64; ++p) {
+                    const int r = (p * 64 + lane) / P, c = lane % P, m = r0 + j * 16 + r;
+                    if (r < 16 && m < rows_now)
+                        *reinterpret_cast<nvx_u32x4*>((A*)a.out + (int64_t)(row_now + m) * a.n_out + tn_now * OUT + wn * WOUT + c * 8) =
+                            *reinterpret_cast<const nvx_u32x4*>(so + r * (WOUT * 2) + ((c ^ (r & (P - 1))) * 16));
+                }
+                wide_lds_wait();
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < FM; ++j) {
+                const int m = r0 + j * 16 + l16;
+                float* at = (float*)a.out + (int64_t)(row_now + m) * a.n_out + tn_now * OUT + wn * WOUT + 4 * quad;
+                if (m < rows_now)
+#pragma unroll
+                    for (int i = 0; i < FN; ++i) *reinterpret_cast<nvx_f32x4*>(at + 16 * i) = acc[i][j];
+            }
+        }
+        return t < last;
+    };
+    place();
+    T::walk((unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)smem, a.k / T::KS, ask,
+            [&]() __attribute__((always_inline)) { m_now = m0, tn_now = tn, row_now = row0, rows_now = n_rows; },
+            [&]() __attribute__((always_inline)) {
+                t += stride;
+                if (t < last) place();
+            },
+            [](nvx_u32x4 w, nvx_u32x4 x, nvx_f32x4 c) __attribute__((always_inline)) { return mfma16(w, x, c, A{}); }, finish);
+}
+
 // out[t] = sum_k wts[t * top + k] * o[dst[t * top + k]]   (wts == null: ones), four columns a thread.  A choice of an expert that does not exist
 // (dst < 0) makes its token's result NaN: nothing on this path reads the choices on the host, and a number would pass for a result.
 template <typename A>
@@ -200,6 +333,35 @@ bool nvx_moe_grouped_fits(int fmt, int64_t n_exp, int64_t width, int64_t ff) {
     return fmt < 2 && n_exp <= 63 && width % GT == 0 && ff % 64 == 0;
 }
 
+template <typename A, bool UP, int TM, int TN, int STAGES>
+static void launch_moe_wide(const MoeWideArgs<A>& a, int64_t m_tiles, hipStream_t st) {
+    const int64_t tiles = m_tiles * (a.n_out / (UP ? TN / 2 : TN));
+    hipLaunchKernelGGL((moe_wide_kernel<A, UP, TM, TN, STAGES>), dim3((unsigned)(tiles < 256 ? (tiles + 7) / 8 * 8 : 256)), dim3(512), 0, st, a);      // (a workgroup a CU)
+}
+
+// One of the two products.  Tile: the fewest rounds of workgroups times what a round costs (us of 1024 columns), an expert's last tile taken as half full; the
+// small tile of four waves, two workgroups a CU, where none of the wide ones fits.
+template <typename A, bool UP>
+static void launch_moe_product(const MoeWideArgs<A>& a, int64_t pairs, int64_t n_tok, hipStream_t st) {
+    const int64_t n = UP ? 2 * (int64_t)a.n_out : a.n_out, live = a.n_exp < pairs ? a.n_exp : pairs;      // (experts that may have pairs)
+    auto most = [&](int64_t tm) { return pairs / tm + live; };                                           // as many tiles as the counts can ask for
+    const bool fits = a.k >= 256 && a.x_stride < (1 << 21) && n_tok * a.x_stride < (1ll << 30) && n * a.k < (1ll << 30);
+    const struct { int m, n; float us; } tiles[] = {{256, 256, 34.f}, {192, 256, 28.f}, {128, 128, 10.8f}};
+    int best = -1;
+    float least = 0.f;
+    for (int i = 0; fits && i < 3; ++i) {
+        if (n % tiles[i].n) continue;
+        const int64_t m2 = 2 * pairs / tiles[i].m + live, m = m2 / 2 > live ? m2 / 2 : live;
+        const float cost = (float)((m * (n / tiles[i].n) + 255) / 256) * tiles[i].us;
+        if (best < 0 || cost < least) best = i, least = cost;
+    }
+    if (best == 0) launch_moe_wide<A, UP, 256, 256, 2>(a, most(256), st);
+    else if (best == 1) launch_moe_wide<A, UP, 192, 256, 2>(a, most(192), st);
+    else if (best == 2) launch_moe_wide<A, UP, 128, 128, 4>(a, most(128), st);
+    else hipLaunchKernelGGL((moe_group_gemm_kernel<A, UP>), dim3((unsigned)((most(GT) * (a.n_out / (UP ? GT / 2 : GT)) + 7) / 8 * 8)), dim3(256), 0, st, a.x, a.x_stride, a.src,
+                            a.src_div, a.scale, a.counts, a.n_exp, a.w, a.k, a.n_out, a.limit, a.alpha, a.shift, a.out);
+}
+
 // The whole mixture (see nvx_moe_expert_rows) for a step of many tokens; ws as there.  The pairs' order is made here too.
 int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
                     int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
@@ -213,18 +375,14 @@ int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx
     int32_t* src = reinterpret_cast<int32_t*>(dst + pairs);
     int32_t* counts = src + pairs;
     if (const int rc = nvx_moe_order_pairs(idx, pairs, n_exp, dst, src, counts, st)) return rc;
-    // as many workgroups as the counts can ask for: an expert's last tile may hold one pair
     const int64_t m_tiles = pairs / GT + (n_exp < pairs ? n_exp : pairs);
-    const int64_t up = (m_tiles * (ff / (GT / 2)) + 7) / 8 * 8, down = (m_tiles * (width / GT) + 7) / 8 * 8;
-    NVX_REQUIRE(up < (1ll << 31) && down < (1ll << 31), NVX_EINVAL, "nvx_moe_expert_rows: too many tiles");
+    NVX_REQUIRE(m_tiles * (ff / (GT / 2)) < (1ll << 30) && m_tiles * (width / GT) < (1ll << 30), NVX_EINVAL, "nvx_moe_expert_rows: too many tiles");
 #define NVX_GROUPED(A_)                                                                                                                            \
     do {                                                                                                                                           \
-        hipLaunchKernelGGL((moe_group_gemm_kernel<A_, true>), dim3((unsigned)up), dim3(256), 0, st, (const A_*)h, h_stride, (const int32_t*)src,   \
-                           (int)top, weight_out ? (const float*)nullptr : wts, (const int32_t*)counts, (int)n_exp, (const A_*)w_gu, (int)width,    \
-                           (int)ff, limit, alpha, shift, (void*)y);                                                                                \
-        hipLaunchKernelGGL((moe_group_gemm_kernel<A_, false>), dim3((unsigned)down), dim3(256), 0, st, (const A_*)y, ff, (const int32_t*)nullptr,  \
-                           1, (const float*)nullptr, (const int32_t*)counts, (int)n_exp, (const A_*)w_d, (int)ff, (int)width, limit, alpha, shift,  \
-                           (void*)o);                                                                                                              \
+        launch_moe_product<A_, true>({(const A_*)h, h_stride, src, (int)top, weight_out ? (const float*)nullptr : wts, counts, (int)n_exp,         \
+                                      (const A_*)w_gu, (int)width, (int)ff, limit, alpha, shift, (void*)y}, pairs, n_tok, st);                     \
+        launch_moe_product<A_, false>({(const A_*)y, ff, (const int32_t*)nullptr, 1, (const float*)nullptr, counts, (int)n_exp, (const A_*)w_d,    \
+                                       (int)ff, (int)width, limit, alpha, shift, (void*)o}, pairs, pairs, st);                                     \
         hipLaunchKernelGGL(moe_pair_gather_kernel<A_>, dim3((unsigned)((n_tok * (width / 4) + 255) / 256)), dim3(256), 0, st, (const float*)o,     \
                            (const int64_t*)dst, weight_out ? wts : (const float*)nullptr, (int)top, (A_*)out, n_tok * (width / 4), (int)(width / 4)); \
     } while (0)
