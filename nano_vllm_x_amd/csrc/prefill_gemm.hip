@@ -10,7 +10,7 @@
 // above some 200 rows, whose products take K in the same order).
 // The products of a layer of Qwen3-0.6B, us, qkv / o / gate | up / down (the library's without SiluAndMul's own 4 us):
 //     64 rows 4.6 / 6.0 / 5.8 / 7.5 (8.8 / 8.4 / 9.0 / 10.1),   216 rows 6.8 / 6.1 / 10.1 / 7.8 (9.4 / 8.9 / 13.4 / 9.4),
-//     459 rows 9.1 / 7.9 / 11.8 / 10.0 (11.2 / 9.7 / 13.6 / 12.5),   1536 rows 20.6 / 13.7 / 29.5 / 20.5 (17.7 / 13.7 / 28.9 / 17.1).
+//     459 rows 9.1 / 7.9 / 11.8 / 10.0 (11.2 / 9.7 / 13.6 / 12.5),   1536 rows 18.7 / 13.8 / 24.4 / 20.1 (17.7 / 13.7 / 28.9 / 17.1).
 #include "prefill_gemm.h"
 
 namespace NVX_NS {
