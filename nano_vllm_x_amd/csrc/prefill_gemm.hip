@@ -164,7 +164,7 @@ static const PrefillTile PREFILL_TILES[] = {{256, 256, 256, 26.f, 26.f}, {192, 2
 // More rows: rounds of a tile's workgroups times what a round costs, by which every tile is chosen somewhere; us of 4096 outputs from 1024 columns, the
 // chosen / 64 x 128: 700 rows 11.8 (128 x 128) / 12.9, 1536 rows 18.7 (128 x 256) / 20.5, 2160 rows 22 (192 x 256) / 30, 4096 rows 32 (256 x 256) / 45; with SILU
 // 6144 from 1024, 1536 rows 24 (192 x 256) / 27, 2160 rows 31 (256 x 256) / 39.
-// QKV: up to 512 rows, where a head's norm and rotation behind the product are less than their own launch (459 rows 12.4, product and launch 14; 1024 rows 17.6
+// QKV: of 129 to 512 rows (prefill_step.hip), where a head's norm and rotation behind the product are less than their own launch (459 rows 12.4, product and launch 14; 1024 rows 17.6
 // and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).
 static int prefill_gemm_rule(int64_t m, int64_t n, bool silu, bool wide) {
     auto tiles = [&](int64_t tm, int64_t tn) { return (m + tm - 1) / tm * (n / tn); };

@@ -32,7 +32,9 @@ extern "C" int NVX_ENTRY(nvx_internal_prefill_step)(const NvxPrefillStep* s, nvx
     int turn = 0;
     for (int64_t l = 0; l < s->n_layers; ++l) {
         const int64_t* w = s->layers + 10 * l;
-        if (t <= 512) {
+        // a head's norm and rotation behind the product: us a step of Qwen3-0.6B, in a launch of their own / there, 40 tokens 1557 / 1594, 128 1700 / 1718, 200 1801 / 1783,
+        // 400 2296 / 2265, 512 2457 / 2400 (up to 128 the product has smaller tiles, which hold no head; beyond 512 see prefill_gemm_rule)
+        if (t > 128 && t <= 512) {
             const NvxQkvOut out = {s->positions, s->slots, s->rope, s->rope_rows, s->n_slots, (const uint16_t*)w[2], (const uint16_t*)w[3], (uint16_t*)s->q,
                                    (uint16_t*)w[8], (uint16_t*)w[9], (int)s->hq, (int)s->hkv, eps};
             NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[1], nullptr, t, qw, hid, NVX_PG_QKV, &out, st));

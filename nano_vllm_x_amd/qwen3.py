@@ -97,8 +97,8 @@ DECODE_LINEAR_MAX_WEIGHT_BYTES = 16 << 20
 # Multiply-adds of a layer's projections up to which a prefill step is queued by one native call with the products of csrc/prefill_gemm.hip
 # (ops.prefill_step), with layers of up to 2048 and of more: 4450 tokens of Qwen3-0.6B, 1390 of Qwen3-1.7B, 124 of Qwen3-8B.  A layer's products, here and the
 # library's with silu_mul: 0.6B, us, 2160 tokens 96 and 115, 4096 tokens 140 and 149, 8000 tokens 228 and 238, 15754 tokens 437 and 432, with SiluAndMul's
-# product from here and the others the library's 221 and 407; up to some 4000 tokens the host is the slower from Python too.  8B, 64 tokens 115 and 120, 216 tokens
-# 184 and 169.
+# product from here and the others the library's 221 and 407; up to some 4000 tokens the host is the slower from Python too.  1.7B, 700 tokens 108 and 113, 1390
+# tokens 170 and 180, SiluAndMul's product of 6000 281 and 333.  8B, 64 tokens 115 and 120, 216 tokens 184 and 169.
 PREFILL_STEP_MAX_WORK, PREFILL_STEP_MAX_WORK_WIDE = int(70e9), int(24e9)
 
 # NVX_FP32_LINEAR=1 (read when a model is built): every dense projection, the LM head included, multiplies in fp32 and
