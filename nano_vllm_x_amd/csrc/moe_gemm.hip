@@ -11,10 +11,12 @@
 // neighbouring tiles (8 row tiles by as many weight tiles share its L2).  Bound: the CU's 64 bytes a clock from L2, at which two workgroups
 // of this tile keep the matrix cores busy for at most as long as they wait.  One library product per expert and direction, with a copy into
 // expert order ahead of them and the activation between, needed 16 + 3 launches and the counts on the host.
-// 8192 pairs over 8 experts of 1536 x 1024: up 93 us (560 TFLOP/s), down 54 (480), the weighted sum 8.6; the library's products with copy,
-// activation and sum took 270 for a layer, and its counts a wait of the host.
+// 8192 pairs over 8 experts of 1536 x 1024: up 93 us (560 TFLOP/s), down 54 (480), the weighted sum 8.6, and with the tiles that the rule below takes (moe_wide_kernel)
+// 74 and 44; the library's products with copy, activation and sum took 270 for a layer, and its counts a wait of the host.
 #include "moe_dev.h"
 #include "wide_dev.h"
+
+#include <algorithm>
 
 namespace NVX_NS {
 
@@ -339,33 +341,49 @@ static void launch_moe_wide(const MoeWideArgs<A>& a, int64_t m_tiles, hipStream_
     hipLaunchKernelGGL((moe_wide_kernel<A, UP, TM, TN, STAGES>), dim3((unsigned)(tiles < 256 ? (tiles + 7) / 8 * 8 : 256)), dim3(512), 0, st, a);      // (a workgroup a CU)
 }
 
-// One of the two products.  Tile: the fewest rounds of workgroups times what a round costs (us of 1024 columns), an expert's last tile taken as half full; the
-// small tile of four waves, two workgroups a CU, where none of the wide ones fits.
+enum { MOE_BY_RULE, MOE_256_256, MOE_192_256, MOE_128_128, MOE_FOUR_WAVES };      // tiles of pairs x rows of weights: of the wide walk, or the kernel of four waves
+static const struct { int m, n, slots; float us; } MOE_TILES[] = {{256, 256, 256, 30.f}, {192, 256, 256, 28.f}, {128, 128, 256, 10.8f}, {GT, GT, 512, 21.f}};      // workgroups that run at once; us of a round of them over 1024 columns
+
+// Which tile a product takes (n rows of weights an expert, k columns): the fewest rounds of workgroups times what a round costs (of the kernel of four waves, two a CU: 0.55 of that
+// where a CU has one).  How many tiles the pairs make the counts decide, which the host does not know: the more of experts alike and of an expert's last tile
+// half full for the wide tiles, whose round too many is the dearer, and the mean for the other.  us of the mixture, the tile above / four waves, where the estimate
+// of half-full tiles alone went wrong: up products of 3200 pairs over 8 experts of 1536 x 1024 (192 x 256: 24 tiles of pairs, not 20) 83 / 71, 3072 x 2048 231 / 207,
+// 12 000 over 60 of 1024 x 512 149 / 135.  Of 360 products measured (65 to 20 000 tokens, 2 to 63 experts, columns of 256 to 4096) four are slower than four waves, by 2 % of the mixture at most.
+static int moe_tile_rule(int64_t pairs, int64_t n_exp, int64_t n, int64_t k, bool fits) {
+    const int64_t live = n_exp < pairs ? n_exp : pairs;      // (experts that may have pairs)
+    int best = MOE_FOUR_WAVES;
+    float least = 0.f;
+    for (int i = fits ? 0 : 3; i < 4; ++i) {
+        const auto& t = MOE_TILES[i];
+        if (i < 3 && n % t.n) continue;
+        const int64_t half = std::max((2 * pairs / t.m + live) / 2, live), alike = live * ((pairs + live * t.m - 1) / (live * t.m));
+        const int64_t tiles = (i == 3 ? (half + alike) / 2 : std::max(half, alike)) * ((n + t.n - 1) / t.n);
+        const float cost = t.us * (i == 3 && tiles <= 256 ? 0.55f : (float)((tiles + t.slots - 1) / t.slots));
+        if (best == MOE_FOUR_WAVES || cost < least) best = MOE_256_256 + i, least = cost;
+    }
+    return best;
+}
+
+// One of the two products, by a tile of MOE_* that fits (BY_RULE: the rule's).
 template <typename A, bool UP>
-static void launch_moe_product(const MoeWideArgs<A>& a, int64_t pairs, int64_t n_tok, hipStream_t st) {
-    const int64_t n = UP ? 2 * (int64_t)a.n_out : a.n_out, live = a.n_exp < pairs ? a.n_exp : pairs;      // (experts that may have pairs)
+static int launch_moe_product(const MoeWideArgs<A>& a, int64_t pairs, int64_t n_tok, int tile, hipStream_t st) {
+    const int64_t n = UP ? 2 * (int64_t)a.n_out : a.n_out, live = a.n_exp < pairs ? a.n_exp : pairs;
     auto most = [&](int64_t tm) { return pairs / tm + live; };                                           // as many tiles as the counts can ask for
     const bool fits = a.k >= 256 && a.x_stride < (1 << 21) && n_tok * a.x_stride < (1ll << 30) && n * a.k < (1ll << 30);
-    const struct { int m, n; float us; } tiles[] = {{256, 256, 34.f}, {192, 256, 28.f}, {128, 128, 10.8f}};
-    int best = -1;
-    float least = 0.f;
-    for (int i = 0; fits && i < 3; ++i) {
-        if (n % tiles[i].n) continue;
-        const int64_t m2 = 2 * pairs / tiles[i].m + live, m = m2 / 2 > live ? m2 / 2 : live;
-        const float cost = (float)((m * (n / tiles[i].n) + 255) / 256) * tiles[i].us;
-        if (best < 0 || cost < least) best = i, least = cost;
-    }
-    if (best == 0) launch_moe_wide<A, UP, 256, 256, 2>(a, most(256), st);
-    else if (best == 1) launch_moe_wide<A, UP, 192, 256, 2>(a, most(192), st);
-    else if (best == 2) launch_moe_wide<A, UP, 128, 128, 4>(a, most(128), st);
+    if (tile == MOE_BY_RULE) tile = moe_tile_rule(pairs, a.n_exp, n, a.k, fits);
+    NVX_REQUIRE(tile == MOE_FOUR_WAVES || (tile >= MOE_256_256 && tile <= MOE_128_128 && fits && n % MOE_TILES[tile - 1].n == 0), NVX_EUNSUPPORTED, "nvx_moe_expert_rows: tile %d", tile);
+    if (tile == MOE_256_256) launch_moe_wide<A, UP, 256, 256, 2>(a, most(256), st);
+    else if (tile == MOE_192_256) launch_moe_wide<A, UP, 192, 256, 2>(a, most(192), st);
+    else if (tile == MOE_128_128) launch_moe_wide<A, UP, 128, 128, 4>(a, most(128), st);
     else hipLaunchKernelGGL((moe_group_gemm_kernel<A, UP>), dim3((unsigned)((most(GT) * (a.n_out / (UP ? GT / 2 : GT)) + 7) / 8 * 8)), dim3(256), 0, st, a.x, a.x_stride, a.src,
                             a.src_div, a.scale, a.counts, a.n_exp, a.w, a.k, a.n_out, a.limit, a.alpha, a.shift, a.out);
+    return nvx_check_launch("nvx_moe_expert_rows");
 }
 
 // The whole mixture (see nvx_moe_expert_rows) for a step of many tokens; ws as there.  The pairs' order is made here too.
-int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
-                    int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
-                    hipStream_t st) {
+static int moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
+                       int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
+                       int up_tile, int down_tile, hipStream_t st) {
     const int64_t pairs = n_tok * top;
     // ws: n_tok * top * (width + ff) floats = the pairs' results (float32), their hidden rows (16 bits), then the order: its counts, source and
     // place of every pair (12 bytes a pair and 256: they fit in the half of the hidden rows that 16 bits leave, 2 * ff >= 128 bytes a pair)
@@ -379,10 +397,10 @@ int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx
     NVX_REQUIRE(m_tiles * (ff / (GT / 2)) < (1ll << 30) && m_tiles * (width / GT) < (1ll << 30), NVX_EINVAL, "nvx_moe_expert_rows: too many tiles");
 #define NVX_GROUPED(A_)                                                                                                                            \
     do {                                                                                                                                           \
-        launch_moe_product<A_, true>({(const A_*)h, h_stride, src, (int)top, weight_out ? (const float*)nullptr : wts, counts, (int)n_exp,         \
-                                      (const A_*)w_gu, (int)width, (int)ff, limit, alpha, shift, (void*)y}, pairs, n_tok, st);                     \
-        launch_moe_product<A_, false>({(const A_*)y, ff, (const int32_t*)nullptr, 1, (const float*)nullptr, counts, (int)n_exp, (const A_*)w_d,    \
-                                       (int)ff, (int)width, limit, alpha, shift, (void*)o}, pairs, pairs, st);                                     \
+        if (const int rc = launch_moe_product<A_, true>({(const A_*)h, h_stride, src, (int)top, weight_out ? (const float*)nullptr : wts, counts, (int)n_exp,         \
+                                      (const A_*)w_gu, (int)width, (int)ff, limit, alpha, shift, (void*)y}, pairs, n_tok, up_tile, st)) return rc; \
+        if (const int rc = launch_moe_product<A_, false>({(const A_*)y, ff, (const int32_t*)nullptr, 1, (const float*)nullptr, counts, (int)n_exp, (const A_*)w_d,    \
+                                       (int)ff, (int)width, limit, alpha, shift, (void*)o}, pairs, pairs, down_tile, st)) return rc; \
         hipLaunchKernelGGL(moe_pair_gather_kernel<A_>, dim3((unsigned)((n_tok * (width / 4) + 255) / 256)), dim3(256), 0, st, (const float*)o,     \
                            (const int64_t*)dst, weight_out ? wts : (const float*)nullptr, (int)top, (A_*)out, n_tok * (width / 4), (int)(width / 4)); \
     } while (0)
@@ -391,3 +409,21 @@ int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx
 #undef NVX_GROUPED
     return nvx_check_launch("nvx_moe_expert_rows");
 }
+
+int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
+                    int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
+                    hipStream_t st) {
+    return moe_grouped(h, h_stride, fmt, idx, wts, top, w_gu, w_d, n_exp, limit, alpha, shift, weight_out, ws, out, n_tok, width, ff, MOE_BY_RULE, MOE_BY_RULE, st);
+}
+
+// The same with tiles of the caller's choice (0: the rule's), and the rule itself for sizes and layouts that the wide walk reads.
+extern "C" int nvx_internal_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu,
+                                        const void* w_d, int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out,
+                                        int64_t n_tok, int64_t width, int64_t ff, int up_tile, int down_tile, nvx_stream_t stream) {
+    NVX_REQUIRE(nvx_moe_grouped_fits(fmt, n_exp, width, ff) && n_tok > 0 && n_tok <= 65535 && top > 0 && n_tok * top < (1ll << 31) && n_exp > 0 && h_stride >= width && h_stride % 8 == 0,
+                NVX_EUNSUPPORTED, "nvx_internal_moe_grouped: sizes");
+    NVX_REQUIRE(h && idx && wts && w_gu && w_d && ws && out && nvx_aligned16(h) && nvx_aligned16(w_gu) && nvx_aligned16(w_d) && nvx_aligned16(ws) && nvx_aligned16(out), NVX_EINVAL,
+                "nvx_internal_moe_grouped: pointers must be 16-byte aligned");
+    return moe_grouped(h, h_stride, fmt, idx, wts, top, w_gu, w_d, n_exp, limit, alpha, shift, weight_out, ws, out, n_tok, width, ff, up_tile, down_tile, (hipStream_t)stream);
+}
+extern "C" int nvx_internal_moe_tile(int64_t pairs, int64_t n_exp, int64_t n, int64_t k) { return moe_tile_rule(pairs, n_exp, n, k, k >= 256); }
