@@ -208,7 +208,12 @@ def linear_decode(x, w, mode: int = 0, k_splits: int = 1, out=None, squares=None
     """x (m <= 256, k) bf16 times w (n, k)^T.  mode 0 -> bf16 (m, n); mode 1 -> SiluAndMul of the
     [gate; up] projection, bf16 (m, n/2); mode 2 -> fp32 partials (k_splits, m, n) for rmsnorm_splitk; mode 3 -> the product + `residual` with the norm
     behind it left open: (that sum times norm_weight, the sum, the squares of its rows), the first and the last being x and `squares` of a product of mode 0
-    or 1, which then is of the normed rows (sizes: decode_boundary_fits)."""
+    or 1, which then is of the normed rows (sizes: decode_boundary_fits).  `out` and `k_splits` belong to modes 0 to 2 without `squares`, `eps` to `squares`."""
+    if mode == 3 or squares is not None:
+        _need(out is None and k_splits == 1, "linear_decode: no out and no k_splits with mode 3 or squares")
+    _need((residual is not None and norm_weight is not None) if mode == 3 else (residual is None and norm_weight is None),
+          "linear_decode: residual and norm_weight with mode 3 and no other")
+    _need(squares is not None or eps == 0.0, "linear_decode: eps without squares")
     _dev(x, w, out)
     if mode == 3 or squares is not None:
         return _decode_boundary(x, w, mode, squares, eps, residual, norm_weight)

@@ -4,6 +4,7 @@ import torch
 from torch import nn
 
 import test_plain_calls as plain_calls
+from nano_vllm_x_amd import ops
 from nano_vllm_x_amd.core.common import ForwardMode
 from nano_vllm_x_amd.layers.attention import AttentionMetadata, PagedDecodeWrapper, PagedPrefillWrapper, attention_kv_cache
 from nano_vllm_x_amd.qwen3 import Qwen3Config, Qwen3ForCausalLM
@@ -56,3 +57,15 @@ def test_other_steps_formats_sizes_and_layouts_keep_the_modules():
         p = getattr(m.model.layers[layer].self_attn, name)
         p.weight = nn.Parameter(torch.zeros(p.weight.shape[1], p.weight.shape[0]).bfloat16().t())
         assert not _plain(m), name
+
+
+@pytest.mark.parametrize("args,what", [
+    (dict(mode=3, out=True, residual=True, norm_weight=True), "no out"), (dict(mode=3, k_splits=2, residual=True, norm_weight=True), "no out"),
+    (dict(mode=0, out=True, squares=True, eps=1e-6), "no out"), (dict(mode=1, k_splits=4, squares=True, eps=1e-6), "no out"),
+    (dict(mode=0, residual=True), "residual and norm_weight"), (dict(mode=1, norm_weight=True), "residual and norm_weight"),
+    (dict(mode=2, residual=True, norm_weight=True), "residual and norm_weight"), (dict(mode=0, squares=True, residual=True), "residual and norm_weight"),
+    (dict(mode=3), "residual and norm_weight"), (dict(mode=3, residual=True), "residual and norm_weight"), (dict(mode=0, eps=1e-6), "eps")])
+def test_an_argument_that_a_product_does_not_take_is_refused(args, what):
+    t = torch.zeros(4, 1024).bfloat16()
+    with pytest.raises(Exception, match=what):
+        ops.linear_decode(t, torch.zeros(32, 1024).bfloat16(), **{k: t if v is True else v for k, v in args.items()})
