@@ -95,11 +95,20 @@ DECODE_LINEAR_MAX_WEIGHT_BYTES = 16 << 20
 
 
 # Multiply-adds of a layer's projections up to which a prefill step is queued by one native call with the products of csrc/prefill_gemm.hip
-# (ops.prefill_step), with layers of up to 2048 and of more: 4450 tokens of Qwen3-0.6B, 1390 of Qwen3-1.7B, 124 of Qwen3-8B.  A layer's products, here and the
-# library's with silu_mul: 0.6B, us, 2160 tokens 96 and 115, 4096 tokens 140 and 149, 8000 tokens 228 and 238, 15754 tokens 437 and 432, with SiluAndMul's
-# product from here and the others the library's 221 and 407; up to some 4000 tokens the host is the slower from Python too.  1.7B, 700 tokens 108 and 113, 1390
-# tokens 170 and 180, SiluAndMul's product of 6000 281 and 333.  8B, 64 tokens 115 and 120, 216 tokens 184 and 169.
-PREFILL_STEP_MAX_WORK, PREFILL_STEP_MAX_WORK_WIDE = int(70e9), int(24e9)
+# (ops.prefill_step) in any case: there the host is the slower from Python.  Up to the second figure it is with layers of up to 1024 whose two products back to the
+# layer's size are one round of 128 x 128 tiles (rows of 128 times columns of 128 up to the CUs).  That is 4096 tokens of Qwen3-0.6B, 476 of Qwen3-1.7B, 124 of
+# Qwen3-8B.  us of 14 layers, native / library with SiluAndMul's product from here / library and silu_mul: layers of 1024 x 3072, 2600 tokens 2438 / 2524 / 2686, 4000
+# 2864 / 2970 / 3280, 4200 (two rounds) 3902 / 3536 / 3678, 4440 3961 / 3523 / 3671; 768 x 2304, 5000 tokens 2314 / 2477 / 2681, 6000 (two rounds) 2995 / 2724 / 2874;
+# 2048 x 6144, 600 tokens 2399 / 2243 / 2340, 1390 3612 / 3353 / 3401; 2048 x 2048, 2100 tokens 3267 / 2603 / 2591; 512 x 1536, 7000 tokens 2103 / 2429 / 2784.
+# 8B, a layer's products, 64 tokens 115 and the library's 120, 216 tokens 184 and 169.
+PREFILL_STEP_MAX_WORK, PREFILL_STEP_MAX_WORK_NARROW = int(24e9), int(70e9)
+
+
+def prefill_step_is_native(tokens: int, hidden: int, n_q_heads: int, n_kv_heads: int, inter: int) -> bool:
+    """Whether a prefill step of sizes that ops.prefill_step_fits accepts is faster through ops.prefill_step than queued from Python."""
+    work = tokens * (hidden * (2 * n_q_heads + 2 * n_kv_heads) * 128 + 3 * hidden * inter)
+    return work <= PREFILL_STEP_MAX_WORK or (work <= PREFILL_STEP_MAX_WORK_NARROW and hidden <= 1024 and -(-tokens // 128) * -(-hidden // 128) <= 256)
+
 
 # NVX_FP32_LINEAR=1 (read when a model is built): every dense projection, the LM head included, multiplies in fp32 and
 # rounds its result to the model's 16-bit format once (the LM head's logits stay fp32).  Not a serving mode: it takes
@@ -429,8 +438,7 @@ class Qwen3Model(nn.Module):
         wrapper, cache, slots = md.wrapper, md.kv_cache, md.output_kv_indices
         hidden_states, residual, t = self.embed_tokens(input_ids), None, input_ids.shape[0]
         hq, hkv, eps, final = first.num_heads, first.num_kv_heads, cfg.rms_norm_eps, weight_of(self.norm)
-        work = t * (cfg.hidden_size * (2 * hq + 2 * hkv) * 128 + 3 * cfg.hidden_size * cfg.intermediate_size)
-        long = work > (PREFILL_STEP_MAX_WORK if cfg.hidden_size <= 2048 else PREFILL_STEP_MAX_WORK_WIDE)
+        long = not prefill_step_is_native(t, cfg.hidden_size, hq, hkv, cfg.intermediate_size)
         if not long and ops.prefill_step_fits(cfg.hidden_size, hq, hkv, cfg.intermediate_size):
             qo_indptr, kv_indptr, kv_indices, n_q, n_kv = wrapper._planned
             full = [(*ws, *cache.get_kv_cache(attn.layer_id)) for ws, attn in zip(layers, attns)]

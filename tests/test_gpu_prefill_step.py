@@ -1,4 +1,4 @@
-"""Prefill steps of a Qwen3 model as the runner queues them (in one native call up to some 1500 tokens of this width, without module calls above) against the module
+"""Prefill steps of a Qwen3 model as the runner queues them (in one native call up to 4096 tokens of this width, without module calls above) against the module
 graph, which a hook on any of its modules brings back."""
 import pytest
 import torch
@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 LAYERS, ROUNDINGS = 2, 9      # 16-bit stores of a layer that another order of summation can turn: norms 2, qkv, q and k, read-out, o, activation, down
 
 
-def _runner(dtype, hidden=1024, inter=3072, heads=16):
+def _runner(dtype, hidden=1024, inter=3072, heads=16, slots=4096):
     from nano_vllm_x_amd.core.model_runner import ModelRunner
     from nano_vllm_x_amd.qwen3 import Qwen3Config
 
@@ -17,8 +17,27 @@ def _runner(dtype, hidden=1024, inter=3072, heads=16):
                                      rope_theta=1e6, tie_word_embeddings=True, torch_dtype=dtype))
     r = ModelRunner(model="random", max_bs=8, enforce_eager=True, context_len=2048, config=cfg, dtype=dtype)
     r.load_model()
-    r.initialize_kv_cache(4096)
+    r.initialize_kv_cache(slots)
     return r
+
+
+@pytest.fixture
+def route(monkeypatch):
+    """How often a step went out natively, and how often a long step took SiluAndMul into its product."""
+    from nano_vllm_x_amd import ops
+
+    calls = {"native": 0, "gated": 0}
+
+    def counted(name, fn):
+        def run(*args):
+            out = fn(*args)
+            calls[name] += out is not None
+            return out
+        return run
+
+    monkeypatch.setattr(ops, "prefill_step", counted("native", ops.prefill_step))
+    monkeypatch.setattr(ops, "gated_product", counted("gated", ops.gated_product))
+    return calls
 
 
 def _step(r, lens, cached):
@@ -28,7 +47,7 @@ def _step(r, lens, cached):
     gen = torch.Generator().manual_seed(sum(lens) + cached)
     r.kv_cache.k_cache.copy_(torch.randn(r.kv_cache.k_cache.shape, generator=gen).to(r.dtype) * 0.1)
     r.kv_cache.v_cache.copy_(torch.randn(r.kv_cache.v_cache.shape, generator=gen).to(r.dtype) * 0.1)
-    slots = torch.randperm(4096, generator=gen).tolist()
+    slots = torch.randperm(r.kv_cache.k_cache.shape[1], generator=gen).tolist()
     seqs, at = [], 0
     for i, n in enumerate(lens):
         ids = torch.randint(0, 1024, (n + cached,), generator=gen).tolist()
@@ -40,8 +59,25 @@ def _step(r, lens, cached):
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 @pytest.mark.parametrize("lens,cached", [((1,), 0), ((1, 1, 1), 7), ((255,), 0), ((256,), 3), ((257,), 0), ((300, 5, 206), 64), ((600,), 0), ((1100,), 0), ((1530,), 0), ((1500, 20, 100), 100)])
-def test_prefill_steps_equal_the_module_graph(dtype, lens, cached):
-    r = _runner(dtype)
+def test_prefill_steps_equal_the_module_graph(dtype, lens, cached, route):
+    _equal_to_the_module_graph(_runner(dtype), dtype, lens, cached)
+    assert route == {"native": 1, "gated": 0}
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("lens,cached,limit", [((2000, 2000, 97), 0, None), ((2000, 1, 2000, 500), 40, None), ((1, 1, 1), 7, 0), ((300, 5, 206), 64, 0), ((1100,), 0, 0)])
+def test_long_steps_equal_the_module_graph(dtype, lens, cached, limit, route, monkeypatch):
+    """Steps past the native call's limit, and shorter ones with the limit taken down."""
+    from nano_vllm_x_amd import qwen3
+
+    if limit is not None:
+        monkeypatch.setattr(qwen3, "PREFILL_STEP_MAX_WORK", limit)
+        monkeypatch.setattr(qwen3, "PREFILL_STEP_MAX_WORK_NARROW", limit)
+    _equal_to_the_module_graph(_runner(dtype, slots=8192), dtype, lens, cached)
+    assert route == {"native": 0, "gated": LAYERS}
+
+
+def _equal_to_the_module_graph(r, dtype, lens, cached):
     got = _step(r, lens, cached)
     hook = r.model.model.layers[1].mlp.register_forward_hook(lambda *_: None)
     ref = _step(r, lens, cached)
@@ -56,10 +92,12 @@ def test_prefill_steps_equal_the_module_graph(dtype, lens, cached):
 
 
 @pytest.mark.parametrize("alone", [1, 33, 65, 200])
-def test_a_prompt_s_logits_do_not_depend_on_what_shares_its_step(alone):
-    """Whatever tile a step's size chooses, a row's sums run in the same order: the same bits alone and among 256, 500, 1000 and 3000 other tokens (the
-    last through the library's products, which take K in that order too for steps of that size)."""
-    r = _runner("bfloat16")
+def test_a_prompt_s_logits_do_not_depend_on_what_shares_its_step(alone, route, monkeypatch):
+    """Whatever tile a step's size chooses, a row's sums run in the same order: the same bits alone and among 256, 500, 1000 and 3000 other tokens, and among 4500
+    and, with the native call's limit taken down, 600 and 2000 (through the library's products, which take K in that order too for steps of such sizes)."""
+    from nano_vllm_x_amd import qwen3
+
+    r = _runner("bfloat16", slots=8192)
     gen = torch.Generator().manual_seed(alone)
     ids = torch.randint(0, 1024, (alone,), generator=gen).tolist()
 
@@ -76,6 +114,13 @@ def test_a_prompt_s_logits_do_not_depend_on_what_shares_its_step(alone):
     want = first([])
     for others in ([256], [500], [400, 600], [1500, 1500]):
         assert torch.equal(first(others), want), others
+    assert route == {"native": 5, "gated": 0}
+    assert torch.equal(first([2000, 2000, 500]), want)
+    monkeypatch.setattr(qwen3, "PREFILL_STEP_MAX_WORK", 0)
+    monkeypatch.setattr(qwen3, "PREFILL_STEP_MAX_WORK_NARROW", 0)
+    for others in ([600], [2000]):
+        assert torch.equal(first(others), want), others
+    assert route == {"native": 5, "gated": 3 * LAYERS}
 
 
 @pytest.mark.parametrize("alone", [1, 33, 100])
