@@ -183,12 +183,19 @@ def prefill_step_fits(hidden: int, n_q_heads: int, n_kv_heads: int, inter: int) 
     return hidden % 256 == 0 and inter % 256 == 0 and n_q_heads % 2 == 0 and n_q_heads % n_kv_heads == 0 and n_q_heads // n_kv_heads in (1, 2, 4, 8)
 
 
+def gated_product_faster(rows: int, n: int, k: int) -> bool:
+    """Whether SiluAndMul of a product of csrc/prefill_gemm.hip, n rows of weights of k columns, beats the library's product and silu_mul.  Up to 1536 columns it
+    does (us, 15754 rows: 6144 x 1024 182, library 159 and 50; 500 to 30 000 rows of 3072 x 512 to 16384 x 1024 and 8192 x 1536: 0.32 to 0.95 of the two, but for 1.03 and
+    1.01 at one size each); with more, where SiluAndMul is the smaller part, up to 2048 where four rounds of 256 x 256 tiles or more make an idle part of the last a small one: 12288 x
+    2048, 600 rows 47 and 40, 1300 97 and 82, 2048 132 and 106, 5500 rows 0.86 of the two, up to 30 000 0.85 to 0.99; 9728 x 1792, 4096 rows 193 and 163, from 7000 0.73 to 0.95."""
+    return k <= 1536 or (k <= 2048 and rows * n >= 4 * 256 * 256 * 256)
+
+
 def gated_product_fits(x, w) -> bool:
-    """Whether SiluAndMul of x W^T, w = [gate; up], is a product of csrc/prefill_gemm.hip that beats the library's and silu_mul: columns of up to 2048, behind
-    which SiluAndMul is the smaller part and the library's lead in the product (a tenth) the larger.  us, 15754 rows: 6144 x 1024 182, library 159 and 50."""
+    """Whether gated_product takes these, and is the faster (gated_product_faster)."""
     return x.dim() == 2 and w.dim() == 2 and x.dtype in H16 and w.dtype == x.dtype and x.is_cuda and w.device == x.device and 0 < x.shape[0] < 1 << 24 \
-        and x.shape[1] == w.shape[1] <= 2048 and w.shape[1] % 256 == 0 and w.shape[0] % 256 == 0 and x.is_contiguous() and w.is_contiguous() \
-        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.numel() < 1 << 30
+        and x.shape[1] == w.shape[1] and gated_product_faster(x.shape[0], w.shape[0], x.shape[1]) and w.shape[1] % 256 == 0 and w.shape[0] % 256 == 0 \
+        and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.numel() < 1 << 30
 
 
 def gated_product(x, w):

@@ -1,6 +1,7 @@
 """Which Qwen3 prefill steps go out in one native call (no GPU: only the choice)."""
 import pytest
 
+from nano_vllm_x_amd import ops
 from nano_vllm_x_amd.qwen3 import prefill_step_is_native
 
 L06B, L17B, L8B = (1024, 16, 8, 3072), (2048, 16, 8, 6144), (4096, 32, 8, 12288)      # hidden, heads, kv heads, intermediate
@@ -19,3 +20,13 @@ def test_steps_that_the_library_s_products_do_faster(layer, tokens):
     """(Measured: the native call takes 2 to 26 % more there than steps queued from Python do.)"""
     hidden, hq, hkv, inter = layer
     assert not prefill_step_is_native(tokens, hidden, hq, hkv, inter)
+
+
+@pytest.mark.parametrize("rows,n,k", [(4200, 6144, 1024), (15754, 6144, 1024), (2600, 8192, 1536), (10000, 3072, 512), (6000, 12288, 2048), (20000, 12288, 2048), (20000, 4096, 2048)])
+def test_gated_products_of_long_steps(rows, n, k):
+    assert ops.gated_product_faster(rows, n, k)
+
+
+@pytest.mark.parametrize("rows,n,k", [(600, 12288, 2048), (1300, 12288, 2048), (2000, 12288, 2048), (4200, 12288, 2048), (4096, 9728, 1792), (6000, 9728, 1792), (30000, 24576, 4096)])
+def test_gated_products_that_the_library_and_silu_mul_do_faster(rows, n, k):
+    assert not ops.gated_product_faster(rows, n, k)
