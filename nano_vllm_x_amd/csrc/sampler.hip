@@ -550,6 +550,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const uint16_t* lrow = logits + row * row_stride;
     auto alike = [](uint32_t v) { return PROBS ? v : uniform(v); };       // (where the registers are short)
+    auto alike64 = [&](unsigned long long v) -> unsigned long long { return PROBS ? v : (unsigned long long)uniform((uint32_t)(v >> 32)) << 32 | uniform((uint32_t)v); };
     const float T = temps[row];
     const bool greedy = !(T > 0.0f);
     const int64_t k64 = top_ks[row];
@@ -629,11 +630,12 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     unsigned int* const my32 = sc.hist.h32 + (lane & 31);
     unsigned long long* const my64 = sc.hist.h64 + (lane & 15);
 
-    // ---- both boundaries from one count: how often each of the 2048 largest scores (a row's positive ones, 16 powers of two down from the maximum)
-    // occurs, and each of as many negative ones from minus the maximum up.  Equal scores have equal masses, so count times mass, in integers, is what the
-    // tokens' own masses add up to; the few tokens of neither kind add theirs up in registers.  A boundary that is not among the largest is found in two
-    // passes each, as below.  us, 224 rows of 151 936 tokens, with two passes each and now: top-k 50 41 and 39, top-p 0.9 at temperature
-    // 0.6 81 and 52, at 1.0 107 and 70, both 58 and 44; a token's own mass is an exponential and a 64-bit atomic among ten bins where most meet. ----
+    // ---- both boundaries from counts of scores: how often each of the 2048 largest occurs (a row's positive ones, 16 powers of two down from the maximum)
+    // and, beside them or in a pass of their own, each of as many negative ones.  Equal scores have equal masses, so count times mass, in integers, is what the
+    // tokens' own masses add up to; the few tokens of neither kind add theirs up in registers.  A boundary of neither kind is found in two
+    // passes each, as below.  us, 224 rows of 151 936 tokens at temperature 0.8, with two passes each and now, scores of deviation 2.5 around 0 / around -8: top-k 50
+    // 41.2 and 40.0 / 40.7 and 39.6, top-p 0.9 85 and 61 / 85 and 60, both 59 and 45 / 59 and 46; of deviation 0.1, top-p 0.9 178 and 159.  A token's own mass is an
+    // exponential and a 64-bit atomic among ten bins where most meet. ----
     constexpr int WINDOW = 2048;
     static_assert(WINDOW == 2 * SMP_THREADS && sizeof(sc.hist) == WINDOW * 16, "a thread has two scores, of four counts each, or two of either kind, of two");
     const bool k_on = k < vocab, p_on = top_p < 1.0f;
@@ -641,52 +643,29 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     uint32_t k_key = 0;                          // key of the k-th largest score: ascending rank vocab - k
     uint32_t p_key = 0;                          // scores with key < p_key are dropped
     unsigned long long before = 0, thr = 0;      // mass of kept scores strictly below p_key; the mass that may be dropped
+    uint32_t n_ties = 0xffffffffu;               // scores with key == p_key, where that is known
     if (!PROBS && (k_on || p_on)) {      // (beside the pass that writes the probabilities it takes registers that are not there)
         const bool both = kmax >= 0x8000u + WINDOW;                        // (else no score is positive, and the largest are among the negative ones)
-        const uint32_t base = kmax >= WINDOW ? kmax - (WINDOW - 1) : 0, base_neg = both ? 0xffffu - kmax : base;
-        __syncthreads();
-        zero_hist();
-        __syncthreads();
-        unsigned long long below = 0;
-        if (k_on) {                              // (what lies below the largest is dropped: no count of it, and four counters a score)
-            unsigned int* const mine = sc.hist.h32 + (lane & 3);
-            each_pair([&](int, uint32_t kw) {
-                const uint32_t b0 = (kw & 0xffffu) - base, b1 = (kw >> 16) - base;
-                atomicAdd(mine + (b0 & (WINDOW - 1)) * 4, b0 < WINDOW ? 1u : 0u);
-                atomicAdd(mine + (b1 & (WINDOW - 1)) * 4, b1 < WINDOW ? 1u : 0u);
-            });
-        } else {
-            unsigned int* const mine = sc.hist.h32 + (lane & 1);
-            const uint32_t upper = both ? 0u : (uint32_t)WINDOW;
-            each_pair([&](int, uint32_t kw) {
-                const uint32_t k0 = kw & 0xffffu, k1 = kw >> 16;
-                const uint32_t b0 = k0 - (k0 & 0x8000u ? base : base_neg), b1 = k1 - (k1 & 0x8000u ? base : base_neg);
-                const uint32_t u0 = (k0 >> 4 & (uint32_t)WINDOW) | upper, u1 = (k1 >> 4 & (uint32_t)WINDOW) | upper;
-                atomicAdd(mine + ((b0 & (WINDOW - 1)) + u0) * 2, b0 < WINDOW ? 1u : 0u);
-                atomicAdd(mine + ((b1 & (WINDOW - 1)) + u1) * 2, b1 < WINDOW ? 1u : 0u);
-                if (__any(b0 >= WINDOW || b1 >= WINDOW)) {
-                    const uint32_t pr = pair_of_keys(kw);
-                    below += b0 >= WINDOW ? mass_fixed(h16lo_to_f32(pr), c1, c2m) : 0u;
-                    below += b1 >= WINDOW ? mass_fixed(h16hi_to_f32(pr), c1, c2m) : 0u;
-                }
-            });
-        }
-        __syncthreads();
-        // a thread has two neighbouring scores: how often they occur, or with `masses` what they weigh
-        const uint32_t key0 = base + 2 * (uint32_t)tid;
-        auto count_of = [&](int score) -> unsigned int {             // (from -WINDOW on: the negative ones)
-            if (k_on) return (sc.hist.h32[score * 4] + sc.hist.h32[score * 4 + 1]) + (sc.hist.h32[score * 4 + 2] + sc.hist.h32[score * 4 + 3]);
+        const uint32_t base = kmax >= WINDOW ? kmax - (WINDOW - 1) : 0;
+        // The negative ones from so far below the maximum that what lies below weighs nothing (2^-32 of it: 22.2 temperatures), and as far as the positive
+        // ones reach, 16 powers of two up from there
+        const uint32_t low = (~__float_as_uint(fminf(lmax - 22.5f * fmaxf(T, 1.0f), -lmax)) >> 16) - 1u;
+        const uint32_t base_neg = alike(both ? (low < 0x8000u - WINDOW ? low : 0x8000u - WINDOW) : base);
+        // a thread has two neighbouring scores, first_key and the next: how often they occur, or with `masses` what they weigh
+        bool four = k_on;                        // counters a score, else two
+        auto count_of = [&](int score) -> unsigned int {             // (of two counters: from -WINDOW on, the negative ones)
+            if (four) return (sc.hist.h32[score * 4] + sc.hist.h32[score * 4 + 1]) + (sc.hist.h32[score * 4 + 2] + sc.hist.h32[score * 4 + 3]);
             return sc.hist.h32[(WINDOW + score) * 2] + sc.hist.h32[(WINDOW + score) * 2 + 1];
         };
         auto mass_of = [&](uint32_t ky, unsigned int n) -> unsigned long long {
             return n && ky >= k_key ? (unsigned long long)n * mass_fixed(logit_of_key(ky), c1, c2m) : 0ull;
         };
-        auto of_score = [&](int q, bool masses) -> unsigned long long {
-            const unsigned int n = count_of(2 * tid + q);
-            return masses ? mass_of(key0 + q, n) : n;
+        auto of_score = [&](int at, uint32_t ky, bool masses) -> unsigned long long {
+            const unsigned int n = count_of(at);
+            return masses ? mass_of(ky, n) : n;
         };
-        auto sum_quads = [&](bool masses) {      // of the scores of four threads -> tot
-            unsigned long long v = of_score(0, masses) + of_score(1, masses);
+        auto sum_quads = [&](int at, uint32_t ky, bool masses) {      // of the scores of four threads -> tot
+            unsigned long long v = of_score(at, ky, masses) + of_score(at + 1, ky + 1, masses);
             v += shfl_xor_u64(v, 1);
             v += shfl_xor_u64(v, 2);
             if ((tid & 3) == 0) sc.tot[tid >> 2] = v;
@@ -694,57 +673,139 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
             __syncthreads();
         };
         // among the eight scores of the quad that select_bin chose, the first up to which all add up to more than target
-        auto boundary = [&](bool masses, unsigned long long target) {
+        auto boundary = [&](int at, uint32_t ky, bool masses, unsigned long long target) {
             __syncthreads();
             if ((unsigned)(tid >> 2) == sc.sel_digit) {
-                const unsigned long long v0 = of_score(0, masses), v1 = of_score(1, masses);
-                unsigned long long at = sc.sel_before;
+                const unsigned long long v0 = of_score(at, ky, masses), v1 = of_score(at + 1, ky + 1, masses);
+                unsigned long long sum = sc.sel_before;
                 for (int j = 0; j < 3; ++j) {
                     const unsigned long long o = shfl_quad_u64(v0 + v1, j);
-                    if (j < (tid & 3)) at += o;
+                    if (j < (tid & 3)) sum += o;
                 }
-                if (at <= target && at + v0 + v1 > target) {
-                    const bool second = at + v0 <= target;
-                    sc.found = (int)(key0 + (second ? 1 : 0));
-                    sc.sel_bucket = second ? at + v0 : at;
+                if (sum <= target && sum + v0 + v1 > target) {
+                    const bool second = sum + v0 <= target;
+                    sc.found = (int)(ky + (second ? 1 : 0));
+                    sc.sel_bucket = second ? sum + v0 : sum;
+                    sc.thr = count_of(at + (second ? 1 : 0));
                 }
             }
             __syncthreads();
         };
+        // top-k: the positive ones, or where fewer than k scores are not negative the negative ones, what is below them in the first counter and what is above
+        // in the last
+        bool k_neg = false;
         if (k_on) {
-            sum_quads(false);
-            const unsigned long long rank = (unsigned long long)(vocab - k);
-            if (tid < 64) {
-                const unsigned long long in = wave_sum_u64(sc.tot[4 * lane] + sc.tot[4 * lane + 1] + sc.tot[4 * lane + 2] + sc.tot[4 * lane + 3]);
-                select_bin(sc, (unsigned long long)vocab - in, rank, lane);
+            unsigned int* const mine = sc.hist.h32 + (lane & 3);
+            auto clear = [&]() { __syncthreads(); zero_hist(); __syncthreads(); };
+            auto search = [&](uint32_t first, int inner) __attribute__((always_inline)) {      // `inner`: first and last are counters of others
+                __syncthreads();
+                const uint32_t ky = first + 2 * (uint32_t)tid;
+                const unsigned long long rank = (unsigned long long)(vocab - k);
+                sum_quads(2 * tid, ky, false);
+                if (tid < 64) {
+                    const unsigned long long in = wave_sum_u64(sc.tot[4 * lane] + sc.tot[4 * lane + 1] + sc.tot[4 * lane + 2] + sc.tot[4 * lane + 3]);
+                    select_bin(sc, (unsigned long long)vocab - in, rank, lane);
+                }
+                boundary(2 * tid, ky, false, rank);
+                const int at = (int)alike(sc.found);
+                k_found = at >= (int)first + inner && at < (int)first + WINDOW - inner;
+                k_key = k_found ? (uint32_t)at : 0;
+            };
+            if (both) {                                // are fewer than k of the scores not negative?  Most rows show as many among their first 16 384 tokens
+                auto total = [&](int n) -> int {
+#pragma unroll
+                    for (int m = 32; m >= 1; m >>= 1) n += __shfl_xor(n, m, 64);
+                    __syncthreads();
+                    if (tid == 0) sc.wave_cnt[0] = 0;
+                    __syncthreads();
+                    if (lane == 0) atomicAdd(&sc.wave_cnt[0], n);
+                    __syncthreads();
+                    return (int)alike(sc.wave_cnt[0]);
+                };
+                constexpr uint32_t P = 0x80008000u;
+                k_neg = total(__popc(raw0.x & P) + __popc(raw0.y & P) + __popc(raw0.z & P) + __popc(raw0.w & P) +
+                              __popc(raw1.x & P) + __popc(raw1.y & P) + __popc(raw1.z & P) + __popc(raw1.w & P)) < k;
+                if (k_neg) {
+                    int n_pos = 0;
+                    each_pair([&](int, uint32_t kw) { n_pos += __popc(kw & P); });
+                    k_neg = total(n_pos) < k;
+                }
             }
-            boundary(false, rank);
-            k_found = (int)alike(sc.found) >= 0;
-            k_key = k_found ? alike(sc.found) : 0;
+            if (k_neg) {
+                clear();
+                each_pair([&](int, uint32_t kw) {
+                    const int b0 = (int)(kw & 0xffffu) - (int)base_neg, b1 = (int)(kw >> 16) - (int)base_neg;
+                    atomicAdd(mine + min(max(b0, 0), WINDOW - 1) * 4, 1u);
+                    atomicAdd(mine + min(max(b1, 0), WINDOW - 1) * 4, 1u);
+                });
+                search(base_neg, 1);
+            }
+            if (!k_found) {
+                clear();
+                each_pair([&](int, uint32_t kw) {          // (what lies below the largest is dropped: no count of it)
+                    const uint32_t b0 = (kw & 0xffffu) - base, b1 = (kw >> 16) - base;
+                    atomicAdd(mine + (b0 & (WINDOW - 1)) * 4, b0 < WINDOW ? 1u : 0u);
+                    atomicAdd(mine + (b1 & (WINDOW - 1)) * 4, b1 < WINDOW ? 1u : 0u);
+                });
+                search(base, 0);
+            }
             __syncthreads();
         }
         if (p_on && k_found) {
-            if (!k_on && both)
-                for (int q = 0; q < 2; ++q) below += mass_of(base_neg + 2 * tid + q, count_of(2 * tid + q - WINDOW));
-            sum_quads(true);
-            below = wave_sum_u64(below);
-            if (lane == 0) atomicAdd(&sc.z_total, below);
-            __syncthreads();
-            if (tid < 64) {
-                const unsigned long long lower = sc.z_total;
-                const unsigned long long z = lower + wave_sum_u64(sc.tot[4 * lane] + sc.tot[4 * lane + 1] + sc.tot[4 * lane + 2] + sc.tot[4 * lane + 3]);
-                const double thr_d = (double)(1.0f - top_p) * (double)z;
-                unsigned long long t = thr_d <= 0.0 ? 0ull : (unsigned long long)thr_d;
-                if (t >= z) t = z > 0 ? z - 1 : 0;   // the largest score always survives
-                if (lane == 0) sc.thr = t;
-                select_bin(sc, lower, t, lane);
+            unsigned long long below = 0;
+            if (!k_on || k_neg) {                // both kinds, two counters a score
+                four = false;
+                __syncthreads();
+                zero_hist();
+                __syncthreads();
+                unsigned int* const mine = sc.hist.h32 + (lane & 1);
+                const uint32_t upper = both ? 0u : (uint32_t)WINDOW;
+                each_pair([&](int, uint32_t kw) {
+                    const uint32_t k0 = kw & 0xffffu, k1 = kw >> 16;
+                    const uint32_t b0 = k0 - (k0 & 0x8000u ? base : base_neg), b1 = k1 - (k1 & 0x8000u ? base : base_neg);
+                    const uint32_t u0 = (k0 >> 4 & (uint32_t)WINDOW) | upper, u1 = (k1 >> 4 & (uint32_t)WINDOW) | upper;
+                    atomicAdd(mine + ((b0 & (WINDOW - 1)) + u0) * 2, b0 < WINDOW ? 1u : 0u);
+                    atomicAdd(mine + ((b1 & (WINDOW - 1)) + u1) * 2, b1 < WINDOW ? 1u : 0u);
+                    if (__any(b0 >= WINDOW || b1 >= WINDOW)) {
+                        const uint32_t pr = pair_of_keys(kw);
+                        below += b0 >= WINDOW && k0 >= k_key ? mass_fixed(h16lo_to_f32(pr), c1, c2m) : 0u;
+                        below += b1 >= WINDOW && k1 >= k_key ? mass_fixed(h16hi_to_f32(pr), c1, c2m) : 0u;
+                    }
+                });
+                __syncthreads();
+                if (both)
+                    for (int q = 0; q < 2; ++q) below += mass_of(base_neg + 2 * tid + q, count_of(2 * tid + q - WINDOW));
             }
-            __syncthreads();
-            thr = sc.thr;
-            boundary(true, thr);
-            p_found = (int)alike(sc.found) >= 0;
+            below = wave_sum_u64(below);
+            // the positive ones, then, where the boundary is below them, the negative ones
+#pragma unroll 1
+            for (int neg = 0;;) {
+                sum_quads(2 * tid - neg, (neg ? base_neg : base) + 2 * (uint32_t)tid, true);
+                if (lane == 0 && !neg) atomicAdd(&sc.z_total, below);
+                __syncthreads();
+                if (tid < 64) {
+                    const unsigned long long lower = sc.z_total;     // (of the negative ones: nothing weighs below them)
+                    if (!neg) {
+                        const unsigned long long z = lower + wave_sum_u64(sc.tot[4 * lane] + sc.tot[4 * lane + 1] + sc.tot[4 * lane + 2] + sc.tot[4 * lane + 3]);
+                        const double thr_d = (double)(1.0f - top_p) * (double)z;
+                        unsigned long long t = thr_d <= 0.0 ? 0ull : (unsigned long long)thr_d;
+                        if (t >= z) t = z > 0 ? z - 1 : 0;   // the largest score always survives
+                        thr = alike64(t);
+                        if (lane == 0) sc.thr = t;
+                    }
+                    select_bin(sc, lower, thr, lane);
+                }
+                __syncthreads();
+                if (!neg) thr = alike64(sc.thr);
+                boundary(2 * tid - neg, (neg ? base_neg : base) + 2 * (uint32_t)tid, true, thr);
+                p_found = (int)alike(sc.found) >= 0;
+                if (p_found || neg || four || !both) break;
+                __syncthreads();
+                neg = WINDOW;
+            }
             p_key = p_found ? alike(sc.found) : 0;
-            before = sc.sel_bucket;
+            before = alike64(sc.sel_bucket);
+            if (p_found) n_ties = alike((uint32_t)sc.thr);
         }
     }
 
@@ -891,7 +952,8 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
             __syncthreads();
             p_cut = (int)alike(sc.found) >= 0 ? (int)alike(sc.found) : vocab;
     };
-    if (PROBS && n_drop > 0) cut_by_passes();
+    constexpr uint32_t TIES = 384;       // of so many the id that parts them is found beside the draw: each is compared with all, and a pass is 2 us
+    if (n_drop > 0 && (PROBS || n_ties > TIES)) cut_by_passes();
 
     auto kept_kp = [&](uint32_t ky, int i) -> bool {
         if (ky < k_key) return false;
@@ -943,10 +1005,11 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
     // Philox code once and reads their logits back from memory.  Four tokens share one Philox block; its counter
     // depends on the token alone, so skipping the blocks without a survivor changes no draw. ----
     uint32_t km[5] = {0, 0, 0, 0, 0};
-    // Where some of the ties at top-p's boundary are to be dropped they are all taken down on the way, and the id that parts them is found among the list (in LDS,
-    // the counts' memory), each against all; ties beyond it leave the draw again.  More than a thousand of them are parted by passes over the row.
+    // Where some of few ties at top-p's boundary are to be dropped they are all taken down on the way, and the id that parts them is found among the list (in LDS,
+    // the counts' memory), each against all; ties beyond it leave the draw again.  More of them have been parted by passes over the row.
     int* const ties = reinterpret_cast<int*>(sc.hist.h32);
-    if (n_drop > 0) {
+    const bool listed = n_drop > 0 && n_ties <= TIES;
+    if (listed) {
         __syncthreads();
         if (tid == 0) { sc.sel_digit = 0; sc.found = -1; }
         __syncthreads();
@@ -957,30 +1020,31 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_resident_kernel(
         const bool a = (kw & 0xffffu) >= lowest, b = (kw >> 16) >= lowest;
         km[pos >> 5] |= ((a ? 1u : 0u) | (b ? 2u : 0u)) << (pos & 31);
     };
-    if (n_drop > 0) each_pair([&](int i, uint32_t kw) {
-        mark(i, kw);
-        const bool ta = (kw & 0xffffu) == p_key, tb = (kw >> 16) == p_key;
-        if (ta || tb) {
-            const int first = (int)atomicAdd(&sc.sel_digit, (ta ? 1u : 0u) + (tb ? 1u : 0u));
-            if (first < SMP_THREADS) ties[first] = ta ? i : i + 1;
-            if (ta && tb && first + 1 < SMP_THREADS) ties[first + 1] = i + 1;
-        }
-    });
-    else each_pair(mark);
-    if (n_drop > 0) {
-        __syncthreads();
-        const int n_ties = (int)sc.sel_digit;
-        if (n_ties <= SMP_THREADS) {
-            if (tid < n_ties) {
-                const int me = ties[tid];
-                int less = 0;
-                for (int j = 0; j < n_ties; ++j) less += ties[j] < me ? 1 : 0;
-                if (less == n_drop) sc.found = me;              // (ids differ: one thread)
+    if (listed) {
+        each_pair([&](int i, uint32_t kw) {
+            mark(i, kw);
+            const bool ta = (kw & 0xffffu) == p_key, tb = (kw >> 16) == p_key;
+            if (ta || tb) {
+                const uint32_t first = atomicAdd(&sc.sel_digit, (ta ? 1u : 0u) + (tb ? 1u : 0u));
+                if (first < TIES) ties[first] = ta ? i : i + 1;
+                if (ta && tb && first + 1 < TIES) ties[first + 1] = i + 1;
             }
-            __syncthreads();
-            p_cut = (int)alike(sc.found) >= 0 ? (int)alike(sc.found) : vocab;
-        } else cut_by_passes();
-    }
+        });
+        if (tid < 4) ties[n_ties + tid] = 0x7fffffff;
+        __syncthreads();
+        if (tid < (int)n_ties) {
+            const int me = ties[tid];
+            int less = 0;
+#pragma unroll 2
+            for (int j = 0; j < (int)n_ties; j += 4) {
+                const int4 t = *reinterpret_cast<const int4*>(ties + j);
+                less += (t.x < me ? 1 : 0) + (t.y < me ? 1 : 0) + (t.z < me ? 1 : 0) + (t.w < me ? 1 : 0);
+            }
+            if (less == n_drop) sc.found = me;              // (ids differ: one thread)
+        }
+        __syncthreads();
+        p_cut = (int)alike(sc.found) >= 0 ? (int)alike(sc.found) : vocab;
+    } else each_pair(mark);
     const uint32_t tie_bits = n_drop > 0 ? __float_as_uint(logit_of_key(p_key)) >> 16 : 0x10000u;      // as the row has it
     const uint2 key = make_uint2((uint32_t)seed, (uint32_t)(seed >> 32));
     float best = -INFINITY; int besti = 0x7fffffff;

@@ -54,6 +54,51 @@ def test_boundaries_outside_the_largest_scores_draw_the_same(shape):
                 assert torch.equal(_draw(lg, T, *a, 3), _draw(wide[:, :vocab], T, *a, 3)), (k, p, m)
 
 
+@pytest.mark.parametrize("shape", ["below zero", "one above", "few above", "around zero", "grid", "small", "large"])
+def test_boundaries_among_negative_scores_draw_the_same(shape):
+    """Largest scores above zero, boundaries below it, above and below the negative scores that are counted, and in between: the general kernel's tokens."""
+    rows, vocab = 24, 65536
+    g = torch.Generator(device="cuda").manual_seed(7 * len(shape))
+    x = torch.randn((rows, vocab), generator=g, device="cuda")
+    few = torch.rand((rows, vocab), generator=g, device="cuda") < 2e-4
+    lg = {"below zero": 2.5 * x - 8, "one above": torch.where(x == x.max(1, keepdim=True).values, 0.75, 0.5 * x - 30), "few above": torch.where(few, x.abs(), x - 12),
+          "around zero": torch.where(few, 3.0, 1e-4 * x), "grid": (4 * x).round() / 2 - 6, "small": torch.where(few, 0.01, -x.abs() / 100),
+          "large": torch.where(few, 1e4, -1e4 * x.abs())}[shape].to(torch.bfloat16)
+    assert bool((lg.float().max(1).values > 0).all())
+    wide = torch.empty((rows, vocab + 1), dtype=torch.bfloat16, device="cuda")
+    wide[:, :vocab] = lg
+    T = torch.tensor([0.05, 0.3, 0.8, 1.0, 2.0, 40.0], device="cuda").repeat(rows // 6)
+    off = lambda v, d=torch.float32: torch.full((rows,), v, dtype=d, device="cuda")
+    for k in (vocab, 1, 20, 200, 30000, vocab - 1):
+        for p in (1.0, 0.999, 0.9, 0.4):
+            for m in (0.0, 0.05):
+                a = (off(k, torch.int64), off(p), off(m))
+                assert torch.equal(_draw(lg, T, *a, 3), _draw(wide[:, :vocab], T, *a, 3)), (k, p, m)
+
+
+@pytest.mark.parametrize("vocab", [32000, 151936])
+@pytest.mark.parametrize("score", [4.0, -4.0])
+def test_ties_at_the_boundary_are_parted_alike(vocab, score):
+    """One to thousands of tokens with the boundary's score, from none to all of them dropped: the general kernel's tokens, by a list of up to 384 or by passes."""
+    counts = (1, 2, 63, 382, 384, 385, 1024, 1025, 9000)
+    g = torch.Generator().manual_seed(vocab)
+    lg, tops = torch.full((3 * len(counts), vocab), -40.0), []
+    for i, n in enumerate(counts):
+        for j, share in enumerate((0.02, 0.5, 0.999)):       # of the ties' mass that is kept
+            at = torch.randperm(vocab, generator=g)[:n + 3]
+            lg[3 * i + j, at[:3]], lg[3 * i + j, at[3:]] = 4.5, score
+            above, ties = 3 * 2.718281828 ** (4.5 - score), n
+            tops.append((above + share * ties) / (above + ties))
+    lg = lg.to(torch.bfloat16).cuda()
+    wide = torch.empty((lg.shape[0], vocab + 1), dtype=torch.bfloat16, device="cuda")
+    wide[:, :vocab] = lg
+    p, one = torch.tensor(tops, device="cuda"), torch.ones(lg.shape[0], device="cuda")
+    for k in (vocab, vocab - 1):
+        for step in range(8):
+            a = (torch.full((lg.shape[0],), k, device="cuda"), p, 0 * one)
+            assert torch.equal(_draw(lg, one, *a, step), _draw(wide[:, :vocab], one, *a, step)), (k, step)
+
+
 def test_min_p_keeps_the_tokens_of_its_ratio():
     """Among logits 0, -1, -2, ... at temperature 1 the ratio of a probability to the largest is e^-i: min_p between e^-3 and e^-2 leaves three tokens."""
     lg = torch.full((64, 1024), -100.0, device="cuda", dtype=torch.bfloat16)
