@@ -1,8 +1,10 @@
 // Products of a Qwen3 decode step with the residual sum and RMSNorm between two of them inside the products themselves.
 //
 // A norm needs whole rows, so as a kernel of its own it stands between two products and costs a launch to move a few KB.  Here the product in front of a norm takes K whole in every workgroup, so it can add the residual itself, and leaves three
-// things: the new residual, the unrounded sum times the norm's weight (rounded once, as the norm's result was), and per row and 16 columns
-// the sum of the squares.  The product behind it adds a row's squares up and multiplies its own sums by 1 / rms: (x w / rms) W = (x w) W / rms.
+// things: the new residual, the unrounded sum times the norm's weight (rounded once, as the norm's result was), and per row and 8 columns (16 from 33 rows
+// on) the sum of the squares.  The product behind it adds a row's squares up and multiplies its own sums by 1 / rms: (x w / rms) W = (x w) W / rms.
+// bfloat16 only: unnormed rows times a norm's weight need its exponents.  Rows of 1024 only: all four products of a layer have to be kernels of this package,
+// which take weights of up to 16 MB (qwen3.py); with rows of 2048 and an inner size of 6144 gate | up is 50 MB and the library's.
 //
 // The products are those of few_rows.hip: eight waves share K, 64 columns (a 128-byte line of every row) at a time, through a ring in LDS that
 // is each wave's own, no barrier until the waves' sums meet, in a fixed order, whatever the number of rows: linear_decode.hip's products over the rms,
@@ -13,7 +15,6 @@
 // what stands between them: 22.2 / 25.6 / 30.3 / 34.2 / 42.2, now 17.7 / 22.6 / 26.3 / 31.6 / 39.7.
 #include "nvx_dev.h"
 
-#ifndef NVX_F16     // bfloat16 only: unnormed rows times a norm's weight need its exponents
 namespace NVX_NS {
 
 constexpr int DB_WAVES = 8;
@@ -195,4 +196,3 @@ extern "C" int nvx_internal_decode_boundary(const void* x, const void* w, void* 
 #undef NVX_DB
     return nvx_check_launch("nvx_internal_decode_boundary");
 }
-#endif

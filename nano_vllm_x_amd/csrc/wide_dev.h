@@ -94,7 +94,7 @@ struct WideTile {
             int asked = STAGES;
             for (int s = 0; s < steps; ++s) {
                 half(even, odd, slot, std::false_type{}, 0, 0);
-                wide_wait_for_all_but<(STAGES - 2) * LOADS>();          // the step behind this one has landed (a tile's other loads and stores count too, and are older)
+                wide_wait_for_all_but<(STAGES - 2) * LOADS>();          // the step behind this one has landed (as have, behind a tile, the stores of its results: they are younger and count too)
                 __builtin_amdgcn_s_barrier();                           // everybody's part of it has, and everybody has read this one (wide_lds_wait)
                 asm volatile("" : : : "memory");
                 const int was = slot;

@@ -248,7 +248,8 @@ BOUNDARY_ROWS = 256       # largest decode step whose norms ride on its products
 
 
 def decode_boundary_fits(rows: int, hidden: int, attn_width: int, inter: int, dtype) -> bool:
-    """Whether a decode step's products may carry its residual sums and norms (linear_decode's mode 3, and modes 0 and 1 with squares)."""
+    """Whether a decode step's products may carry its residual sums and norms (linear_decode's mode 3, and modes 0 and 1 with squares): in bfloat16 with rows of
+    1024, the width whose four products are all of csrc/decode_boundary.hip and csrc/linear_decode.hip (see there)."""
     return dtype == torch.bfloat16 and 0 < rows <= BOUNDARY_ROWS and hidden == 1024 and attn_width % 512 == 0 and inter % 512 == 0
 
 

@@ -465,7 +465,8 @@ class Qwen3Model(nn.Module):
 
     def _decode(self, layers, residual, positions):
         """What the module graph computes for a decode step (embedding rows `residual`), with the residual sums and norms between two products inside
-        these (csrc/decode_boundary.hip): two launches a layer fewer.  `layers`: as _plain_decode gives them."""
+        these (csrc/decode_boundary.hip): two launches a layer fewer.  As many roundings as there, in other places, and sums of K in another order: a step that
+        the modules compute (a hook, a parallel stage) agrees with it to the rounding of bfloat16, not bit for bit.  `layers`: as _plain_decode gives them."""
         eps, attns = self.config.rms_norm_eps, [layer._modules["self_attn"]._modules["attn"] for layer in self.layers]
         md = attns[0].attention_metadata
         qkv = decode_linear(ops.rmsnorm(residual, layers[0][0], eps), layers[0][1], "qkv")
