@@ -376,7 +376,8 @@ class Qwen3Model(nn.Module):
         """_plain_layers of a decode step (embedding rows x) whose norms may ride on its products (_decode); else None."""
         c = self.config
         hidden, aw, inter = c.hidden_size, c.num_attention_heads * 128, c.intermediate_size
-        if not ops.decode_boundary_fits(x.shape[0], hidden, aw, inter, x.dtype) or x.shape[1:] != (hidden,) or not x.is_contiguous():
+        if not ops.decode_boundary_fits(x.shape[0], hidden, aw, inter, x.dtype) or x.shape[0] > min(DECODE_LINEAR_MAX_ROWS.values()) or x.shape[1:] != (hidden,) \
+                or not x.is_contiguous():
             return None
         plain = self._plain_layers(ForwardMode.DECODE, PagedDecodeWrapper, "run_qkv")
         if not plain or not self.layers[0].self_attn.attn.attention_metadata.wrapper.qkv_fused:

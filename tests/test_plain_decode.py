@@ -4,7 +4,7 @@ import torch
 from torch import nn
 
 import test_plain_calls as plain_calls
-from nano_vllm_x_amd import ops
+from nano_vllm_x_amd import ops, qwen3
 from nano_vllm_x_amd.core.common import ForwardMode
 from nano_vllm_x_amd.layers.attention import AttentionMetadata, PagedDecodeWrapper, PagedPrefillWrapper, attention_kv_cache
 from nano_vllm_x_amd.qwen3 import Qwen3Config, Qwen3ForCausalLM
@@ -57,6 +57,13 @@ def test_other_steps_formats_sizes_and_layouts_keep_the_modules():
         p = getattr(m.model.layers[layer].self_attn, name)
         p.weight = nn.Parameter(torch.zeros(p.weight.shape[1], p.weight.shape[0]).bfloat16().t())
         assert not _plain(m), name
+
+
+@pytest.mark.parametrize("kind", ["qkv", "o", "gate_up", "down"])
+def test_rows_that_a_projection_leaves_to_the_library(kind, monkeypatch):
+    m = _model()
+    monkeypatch.setitem(qwen3.DECODE_LINEAR_MAX_ROWS, kind, 3)
+    assert not _plain(m) and _plain(m, torch.zeros(3, 1024).bfloat16())
 
 
 @pytest.mark.parametrize("args,what", [
