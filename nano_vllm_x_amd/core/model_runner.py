@@ -73,6 +73,8 @@ class ModelRunner:
         self.block_table: Optional[BlockTable] = None
         self._sp_key, self._sp_dev, self._sp_unfiltered = None, None, False
         self._stage_output, self._defer_stage_send = None, False
+        self.decode_chain: Optional[ops.DecodeChain] = None      # decode steps whose layers are one launch, and their graphs
+        self.chain_graph: Optional[HIPGraph] = None
         self._last_done = 0.0
         self.stats = {"prefill_steps": 0, "decode_steps": 0, "graph_steps": 0, "eager_decode_steps": 0, "prefill_s": 0.0, "decode_s": 0.0}
         self.graph_sizes_dropped: list = []               # decode batch sizes whose graph was slower than a larger one's
@@ -198,6 +200,10 @@ class ModelRunner:
         n_rows = max(1024, 4 * self.max_bs) + 1
         self.block_table = BlockTable(self.max_bs, n_rows, 2 * self.context_len, self.device)
         self.decode_ws = ops.DecodeWorkspace(self.max_bs, self.num_heads, self.num_kv_heads, self.device)
+        cfg = self.hf_config
+        if self.tp_size * self.pp_size == 1 and not self.enforce_eager and ops.DecodeChain.available() \
+                and ops.DecodeChain.fits(1, self.num_layers, cfg.hidden_size, self.num_heads, self.num_kv_heads, cfg.intermediate_size, self.dtype):
+            self.decode_chain = ops.DecodeChain(self.device)
         if not self.enforce_eager:
             self.graph = HIPGraph()
             try:
@@ -275,6 +281,8 @@ class ModelRunner:
         None on a pipeline stage other than the last."""
         decode = batch.forward_mode == ForwardMode.DECODE
         tpd.check_peer_status()      # results leave through here too (tests, tools): never on top of a failed exchange
+        if self.decode_chain is not None:
+            self.decode_chain.check()
         if self.graph_step_possible(batch):
             hidden = self._execute_model_graph(batch, ids_on_device)
             self.stats["graph_steps"] += 1
@@ -398,6 +406,8 @@ class ModelRunner:
             tpd.check_peer_status()      # a direct-peer exchange that gave up waiting must not pass as a result
         except RuntimeError as e:
             raise RuntimeError(f"{e} [rank {self.rank}, {key[:-2]} step of {n} sequences, steps so far {self.stats}]") from None
+        if self.decode_chain is not None:
+            self.decode_chain.check()
         # launch to completion; a step queued behind another is charged from the moment that one completed
         now = time.perf_counter()
         self.stats[key] = self.stats.get(key, 0.0) + (now - max(t0, self._last_done))
@@ -452,11 +462,16 @@ class ModelRunner:
             host.fill_(-1)                    # rows past the batch are padding: no state is read or written for them
             host[:bs] = torch.tensor([s.state_slot for s in batch.seqs], dtype=torch.int32)
             self._state_slot_dev.copy_(host, non_blocking=True)
-        self.graph.replay(padded)
+        chain = self.chain_graph
+        if chain is not None and bs <= chain.max_bs and self.decode_chain.faster(bs, sum(len(s.kv_indices) for s in batch.seqs)):
+            self.decode_chain.in_turn(lambda: chain.replay(chain.match_bs(bs)))
+            self.stats["chain_steps"] = self.stats.get("chain_steps", 0) + 1
+        else:
+            self.graph.replay(padded)
         return self.graph.get_output_buffer("hidden_states")[:bs]
 
-    def _decode_forward(self, bs: int) -> torch.Tensor:
-        """The body of a captured decode step for a padded batch of `bs` rows."""
+    def _decode_forward(self, bs: int, chain: Optional[ops.DecodeChain] = None) -> torch.Tensor:
+        """The body of a captured decode step for a padded batch of `bs` rows, its layers in one launch if there is a `chain`."""
         bt = self.block_table
         torch.ops.nvx.decode_step_setup(bt.step_dev, bt.max_bs, bs, bt.table, bt.pad_start, bt.kv_start, bt.kv_len, bt.out_slots,
                                         bt.positions, bt.input_ids, self._sample_out)
@@ -468,8 +483,8 @@ class ModelRunner:
                                   out_slots=bt.out_slots[:bs], kv_indptr=None)
             with attention_kv_cache(self.model, md):
                 return self.model(bt.input_ids[:bs], bt.positions[:bs])
-        torch.ops.nvx.decode_plan(bt.kv_len[:bs], bt.kv_start[:bs], bt.out_slots[:bs], self.num_kv_heads, self.decode_ws.plan)
         wrapper = self._graph_wrappers[bs]
+        wrapper.bind_step(bt.out_slots, self.num_kv_heads, chain)
         md = AttentionMetadata(forward_mode=ForwardMode.DECODE, kv_cache=self.kv_cache, output_kv_indices=bt.out_slots[:bs],
                                wrapper=wrapper)
         with attention_kv_cache(self.model, md):
@@ -505,11 +520,20 @@ class ModelRunner:
                     w.bind_table(bt.table.view(-1), bt.kv_start, bt.kv_len, bs, self.decode_ws, qkv_fused=True)
                     self._graph_wrappers[bs] = w
                 self._decode_forward(bs)   # warm-up outside capture (library handles, allocator pool)
+                if self.decode_chain is not None and bs <= ops.DecodeChain.ROWS:
+                    self.decode_chain.in_turn(lambda: self._decode_forward(bs, self.decode_chain))
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         for bs in reversed(sizes):
             with self.graph.capture(bs):
                 hidden_out[:bs] = self._decode_forward(bs)
+        if self.decode_chain is not None:
+            self.chain_graph = HIPGraph()
+            self.chain_graph.graph_pool = self.graph.graph_pool      # (steps of either follow each other on a stream)
+            for bs in reversed(sizes):
+                if bs <= ops.DecodeChain.ROWS:
+                    with self.chain_graph.capture(bs):
+                        hidden_out[:bs] = self._decode_forward(bs, self.decode_chain)
         torch.cuda.synchronize()
         if os.environ.get("NVX_GRAPH_PRUNE", "1") != "0":
             self.prune_slow_graph_sizes()
@@ -553,6 +577,8 @@ class ModelRunner:
     def shutdown(self):
         if self.graph is not None:
             self.graph.clear()
+        if self.chain_graph is not None:
+            self.chain_graph.clear()
         tpd.shutdown()
 
 

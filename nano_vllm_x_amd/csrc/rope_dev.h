@@ -45,10 +45,9 @@ __device__ __forceinline__ int64_t clamp_pos(int64_t p, int64_t max_pos) {
 
 // RMSNorm over the 128 elements of a head (ss = their sum of squares, already reduced over the 16
 // lanes), rounded to bf16 as the unfused norm hands it to the rotary op, then rotated and interleaved.
-__device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float ss, const uint16_t* __restrict__ w, float eps,
+// (wa, wb: the norm's weights of the lane's elements)
+__device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float ss, const uint2& wa, const uint2& wb, float eps,
                                                         const float* cs_row, int l16) {
-    const uint2 wa = *reinterpret_cast<const uint2*>(w + 4 * l16);
-    const uint2 wb = *reinterpret_cast<const uint2*>(w + 64 + 4 * l16);
     const float wA[4] = {h16lo_to_f32(wa.x), h16hi_to_f32(wa.x), h16lo_to_f32(wa.y), h16hi_to_f32(wa.y)};
     const float wB[4] = {h16lo_to_f32(wb.x), h16hi_to_f32(wb.x), h16lo_to_f32(wb.y), h16hi_to_f32(wb.y)};
     const float inv = 1.0f / sqrtf(ss / 128.0f + eps);
@@ -59,6 +58,10 @@ __device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float
         n.b[j] = round_h16((x.b[j] * inv) * wB[j]);
     }
     return rotate_interleave(n, cs_row, l16);
+}
+__device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float ss, const uint16_t* __restrict__ w, float eps,
+                                                        const float* cs_row, int l16) {
+    return norm_rotate_interleave(x, ss, *reinterpret_cast<const uint2*>(w + 4 * l16), *reinterpret_cast<const uint2*>(w + 64 + 4 * l16), eps, cs_row, l16);
 }
 
 __device__ __forceinline__ float half_quad_sumsq(const HalfQuad& x) {

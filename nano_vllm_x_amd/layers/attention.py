@@ -122,6 +122,8 @@ class PagedDecodeWrapper:
         self._batch = 0
         self.qkv_fused = False
         self._new_slots = None
+        self.chain: Optional[ops.DecodeChain] = None
+        self._plan_due = None
 
     def _ensure(self, batch: int, hq: int, hkv: int, device):
         if self._ws is None or self._ws.max_batch < batch or (self._ws.n_q_heads, self._ws.n_kv_heads) != (hq, hkv):
@@ -160,9 +162,25 @@ class PagedDecodeWrapper:
         self._kv_indices, self._kv_start, self._kv_len, self._batch, self._ws = kv_indices, kv_start, kv_len, batch, ws
         self.qkv_fused = qkv_fused
 
+    def bind_step(self, out_slots, num_kv_heads: int, chain=None):
+        """After bind_table: the slots of the step's new rows, and what its layers may go through in one launch (ops.decode_chain).  The plan is launched
+        by the step's first run or run_qkv; a step that needs neither launches none."""
+        self._plan_due, self.chain = (out_slots, num_kv_heads), chain
+
+    def table_of_step(self):
+        """(kv_start, kv_len, out_slots, kv_indices) as bind_table and bind_step left them."""
+        b = self._batch
+        return self._kv_start[:b], self._kv_len[:b], self._plan_due[0][:b], self._kv_indices
+
+    def _launch_due_plan(self):
+        if self._plan_due is not None:
+            (slots, hkv), self._plan_due, b = self._plan_due, None, self._batch
+            torch.ops.nvx.decode_plan(self._kv_len[:b], self._kv_start[:b], slots[:b], hkv, self._ws.plan)
+
     def run_qkv(self, qkv, positions, cos_sin_cache, q_weight, k_weight, eps, paged_kv_cache, out=None):
         """Attention straight from the raw fused projection (see ops.paged_decode_qkv): replaces the
         q/k norm + rotary + scatter launch and run()."""
+        self._launch_due_plan()
         k_cache, v_cache = (_as_nhd(c) for c in paged_kv_cache)
         scale = self._sm_scale if self._sm_scale is not None else 128 ** -0.5
         if out is None and qkv.shape[0] == self._batch:
@@ -173,6 +191,7 @@ class PagedDecodeWrapper:
                                     self._batch, self._ws, scale, out=out)
 
     def run(self, q, paged_kv_cache, out=None):
+        self._launch_due_plan()
         k_cache, v_cache = (_as_nhd(c) for c in paged_kv_cache)
         b = self._batch
         ws = self._ws

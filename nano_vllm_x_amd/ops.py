@@ -9,6 +9,8 @@ capturable into a hipGraph.  `nano_vllm_x_amd.torch_ops` registers the stateless
 from __future__ import annotations
 
 import ctypes as _ctypes
+import threading as _threading
+import weakref as _weakref
 from typing import Optional
 
 import torch
@@ -274,6 +276,93 @@ def _decode_boundary(x, w, mode, squares, eps, residual, norm_weight):
         rc = lib.nvx_internal_linear_decode_scaled(_ptr(x), _ptr(w), _ptr(y), m, n, k, mode, _ptr(squares), float(eps), _stream())
     _lib.check(rc, "linear_decode")
     return y
+
+
+class DecodeChain:
+    """What steps of csrc/decode_chain.hip keep from one to the next: the words that their workgroups leave each other, the number of layers computed so far (no
+    word is ever marked with a number twice) and, in host memory, whether a wait ran out.  Steps that share one follow each other on a stream.
+
+    The workgroups of a step wait for each other, so all of them must find room on the device.  There is room for two steps; where a process keeps more than
+    two of these on a device, its steps take turns (in_turn), whatever their streams."""
+
+    ROWS, LAYERS, SECONDS = 8, 32, 10.0
+    _alive, _turn, _lock = _weakref.WeakSet(), {}, _threading.Lock()
+
+    def __init__(self, device):
+        self.words = torch.zeros(_lib.load().nvx_internal_decode_chain_words(), dtype=torch.int64, device=device)
+        self.epoch = torch.ones(1, dtype=torch.int32, device=device)
+        self.status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._status = self.status.numpy()
+        with self._lock:
+            self._alive.add(self)
+            if self._crowded():        # steps under way went without an event that the next ones could wait for
+                torch.cuda.synchronize(self.words.device)
+
+    def _crowded(self) -> bool:
+        return sum(c.words.device == self.words.device for c in self._alive) > 2
+
+    def in_turn(self, launch):
+        """launch(), which queues a step of this chain on the current stream; behind every other chain's where more than two are kept on the device."""
+        with self._lock:
+            crowded, device = self._crowded(), self.words.device
+            if crowded:
+                stream, last = torch.cuda.current_stream(device), self._turn.get(device)
+                if last is not None and last[0] != stream:
+                    stream.wait_event(last[1])
+            out = launch()
+            if crowded:
+                event = torch.cuda.Event()
+                event.record(stream)
+                self._turn[device] = (stream, event)
+            return out
+
+    @staticmethod
+    def fits(rows: int, layers: int, hidden: int, n_q_heads: int, n_kv_heads: int, inter: int, dtype) -> bool:
+        """Whether the kernel is built for a model of these sizes (its registers and LDS hold each weight's rows) and a step of this many sequences."""
+        return dtype == torch.bfloat16 and 0 < rows <= DecodeChain.ROWS and 0 < layers <= DecodeChain.LAYERS and (hidden, n_q_heads, n_kv_heads, inter) == (1024, 16, 8, 3072)
+
+    @staticmethod
+    def faster(rows: int, tokens: int) -> bool:
+        """Whether it beats the layers launch by launch for sequences of so many tokens together: 128 workgroups read keys and values, and the words grow with the rows.
+        us before and now: 8 sequences of 1200 1023 and 969, of 1500 1047 and 1040, 6 of 2000 1057 and 1122, 5 of 3000 1165 and 1126, of 8000 1688 and 1860, 4 of 8000 1616 and 1526,
+        of 16 000 2176 and 2384, 3 of 16 000 1979 and 2166, 2 of 30 000 2389 and 2232, 1 of 30 000 2225 and 1414."""
+        return rows <= DecodeChain.ROWS and tokens <= (60000 if rows <= 2 else 32000 if rows <= 4 else 10000)
+
+    @staticmethod
+    def available() -> bool:
+        return bool(_lib.load().nvx_internal_decode_chain_fits())
+
+    def check(self):
+        if self._status[0]:
+            raise RuntimeError("a decode step gave up waiting for its own workgroups: the device was taken by other work, and the step's results are not whole")
+
+
+def decode_chain(chain, layers, qkv, residual, positions, kv_start, kv_len, out_slots, kv_indices, cos_sin_cache, eps, sm_scale):
+    """The layers of a decode step of the sizes of DecodeChain.fits from the first one's attention to the last one's SiluAndMul, in one launch.  `layers`: per layer (input norm,
+    qkv, q norm, k norm, o, post-attention norm, gate | up, down, k rows, v rows); qkv (rows, 4096) the first layer's projections, residual (rows, 1024) the embedding rows.
+    Returns (activations (rows, 3072), residual (rows, 1024))."""
+    m = qkv.shape[0]
+    flat = [w for layer in layers for w in layer]
+    _dev(chain.words, qkv, residual, positions, kv_start, kv_len, out_slots, kv_indices, cos_sin_cache, *flat)
+    n_slots = layers[0][8].shape[0]
+    rows, bf = (n_slots, 8, 128), torch.bfloat16
+    shapes = ((1024,), (4096, 1024), (128,), (128,), (1024, 2048), (1024,), (6144, 1024), (1024, 3072), rows, rows)
+    _need(0 < m <= DecodeChain.ROWS and qkv.shape == (m, 4096) and residual.shape == (m, 1024) and all(t.dtype == bf and t.is_contiguous() for t in (qkv, residual)),
+          "decode_chain: projections, residual")
+    _need(0 < len(layers) <= DecodeChain.LAYERS and all(w.shape == shape and w.dtype == bf and w.is_contiguous() for layer in layers for w, shape in zip(layer, shapes)),
+          "decode_chain: weights, caches")
+    _need(all(t.dtype == torch.int64 and t.is_contiguous() and t.numel() == m for t in (positions, kv_start, out_slots)) and kv_len.dtype == torch.int32 and kv_len.is_contiguous()
+          and kv_len.numel() == m and kv_indices.dtype == torch.int32 and kv_indices.is_contiguous(), "decode_chain: positions, table")
+    _need(cos_sin_cache.dtype == torch.float32 and cos_sin_cache.dim() == 2 and cos_sin_cache.shape[1] == 128 and cos_sin_cache.is_contiguous(), "decode_chain: rotary table")
+    table = (_ctypes.c_int64 * (10 * len(layers)))()
+    for i, (_, _, nq, nk, o, n2, gate_up, down, k, v) in enumerate(layers):
+        n1, w = layers[i + 1][:2] if i + 1 < len(layers) else (None, None)
+        table[10 * i:10 * i + 10] = [t.data_ptr() if t is not None else 0 for t in (o, n2, gate_up, down, n1, w, nq, nk, k, v)]
+    act, new = torch.empty((m, 3072), dtype=bf, device=qkv.device), torch.empty_like(residual)
+    _lib.check(_lib.load().nvx_internal_decode_chain(table, len(layers), m, _ptr(qkv), _ptr(residual), _ptr(act), _ptr(new), _ptr(positions), _ptr(kv_start), _ptr(kv_len),
+                                                     _ptr(out_slots), _ptr(kv_indices), _ptr(cos_sin_cache), cos_sin_cache.shape[0], n_slots, _ptr(chain.words),
+                                                     _ptr(chain.epoch), chain.status.data_ptr(), DecodeChain.SECONDS, float(eps), float(sm_scale), _stream()), "decode_chain")
+    return act, new
 
 
 def rmsnorm_splitk(partials, weight, eps, residual=None):

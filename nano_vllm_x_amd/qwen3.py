@@ -471,6 +471,12 @@ class Qwen3Model(nn.Module):
         eps, attns = self.config.rms_norm_eps, [layer._modules["self_attn"]._modules["attn"] for layer in self.layers]
         md = attns[0].attention_metadata
         qkv = decode_linear(ops.rmsnorm(residual, layers[0][0], eps), layers[0][1], "qkv")
+        wrapper, first = md.wrapper, self.layers[0].self_attn
+        if wrapper.chain is not None and ops.DecodeChain.fits(residual.shape[0], len(layers), residual.shape[1], first.num_heads, first.num_kv_heads, layers[0][7].shape[1],
+                                                              residual.dtype):
+            act, residual = ops.decode_chain(wrapper.chain, [(*ws, *md.kv_cache.get_kv_cache(attn.layer_id)) for ws, attn in zip(layers, attns)], qkv, residual, positions,
+                                             *wrapper.table_of_step(), self.rope_table, eps, attns[0].scaling)
+            return self.norm(decode_linear(act, layers[-1][7], "down"), residual)[0]
         for i, ((_, _, nq, nk, o, n2, gate_up, down), attn) in enumerate(zip(layers, attns)):
             md.wrapper._sm_scale = attn.scaling
             read_out = md.wrapper.run_qkv(qkv, positions, self.rope_table, nq, nk, eps, md.kv_cache.get_kv_cache(attn.layer_id))
