@@ -4,13 +4,13 @@
 // Such a product is a few microseconds of matrix work, and what decides its time is how many workgroups the tile leaves to 256 CUs and what a
 // workgroup does between two steps of K.  So the tile follows the size, a workgroup keeps STAGES - 1 steps of both operands on their way (memory
 // -> LDS without registers, waited for by count, one barrier a step), and the next step's operands are read from LDS while the present one is
-// multiplied.  16-byte pieces are XOR-swizzled on the global side.  Small tiles are bound by LDS (a wave reads 3 bytes for every 2 it
-// multiplies), which splitting K over the waves would halve; but K is never split: a row's sum runs over K in order, in one chain of
+// multiplied.  16-byte pieces are XOR-swizzled on the global side.  Small tiles are bound by what they bring into a CU (see PREFILL_TILES) and by LDS (a wave reads 3 bytes for every 2
+// it multiplies), which splitting K over the waves would halve; but K is never split: a row's sum runs over K in order, in one chain of
 // v_mfma_f32_16x16x32, whatever the tile, so that a token's result does not depend on how many tokens share its step (and equals the library's
 // above some 200 rows, whose products take K in the same order).
-// The products of a layer of Qwen3-0.6B, us, qkv / o / gate | up / down (the library's without SiluAndMul's own 4 us):
-//     64 rows 4.6 / 6.0 / 5.8 / 7.5 (8.8 / 8.4 / 9.0 / 10.1),   216 rows 6.8 / 6.1 / 10.1 / 7.8 (9.4 / 8.9 / 13.4 / 9.4),
-//     459 rows 9.1 / 7.9 / 11.8 / 10.0 (11.2 / 9.7 / 13.6 / 12.5),   1536 rows 18.7 / 13.8 / 24.4 / 20.1 (17.7 / 13.7 / 28.9 / 17.1).
+// The products of a layer of Qwen3-0.6B with weights that no cache holds, us, qkv / o / gate | up / down: 100 rows 5.4 / 5.7 / 7.8 / 7.1, 200 rows 6.4 / 5.8 / 10.4 / 7.5,
+//     459 rows 8.9 / 7.5 / 12.4 / 9.8, 1500 rows 18.8 / 11.7 / 28.7 / 16.4 (the library with weights in its caches: 64 rows 8.8 / 8.4 / 9.0 and SiluAndMul's 4 / 10.1, 459 rows
+//     11.2 / 9.7 / 13.6 and 4 / 12.5, 1536 rows 17.7 / 13.7 / 28.9 and 4 / 17.1).
 #include "prefill_gemm.h"
 
 namespace NVX_NS {
@@ -153,33 +153,31 @@ static void launch_prefill_gemm(const void* x, int64_t x_stride, const void* w, 
 
 using namespace NVX_NS;
 
-struct PrefillTile { int m, n, slots; float us, us_silu; };
-// Tiles of many rows: workgroups that run at once, us of 1024 columns of K with the chip full of them (SILU: 64 x 128 in two stages, three a CU)
-static const PrefillTile PREFILL_TILES[] = {{256, 256, 256, 26.f, 26.f}, {192, 256, 256, 20.f, 20.f}, {128, 256, 256, 15.5f, 15.5f}, {128, 128, 256, 8.4f, 8.4f}, {64, 128, 512, 10.5f, 13.5f}};
+// What a tile costs, us of 1024 columns of K with weights that no cache holds: the first `slots` workgroups, and every further as many (0: not built).  Fitted to
+// 100 to 2560 rows of 4096, 2048 and 1024 outputs and, with SILU, of 6144 (deeper K: the same order).  Up to one workgroup a CU a product costs what its tile brings
+// into a CU, 82 KB a us whatever the kernel (rows of w straight to registers in operand order: the same times), so the tile that just fills the CUs is the best.
+struct PrefillTile { int tile, m, n, slots, silu_slots; float us, more, us_silu, more_silu; bool wide; };
+static const PrefillTile PREFILL_TILES[] = {
+    {NVX_PG_32_32, 32, 32, 256, 0, 4.2f, 1.65f, 0.f, 0.f, false},       {NVX_PG_32_64, 32, 64, 256, 256, 5.3f, 3.6f, 6.0f, 4.6f, false},
+    {NVX_PG_64_64, 64, 64, 256, 256, 6.4f, 2.9f, 7.7f, 3.6f, false},    {NVX_PG_96_64, 96, 64, 256, 0, 7.5f, 4.0f, 0.f, 0.f, false},
+    {NVX_PG_64_128, 64, 128, 256, 768, 9.2f, 4.9f, 20.5f, 17.f, false}, {NVX_PG_128_128, 128, 128, 256, 256, 10.6f, 8.4f, 12.5f, 9.5f, true},
+    {NVX_PG_128_256, 128, 256, 256, 256, 16.8f, 17.f, 25.f, 15.5f, true}, {NVX_PG_192_256, 192, 256, 256, 256, 18.6f, 7.f, 27.5f, 19.f, true},
+    {NVX_PG_256_256, 256, 256, 256, 256, 22.7f, 12.f, 31.f, 18.f, true}};
 
-// Few rows: the smallest tile whose workgroups all run at once (256 CUs; two a CU for 64 x 64) is the fastest at every size measured: us at
-// 459 rows of 1024 outputs from 2048 columns, 240 workgroups of 32 x 64: 7.9, 480 of 32 x 32: 8.4, 128 of 64 x 64: 9.9; 300 rows of 4096
-// outputs from 1024, 320 of 64 x 64: 8.8, 640 of 32 x 64: 13.6.  With SILU 64 x 64 in two stages (four workgroups a CU) holds on to 800 workgroups (459 rows 12.2,
-// 128 x 128 13.5; 600 rows, 960 workgroups, 14.4 and 13.8).
-// More rows: rounds of a tile's workgroups times what a round costs, by which every tile is chosen somewhere; us of 4096 outputs from 1024 columns, the
-// chosen / 64 x 128: 700 rows 11.8 (128 x 128) / 12.9, 1536 rows 18.7 (128 x 256) / 20.5, 2160 rows 22 (192 x 256) / 30, 4096 rows 32 (256 x 256) / 45; with SILU
-// 6144 from 1024, 1536 rows 24 (192 x 256) / 27, 2160 rows 31 (256 x 256) / 39.
+// The least of those.  us with cold weights, the rule before (the smallest tile whose workgroups all run at once, from some size on rounds times a round's cost) and
+// this one: SILU 6144 x 1024, 384 rows 14.9 and 12.9, 459 15.2 and 12.4, 512 16.2 and 13.0, 1100 25.6 and 22.1, 1200 25.5 and 24.7; 1024 x 3072, 1100 rows 20.2 and 15.9, 1500
+// 20.3 and 16.3, 2000 23.3 and 20.9; 1024 x 2048, 1500 rows 13.2 and 11.7, 2560 18.9 and 17.1; 4096 x 1024, 700 rows 11.1 and 10.6, 1100 17.6 and 16.6.
 // QKV: of 129 to 512 rows (prefill_step.hip), where a head's norm and rotation behind the product are less than their own launch (459 rows 12.4, product and launch 14; 1024 rows 17.6
-// and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).
+// and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).  Its tiles of 64, 96 and 128 rows: 0.99 to 1.02 of a step of 300 to 1024 tokens.
 static int prefill_gemm_rule(int64_t m, int64_t n, bool silu, bool wide) {
-    auto tiles = [&](int64_t tm, int64_t tn) { return (m + tm - 1) / tm * (n / tn); };
-    if (!silu && tiles(32, 32) <= 256) return NVX_PG_32_32;
-    if (tiles(32, 64) <= 256) return NVX_PG_32_64;
-    if (tiles(64, 64) <= 512) return NVX_PG_64_64;
-    if (silu && tiles(64, 64) <= 800) return NVX_PG_64_64_TWO;
     int best = NVX_PG_64_128;
     float least = 0.f;
-    for (int i = 4; i >= 0; --i) {
-        const PrefillTile& t = PREFILL_TILES[i];
-        if (n % t.n || (i < 4 && !wide)) continue;
-        const int slots = silu && i == 4 ? 768 : t.slots;
-        const float cost = (float)((tiles(t.m, t.n) + slots - 1) / slots) * (silu ? t.us_silu : t.us);
-        if (i == 4 || cost < least) best = NVX_PG_256_256 + i, least = cost;
+    for (const PrefillTile& t : PREFILL_TILES) {
+        const int slots = silu ? t.silu_slots : t.slots;
+        if (!slots || n % t.n || (t.wide && !wide)) continue;
+        const int64_t rounds = ((m + t.m - 1) / t.m * (n / t.n) + slots - 1) / slots;
+        const float cost = (silu ? t.us_silu : t.us) + (float)(rounds - 1) * (silu ? t.more_silu : t.more);
+        if (least == 0.f || cost < least) best = t.tile, least = cost;
     }
     return best;
 }
@@ -196,13 +194,13 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
     if (mode == NVX_PG_QKV) tile = NVX_PG_32_128;
     else if (tile == 0) tile = prefill_gemm_rule(m, n, silu, x_stride < (1 << 21) && n * k < (1ll << 30));       // (what the wide tiles' offsets hold)
     if (tile >= NVX_PG_256_256 && tile < NVX_PG_64_128)
-        return NVX_ENTRY(nvx_prefill_wide)(x, x_stride, w, y, m, n, k, silu, PREFILL_TILES[tile - NVX_PG_256_256].m, PREFILL_TILES[tile - NVX_PG_256_256].n, st);
+        return NVX_ENTRY(nvx_prefill_wide)(x, x_stride, w, y, m, n, k, silu, tile == NVX_PG_256_256 ? 256 : tile == NVX_PG_192_256 ? 192 : 128, tile == NVX_PG_128_128 ? 128 : 256, st);
 #define NVX_PG(TM, TN, KS, ST, MODE) launch_prefill_gemm<TM, TN, KS, ST, 2, MODE>(x, x_stride, w, y, m, n, k, qkv, st)
     switch (tile) {
         case NVX_PG_64_128: if (silu) NVX_PG(64, 128, 64, 2, NVX_PG_SILU); else NVX_PG(64, 128, 64, 3, NVX_PG_PLAIN); break;
         case NVX_PG_64_64: if (silu) NVX_PG(64, 64, 64, 4, NVX_PG_SILU); else NVX_PG(64, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_64: if (silu) NVX_PG(32, 64, 128, 4, NVX_PG_SILU); else NVX_PG(32, 64, 128, 4, NVX_PG_PLAIN); break;
-        case NVX_PG_64_64_TWO: NVX_REQUIRE(silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(64, 64, 64, 2, NVX_PG_SILU); break;
+        case NVX_PG_96_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(96, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_32: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 32, 128, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_128: NVX_REQUIRE(mode == NVX_PG_QKV, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 128, 64, 4, NVX_PG_QKV); break;
         default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);

@@ -1,0 +1,24 @@
+"""The tile of 96 x 64 of csrc/prefill_gemm.hip: edges of tiles, one and several rounds of workgroups, rows apart, against the tile of 64 x 64 (held to float64 elsewhere)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 256), (95, 128, 256), (96, 256, 512), (97, 128, 768), (1025, 1024, 2048), (1100, 4096, 256), (1536, 1024, 256)])
+def test_one_order_of_summation(dtype, m, n, k):
+    from nano_vllm_x_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 64, generator=gen, device="cuda").to(dtype)[:, 32:32 + k]
+    w = (torch.randn(n, k, generator=gen, device="cuda") * k ** -0.5).to(dtype)
+    fn, out = getattr(_lib.load(), "nvx_internal_prefill_gemm" + ("_f16" if dtype == torch.float16 else "")), []
+    for tile in (6, 7, 0):       # 64 x 64, 96 x 64, by the rule
+        y = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+        _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 0, tile, ops._stream()))
+        out.append(y)
+    assert bool(torch.isfinite(out[0]).all()) and torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    y = torch.empty((m, n // 2), dtype=dtype, device="cuda")
+    with pytest.raises(RuntimeError):
+        _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 1, 7, ops._stream()))
