@@ -23,6 +23,8 @@ namespace NVX_NS {
 
 
 #define PF_KVBLK 64
+#define PF_RING 3               // tiles of a workgroup with waves that only fetch
+#define PF_IDS (2 * PF_RING)    // tiles whose slot ids such a wave keeps
 #define PF_LOG2E 1.4426950408889634f
 
 typedef __attribute__((ext_vector_type(4))) short pf_s16x4;
@@ -156,17 +158,20 @@ extern "C" int nvx_debug_pf_stamps(unsigned long long* host) { return (int)hipMe
 #endif
 
 // ---------------------------------------------------------------------------------------------
-template <int G, int NWAVES>
-__global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
+// LOADERS > 0: that many more waves fetch the tiles, PF_RING of them in LDS, and the others only compute.  For launches that leave a CU one workgroup or little
+// more: there nothing runs beside a workgroup's own chain of tiles, of whose 3450 clocks a tile the copies' addresses and issue are 600 and the wait for them 340.  With two
+// workgroups a CU either hides the other's and the registers of eight more waves would not fit.  The sums are the same, bit for bit.
+template <int G, int NWAVES, int LOADERS>
+__global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void paged_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t q_stride, const uint16_t* __restrict__ k_cache,
     const uint16_t* __restrict__ v_cache, int64_t n_slots, const int32_t* __restrict__ qo_indptr,
     const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_indices, const int32_t* __restrict__ plan,
     uint16_t* __restrict__ out, int batch, int hkv, float scale_log2) {
-    constexpr int NT = NWAVES * 64;
+    constexpr int NT = (NWAVES + LOADERS) * 64;
     constexpr int POSB = NWAVES / G;          // 32-row position blocks per workgroup
     constexpr int QPOS = 32 * POSB;           // query positions per workgroup
     constexpr int TAB = QPOS == 32 ? 0 : (QPOS == 64 ? 1 : 2);
-    constexpr int KEYS_PER_PASS = NT / 16;    // 16 lanes move one 256-byte row
+    constexpr int KEYS_PER_PASS = (LOADERS ? LOADERS : NWAVES) * 4;    // 16 lanes move one 256-byte row
     constexpr int PASSES = PF_KVBLK / KEYS_PER_PASS;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     // two tile buffers of [K: 64 keys x 256 B, pieces swizzled by key & 15][V: same, swizzled by (key & 3) << 2],
@@ -187,7 +192,8 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
     // of every workgroup's first tile; this is one.)
     // (the counters sit behind the tile buffers: the fragment addressing XORs address bits and needs the
     // buffers at a 256-byte boundary, which a static LDS array in front of them would break)
-    int* owner_count = reinterpret_cast<int*>(smem + 2 * BUF_BYTES + 2 * IDS_BYTES);
+    constexpr int RING = LOADERS ? PF_RING : 2, ID_TILES = LOADERS ? LOADERS * PF_IDS : 2;
+    int* owner_count = reinterpret_cast<int*>(smem + RING * BUF_BYTES + ID_TILES * IDS_BYTES);
     int below = 0;
     for (int i = tid; i < batch; i += NT) below += tab[1 + i] <= gblk ? 1 : 0;
 #pragma unroll
@@ -196,7 +202,7 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
     __syncthreads();
     int b = -1;
 #pragma unroll
-    for (int w = 0; w < NWAVES; ++w) b += owner_count[w];
+    for (int w = 0; w < NWAVES + LOADERS; ++w) b += owner_count[w];
     b = __builtin_amdgcn_readfirstlane(b < 0 ? 0 : b);
     // blocks of a sequence are taken last first: the last query block sees the most keys, and the launch should end
     // on short blocks, not on the longest ones
@@ -215,6 +221,40 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
     const int wave_first_vis = qb * QPOS + pb * 32 + offset;      // last key the wave's FIRST query sees
     const int n_tiles = (kmax + PF_KVBLK - 1) / PF_KVBLK;
 
+    if constexpr (LOADERS > 0) {
+        if (wave >= NWAVES) {
+            // A loader wave has the same keys of every tile, and every tile's ids in LDS of its own, PF_RING tiles before their rows (operations complete
+            // in order, so the wait for a tile's rows is a wait for the ids of the rows that are asked for next).
+            const int me = wave - NWAVES, pos = lane & 15, krow0 = me * 4 + (lane >> 4);
+            const int32_t* seq_slots = kv_indices + kv0;
+            const unsigned char* kg = reinterpret_cast<const unsigned char*>(k_cache) + head * 256 + ((pos ^ (krow0 & 15)) << 4);
+            const unsigned char* vg = reinterpret_cast<const unsigned char*>(v_cache) + head * 256 + ((pos ^ ((krow0 & 3) << 2)) << 4);
+            const unsigned n_slots_u = n_slots > 0xffffffffll ? 0xffffffffu : (unsigned)n_slots;
+            const unsigned lds0 = pf_lds_addr(smem), rows = (unsigned)__builtin_amdgcn_readfirstlane(me * 4 * 256);
+            const unsigned ids = lds0 + (unsigned)__builtin_amdgcn_readfirstlane(RING * BUF_BYTES + me * PF_IDS * IDS_BYTES);
+            auto fetch_ids = [&](int t) { pf_fetch_slot_ids(seq_slots, t, lkv, lane, ids + (t % PF_IDS) * IDS_BYTES); };
+            auto fetch_rows = [&](int t) {
+                const unsigned at = lds0 + (unsigned)(t % RING) * BUF_BYTES + rows;
+                pf_gather<PASSES, KEYS_PER_PASS>(ids + (t % PF_IDS) * IDS_BYTES, krow0, n_slots_u, kg, vg, (unsigned)hkv * 256u, at, at + PF_KVBLK * 256);
+            };
+            for (int t = 0; t < n_tiles && t < 2 * RING - 1; ++t) fetch_ids(t);
+            pf_wait_copies();
+            for (int t = 0; t < n_tiles && t < RING - 1; ++t) fetch_rows(t);
+            if (n_tiles > RING - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "n"((RING - 2) * 2 * PASSES) : "memory");
+            else pf_wait_copies();
+            __syncthreads();
+            for (int t = 0; t < n_tiles; ++t) {
+                if (t + RING - 1 < n_tiles) fetch_rows(t + RING - 1);              // (to where tile t - 1 was)
+                if (t + 2 * RING - 1 < n_tiles) {
+                    fetch_ids(t + 2 * RING - 1);
+                    // since the rows of tile t + 1: the ids asked for behind them, RING - 2 tiles
+                    asm volatile("s_waitcnt vmcnt(%0)" : : "n"((RING - 2) * (2 * PASSES + 1)) : "memory");
+                } else pf_wait_copies();
+                __syncthreads();
+            }
+            return;
+        }
+    }
     // Q^T fragments: 8 k-steps of 16 dims; lane holds dims 16*ks + 8*half .. +7 of its query row
     nvx_h16x8 qf[8];
     {
@@ -234,7 +274,7 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
         for (int r = 0; r < 16; ++r) o_acc[d][r] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
 
-    static_assert(PASSES == 2 || PASSES == 4, "tile gather is written for 256- or 512-thread workgroups");
+    static_assert(PASSES == 2 || PASSES == 4, "tile gather is written for four or eight waves");
     // Pipeline, one barrier per tile: while tile t is computed from one buffer, the rows of tile t + 1 travel
     // pool -> LDS into the other and the slot ids of tile t + 2 block table -> LDS.
     const int pos = tid & 15, krow0 = tid >> 4;
@@ -256,7 +296,7 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
     }();
     unsigned ring0 = lds0, ring1 = lds0 + BUF_BYTES;                 // tile being computed, tile arriving
     unsigned ids0 = lds0 + 2 * BUF_BYTES, ids1 = ids0 + IDS_BYTES;     // slot ids of the next tile, of the one after
-    if (n_tiles > 0) {
+    if (LOADERS == 0 && n_tiles > 0) {
         if (wave == 0) {
             pf_fetch_slot_ids(seq_slots, 0, lkv, lane, ids0);
             if (n_tiles > 1) pf_fetch_slot_ids(seq_slots, 1, lkv, lane, ids1);
@@ -281,7 +321,7 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
         PF_STAMP(0);
         const unsigned k_lds = ring0;   // LDS byte addresses
         const unsigned v_lds = k_lds + PF_KVBLK * 256;
-        if (tile + 1 < n_tiles) {   // the other buffer held tile t - 1: every wave left it before the last barrier
+        if (LOADERS == 0 && tile + 1 < n_tiles) {   // the other buffer held tile t - 1: every wave left it before the last barrier
             if (tile > 0)           // (tile 1 came with tile 0)
                 pf_gather<PASSES, KEYS_PER_PASS>(ids0, krow0, n_slots_u, kg, vg, row_bytes, ring1 + wave_rows, ring1 + PF_KVBLK * 256 + wave_rows);
             if (tile + 2 < n_tiles && wave == 0) pf_fetch_slot_ids(seq_slots, tile + 2, lkv, lane, ids1);
@@ -419,11 +459,12 @@ __global__ __launch_bounds__(NWAVES * 64, 2) void paged_prefill_kernel(
         };
         if (key_base + 32 <= wave_last_key) tile_body(std::integral_constant<int, 2>{});        // wave-uniform
         else if (key_base <= wave_last_key) tile_body(std::integral_constant<int, 1>{});        // else: nothing visible
-        pf_wait_copies();
+        if (LOADERS == 0) pf_wait_copies();
         PF_STAMP(6);
         __syncthreads();   // tile + 1 and the ids of tile + 2 visible; this tile's buffer free
         PF_STAMP(7);
-        { const unsigned t0 = ring0; ring0 = ring1; ring1 = t0; }
+        if (LOADERS) ring0 = ring0 == lds0 + (RING - 1) * BUF_BYTES ? lds0 : ring0 + BUF_BYTES;
+        else { const unsigned t0 = ring0; ring0 = ring1; ring1 = t0; }
         { const unsigned t0 = ids0; ids0 = ids1; ids1 = t0; }
     }
 
@@ -480,26 +521,39 @@ extern "C" int NVX_ENTRY(nvx_paged_prefill)(const void* q, int64_t q_row_stride,
     // two tile buffers of K and V, two tiles of slot ids, per-wave counters; at the end the same memory
     // stages the output, 32 rows of 272 B per wave
     const size_t loop_bytes = 2 * 2 * PF_KVBLK * 256 + 2 * 4 * PF_KVBLK + 64;
-#define NVX_PF(GG, NW, QPOS)                                                                                           \
+#define NVX_PF(GG, NW, QPOS, LD)                                                                                       \
     do {                                                                                                                \
-        const size_t lds_bytes = loop_bytes > (size_t)(NW) * 32 * 272 ? loop_bytes : (size_t)(NW) * 32 * 272;           \
-        static const hipError_t attr = hipFuncSetAttribute((const void*)paged_prefill_kernel<GG, NW>,                   \
+        const size_t need = (LD) ? (size_t)PF_RING * 2 * PF_KVBLK * 256 + (size_t)(LD) * PF_IDS * 4 * PF_KVBLK + 64 : loop_bytes; \
+        const size_t lds_bytes = need > (size_t)(NW) * 32 * 272 ? need : (size_t)(NW) * 32 * 272;                       \
+        static const hipError_t attr = hipFuncSetAttribute((const void*)paged_prefill_kernel<GG, NW, LD>,               \
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes); \
         NVX_REQUIRE(attr == hipSuccess, NVX_ELAUNCH, "nvx_paged_prefill: cannot reserve %d KB of LDS", (int)(lds_bytes / 1024)); \
         const int64_t blocks = ((n_tokens + (QPOS) - 1) / (QPOS) + batch) * n_kv_heads;                                 \
-        hipLaunchKernelGGL((paged_prefill_kernel<GG, NW>), dim3((unsigned)blocks), dim3((NW) * 64), lds_bytes, st,      \
+        hipLaunchKernelGGL((paged_prefill_kernel<GG, NW, LD>), dim3((unsigned)blocks), dim3(((NW) + (LD)) * 64), lds_bytes, st, \
                            (const uint16_t*)q, q_row_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache,        \
                            n_slots, qo_indptr, kv_indptr, kv_indices, plan_ws, (uint16_t*)out, (int)batch, n_kv_heads,  \
                            scale_log2);                                                                                 \
     } while (0)
+    // Few workgroups (of so many query positions, at most): waves of their own for the copies, and 32 positions of two heads as two waves, which read half as much LDS a tile.  us a
+    // step of Qwen3-0.6B before and now: 40 tokens 1378 and 1327, 459 2041 and 1970, 1024 2963 and 2843, 3000 6431 and 6068; 2160 tokens behind 900-3000 cached ones (320 workgroups)
+    // 5591 and 5382, 480 behind as many 3330 and 3057; 32 positions at 328 workgroups 3051 where 64 are 3031; 64 at 392 workgroups 5512 and 5338, at 488 5320 and 5330, at 592 7545 and 7734.
+    // Qwen3-8B, four layers: 459 tokens 1345 and 1324, 1500 2671 and 2634.
+    const auto groups = [&](int64_t positions) { return ((n_tokens + positions - 1) / positions + batch - 1) * n_kv_heads; };
     switch (g) {
-        case 1: NVX_PF(1, 4, 128); break;
+        case 1: NVX_PF(1, 4, 128, 0); break;
         // two 4-wave workgroups per CU (each in its own phase of the tile loop) measured faster than one
         // 8-wave workgroup of 128 queries (0.75 vs 0.86 ms on the bench prompts); a third tile buffer (row
         // copies two tiles ahead) changed neither
-        case 2: NVX_PF(2, 4, 64); break;
-        case 4: NVX_PF(4, 4, 32); break;   // 8 waves / 64 queries measured slower here too (1.77 vs 1.57 ms at 32 q heads)
-        case 8: NVX_PF(8, 8, 32); break;
+        case 2:
+            if (groups(32) <= 256) NVX_PF(2, 2, 32, 4);
+            else if (groups(64) <= 392) NVX_PF(2, 4, 64, 4);
+            else NVX_PF(2, 4, 64, 0);
+            break;
+        case 4:
+            if (groups(32) <= 392) NVX_PF(4, 4, 32, 4);
+            else NVX_PF(4, 4, 32, 0);
+            break;   // 8 waves / 64 queries measured slower here too (1.77 vs 1.57 ms at 32 q heads)
+        case 8: NVX_PF(8, 8, 32, 0); break;
         default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_paged_prefill: query/kv head ratio %d not in {1,2,4,8}", g);
     }
 #undef NVX_PF

@@ -1,0 +1,43 @@
+"""Attention of prompts in launches of few workgroups, whose tiles are fetched by waves of their own: the bits of the same sequences among many others."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(q, k, v, parts, slots, hq, hkv):
+    """parts: (queries, keys) of each sequence, whose queries are the next rows of q and keys the next of the slot list."""
+    from nano_vllm_x_amd import ops
+
+    ends = torch.tensor([(0, 0)] + list(parts)).cumsum(0).to(torch.int32).cuda()
+    qo, kv = ends[:, 0].contiguous(), ends[:, 1].contiguous()
+    plan = ops.prefill_plan_ws(len(parts), "cuda")
+    ops.prefill_plan(qo, plan)
+    return ops.paged_prefill(q, k, v, qo, kv, slots, plan, hq, hkv, 128 ** -0.5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv", [(4, 2), (8, 2)])
+@pytest.mark.parametrize("parts", [((1, 1),), ((31, 31),), ((33, 64),), ((64, 65),), ((1, 128),), ((129, 129),), ((200, 700),), ((449, 449), (2, 300)), ((3, 3), (65, 1000), (1, 64), (640, 641)),
+                                   ((1000, 1400), (500, 500), (300, 2000))])
+def test_the_same_alone_and_among_others(dtype, hq, hkv, parts):
+    gen = torch.Generator(device="cuda").manual_seed(sum(a + 7 * b for a, b in parts))
+    filler = ((64, 64),) * 200           # so many workgroups that the copies are every wave's
+    nq, nk = (sum(p[i] for p in parts + filler) for i in (0, 1))
+    q = torch.randn(nq, hq * 128, generator=gen, device="cuda").to(dtype)
+    k, v = (torch.randn(nk, hkv, 128, generator=gen, device="cuda").to(dtype) for _ in range(2))
+    slots = torch.randperm(nk, generator=gen, device="cuda").to(torch.int32)
+    n = sum(p[0] for p in parts)
+    alone = _run(q[:n], k, v, parts, slots, hq, hkv)
+    among = _run(q, k, v, parts + filler, slots, hq, hkv)
+    assert bool(torch.isfinite(alone).all()) and torch.equal(alone, among[:n])
+    # one sequence against float64
+    (a, b), heads = parts[0], hq // hkv
+    rows = slots[:b].long()
+    s = torch.einsum("ihd,jhd->hij", q[:a].view(a, hq, 128).double(), k[rows].double().repeat_interleave(heads, 1)) * 128 ** -0.5
+    s = s.masked_fill(torch.arange(b, device="cuda")[None] > torch.arange(a, device="cuda")[:, None] + b - a, -torch.inf).softmax(2)
+    want = torch.einsum("hij,jhd->ihd", s, v[rows].double().repeat_interleave(heads, 1)).reshape(a, -1)
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    size = torch.einsum("hij,jhd->ihd", s, v[rows].double().abs().repeat_interleave(heads, 1)).reshape(a, -1)
+    # weights rounded to the format (half a unit each, the sum of them is not), the result once more; scores in float32
+    assert bool(((alone[:a].double() - want).abs() <= unit * size + unit * want.abs() + 2.0 ** -14 * size).all())
