@@ -158,6 +158,66 @@ extern "C" int nvx_debug_pf_stamps(unsigned long long* host) { return (int)hipMe
 #endif
 
 // ---------------------------------------------------------------------------------------------
+// Blocks of up to PF_SORTED sequences, longest first over all of them: sequence b has one block at each of the levels (its first query's position over
+// QPOS) from its cached tokens on.  In the order of the sequences a launch of two workgroups a CU ended on whatever came last: 32 prompts of 100 to 1024 tokens, 2088
+// workgroups of 15 us in the mean, 512 at a time, took 82 us.  Many short blocks (more than PF_SORT_BLOCKS, none that sees PF_SORT_KEYS) stay in the order of the
+// sequences, whose neighbours share their keys in an XCD's L2.  No plan is read (two trips to memory less ahead of the first keys, and no launch of the plan).  Qwen3-0.6B, us a step by
+// the plan, in order of length throughout, and by this rule: 8 prompts of 200-900 tokens 7086 / 6938 / 6918, 32 of 100-1024 21620 / 21395 / 21427, 64 of 20-400 13597 / 13595 / 13488, 20 of
+// 100-400 behind 30-1000 cached ones 7739 / 7508 / 7498; with the waves for the copies (below) 9 of 100-400 behind 900-3000 6326 / - / 5330.
+#define PF_SORTED 64
+#define PF_SORT_BLOCKS 128
+#define PF_SORT_KEYS 704
+struct PfBlock { int qb, q0, lq, kv0, lkv; };       // qb < 0: there is none
+__device__ __forceinline__ int pf_wave_sum(int v) {
+    float f = __builtin_bit_cast(float, v);
+    auto add = [&](float o) { f = __builtin_bit_cast(float, __builtin_bit_cast(int, f) + __builtin_bit_cast(int, o)); };
+    add(dpp_move<0xB1>(f));
+    add(dpp_move<0x4E>(f));
+    add(dpp_move<0x141>(f));
+    add(dpp_move<0x140>(f));
+    add(xor16(f));
+    add(xor32(f));
+    return __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f));
+}
+template <int QPOS>
+__device__ __forceinline__ PfBlock pf_block_of(const int32_t* __restrict__ qo_indptr, const int32_t* __restrict__ kv_indptr, int batch, int gblk, int lane) {
+    int q0 = 0, q1 = 0, k0 = 0, k1 = 0;
+    if (lane < batch) { q0 = qo_indptr[lane]; q1 = qo_indptr[lane + 1]; k0 = kv_indptr[lane]; k1 = kv_indptr[lane + 1]; }
+    const int lq = q1 - q0, lkv = k1 - k0, nb = lq > 0 ? (lq + QPOS - 1) / QPOS : 0, base = lkv > lq ? (lkv - lq) / QPOS : 0, end = nb ? base + nb : 0;
+    PfBlock w = {-1, 0, 0, 0, 0};
+    const int total = pf_wave_sum(nb);
+    if (gblk >= total) return w;
+    auto take = [&](int b, int qb) {
+        w.qb = qb;
+        w.q0 = __builtin_amdgcn_readlane(q0, b);
+        w.lq = __builtin_amdgcn_readlane(lq, b);
+        w.kv0 = __builtin_amdgcn_readlane(k0, b);
+        w.lkv = __builtin_amdgcn_readlane(lkv, b);
+    };
+    if (total > PF_SORT_BLOCKS && !__any(end * QPOS >= PF_SORT_KEYS)) {
+        int upto = nb;
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) { const int o = __shfl_up(upto, s, 64); if (lane >= s) upto += o; }
+        const int b = __popcll(__ballot(upto <= gblk));
+        take(b, __builtin_amdgcn_readlane(upto, b) - 1 - gblk);
+        return w;
+    }
+    auto from_level = [&](int level) { return pf_wave_sum(min(max(end - level, 0), nb)); };
+    int lo = 0, hi = 1;                              // the highest level with more than gblk blocks from it on
+    while (__any(end > hi)) hi *= 2;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (from_level(mid) > gblk) lo = mid;
+        else hi = mid;
+    }
+    const int nth = gblk - from_level(lo + 1);       // of the sequences that have a block of this level (a sum over the wave: not behind &&)
+    const bool has = nb && base <= lo && lo < end;
+    const unsigned long long there = __ballot(has);
+    const int rank = __popcll(there & ((1ull << lane) - 1)), b = __ffsll((long long)__ballot(has && rank == nth)) - 1;
+    take(b, lo - __builtin_amdgcn_readlane(base, b));
+    return w;
+}
+
 // LOADERS > 0: that many more waves fetch the tiles, PF_RING of them in LDS, and the others only compute.  For launches that leave a CU one workgroup or little
 // more: there nothing runs beside a workgroup's own chain of tiles, of whose 3450 clocks a tile the copies' addresses and issue are 600 and the wait for them 340.  With two
 // workgroups a CU either hides the other's and the registers of eight more waves would not fit.  The sums are the same, bit for bit.
@@ -181,34 +241,41 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int half = lane >> 5, l32 = lane & 31;
-    const int32_t* tab = plan + TAB * (batch + 2);
-    const int total_blocks = tab[0];
     const int unit = blockIdx.x;
     const int gblk = unit / hkv, head = unit % hkv;
-    if (gblk >= total_blocks) return;
-    // Sequence that owns query block gblk: the last b with tab[1 + b] <= gblk.  The table is
-    // non-decreasing, so b + 1 is the number of entries <= gblk: every thread tests some entries and the
-    // workgroup adds up.  (A binary search is log2(batch) dependent loads, several microseconds in front
-    // of every workgroup's first tile; this is one.)
     // (the counters sit behind the tile buffers: the fragment addressing XORs address bits and needs the
     // buffers at a 256-byte boundary, which a static LDS array in front of them would break)
     constexpr int RING = LOADERS ? PF_RING : 2, ID_TILES = LOADERS ? LOADERS * PF_IDS : 2;
-    int* owner_count = reinterpret_cast<int*>(smem + RING * BUF_BYTES + ID_TILES * IDS_BYTES);
-    int below = 0;
-    for (int i = tid; i < batch; i += NT) below += tab[1 + i] <= gblk ? 1 : 0;
+    int qb, q0, lq, kv0, lkv;
+    if (batch <= PF_SORTED) {
+        // Every wave finds the block for itself, in one trip to memory: of all sequences' blocks the one that sees the gblk-th most keys.
+        const PfBlock w = pf_block_of<QPOS>(qo_indptr, kv_indptr, batch, gblk, lane);
+        if (w.qb < 0) return;
+        qb = w.qb; q0 = w.q0; lq = w.lq; kv0 = w.kv0; lkv = w.lkv;
+    } else {
+        const int32_t* tab = plan + TAB * (batch + 2);
+        if (gblk >= tab[0]) return;
+        // Sequence that owns query block gblk: the last b with tab[1 + b] <= gblk.  The table is
+        // non-decreasing, so b + 1 is the number of entries <= gblk: every thread tests some entries and the
+        // workgroup adds up.  (A binary search is log2(batch) dependent loads, several microseconds in front
+        // of every workgroup's first tile; this is one.)
+        int* owner_count = reinterpret_cast<int*>(smem + RING * BUF_BYTES + ID_TILES * IDS_BYTES);
+        int below = 0;
+        for (int i = tid; i < batch; i += NT) below += tab[1 + i] <= gblk ? 1 : 0;
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) below += __shfl_xor(below, m, 64);
-    if (lane == 0) owner_count[wave] = below;
-    __syncthreads();
-    int b = -1;
+        for (int m = 32; m >= 1; m >>= 1) below += __shfl_xor(below, m, 64);
+        if (lane == 0) owner_count[wave] = below;
+        __syncthreads();
+        int b = -1;
 #pragma unroll
-    for (int w = 0; w < NWAVES + LOADERS; ++w) b += owner_count[w];
-    b = __builtin_amdgcn_readfirstlane(b < 0 ? 0 : b);
-    // blocks of a sequence are taken last first: the last query block sees the most keys, and the launch should end
-    // on short blocks, not on the longest ones
-    const int qb = tab[2 + b] - 1 - gblk;
-    const int q0 = qo_indptr[b], lq = qo_indptr[b + 1] - q0;
-    const int kv0 = kv_indptr[b], lkv = kv_indptr[b + 1] - kv0;
+        for (int w = 0; w < NWAVES + LOADERS; ++w) b += owner_count[w];
+        b = __builtin_amdgcn_readfirstlane(b < 0 ? 0 : b);
+        // blocks of a sequence are taken last first: the last query block sees the most keys, and the launch should end
+        // on short blocks, not on the longest ones
+        qb = tab[2 + b] - 1 - gblk;
+        q0 = qo_indptr[b]; lq = qo_indptr[b + 1] - q0;
+        kv0 = kv_indptr[b]; lkv = kv_indptr[b + 1] - kv0;
+    }
     const int offset = lkv - lq;              // query i sees keys 0 .. i + offset
     const int g = wave % G, pb = wave / G;
     const int qi = qb * QPOS + pb * 32 + l32;  // this lane's query (position within the new tokens)

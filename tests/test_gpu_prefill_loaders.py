@@ -41,3 +41,20 @@ def test_the_same_alone_and_among_others(dtype, hq, hkv, parts):
     size = torch.einsum("hij,jhd->ihd", s, v[rows].double().abs().repeat_interleave(heads, 1)).reshape(a, -1)
     # weights rounded to the format (half a unit each, the sum of them is not), the result once more; scores in float32
     assert bool(((alone[:a].double() - want).abs() <= unit * size + unit * want.abs() + 2.0 ** -14 * size).all())
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130])
+def test_blocks_in_order_of_length(n):
+    """Up to 64 sequences the longest blocks of all go first, more in the order of the sequences: every row is computed, empty sequences among them, and gives the bits it gives alone."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    parts = [(0 if i % 7 == 3 else (17 * i * i + 5) % 210 + 1, 0) for i in range(n)]
+    parts = [(a, a + (61 * i) % 400) for i, (a, _) in enumerate(parts)]
+    nq, nk = (sum(p[i] for p in parts) for i in (0, 1))
+    q = torch.randn(nq, 4 * 128, generator=gen, device="cuda").bfloat16()
+    k, v = (torch.randn(nk, 2, 128, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    slots = torch.randperm(nk, generator=gen, device="cuda").to(torch.int32)
+    got, at_q, at_k = _run(q, k, v, parts, slots, 4, 2), 0, 0
+    for a, b in parts:
+        if a:
+            assert torch.equal(_run(q[at_q:at_q + a], k, v, [(a, b)], slots[at_k:at_k + b].clone(), 4, 2), got[at_q:at_q + a])
+        at_q, at_k = at_q + a, at_k + b
