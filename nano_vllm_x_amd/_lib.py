@@ -189,6 +189,14 @@ class TableChoices(ctypes.Structure):
                 ("top", _c_i32 * TABLE_LAYERS), ("share", ctypes.c_float * TABLE_LAYERS)]
 
 
+class MemoryStep(ctypes.Structure):
+    """NvxMemoryStep of csrc/state_scan.hip, field by field."""
+    _fields_ = [(n, _c_vp) for n in ("x", "h", "w1", "w2", "bias", "norm", "S", "N", "M", "pos0", "state_slot", "out")] \
+        + [(n, _c_i64) for n in ("x_stride", "h_stride", "out_stride", "n_seq", "n_slots")] \
+        + [(n, _c_i32) for n in ("kind", "fmt", "q_off", "k_off", "v_off", "g_off", "heads", "dim", "vdim", "k_in", "rank", "norm_shared")] \
+        + [(n, _c_f32) for n in ("q_mul", "cap", "power", "eps")]
+
+
 # What the host of this package calls beside the C ABI; not declared in include/nvx.h
 INTERNAL = {name: (_c_i32, [ctypes.POINTER(PrefillStep), _c_vp]) for name in ("nvx_internal_prefill_step", "nvx_internal_prefill_step_f16")}
 INTERNAL.update({name: (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_vp])
@@ -199,6 +207,7 @@ INTERNAL["nvx_internal_moe_grouped"] = (_c_i32, SIGNATURES["nvx_moe_expert_rows"
 INTERNAL["nvx_internal_moe_tile"] = (_c_i32, [_c_i64] * 4)
 INTERNAL["nvx_internal_decode_boundary"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_vp, _c_f32, _c_vp, _c_vp, _c_vp, _c_vp])
 INTERNAL["nvx_internal_linear_decode_scaled"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_vp, _c_f32, _c_vp])
+INTERNAL["nvx_internal_memory_step"] = (_c_i32, [ctypes.POINTER(MemoryStep), _c_vp])
 INTERNAL["nvx_internal_decode_chain_words"] = (_c_i64, [])
 INTERNAL["nvx_internal_decode_chain_fits"] = (_c_i32, [])
 INTERNAL["nvx_internal_decode_chain"] = (_c_i32, [_c_vp, _c_i64, _c_i64] + [_c_vp] * 10 + [_c_i64, _c_i64, _c_vp, _c_vp, _c_vp, ctypes.c_double, _c_f32, _c_f32, _c_vp])

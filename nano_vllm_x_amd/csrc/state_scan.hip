@@ -706,10 +706,61 @@ __global__ __launch_bounds__(256) void decay_step_kernel(const A* __restrict__ x
 // step costs is the memory, read and written once: a workgroup has one head of one sequence, a thread four columns of every n_groups-th
 // row, eight rows' loads in flight together, and the groups' partial read-outs are added through LDS.  The scan kernels keep a column of 32
 // rows a thread (loads of 4 bytes) and stage for many tokens.  16 sequences, 8 heads of 64 x 128, us: gla 13.9 -> 6.6, mlstm 14.3 -> 7.6; 16 heads, decay 14.7 -> 7.7.
-template <typename A, int KIND>
-__global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
+//
+// ENDS: the small float32 projections in front (mlstm's two gates of the head; gla's decays through `rank` numbers, computed again by every
+// head) and the norm and gate of the read-out (as at decay_step_kernel) are part of the launch.  Everything that waits for nothing is asked
+// for first: the memory's first rows, the gate, the weights.  16 sequences, 8 heads of 64 x 128, rows of 1024, us of all launches (and the gaps between them
+// fall away): gla with 16 numbers 6.8 + 5.3 + 4.8 + 3.6 -> 11.9, mlstm 7.4 + 5.3 + 3.6 -> 9.6; bound: the chain projections, decays, memory, norm in one workgroup.
+constexpr int STEP_RANK = 32;              // most numbers that gla's decays pass through: a key channel's weights wait in a thread's registers
+struct StepEnds {
+    const void* h;                         // rows the projections read
+    int64_t h_stride;
+    int k_in, rank;
+    const float *w1, *w2, *w2_bias;        // mlstm: w1 (2 heads, k_in); gla: w1 (rank, k_in), w2 (heads * dim, rank) and its bias
+    float power;
+    const float* norm;
+    int norm_shared, g_off, kind;          // kind 1: sigmoid, 2: silu of x's columns at g_off
+    float eps;
+    void* out;
+    int64_t out_stride;
+};
+
+// part[wave][j] <- the wave's share of outputs first, first + step, ... (`count` of them) of the rows of w on one row h: four neighbouring
+// inputs a lane, every fourth piece of 256 inputs a wave -- the order of skinny_wide_kernel's sums
+template <typename A, int N>
+__device__ __forceinline__ void step_project(const A* __restrict__ h, const float* __restrict__ w, int first, int step, int count, int k_in,
+                                             float (*part)[STEP_RANK]) {
+    typedef A veca __attribute__((ext_vector_type(4)));
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int j0 = 0; j0 < count; j0 += N) {
+        float acc[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) acc[n] = 0.f;
+        for (int k = wave * 256 + lane * 4; k < k_in; k += 1024) {
+            const veca hv = *reinterpret_cast<const veca*>(h + k);
+            nvx_f32x4 wv[N];
+#pragma unroll
+            for (int n = 0; n < N; ++n) wv[n] = *reinterpret_cast<const nvx_f32x4*>(w + (int64_t)(first + (j0 + n < count ? j0 + n : count - 1) * step) * k_in + k);
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[n] += (float)hv[i] * wv[n][i];
+        }
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            float v = quarter_sum(acc[n]);
+            v += xor16(v);
+            v += xor32(v);
+            if (lane == 0 && j0 + n < count) part[wave][j0 + n] = v;
+        }
+    }
+}
+
+template <typename A, int KIND, bool ENDS>
+__global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a, StepEnds ends) {
     extern __shared__ __align__(16) float sm[];
     __shared__ float red[4];
+    __shared__ float few[4][STEP_RANK];
     const int hd = blockIdx.x, dim = a.dim, vdim = a.vdim, pieces = vdim / 4, n_groups = 256 / pieces;
     float* part = sm;                      // n_groups x vdim
     float* sq = part + n_groups * vdim;    // dim
@@ -717,10 +768,49 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
     float* sa = sk + dim;                  // dim (gla)
     const int64_t b = blockIdx.y;
     const int slot = a.state_slot[b];
-    if (slot < 0) return;
+    A* orow = ENDS ? (A*)ends.out + b * ends.out_stride + (int64_t)hd * vdim : nullptr;
+    if (slot < 0) {                        // (a padding row: its output is read by the products behind it, nothing else)
+        if (ENDS)
+            for (int e = threadIdx.x; e < vdim; e += 256) st_f(orow, e, 0.f);
+        return;
+    }
     const A* xr = (const A*)a.x + b * a.x_stride;
     const bool cont = a.pos0[b] > 0;
     const int64_t at = (int64_t)slot * a.heads + hd;
+    const int grp = threadIdx.x / pieces, e0 = threadIdx.x % pieces * 4;
+    float* Sp = a.S + at * dim * vdim;
+    constexpr int U = 8;                   // rows of the memory in flight a thread
+    nvx_f32x4 s[U], val, acc = {0.f, 0.f, 0.f, 0.f};
+    const auto load_rows = [&](int r0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int r = r0 + u * n_groups;
+            s[u] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+            if (cont && r < dim) s[u] = *reinterpret_cast<const nvx_f32x4*>(Sp + (int64_t)r * vdim + e0);
+        }
+    };
+    if (grp < n_groups) {
+        load_rows(grp);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) val[i] = scan_act(ld_f(xr, a.v_off + hd * vdim + e0 + i), a.act);
+    }
+    nvx_f32x4 w2[STEP_RANK / 4];
+    float z[4], wn[4], w2_bias = 0.f;
+    if (ENDS) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = threadIdx.x + 256 * i;
+            if (e < vdim) z[i] = ld_f(xr, ends.g_off + hd * vdim + e);
+            if (e < vdim) wn[i] = ends.norm[(ends.norm_shared ? 0 : hd * vdim) + e];
+        }
+        if (KIND == SCAN_GLA && (int)threadIdx.x < dim) {
+            const float* w2_row = ends.w2 + (int64_t)(hd * dim + threadIdx.x) * ends.rank;
+            w2_bias = ends.w2_bias[hd * dim + threadIdx.x];
+#pragma unroll
+            for (int i = 0; i < STEP_RANK / 4; ++i)
+                if (4 * i < ends.rank) w2[i] = *reinterpret_cast<const nvx_f32x4*>(w2_row + 4 * i);
+        }
+    }
     for (int d = threadIdx.x; d < dim; d += 256) {
         float qv = scan_act(ld_f(xr, a.q_off + hd * dim + d), a.act), kv = scan_act(ld_f(xr, a.k_off + hd * dim + d), a.act);
         if (KIND == SCAN_DECAY && d < 2 * a.half) {
@@ -733,7 +823,20 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
         }
         sq[d] = qv * a.q_mul;
         sk[d] = kv * a.k_mul;
-        if (KIND == SCAN_GLA) sa[d] = a.alpha[(b * a.heads + hd) * dim + d];
+        if (KIND == SCAN_GLA && !ENDS) sa[d] = a.alpha[(b * a.heads + hd) * dim + d];
+    }
+    if (ENDS) {
+        const A* hr = (const A*)ends.h + b * ends.h_stride;
+        if (KIND == SCAN_GLA) step_project<A, 8>(hr, ends.w1, 0, 1, ends.rank, ends.k_in, few);
+        else step_project<A, 2>(hr, ends.w1, hd, a.heads, 2, ends.k_in, few);
+        __syncthreads();
+        if (KIND == SCAN_GLA && (int)threadIdx.x < dim) {
+            float t = 0.f;
+#pragma unroll
+            for (int j = 0; j < STEP_RANK; ++j)
+                if (j < ends.rank) t += w2[j / 4][j % 4] * (few[0][j] + few[1][j] + few[2][j] + few[3][j]);
+            sa[threadIdx.x] = expf(ends.power * logsigmoid_f(t + w2_bias));
+        }
     }
     float keep = 1.f, put = 1.f, bottom = 1.f;
     if (KIND == SCAN_DECAY) keep = a.decay[hd];
@@ -741,8 +844,9 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
         // the gates are rounded before they meet their maximum: contracted into the exponents' subtractions, the larger one would not weigh exactly 1
 #pragma clang fp contract(off)
         const float* g = a.gates + b * 2 * a.heads;
-        const float gi = a.cap * tanhf((g[hd] + a.gate_bias[hd]) / a.cap);
-        const float gf = logsigmoid_f(a.cap * tanhf((g[a.heads + hd] + a.gate_bias[a.heads + hd]) / a.cap));
+        const float zi = ENDS ? few[0][0] + few[1][0] + few[2][0] + few[3][0] : g[hd], zf = ENDS ? few[0][1] + few[1][1] + few[2][1] + few[3][1] : g[a.heads + hd];
+        const float gi = a.cap * tanhf((zi + a.gate_bias[hd]) / a.cap);
+        const float gf = logsigmoid_f(a.cap * tanhf((zf + a.gate_bias[a.heads + hd]) / a.cap));
         const float m = cont ? a.M_in[at] : 0.f, m_new = fmaxf(gf + m, gi);
         keep = expf(gf + m - m_new);
         put = expf(gi - m_new);
@@ -756,22 +860,10 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
         bottom = fmaxf(fabsf(nq), expf(-m_new)) + 1e-6f;
         if (threadIdx.x == 0) a.M[at] = m_new;                  // (everybody has read it: block256_sum has passed its barriers)
     }
-    const int grp = threadIdx.x / pieces, e0 = threadIdx.x % pieces * 4;
-    float* Sp = a.S + at * dim * vdim;
     __syncthreads();
     if (grp < n_groups) {
-        nvx_f32x4 val, acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) val[i] = scan_act(ld_f(xr, a.v_off + hd * vdim + e0 + i), a.act);
-        constexpr int U = 8;
         for (int r0 = grp; r0 < dim; r0 += n_groups * U) {
-            nvx_f32x4 s[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int r = r0 + u * n_groups;
-                s[u] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
-                if (cont && r < dim) s[u] = *reinterpret_cast<const nvx_f32x4*>(Sp + (int64_t)r * vdim + e0);
-            }
+            if (r0 != grp) load_rows(r0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int r = r0 + u * n_groups;
@@ -788,10 +880,30 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
         *reinterpret_cast<nvx_f32x4*>(part + grp * vdim + e0) = acc;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < vdim; e += 256) {
-        float o = 0.f;
-        for (int g = 0; g < n_groups; ++g) o += part[g * vdim + e];
-        a.out[(b * a.heads + hd) * vdim + e] = KIND == SCAN_MLSTM ? o / bottom : o;
+    if (!ENDS) {
+        for (int e = threadIdx.x; e < vdim; e += 256) {
+            float o = 0.f;
+            for (int g = 0; g < n_groups; ++g) o += part[g * vdim + e];
+            a.out[(b * a.heads + hd) * vdim + e] = KIND == SCAN_MLSTM ? o / bottom : o;
+        }
+        return;
+    }
+    float o[4], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = threadIdx.x + 256 * i;
+        o[i] = 0.f;
+        if (e < vdim) {
+            for (int g = 0; g < n_groups; ++g) o[i] += part[g * vdim + e];
+            if (KIND == SCAN_MLSTM) o[i] /= bottom;
+        }
+        ss += o[i] * o[i];
+    }
+    const float rn = 1.f / sqrtf(block256_sum(ss, red) / (float)vdim + ends.eps);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = threadIdx.x + 256 * i;
+        if (e < vdim) st_f(orow, e, o[i] * rn * wn[i] * (ends.kind == 1 ? sigmoid_f(z[i]) : z[i] * sigmoid_f(z[i])));
     }
 }
 
@@ -799,10 +911,10 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a) {
 static bool memory_step_fits(const ScanArgs& a) {
     return !a.qo_indptr && !a.chunk && a.vdim % 4 == 0 && a.vdim <= 1024 && a.dim <= 512 && nvx_aligned16(a.S);
 }
-template <int KIND>
-static void launch_memory_step(const ScanArgs& a, int fmt, int64_t n_seq, hipStream_t st) {
+template <int KIND, bool ENDS = false>
+static void launch_memory_step(const ScanArgs& a, int fmt, int64_t n_seq, hipStream_t st, const StepEnds& ends = StepEnds{}) {
     const size_t lds = (size_t)((KIND == SCAN_GLA ? 3 : 2) * a.dim + 256 / (a.vdim / 4) * a.vdim) * sizeof(float);
-    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((memory_step_kernel<A_, KIND>), dim3((unsigned)a.heads, (unsigned)n_seq), dim3(256), lds, st, a));
+    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((memory_step_kernel<A_, KIND, ENDS>), dim3((unsigned)a.heads, (unsigned)n_seq), dim3(256), lds, st, a, ends));
 }
 
 // Between the two chunked phases: ws[sequence][chunk] holds every chunk's own contribution and is replaced by the state at the chunk's
@@ -1247,4 +1359,48 @@ extern "C" int nvx_gla_scan(const void* x, int64_t x_stride, int fmt, int64_t q_
     }
 #undef NVX_GLA_SCAN
     return nvx_check_launch("nvx_gla_scan");
+}
+
+// mlstm (kind 0) or gla (kind 1) for a step of one token per sequence with its small projections and the norm and gate of its read-out, one
+// launch; the host of this package calls it, see ops.memory_step
+struct NvxMemoryStep {
+    const void *x, *h;
+    const float *w1, *w2, *bias, *norm;    // mlstm: w1 the gates' weights, bias the gates'; gla: bias that of w2
+    float *S, *N, *M;                      // (mlstm: N and M)
+    const int64_t* pos0;
+    const int32_t* state_slot;
+    void* out;
+    int64_t x_stride, h_stride, out_stride, n_seq, n_slots;
+    int32_t kind, fmt, q_off, k_off, v_off, g_off, heads, dim, vdim, k_in, rank, norm_shared;
+    float q_mul, cap, power, eps;
+};
+
+extern "C" int nvx_internal_memory_step(const NvxMemoryStep* m, nvx_stream_t stream) {
+    NVX_REQUIRE(m && m->fmt >= 0 && m->fmt <= 2 && (m->kind == 0 || m->kind == 1), NVX_EINVAL, "nvx_internal_memory_step: kind or fmt");
+    const int64_t hd = (int64_t)m->heads * m->dim, he = (int64_t)m->heads * m->vdim;
+    NVX_REQUIRE(m->n_seq >= 0 && m->n_seq <= 65535 && m->heads > 0 && m->dim > 0 && m->vdim > 0 && m->n_slots >= 0 && hd < (1 << 24) && he < (1 << 24), NVX_EINVAL,
+                "nvx_internal_memory_step: bad sizes");
+    if (m->n_seq == 0) return NVX_OK;
+    NVX_REQUIRE(m->x && m->h && m->w1 && m->bias && m->norm && m->S && m->pos0 && m->state_slot && m->out, NVX_EINVAL, "nvx_internal_memory_step: null pointer");
+    NVX_REQUIRE(m->q_off >= 0 && m->k_off >= 0 && m->v_off >= 0 && m->g_off >= 0 && m->x_stride >= m->q_off + hd && m->x_stride >= m->k_off + hd &&
+                    m->x_stride >= m->v_off + he && m->x_stride >= m->g_off + he && m->out_stride >= he, NVX_EINVAL,
+                "nvx_internal_memory_step: q, k, v or the gate lies outside a row");
+    const uintptr_t row_border = m->fmt == 2 ? 15u : 7u;
+    NVX_REQUIRE(m->k_in > 0 && m->k_in % 4 == 0 && m->h_stride >= m->k_in && m->h_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(m->h) & row_border) == 0 &&
+                    nvx_aligned16(m->w1), NVX_EUNSUPPORTED, "nvx_internal_memory_step: the projections read four inputs at a time");
+    ScanArgs a = {};
+    a.x = m->x; a.x_stride = m->x_stride; a.q_off = m->q_off; a.k_off = m->k_off; a.v_off = m->v_off; a.heads = m->heads; a.dim = m->dim; a.vdim = m->vdim;
+    a.q_mul = m->q_mul; a.k_mul = 1.0f; a.cap = m->cap; a.gate_bias = m->bias; a.S = m->S; a.N_in = a.N = m->N; a.M_in = a.M = m->M; a.pos0 = m->pos0;
+    a.state_slot = m->state_slot;
+    NVX_REQUIRE(memory_step_fits(a), NVX_EUNSUPPORTED, "nvx_internal_memory_step: head sizes");
+    StepEnds e = {m->h, m->h_stride, m->k_in, m->rank, m->w1, m->w2, m->bias, m->power, m->norm, m->norm_shared, m->g_off, m->kind == 0 ? 1 : 2, m->eps, m->out, m->out_stride};
+    if (m->kind == 0) {
+        NVX_REQUIRE(m->N && m->M && m->cap > 0.f, NVX_EINVAL, "nvx_internal_memory_step: mlstm's normaliser, maximum and cap");
+        launch_memory_step<SCAN_MLSTM, true>(a, m->fmt, m->n_seq, (hipStream_t)stream, e);
+    } else {
+        NVX_REQUIRE(m->w2 && m->dim <= 256 && m->rank > 0 && m->rank <= STEP_RANK && m->rank % 4 == 0 && nvx_aligned16(m->w2), NVX_EUNSUPPORTED,
+                    "nvx_internal_memory_step: gla's decays pass through a multiple of four numbers, at most 32, and its keys have at most 256 channels");
+        launch_memory_step<SCAN_GLA, true>(a, m->fmt, m->n_seq, (hipStream_t)stream, e);
+    }
+    return nvx_check_launch("nvx_internal_memory_step");
 }

@@ -58,9 +58,12 @@ class MLSTM(nn.Module):
     def forward(self, h: torch.Tensor, md, at=None) -> torch.Tensor:
         hd, he, n = self.heads * self.dim, self.heads * self.vdim, self.state_name if at is None else at
         x = self.qkvg_proj(h)
+        S, norm, peak = (md.cache.state((n, which)) for which in ("S", "n", "m"))
+        if ops.memory_step_fits(md.layout, h, S, self.gate_w):
+            return self.o_proj(ops.mlstm_step(x, (0, hd, 2 * hd), 2 * hd + he, h, self.gate_w, self.gate_b, self.gate_cap, self.norm, self.eps, S, norm, peak,
+                                              md.layout, self.heads, self.dim, self.vdim))
         gates = ops.skinny_proj(h, self.gate_w)
-        o = ops.mlstm_scan(x, (0, hd, 2 * hd), gates, self.gate_b, self.gate_cap, md.cache.state((n, "S")), md.cache.state((n, "n")),
-                           md.cache.state((n, "m")), md.layout, self.heads, self.dim, self.vdim)
+        o = ops.mlstm_scan(x, (0, hd, 2 * hd), gates, self.gate_b, self.gate_cap, S, norm, peak, md.layout, self.heads, self.dim, self.vdim)
         y = ops.head_norm_gate(o, self.norm, self.eps, gate=x[:, 2 * hd + he:], kind="sigmoid")
         return self.o_proj(y)
 
@@ -236,9 +239,12 @@ class GatedLinearAttention(nn.Module):
 
     def forward(self, h: torch.Tensor, md, at=None) -> torch.Tensor:
         hd, he, n = self.heads * self.dim, self.heads * self.vdim, self.state_name if at is None else at
-        x = self.qkvg_proj(h)
+        x, S = self.qkvg_proj(h), md.cache.state((n, "S"))
+        if ops.memory_step_fits(md.layout, h, S, self.a1, self.a2):
+            return self.o_proj(ops.gla_step(x, (0, hd, 2 * hd), 2 * hd + he, h, self.a1, self.a2, self.a2_b, 1.0 / self.tau, self.norm, self.eps, S, md.layout,
+                                            self.heads, self.dim, self.vdim, q_mul=self.dim ** -0.5))
         alpha = ops.skinny_proj(ops.skinny_proj(h, self.a1), self.a2, bias=self.a2_b, out_act="sigmoid_pow", power=1.0 / self.tau)
-        o = ops.gla_scan(x, (0, hd, 2 * hd), alpha, md.cache.state((n, "S")), md.layout, self.heads, self.dim, self.vdim, q_mul=self.dim ** -0.5)
+        o = ops.gla_scan(x, (0, hd, 2 * hd), alpha, S, md.layout, self.heads, self.dim, self.vdim, q_mul=self.dim ** -0.5)
         y = ops.head_norm_gate(o, self.norm, self.eps, gate=x[:, 2 * hd + he:], kind="silu")
         return self.o_proj(y)
 

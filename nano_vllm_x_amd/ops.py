@@ -2001,6 +2001,56 @@ def gla_scan(x, offsets, alpha, mem, layout: StepLayout, heads: int, dim: int, v
     return out
 
 
+def memory_step_fits(layout: StepLayout, h, mem, w1, w2=None) -> bool:
+    """Whether mlstm_step (w1: its gates' weights) or gla_step (w1, w2: its decays') serves this step: one token per sequence, heads and rows that
+    their kernel is built for.  Every head of every sequence computes gla's `rank` numbers again, so they must be few."""
+    heads, dim, vdim = mem.shape[1:]
+    item = 4 * h.element_size()
+    if layout.qo_indptr is not None or vdim % 4 or vdim > 1024 or dim > 512 or h.shape[1] % 4 or h.stride(0) % 4 or h.stride(1) != 1 or layout.n_tok > 65535:
+        return False
+    if h.data_ptr() % item or any(t.data_ptr() % 16 for t in (mem, w1) + (() if w2 is None else (w2,))):
+        return False
+    return w2 is None or (dim <= 256 and w1.shape[0] % 4 == 0 and 0 < w1.shape[0] <= 32 and w1.numel() <= 1 << 16)
+
+
+def _memory_step(what, kind, x, offsets, gate_off, h, w1, w2, bias, norm, eps, mem, layout, heads, dim, vdim, nrm=None, peak=None, **scalars):
+    _dev(x, h, w1, w2, bias, norm, mem, nrm, peak)
+    t = x.shape[0]
+    _need(x.dim() == 2 and x.stride(1) == 1 and t == layout.n_tok and layout.qo_indptr is None, what + ": x must be (T, columns), one token per sequence")
+    _need(h.dim() == 2 and h.stride(1) == 1 and h.shape[0] == t and h.dtype == x.dtype and w1.shape[1] == h.shape[1], what + ": h must be (T, inputs) in x's format")
+    for a in (w1, bias, norm, mem) + tuple(a for a in (w2, nrm, peak) if a is not None):
+        _f32c(a, what)
+    n_slots = mem.shape[0]
+    _need(mem.shape == (n_slots, heads, dim, vdim) and norm.numel() in (vdim, heads * vdim), what + ": shapes")
+    out = torch.empty((t, heads * vdim), dtype=x.dtype, device=x.device)
+    if not t:
+        return out
+    a = _lib.MemoryStep(kind=kind, fmt=_fmt(x), q_off=offsets[0], k_off=offsets[1], v_off=offsets[2], g_off=gate_off, heads=heads, dim=dim, vdim=vdim, k_in=h.shape[1],
+                        rank=w1.shape[0], norm_shared=int(norm.numel() == vdim), x_stride=x.stride(0), h_stride=h.stride(0), out_stride=out.stride(0), n_seq=t,
+                        n_slots=n_slots, eps=eps, **scalars)
+    for name, v in (("x", x), ("h", h), ("w1", w1), ("w2", w2), ("bias", bias), ("norm", norm), ("S", mem), ("N", nrm), ("M", peak), ("pos0", layout.pos0),
+                    ("state_slot", layout.state_slot), ("out", out)):
+        setattr(a, name, None if v is None else v.data_ptr())
+    _lib.check(_lib.load().nvx_internal_memory_step(a, _stream()), what)
+    return out
+
+
+def mlstm_step(x, offsets, gate_off: int, h, gate_w, gate_bias, cap: float, norm_w, eps: float, mem, norm, peak, layout: StepLayout, heads: int, dim: int, vdim: int):
+    """skinny_proj (the two gates of every head, of the rows h), mlstm_scan and head_norm_gate (sigmoid of x's columns at `gate_off`) in one launch, where
+    memory_step_fits says so.  Returns (T, heads * vdim) in x's format."""
+    _need(gate_w.shape[0] == 2 * heads and gate_bias.numel() == 2 * heads and norm.shape == mem.shape[:3] and peak.shape == mem.shape[:2], "mlstm_step: shapes")
+    return _memory_step("mlstm_step", 0, x, offsets, gate_off, h, gate_w, None, gate_bias, norm_w, eps, mem, layout, heads, dim, vdim, norm, peak,
+                        q_mul=dim ** -0.5, cap=float(cap))
+
+
+def gla_step(x, offsets, gate_off: int, h, a1, a2, a2_bias, power: float, norm_w, eps: float, mem, layout: StepLayout, heads: int, dim: int, vdim: int,
+             q_mul: float = 1.0):
+    """skinny_proj twice (the decays sigmoid(a2 (a1 h) + a2_bias)^power), gla_scan and head_norm_gate (silu of x's columns at `gate_off`) in one launch, where
+    memory_step_fits says so.  Returns (T, heads * vdim) in x's format."""
+    _need(a2.shape == (heads * dim, a1.shape[0]) and a2_bias.numel() == heads * dim, "gla_step: shapes")
+    return _memory_step("gla_step", 1, x, offsets, gate_off, h, a1, a2, a2_bias, norm_w, eps, mem, layout, heads, dim, vdim, q_mul=float(q_mul), power=float(power))
+
+
 def moe_route_sigmoid(logits, correction, top: int, n_groups: int = 0, keep_groups: int = 0, scale: float = 1.0):
     """logits (T, experts) float32 -> (ids (T, top) int32, weights (T, top) float32).  Scores are sigmoids; choice scores are score +
     correction (experts, float32).  With n_groups > 1 the experts form equal groups of neighbours, a group counts as the sum of its two
