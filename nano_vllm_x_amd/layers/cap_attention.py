@@ -10,6 +10,7 @@ from torch import nn
 
 from .. import ops
 from .linear import Linear
+from .plain import bypassable
 from .rotary_embedding import rotary_frequencies
 
 
@@ -145,6 +146,7 @@ def geometric_slopes(heads: int, base: float = 8.0):
     return [2.0 ** (-base * (h + 1) / heads) for h in range(heads)]
 
 
+@bypassable
 class TiedAttention(nn.Module):
     """Grouped-head softmax attention whose VALUES ARE ITS KEYS as projected: q = W_q h, k = W_k h (optional biases); queries and keys are
     scored after an RMS norm per head (weights of `dim` entries shared by the heads), the read-out sums the keys as they came out of the
@@ -177,10 +179,11 @@ class TiedAttention(nn.Module):
         n = self.cache_name if at is None else at
         return {(n, "k"): self.kv_heads * self.dim, (n, "rn"): (self.kv_heads, torch.float32)}
 
-    def forward(self, h: torch.Tensor, md, at=None) -> torch.Tensor:
-        n = self.cache_name if at is None else at
+    def forward(self, h: torch.Tensor, md, at=None, made=None) -> torch.Tensor:
+        """`made`: in_proj's result where it came with the norm in front."""
+        qk, n = self.in_proj(h) if made is None else made, self.cache_name if at is None else at
         rows, rn = md.cache.latent((n, "k")), md.cache.latent((n, "rn"))
-        q = ops.tied_prep_store(self.in_proj(h), (0, self.q_cols), self.q_norm, self.k_norm, self.eps, md.out_slots, rows, rn, self.heads,
+        q = ops.tied_prep_store(qk, (0, self.q_cols), self.q_norm, self.k_norm, self.eps, md.out_slots, rows, rn, self.heads,
                                 self.kv_heads, self.dim)
         o = ops.softcap_attn(q, rows, rows, md.kv_indices, md.kv_start, md.kv_len, md.layout, self.scale, 0.0, self.heads, self.kv_heads, self.dim,
                              self.dim, window=self.window, chunk=self.chunk, slopes=self.slopes, k_rn=rn)

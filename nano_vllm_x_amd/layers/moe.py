@@ -10,6 +10,7 @@ from torch import nn
 
 from .. import ops
 from .linear import Linear, gated_rows_fit
+from .plain import bypassable
 
 
 class DenseGLU(nn.Module):
@@ -27,6 +28,7 @@ class DenseGLU(nn.Module):
         return self.down(ops.moe_glu(self.gu_proj(h), self.limit, self.alpha, 1.0))
 
 
+@bypassable
 class GeluGLU(nn.Module):
     """W_down (gelu_tanh(W_gate h) * (W_up h)); gate and up are one product."""
 
@@ -36,7 +38,10 @@ class GeluGLU(nn.Module):
         self.gu_proj = Linear(width, 2 * ff, bias=False)      # rows: gate | up
         self.down = Linear(ff, width, bias=False)
 
-    def forward(self, h: torch.Tensor) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, made=None) -> torch.Tensor:
+        """`made`: the activation of gu_proj's result where it came with the norm in front."""
+        if made is not None:
+            return self.down(made)
         if gated_rows_fit(h, self.gu_proj):
             return self.down(ops.few_rows_glu(h, self.gu_proj.weight, gelu=True))
         return self.down(ops.gelu_glu(self.gu_proj(h)))

@@ -7,6 +7,7 @@ from torch import nn
 
 from .. import ops
 from .linear import Linear
+from .plain import bypassable
 
 
 class MinGRU(nn.Module):
@@ -34,6 +35,7 @@ def _f32(*shape):
     return nn.Parameter(torch.zeros(*shape, dtype=torch.float32))
 
 
+@bypassable
 class MLSTM(nn.Module):
     """Matrix memory per head with an exponential input gate and a sigmoid forget gate, both capped, kept finite by a
     running maximum m (which starts at 0):  i = cap tanh((W_i h + b_i) / cap), f = logsigmoid(cap tanh((W_f h + b_f) / cap)),
@@ -55,9 +57,10 @@ class MLSTM(nn.Module):
         n = self.state_name if at is None else at
         return {(n, "S"): (self.heads, self.dim, self.vdim), (n, "n"): (self.heads, self.dim), (n, "m"): (self.heads,)}
 
-    def forward(self, h: torch.Tensor, md, at=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, md, at=None, made=None) -> torch.Tensor:
+        """`made`: qkvg_proj's result where it came with the norm in front."""
         hd, he, n = self.heads * self.dim, self.heads * self.vdim, self.state_name if at is None else at
-        x = self.qkvg_proj(h)
+        x = self.qkvg_proj(h) if made is None else made
         S, norm, peak = (md.cache.state((n, which)) for which in ("S", "n", "m"))
         if ops.memory_step_fits(md.layout, h, S, self.gate_w):
             return self.o_proj(ops.mlstm_step(x, (0, hd, 2 * hd), 2 * hd + he, h, self.gate_w, self.gate_b, self.gate_cap, self.norm, self.eps, S, norm, peak,
@@ -218,6 +221,7 @@ class RGLRU(nn.Module):
         return self.o_proj(s)
 
 
+@bypassable
 class GatedLinearAttention(nn.Module):
     """Linear attention with a decay per key channel and token: q = W_q h / sqrt(dim), k = W_k h (heads x dim), v = W_v h (heads x vdim),
     alpha = sigmoid(W_a2 (W_a1 h) + b)^(1 / tau) (heads x dim); per head S <- diag(alpha) S + k v^T, o = S^T q (the read sees the
@@ -237,9 +241,10 @@ class GatedLinearAttention(nn.Module):
     def state_shapes(self, at=None) -> dict:
         return {(self.state_name if at is None else at, "S"): (self.heads, self.dim, self.vdim)}
 
-    def forward(self, h: torch.Tensor, md, at=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, md, at=None, made=None) -> torch.Tensor:
+        """`made`: as at MLSTM."""
         hd, he, n = self.heads * self.dim, self.heads * self.vdim, self.state_name if at is None else at
-        x, S = self.qkvg_proj(h), md.cache.state((n, "S"))
+        x, S = self.qkvg_proj(h) if made is None else made, md.cache.state((n, "S"))
         if ops.memory_step_fits(md.layout, h, S, self.a1, self.a2):
             return self.o_proj(ops.gla_step(x, (0, hd, 2 * hd), 2 * hd + he, h, self.a1, self.a2, self.a2_b, 1.0 / self.tau, self.norm, self.eps, S, md.layout,
                                             self.heads, self.dim, self.vdim, q_mul=self.dim ** -0.5))

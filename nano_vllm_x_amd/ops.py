@@ -2133,6 +2133,36 @@ def few_rows_glu(x, w, limit: float = 0.0, alpha: float = 0.0, shift: float = 0.
     return y
 
 
+def lead_rows_fit(x, y, add, x_bias, w_norm, w, bias=None, gelu: bool = False) -> bool:
+    """Whether residual_norm(x, y, add=add, bias=x_bias, w=w_norm) and few_rows_product (gelu: few_rows_glu) of its result are one launch (few_rows_lead): rows that
+    every workgroup can form for itself in less time than the boundary's launch takes."""
+    rows, k = x.shape
+    n, dtype = w.shape[0], w.dtype
+    return (0 < rows <= LEAD_ROWS and k == LEAD_WIDTH and dtype in H16 and w.dim() == 2 and w.shape[1] == k and w.is_contiguous()
+            and n % (32 if gelu else 16) == 0 and n // (32 if gelu else 16) >= 16 and n < 12288 and not (gelu and bias is not None)
+            and (gated_rows_faster if gelu else few_rows_faster)(rows, n, k) and not torch.is_grad_enabled() and operators_are_plain()
+            and all(type(a) in (torch.Tensor, torch.nn.Parameter) and a.is_cuda and a.device == x.device and a.data_ptr() % 16 == 0
+                    for a in (x, y, add, x_bias, w_norm, w) if a is not None)
+            and all(a is None or (a.dtype == F32 and a.is_contiguous()) for a in (x, add, x_bias, w_norm))
+            and (y is None or (y.dtype == dtype and y.shape == x.shape and y.stride(1) == 1 and y.stride(0) % 8 == 0 and y.stride(0) >= k))
+            and (add is None or add.shape == x.shape) and (x_bias is None or x_bias.shape == (k,)) and w_norm.shape == (k,)
+            and (bias is None or (type(bias) in (torch.Tensor, torch.nn.Parameter) and bias.dtype == dtype and bias.is_contiguous() and bias.shape == (n,) and bias.device == x.device)))
+
+
+LEAD_ROWS, LEAD_WIDTH = 16, 1024      # what few_rows_lead's workgroups form, each for itself
+
+
+def few_rows_lead(x, y, add, x_bias, w_norm, eps: float, w, bias=None, gelu: bool = False):
+    """(new stream, its norm h, product of h with w): see lead_rows_fit.  The stream x stays as it is."""
+    _need(lead_rows_fit(x, y, add, x_bias, w_norm, w, bias, gelu), "few_rows_lead: sizes and layouts of lead_rows_fit")
+    (rows, k), n = x.shape, w.shape[0]
+    new, h = torch.empty_like(x), torch.empty((rows, k), dtype=w.dtype, device=x.device)
+    out = torch.empty((rows, n // 2 if gelu else n), dtype=w.dtype, device=x.device)
+    _lib.check(_lib.load().nvx_internal_few_rows_lead(_ptr(x), _ptr(y), 0 if y is None else y.stride(0), _ptr(add), _ptr(x_bias), _ptr(w_norm), float(eps), _ptr(new), _ptr(h),
+                                                      _ptr(w), _ptr(bias), _ptr(out), _FMT[w.dtype], rows, n, k, int(gelu), _stream()), "few_rows_lead")
+    return new, h, out
+
+
 def product_f32(x, w):
     """x @ w.T as its float32 sums, unrounded; x (T, k), w (n, k) in one format.  A library product except for few rows (few_rows_product)."""
     if x.dim() == 2 and x.shape[0] <= FEW_ROWS and few_rows_faster(x.shape[0], *w.shape) and few_rows_fits(x, w):

@@ -16,7 +16,8 @@ passes, or absent.
 
 config.json gives every size, the order of the layers and the constants; the mechanisms live in layers/ (cap_attention.py,
 recurrent.py, moe.py) with their constants as arguments.  Between the matrix products (library GEMMs; all input projections of a mixer
-are ONE product) every step is a HIP kernel of this package, one launch per sublayer boundary (ops.residual_norm).  The stream, norms,
+are ONE product) every step is a HIP kernel of this package, one launch per sublayer boundary (ops.residual_norm), or none where the product behind it forms
+its few rows itself (ops.few_rows_lead).  The stream, norms,
 attention scores, positions, routers, gates and decays of the recurrences and their states are float32 in every activation format, and
 the product that joins x and x0 ahead of a pass sees the stream as a hi + lo pair of 16-bit numbers and returns float32.
 """
@@ -32,11 +33,14 @@ from torch import nn
 from . import distributed as tpd
 from . import ops
 from .layers.cap_attention import TiedAttention, geometric_slopes
+from .layers.linear import Linear
 from .layers.moe import DenseGLU, GeluGLU, GroupedSigmoidMoE
+from .layers.plain import as_written, calls_are_plain, untouched
 from .layers.recurrent import MLSTM, GatedLinearAttention
 
 MIXERS = ("attention", "gla", "mlstm")
 GLU_SLOPE = 1.702         # expert: y = g sigmoid(1.702 g) (u + 1)
+FIRST_PRODUCT = {TiedAttention: "in_proj", MLSTM: "qkvg_proj", GatedLinearAttention: "qkvg_proj", GeluGLU: "gu_proj"}      # what reads the module's input
 DECAY_RANK = 16           # inner size of the decay's two projections in a model that is built without a checkpoint
 
 
@@ -231,35 +235,46 @@ class ZenedraForCausalLM(nn.Module):
         x, h = ops.embed_sum(input_ids, self.embed, md.layout, pair=self.pair, mul_prev=b["mul_prev"], mul_cur=b["mul_cur"],
                              prev_id=md.cache.state("prev_id") if self.pair is not None else None, pos_table=self.pos, positions=positions,
                              w=None if cfg.loop else norms[0], eps=eps, split=bool(cfg.loop) and pairs)
-        from_x0 = None
+        from_x0, made = None, None
         if cfg.loop:
             from_x0 = self._join(x, h if pairs else None, 1)       # the same for every pass
             if starts[0] is None:
                 h = ops.residual_norm(x, w=norms[0], eps=eps, dtype=dtype)
             else:
-                x, h = self._begin_pass(x, h if pairs else None, from_x0, starts[0], norms[0])
+                x, h, made = self._begin_pass(x, h if pairs else None, from_x0, starts[0], norms[0], layers[runs[0][0]].mixer)
         for n, (i, name, _) in enumerate(runs):
             layer = layers[i]
-            y, y2 = layer.mixer(h, md, at=name), None
+            y, y2 = layer.mixer(h, md, at=name) if made is None else layer.mixer(h, md, at=name, made=made), None
             if layer.mlp is not None:
-                h = ops.residual_norm(x, y, w=layer.norm2, eps=eps)
-                y = layer.mlp(h) if layer.mlp_kind == "dense" else layer.mlp(h, decode_step)
-                if layer.mlp_kind == "moe":
-                    y, y2 = y
+                x, h, made = self._boundary(layer.mlp, x, y, norm=layer.norm2)
+                if layer.mlp_kind == "dense":
+                    y = layer.mlp(h) if made is None else layer.mlp(h, made=made)
+                else:
+                    y, y2 = layer.mlp(h, decode_step)
             if starts[n + 1] is None:
-                h = ops.residual_norm(x, y, y2, w=norms[n + 1], eps=eps)
+                x, h, made = self._boundary(layers[runs[n + 1][0]].mixer if n + 1 < len(runs) else None, x, y, y2, norm=norms[n + 1])
             else:
                 h = ops.residual_norm(x, y, y2, split=pairs, dtype=dtype)
             if self.layer_streams is not None:
                 self.layer_streams.append(x.clone())
             if starts[n + 1] is not None:
-                x, h = self._begin_pass(x, h, from_x0, starts[n + 1], norms[n + 1])
+                x, h, made = self._begin_pass(x, h, from_x0, starts[n + 1], norms[n + 1], layers[runs[n + 1][0]].mixer)
         return h
 
-    def _begin_pass(self, x, pair_rows, from_x0, t: int, norm):
-        """(stream, its norm) at the head of pass t: x <- W_x x + W_0 x0 + step[t]."""
-        x = self._join(x, pair_rows, 0)
-        return x, ops.residual_norm(x, add=from_x0, bias=self.loop_step[t], w=norm, eps=self.config.eps, dtype=self.embed.dtype)
+    def _begin_pass(self, x, pair_rows, from_x0, t: int, norm, mixer):
+        """_boundary at the head of pass t: x <- W_x x + W_0 x0 + step[t]."""
+        return self._boundary(mixer, self._join(x, pair_rows, 0), add=from_x0, bias=self.loop_step[t], norm=norm)
+
+    def _boundary(self, reader, x, y=None, y2=None, add=None, bias=None, norm=None):
+        """(stream, its norm, None), or (stream, norm, the product of it that `reader` starts with) where both are one launch and the module
+        would call that product as it was written."""
+        name = FIRST_PRODUCT.get(type(reader))
+        if name is not None and y2 is None and x.shape[0] <= ops.LEAD_ROWS:
+            proj, gelu = getattr(reader, name), type(reader) is GeluGLU
+            if (untouched(reader, type(reader)) and untouched(proj, Linear) and as_written(type(reader), Linear) and calls_are_plain()
+                    and ops.lead_rows_fit(x, y, add, bias, norm, proj.weight, proj.bias, gelu)):
+                return ops.few_rows_lead(x, y, add, bias, norm, self.config.eps, proj.weight, proj.bias, gelu)
+        return x, ops.residual_norm(x, y, y2, add=add, bias=bias, w=norm, eps=self.config.eps, dtype=self.embed.dtype if y is None else y.dtype), None
 
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """float32 logits."""
