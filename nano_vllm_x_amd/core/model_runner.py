@@ -182,11 +182,8 @@ class ModelRunner:
                                           self.model.state_shapes())
             self.attn_backend = SeqStateBackend(self.kv_cache, self.device)
             # decode steps as one hipGraph per batch size, as for paged attention: the device block table gives every
-            # running sequence a row of slot ids, and the state slot of each row of the step travels in a buffer of its own
-            self.block_table = BlockTable(self.max_bs, 2 * self.max_bs + 1, 2 * self.context_len, self.device)
-            self._state_slot_dev = torch.full((self.max_bs,), -1, dtype=torch.int32, device=self.device)
-            self._state_slot_hosts = [torch.full((self.max_bs,), -1, dtype=torch.int32, pin_memory=True) for _ in range(2)]
-            self._state_slot_turn = 0
+            # running sequence a row of slot ids, and the state slot of each row travels with the step's other integers
+            self.block_table = BlockTable(self.max_bs, 2 * self.max_bs + 1, 2 * self.context_len, self.device, with_states=True)
             if not self.enforce_eager:
                 self.graph = HIPGraph()
                 self.capture_graph()
@@ -456,19 +453,14 @@ class ModelRunner:
         bs = batch.num_seqs
         padded = self.graph.match_bs(bs)
         self.block_table.stage_decode_step(batch.seqs, ids_on_device)
-        if self.family == "seq_state":
-            self._state_slot_turn ^= 1
-            host = self._state_slot_hosts[self._state_slot_turn]
-            host.fill_(-1)                    # rows past the batch are padding: no state is read or written for them
-            host[:bs] = torch.tensor([s.state_slot for s in batch.seqs], dtype=torch.int32)
-            self._state_slot_dev.copy_(host, non_blocking=True)
         chain = self.chain_graph
         if chain is not None and bs <= chain.max_bs and self.decode_chain.faster(bs, sum(len(s.kv_indices) for s in batch.seqs)):
-            self.decode_chain.in_turn(lambda: chain.replay(chain.match_bs(bs)))
+            padded = chain.match_bs(bs)
+            self.decode_chain.in_turn(lambda: chain.replay(padded))
             self.stats["chain_steps"] = self.stats.get("chain_steps", 0) + 1
-        else:
-            self.graph.replay(padded)
-        return self.graph.get_output_buffer("hidden_states")[:bs]
+            return chain.get_output_buffer(f"hidden_states {padded}")[:bs]
+        self.graph.replay(padded)
+        return self.graph.get_output_buffer(f"hidden_states {padded}")[:bs]
 
     def _decode_forward(self, bs: int, chain: Optional[ops.DecodeChain] = None) -> torch.Tensor:
         """The body of a captured decode step for a padded batch of `bs` rows, its layers in one launch if there is a `chain`."""
@@ -478,7 +470,7 @@ class ModelRunner:
         if self.family == "seq_state":
             from ..layers.seq_state import SeqStateMetadata
             md = SeqStateMetadata(forward_mode=ForwardMode.DECODE, cache=self.kv_cache,
-                                  layout=ops.StepLayout(bs, bs, bt.positions[:bs], self._state_slot_dev[:bs]),
+                                  layout=ops.StepLayout(bs, bs, bt.positions[:bs], bt.state_slots[:bs]),
                                   kv_indices=bt.table.view(-1), kv_start=bt.kv_start[:bs], kv_len=bt.kv_len[:bs],
                                   out_slots=bt.out_slots[:bs], kv_indptr=None)
             with attention_kv_cache(self.model, md):
@@ -493,8 +485,9 @@ class ModelRunner:
     @torch.inference_mode()
     def capture_graph(self):
         """Capture one decode graph per ladder size, largest first so the pool is sized once
-        (model_runner.py:393).  Static inputs: the step buffer of the block table; static output:
-        `hidden_states` (max_bs, hidden)."""
+        (model_runner.py:393).  Static inputs: the step buffer of the block table; output: `hidden_states <bs>` (bs, hidden) of each
+        graph, the tensor that its last launch writes, good until the next replay of any of them (a copy into one buffer for all
+        was a launch of 4 us at the end of every step)."""
         assert self.graph is not None
         bt = self.block_table
         sizes = decode_batch_ladder(self.max_bs)
@@ -504,13 +497,11 @@ class ModelRunner:
             sizes = [bs for bs in sizes if tpd.decode_graph_capturable(bs)]
             if not sizes:
                 raise RuntimeError("the all-reduce of this group cannot be captured at any decode batch size")
-        hidden_out = torch.zeros((self.max_bs, self.hf_config.hidden_size), dtype=self.dtype, device=self.device)
         self.graph.set_input_buffer("step", bt.step_dev)
         self.graph.set_input_buffer("input_ids", bt.input_ids)
         self.graph.set_input_buffer("positions", bt.positions)
-        self.graph.set_output_buffer("hidden_states", hidden_out)
         self._graph_wrappers = {}
-        bt.step_dev.zero_()   # batch = 0: every row is a padding row during warm-up and capture
+        bt.clear_step()   # every row is a padding row during warm-up and capture
         side = torch.cuda.Stream(device=self.device)
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
@@ -526,14 +517,14 @@ class ModelRunner:
         torch.cuda.synchronize()
         for bs in reversed(sizes):
             with self.graph.capture(bs):
-                hidden_out[:bs] = self._decode_forward(bs)
+                self.graph.set_output_buffer(f"hidden_states {bs}", self._decode_forward(bs))
         if self.decode_chain is not None:
             self.chain_graph = HIPGraph()
             self.chain_graph.graph_pool = self.graph.graph_pool      # (steps of either follow each other on a stream)
             for bs in reversed(sizes):
                 if bs <= ops.DecodeChain.ROWS:
                     with self.chain_graph.capture(bs):
-                        hidden_out[:bs] = self._decode_forward(bs, self.decode_chain)
+                        self.chain_graph.set_output_buffer(f"hidden_states {bs}", self._decode_forward(bs, self.decode_chain))
         torch.cuda.synchronize()
         if os.environ.get("NVX_GRAPH_PRUNE", "1") != "0":
             self.prune_slow_graph_sizes()
@@ -547,7 +538,7 @@ class ModelRunner:
         sizes = list(self.graph.captured_bs)
         if len(sizes) < 2:
             return
-        self.block_table.step_dev.zero_()     # batch = 0: every row is a padding row, as during capture
+        self.block_table.clear_step()     # every row is a padding row, as during capture
         times = {}
         for bs in sizes:
             self.graph.replay(bs)             # (first replay of a graph uploads it)

@@ -217,9 +217,11 @@ class AttentionMetadata:
 
 class BlockTable:
     """Device-resident block table: one row of `row_capacity` slot ids per running sequence, plus the
-    static per-step buffers a captured decode graph reads.  Row `n_rows - 1` is the padding row."""
+    static per-step buffers a captured decode graph reads.  Row `n_rows - 1` is the padding row.
+    `with_states`: the sequences' state slots travel behind the step's other integers (one upload, one copy a step;
+    an upload of their own was another copy of 3.3 us)."""
 
-    def __init__(self, max_bs: int, n_rows: int, row_capacity: int, device):
+    def __init__(self, max_bs: int, n_rows: int, row_capacity: int, device, with_states: bool = False):
         self.max_bs, self.n_rows, self.row_capacity, self.device = max_bs, n_rows, row_capacity, device
         self.table = torch.zeros((n_rows, row_capacity), dtype=torch.int32, device=device)
         self.pad_start = (n_rows - 1) * row_capacity
@@ -230,13 +232,22 @@ class BlockTable:
         self.out_slots = torch.full((max_bs,), -1, dtype=torch.int64, device=device)
         self.positions = torch.zeros(max_bs, dtype=torch.int64, device=device)
         self.input_ids = torch.zeros(max_bs, dtype=torch.int64, device=device)
-        self.step_dev = torch.zeros(4 + 4 * max_bs, dtype=torch.int32, device=device)
+        ints = 4 + (5 if with_states else 4) * max_bs
+        self.step_dev = torch.zeros(ints, dtype=torch.int32, device=device)
+        self.state_slots = self.step_dev[4 + 4 * max_bs:] if with_states else None       # per row of the step, -1 for padding
         # two pinned staging buffers, used in turn: with one step queued behind another the upload of the
         # first may not have run yet when the host fills in the second
         pin = torch.device(device).type == "cuda"
-        self._step_hosts = [torch.zeros(4 + 4 * max_bs, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
+        self._step_hosts = [torch.zeros(ints, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
         self._step_nps = [h.numpy() for h in self._step_hosts]
         self._step_turn = 0
+        self.clear_step()
+
+    def clear_step(self):
+        """A step without sequences: every row is a padding row."""
+        self.step_dev.zero_()
+        if self.state_slots is not None:
+            self.state_slots.fill_(-1)
 
     def assign(self, seq_id: str) -> int:
         if seq_id in self.row_of:
@@ -273,7 +284,7 @@ class BlockTable:
                                        upload((np.asarray(rows, dtype=np.int32),), self.device)[0], self.table)
 
     def stage_decode_step(self, seqs, ids_on_device=None):
-        """Fill a pinned step buffer [batch | row | pos | slot | token] and start its upload.  With
+        """Fill a pinned step buffer [batch | row | pos | slot | token (| state slot)] and start its upload.  With
         `ids_on_device` (a list: for every sequence its row in the step before) the token of a row is
         written as -1-j: the id that step sampled for its row j and that has not reached the host yet."""
         n, m = len(seqs), self.max_bs
@@ -288,6 +299,9 @@ class BlockTable:
             buf[4 + 3 * m:4 + 3 * m + n] = [-1 - j for j in ids_on_device]
         else:
             buf[4 + 3 * m:4 + 3 * m + n] = [s.token_ids[-1] for s in seqs]
+        if self.state_slots is not None:
+            buf[4 + 4 * m:4 + 4 * m + n] = [s.state_slot for s in seqs]
+            buf[4 + 4 * m + n:] = -1          # no state is read or written for padding rows
         self.step_dev.copy_(self._step_hosts[self._step_turn], non_blocking=True)
 
     def fits(self, seqs) -> bool:
