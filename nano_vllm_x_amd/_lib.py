@@ -203,6 +203,7 @@ INTERNAL.update({name: (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_i64, _c_i64, _c
                  for name in ("nvx_internal_prefill_gemm", "nvx_internal_prefill_gemm_f16")})
 INTERNAL["nvx_internal_table_choices"] = (_c_i32, [ctypes.POINTER(TableChoices), _c_i32, _c_vp, _c_i64, _c_vp])
 INTERNAL["nvx_internal_moe_decode"] = SIGNATURES["nvx_moe_expert_rows"]
+INTERNAL["nvx_internal_moe_postnorm"] = (_c_i32, SIGNATURES["nvx_moe_expert_rows"][1][:-1] + [_c_i32, _c_vp, _c_vp, _c_i64, _c_vp, _c_i64, _c_f32, _c_vp, _c_vp])
 INTERNAL["nvx_internal_moe_grouped"] = (_c_i32, SIGNATURES["nvx_moe_expert_rows"][1][:-1] + [_c_i32, _c_i32, _c_vp])
 INTERNAL["nvx_internal_moe_tile"] = (_c_i32, [_c_i64] * 4)
 INTERNAL["nvx_internal_decode_boundary"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_vp, _c_f32, _c_vp, _c_vp, _c_vp, _c_vp])

@@ -10,7 +10,7 @@
 //     or the stream handed out as a hi + lo pair of 16-bit rows for a matrix product that must see more than 16 bits of it;
 //   - the embedding of such a stack: token row + row of a table of token pairs + learned position row, with that first norm.
 // Norms, gates and the stream are float32 in every activation format.
-#include "fmt_dev.h"
+#include "moe_dev.h"
 
 namespace NVX_NS {
 
@@ -110,38 +110,77 @@ __global__ __launch_bounds__(256) void postnorm_residual_kernel(const A* __restr
 // waits for.  The kernel above reads its rows two elements at a time and some of them three times.  Bound: HBM on long steps (14 bytes an
 // element with one 16-bit result), one trip to memory and two sums on short ones.  4096 rows of 1024: 17.1 -> 11.0 us; 16 rows of 2048:
 // 9.3 -> 5.0 us.
-template <typename A, int NC>
+// PAIRS: the result is the weighted sum of a token's choices of experts, rounded to A as where a launch of its own leaves it (moe_pair_sum_kernel,
+// moe_pair_gather_kernel), added up where it is used, a pair's two rows asked for together.
+struct PairRows {
+    const float* o;             // (pairs, width)
+    const int64_t* dst;         // the row of every pair, below zero: none (null: pair p has row p)
+    const float* wts;           // (null: ones)
+    int top;
+};
+template <typename A, int NC, bool PAIRS>
 __global__ __launch_bounds__(256) void postnorm_residual_wide_kernel(const A* __restrict__ y, int64_t y_stride, const A* __restrict__ y2,
                                                                     int64_t y2_stride, float a, float b, const float* __restrict__ w_post,
                                                                     int w_post_n, float* __restrict__ x, const float* __restrict__ w_next,
-                                                                    int w_next_n, float eps, A* __restrict__ h_out, int width) {
+                                                                    int w_next_n, float eps, A* __restrict__ h_out, int width, PairRows pairs) {
     typedef A veca __attribute__((ext_vector_type(4)));
     __shared__ float red[2][4];
     const int64_t t = blockIdx.x;
     float* xr = x + t * (int64_t)width;
     nvx_f32x4 v[NC], r[NC], wp[NC], wn[NC];
-    const float wp1 = y && w_post_n == 1 ? w_post[0] : 0.f, wn1 = w_next && w_next_n == 1 ? w_next[0] : 0.f;
+    const bool result = PAIRS || y;
+    const float wp1 = result && w_post_n == 1 ? w_post[0] : 0.f, wn1 = w_next && w_next_n == 1 ? w_next[0] : 0.f;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         const int c = (threadIdx.x + i * 256) * 4;
         v[i] = r[i] = wp[i] = wn[i] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
         if (c < width) {
             v[i] = *reinterpret_cast<const nvx_f32x4*>(xr + c);
-            if (y) {
-                const veca u = *reinterpret_cast<const veca*>(y + t * y_stride + c);
+            if constexpr (!PAIRS) {
+                if (y) {
+                    const veca u = *reinterpret_cast<const veca*>(y + t * y_stride + c);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) r[i][k] = a * (float)u[k];
+                    for (int k = 0; k < 4; ++k) r[i][k] = a * (float)u[k];
+                }
+                if (y2) {
+                    const veca u = *reinterpret_cast<const veca*>(y2 + t * y2_stride + c);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) r[i][k] += b * (float)u[k];
+                }
+            }
+            if (result)
                 wp[i] = w_post_n == 1 ? nvx_f32x4{wp1, wp1, wp1, wp1} : *reinterpret_cast<const nvx_f32x4*>(w_post + c);
-            }
-            if (y2) {
-                const veca u = *reinterpret_cast<const veca*>(y2 + t * y2_stride + c);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) r[i][k] += b * (float)u[k];
-            }
             if (w_next) wn[i] = w_next_n == 1 ? nvx_f32x4{wn1, wn1, wn1, wn1} : *reinterpret_cast<const nvx_f32x4*>(w_next + c);
         }
     }
-    if (y) {
+    if constexpr (PAIRS) {
+        for (int k = 0; k < pairs.top; k += 2) {
+            const bool two = k + 1 < pairs.top;
+            const int64_t p0 = t * pairs.top + k, p1 = two ? p0 + 1 : p0;
+            const int64_t at0 = pairs.dst ? pairs.dst[p0] : p0, at1 = pairs.dst ? pairs.dst[p1] : p1;
+            const float f0 = pairs.wts ? pairs.wts[p0] : 1.0f, f1 = pairs.wts ? pairs.wts[p1] : 1.0f;
+            const float *o0 = pairs.o + (at0 < 0 ? 0 : at0) * width, *o1 = pairs.o + (at1 < 0 ? 0 : at1) * width;
+            nvx_f32x4 v0[NC], v1[NC];
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int c = (threadIdx.x + i * 256) * 4;
+                v0[i] = v1[i] = nvx_f32x4{0.f, 0.f, 0.f, 0.f};
+                if (c < width) v0[i] = *reinterpret_cast<const nvx_f32x4*>(o0 + c), v1[i] = *reinterpret_cast<const nvx_f32x4*>(o1 + c);
+            }
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    r[i][j] += f0 * (at0 < 0 ? NAN : v0[i][j]);
+                    if (two) r[i][j] += f1 * (at1 < 0 ? NAN : v1[i][j]);
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r[i][j] = (threadIdx.x + i * 256) * 4 < width ? (float)(A)r[i][j] : 0.f;      // (past the row: no NaN into its sum)
+    }
+    if (result) {
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < NC; ++i) ss += r[i][0] * r[i][0] + r[i][1] * r[i][1] + r[i][2] * r[i][2] + r[i][3] * r[i][3];
@@ -694,9 +733,9 @@ extern "C" int nvx_postnorm_residual(const void* y, int64_t y_stride, const void
     if (width % 4 == 0 && width <= 4096 && ok4(x, 4) && ok4(y, item) && ok4(y2, item) && ok4(h_out, item) && (!y || y_stride % 4 == 0) &&
         (!y2 || y2_stride % 4 == 0) && (!y || w_post_n == 1 || ok4(w_post, 4)) && (w_next_n == 1 || ok4(w_next, 4))) {
 #define NVX_POSTNORM(NC)                                                                                                                        \
-    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((postnorm_residual_wide_kernel<A_, NC>), dim3((unsigned)n_tok), dim3(256), 0, (hipStream_t)stream, (const A_*)y, \
+    NVX_FMT_CALL(fmt, hipLaunchKernelGGL((postnorm_residual_wide_kernel<A_, NC, false>), dim3((unsigned)n_tok), dim3(256), 0, (hipStream_t)stream, (const A_*)y, \
                                          y_stride, (const A_*)y2, y2_stride, a, b, w_post, (int)w_post_n, x, w_next, (int)w_next_n, eps, (A_*)h_out,  \
-                                         (int)width))
+                                         (int)width, PairRows{}))
         if (width <= 1024) NVX_POSTNORM(1);
         else if (width <= 2048) NVX_POSTNORM(2);
         else NVX_POSTNORM(4);
@@ -707,6 +746,31 @@ extern "C" int nvx_postnorm_residual(const void* y, int64_t y_stride, const void
                                          y_stride, (const A_*)y2, y2_stride, a, b, w_post, (int)w_post_n, x, w_next, (int)w_next_n, eps, (A_*)h_out,
                                          (int)width));
     return nvx_check_launch("nvx_postnorm_residual");
+}
+
+// Sums of a token's choices (see PairRows) as the result of nvx_postnorm_residual.  Rows as nvx_pairs_postnorm_fits wants them, 16-bit formats.
+bool nvx_pairs_postnorm_fits(int fmt, const NvxMoeEnd& e, int64_t width) {
+    return fmt < 2 && width % 4 == 0 && width <= 4096 && nvx_aligned16(e.x) && (reinterpret_cast<uintptr_t>(e.h_out) & 7) == 0 &&
+           (e.w_post_n == 1 || nvx_aligned16(e.w_post)) && (e.w_next_n == 1 || nvx_aligned16(e.w_next));
+}
+
+int nvx_pairs_postnorm(int fmt, const float* o, const int64_t* dst, const float* wts, int64_t top, const NvxMoeEnd& e, int64_t n_tok, int64_t width,
+                       hipStream_t stream) {
+    const PairRows pairs{o, dst, wts, (int)top};
+#define NVX_PAIRS(A_, NC)                                                                                                                      \
+    hipLaunchKernelGGL((postnorm_residual_wide_kernel<A_, NC, true>), dim3((unsigned)n_tok), dim3(256), 0, stream, (const A_*)nullptr, (int64_t)0, (const A_*)nullptr, \
+                       (int64_t)0, 1.f, 0.f, e.w_post, (int)e.w_post_n, e.x, e.w_next, (int)e.w_next_n, e.eps, (A_*)e.h_out, (int)width, pairs)
+#define NVX_PAIRS_FMT(NC)                              \
+    do {                                               \
+        if (fmt == 0) NVX_PAIRS(__bf16, NC);           \
+        else NVX_PAIRS(_Float16, NC);                  \
+    } while (0)
+    if (width <= 1024) NVX_PAIRS_FMT(1);
+    else if (width <= 2048) NVX_PAIRS_FMT(2);
+    else NVX_PAIRS_FMT(4);
+#undef NVX_PAIRS_FMT
+#undef NVX_PAIRS
+    return nvx_check_launch("nvx_internal_moe_postnorm");
 }
 
 extern "C" int nvx_hyper_mix(const float* x_in, int64_t in_tok_stride, int64_t in_stream_stride, const void* y, int64_t y_stride, int fmt,

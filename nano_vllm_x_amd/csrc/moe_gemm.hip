@@ -383,7 +383,7 @@ static int launch_moe_product(const MoeWideArgs<A>& a, int64_t pairs, int64_t n_
 // The whole mixture (see nvx_moe_expert_rows) for a step of many tokens; ws as there.  The pairs' order is made here too.
 static int moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
                        int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
-                       int up_tile, int down_tile, hipStream_t st) {
+                       int up_tile, int down_tile, const NvxMoeEnd* end, hipStream_t st) {
     const int64_t pairs = n_tok * top;
     // ws: n_tok * top * (width + ff) floats = the pairs' results (float32), their hidden rows (16 bits), then the order: its counts, source and
     // place of every pair (12 bytes a pair and 256: they fit in the half of the hidden rows that 16 bits leave, 2 * ff >= 128 bytes a pair)
@@ -401,6 +401,7 @@ static int moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* 
                                       (const A_*)w_gu, (int)width, (int)ff, limit, alpha, shift, (void*)y}, pairs, n_tok, up_tile, st)) return rc; \
         if (const int rc = launch_moe_product<A_, false>({(const A_*)y, ff, (const int32_t*)nullptr, 1, (const float*)nullptr, counts, (int)n_exp, (const A_*)w_d,    \
                                        (int)ff, (int)width, limit, alpha, shift, (void*)o}, pairs, pairs, down_tile, st)) return rc; \
+        if (end) return nvx_pairs_postnorm(fmt, (const float*)o, dst, weight_out ? wts : (const float*)nullptr, top, *end, n_tok, width, st);        \
         hipLaunchKernelGGL(moe_pair_gather_kernel<A_>, dim3((unsigned)((n_tok * (width / 4) + 255) / 256)), dim3(256), 0, st, (const float*)o,     \
                            (const int64_t*)dst, weight_out ? wts : (const float*)nullptr, (int)top, (A_*)out, n_tok * (width / 4), (int)(width / 4)); \
     } while (0)
@@ -412,8 +413,8 @@ static int moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* 
 
 int nvx_moe_grouped(const void* h, int64_t h_stride, int fmt, const int32_t* idx, const float* wts, int64_t top, const void* w_gu, const void* w_d,
                     int64_t n_exp, float limit, float alpha, float shift, int weight_out, float* ws, void* out, int64_t n_tok, int64_t width, int64_t ff,
-                    hipStream_t st) {
-    return moe_grouped(h, h_stride, fmt, idx, wts, top, w_gu, w_d, n_exp, limit, alpha, shift, weight_out, ws, out, n_tok, width, ff, MOE_BY_RULE, MOE_BY_RULE, st);
+                    const NvxMoeEnd* end, hipStream_t st) {
+    return moe_grouped(h, h_stride, fmt, idx, wts, top, w_gu, w_d, n_exp, limit, alpha, shift, weight_out, ws, out, n_tok, width, ff, MOE_BY_RULE, MOE_BY_RULE, end, st);
 }
 
 // The same with tiles of the caller's choice (0: the rule's), and the rule itself for sizes and layouts that the wide walk reads.
@@ -424,6 +425,6 @@ extern "C" int nvx_internal_moe_grouped(const void* h, int64_t h_stride, int fmt
                 NVX_EUNSUPPORTED, "nvx_internal_moe_grouped: sizes");
     NVX_REQUIRE(h && idx && wts && w_gu && w_d && ws && out && nvx_aligned16(h) && nvx_aligned16(w_gu) && nvx_aligned16(w_d) && nvx_aligned16(ws) && nvx_aligned16(out), NVX_EINVAL,
                 "nvx_internal_moe_grouped: pointers must be 16-byte aligned");
-    return moe_grouped(h, h_stride, fmt, idx, wts, top, w_gu, w_d, n_exp, limit, alpha, shift, weight_out, ws, out, n_tok, width, ff, up_tile, down_tile, (hipStream_t)stream);
+    return moe_grouped(h, h_stride, fmt, idx, wts, top, w_gu, w_d, n_exp, limit, alpha, shift, weight_out, ws, out, n_tok, width, ff, up_tile, down_tile, nullptr, (hipStream_t)stream);
 }
 extern "C" int nvx_internal_moe_tile(int64_t pairs, int64_t n_exp, int64_t n, int64_t k) { return moe_tile_rule(pairs, n_exp, n, k, k >= 256); }

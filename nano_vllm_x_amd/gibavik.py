@@ -244,8 +244,12 @@ class GibavikForCausalLM(nn.Module):
             else:
                 h = ops.postnorm_residual(x, y=layer.mixer(h, positions, md), w_post=layer.norm1, eps=eps, w_next=closing)
             if layer.mlp is not None:
-                y = layer.mlp(h) if layer.mlp_kind == "dense" else layer.mlp(h, input_ids, decode_step, plan=plans[i])
-                h = ops.postnorm_residual(x, y=y, w_post=layer.norm2, eps=eps, w_next=self.final_norm if last else None)
+                closing = self.final_norm if last else None
+                done = layer.mlp.into_stream(h, decode_step, plans[i], x, layer.norm2, eps, closing) if layer.mlp_kind == "moe" else None
+                if done is None:
+                    y = layer.mlp(h) if layer.mlp_kind == "dense" else layer.mlp(h, input_ids, decode_step, plan=plans[i])
+                    done = ops.postnorm_residual(x, y=y, w_post=layer.norm2, eps=eps, w_next=closing)
+                h = done
             if self.layer_streams is not None:
                 self.layer_streams.append(x.clone())
         return h

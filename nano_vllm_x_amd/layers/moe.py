@@ -10,7 +10,7 @@ from torch import nn
 
 from .. import ops
 from .linear import Linear, gated_rows_fit
-from .plain import bypassable
+from .plain import as_written, bypassable, calls_are_plain, untouched
 
 
 class DenseGLU(nn.Module):
@@ -152,6 +152,7 @@ class SigmoidInputMoE(ExpertBank):
         return self.run(h, idx, wts, decode_step, weight_out=False)
 
 
+@bypassable
 class TableMoE(ExpertBank):
     """No router: `table` (vocab, top) int32 names the experts of every token id (the entries of a row differ); each chosen expert
     weighs 1 / top and the weights apply to the experts' OUTPUTS.  Expert: W_down (silu(W_gate x) * (W_up x))."""
@@ -203,6 +204,15 @@ class TableMoE(ExpertBank):
             idx, wts = self.choices(input_ids)
             return self.run(h, idx, wts, decode_step, weight_out=True)
         return self.run(h, plan["idx"], plan["wts"], decode_step, weight_out=True, order=plan["order"])
+
+    def into_stream(self, h: torch.Tensor, decode_step: bool, plan: dict, x: torch.Tensor, w_post: torch.Tensor, eps: float, w_next=None):
+        """ops.postnorm_residual of what calling this module gives, without the call; None where something else hangs on the call or the step is not
+        one of ops.moe_expert_rows."""
+        if not (untouched(self, TableMoE) and as_written(TableMoE) and calls_are_plain() and type(self.w_gu) is type(self.w_d) is nn.Parameter
+                and self.by_rows(h.shape[0], decode_step, h)):
+            return None
+        return ops.moe_expert_rows_postnorm(h, plan["idx"], plan["wts"], self.w_gu, self.w_d, self.limit, self.alpha, x, w_post, eps, self.shift, True,
+                                            decode_step, w_next)
 
 
 class GroupedSoftmaxMoE(ExpertBank):

@@ -1661,17 +1661,41 @@ def moe_expert_rows(h, idx, wts, w_gu, w_d, limit: float, alpha: float, shift: f
     (clamp(u, +-limit) + shift).  Without a host read, in 16-bit formats: up to 64 tokens an expert's rows are read once for up to 16 of its
     (token, choice) pairs, more tokens are grouped products over the pairs in expert order where these take the sizes (a `decode` step: where
     they are also the faster); float32 and other sizes pair by pair."""
-    _dev(h, idx, wts, w_gu, w_d)
-    n_exp, ff, width = _moe_weights(w_gu, w_d, "moe_expert_rows")
-    t, top = idx.shape
-    _need(h.shape == (t, width) and h.stride(1) == 1 and h.dtype == w_gu.dtype, "moe_expert_rows: h shape / format")
-    _need(idx.dtype == torch.int32 and idx.is_contiguous() and wts.dtype == F32 and wts.is_contiguous() and wts.shape == idx.shape, "moe_expert_rows: choices")
-    out = torch.empty((t, width), dtype=h.dtype, device=h.device)
-    ws = torch.empty((t * top * (ff + width),), dtype=F32, device=h.device)      # hidden activations and output rows between the launches
+    ws, args, out = _moe_rows_args(h, idx, wts, w_gu, w_d, limit, alpha, shift, weight_out, "moe_expert_rows")
     lib = _lib.load()
     run = lib.nvx_internal_moe_decode if decode else lib.nvx_moe_expert_rows
-    _lib.check(run(_ptr(h), h.stride(0), _fmt(h), _ptr(idx), _ptr(wts), top, _ptr(w_gu), _ptr(w_d), n_exp, float(limit), float(alpha), float(shift),
-                   int(bool(weight_out)), _ptr(ws), _ptr(out), t, width, ff, _stream()), "nvx_moe_expert_rows")
+    _lib.check(run(*args, _stream()), "nvx_moe_expert_rows")
+    return out
+
+
+def _moe_rows_args(h, idx, wts, w_gu, w_d, limit, alpha, shift, weight_out, what: str):
+    """(workspace, which has to outlive the call; arguments up to ff; the result)."""
+    _dev(h, idx, wts, w_gu, w_d)
+    n_exp, ff, width = _moe_weights(w_gu, w_d, what)
+    t, top = idx.shape
+    _need(h.shape == (t, width) and h.stride(1) == 1 and h.dtype == w_gu.dtype, what + ": h shape / format")
+    _need(idx.dtype == torch.int32 and idx.is_contiguous() and wts.dtype == F32 and wts.is_contiguous() and wts.shape == idx.shape, what + ": choices")
+    out = torch.empty((t, width), dtype=h.dtype, device=h.device)
+    ws = torch.empty((t * top * (ff + width),), dtype=F32, device=h.device)      # hidden activations and output rows between the launches
+    return ws, (_ptr(h), h.stride(0), _fmt(h), _ptr(idx), _ptr(wts), top, _ptr(w_gu), _ptr(w_d), n_exp, float(limit), float(alpha), float(shift),
+                int(bool(weight_out)), _ptr(ws), _ptr(out), t, width, ff), out
+
+
+def moe_expert_rows_postnorm(h, idx, wts, w_gu, w_d, limit: float, alpha: float, x, w_post, eps: float, shift: float = 1.0, weight_out: bool = False,
+                             decode: bool = False, w_next=None):
+    """postnorm_residual(x, y=moe_expert_rows(h, ...), w_post=w_post, eps=eps, w_next=w_next), the sums of a token's choices in the norm's launch where both
+    are made for the sizes: the same bits in one launch and one pass of the result less."""
+    _dev(x, w_post, w_next)
+    _f32c(x, "moe_expert_rows_postnorm: x")
+    for name, w in (("w_post", w_post), ("w_next", w_next)):
+        if w is not None:
+            _f32c(w, "moe_expert_rows_postnorm: " + name)
+            _need(w.numel() in (1, h.shape[1]), f"moe_expert_rows_postnorm: {name} has one entry or one per channel")
+    _need(w_post is not None and x.shape == h.shape, "moe_expert_rows_postnorm: x has the shape of h, the result its norm weight")
+    ws, args, y = _moe_rows_args(h, idx, wts, w_gu, w_d, limit, alpha, shift, weight_out, "moe_expert_rows_postnorm")
+    out = torch.empty_like(y)
+    _lib.check(_lib.load().nvx_internal_moe_postnorm(*args, int(bool(decode)), _ptr(x), _ptr(w_post), w_post.numel(), _ptr(w_next),
+                                                     w_next.numel() if w_next is not None else 0, float(eps), _ptr(out), _stream()), "nvx_moe_expert_rows")
     return out
 
 
