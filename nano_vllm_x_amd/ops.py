@@ -2028,9 +2028,11 @@ def gla_scan(x, offsets, alpha, mem, layout: StepLayout, heads: int, dim: int, v
 def memory_step_fits(layout: StepLayout, h, mem, w1, w2=None) -> bool:
     """Whether mlstm_step (w1: its gates' weights) or gla_step (w1, w2: its decays') serves this step: one token per sequence, heads and rows that
     their kernel is built for.  Every head of every sequence computes gla's `rank` numbers again, so they must be few."""
+    if layout.qo_indptr is not None:
+        return False
     heads, dim, vdim = mem.shape[1:]
     item = 4 * h.element_size()
-    if layout.qo_indptr is not None or vdim % 4 or vdim > 1024 or dim > 512 or h.shape[1] % 4 or h.stride(0) % 4 or h.stride(1) != 1 or layout.n_tok > 65535:
+    if vdim % 4 or vdim > 1024 or dim > 512 or h.shape[1] % 4 or h.stride(0) % 4 or h.stride(1) != 1 or layout.n_tok > 65535:
         return False
     if h.data_ptr() % item or any(t.data_ptr() % 16 for t in (mem, w1) + (() if w2 is None else (w2,))):
         return False

@@ -235,30 +235,36 @@ class ZenedraForCausalLM(nn.Module):
         x, h = ops.embed_sum(input_ids, self.embed, md.layout, pair=self.pair, mul_prev=b["mul_prev"], mul_cur=b["mul_cur"],
                              prev_id=md.cache.state("prev_id") if self.pair is not None else None, pos_table=self.pos, positions=positions,
                              w=None if cfg.loop else norms[0], eps=eps, split=bool(cfg.loop) and pairs)
+        few = x.shape[0] <= ops.LEAD_ROWS      # (longer steps, the short ones of them bound by the host, ask nothing of the modules at a boundary)
         from_x0, made = None, None
         if cfg.loop:
             from_x0 = self._join(x, h if pairs else None, 1)       # the same for every pass
             if starts[0] is None:
                 h = ops.residual_norm(x, w=norms[0], eps=eps, dtype=dtype)
             else:
-                x, h, made = self._begin_pass(x, h if pairs else None, from_x0, starts[0], norms[0], layers[runs[0][0]].mixer)
+                x, h, made = self._begin_pass(x, h if pairs else None, from_x0, starts[0], norms[0], layers[runs[0][0]].mixer if few else None)
         for n, (i, name, _) in enumerate(runs):
             layer = layers[i]
             y, y2 = layer.mixer(h, md, at=name) if made is None else layer.mixer(h, md, at=name, made=made), None
             if layer.mlp is not None:
-                x, h, made = self._boundary(layer.mlp, x, y, norm=layer.norm2)
+                if few:
+                    x, h, made = self._boundary(layer.mlp, x, y, norm=layer.norm2)
+                else:
+                    h = ops.residual_norm(x, y, w=layer.norm2, eps=eps)
                 if layer.mlp_kind == "dense":
                     y = layer.mlp(h) if made is None else layer.mlp(h, made=made)
                 else:
                     y, y2 = layer.mlp(h, decode_step)
-            if starts[n + 1] is None:
+            if starts[n + 1] is None and not few:
+                h = ops.residual_norm(x, y, y2, w=norms[n + 1], eps=eps)
+            elif starts[n + 1] is None:
                 x, h, made = self._boundary(layers[runs[n + 1][0]].mixer if n + 1 < len(runs) else None, x, y, y2, norm=norms[n + 1])
             else:
                 h = ops.residual_norm(x, y, y2, split=pairs, dtype=dtype)
             if self.layer_streams is not None:
                 self.layer_streams.append(x.clone())
             if starts[n + 1] is not None:
-                x, h, made = self._begin_pass(x, h, from_x0, starts[n + 1], norms[n + 1], layers[runs[n + 1][0]].mixer)
+                x, h, made = self._begin_pass(x, h, from_x0, starts[n + 1], norms[n + 1], layers[runs[n + 1][0]].mixer if few else None)
         return h
 
     def _begin_pass(self, x, pair_rows, from_x0, t: int, norm, mixer):
