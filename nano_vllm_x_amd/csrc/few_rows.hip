@@ -1,14 +1,14 @@
 // y = x W^T (+ bias) for the few rows of a decode step, in the 16-bit format or as unrounded float32 sums: the projections of the models
 // with per-sequence state.
 //
-// Such a product is one pass over W.  A workgroup of eight waves takes 16 rows of W whole: every wave a strided eighth of K, 64 columns
+// Such a product is one pass over W.  A workgroup of eight waves takes 16 rows of W whole (eight where there are few): every wave a strided eighth of K, 64 columns
 // (a 128-byte line of every row) at a time, of W and of x, through a ring in LDS that is its own: no barrier until the waves' sums meet,
 // in a fixed order.  A layer of 1024 outputs is 64 workgroups whose loads are nearly all in flight at once, where tiles that take K in
 // sequence wait once per step.  Lines travel to LDS without registers; loaded straight in operand order (64 separate 16-byte requests an
 // instruction, which the address unit serves one a clock) 1024 x 2048 took 5.8 us instead of 3.8.
-// 16 rows, N x K, us here and the library's (and the time of W's bytes at 4.9 TB/s): 1024 x 1024 3.2, 5.9 (0.4); 4096 x 1024 4.2, 7.6 (1.7);
-// 1024 x 2048 3.8, 8.2 (0.9); 2048 x 2048 5.0, 11.0 (1.7); 9216 x 2048 11.7, 16.1 (7.7); 1024 x 3072 4.6, 9.7 (1.3); 2048 x 6144 11.7, 12.0 (5.1);
-// 32000 x 2048 28.8, 34.0 (26.7).  32 rows: 1024 x 2048 4.5, 8.4; 2048 x 6144 13.5, 16.6; 32000 x 1024 17, 25.
+// 16 rows, N x K, us here and the library's (and the time of W's bytes at 4.9 TB/s): 1024 x 1024 2.9, 5.9 (0.4); 4096 x 1024 4.2, 7.6 (1.7);
+// 1024 x 2048 3.7, 8.2 (0.9); 2048 x 2048 4.7, 11.0 (1.7); 9216 x 2048 11.7, 16.1 (7.7); 1024 x 3072 5.3, 9.7 (1.3); 2048 x 6144 10.1, 12.0 (5.1);
+// 32000 x 2048 28.8, 34.0 (26.7).  32 rows: 1024 x 2048 4.6, 8.4; 2048 x 6144 12.0, 16.6; 32000 x 1024 17, 25.
 #include "fmt_dev.h"
 
 namespace NVX_NS {
@@ -32,7 +32,7 @@ __device__ __forceinline__ void line_to_lds(const void* g, unsigned lds) {
 }
 
 // the waves' sums meet in `smem` (their rings, which nobody reads any more), in a fixed order, and leave as the product's rows
-template <typename A, int MT, int NT, int GLU>
+template <typename A, int MT, int NT, int GLU, int WR = 16>
 __device__ __forceinline__ void few_rows_end(unsigned char* smem, const nvx_f32x4 (&acc)[NT][MT], const A* __restrict__ bias, void* __restrict__ y, int f32_out,
                                              int rows, int n, int n0, float limit, float alpha, float shift) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
@@ -50,7 +50,7 @@ __device__ __forceinline__ void few_rows_end(unsigned char* smem, const nvx_f32x
 #pragma unroll
             for (int i = 1; i < FR_WAVES; ++i) { g += part[i][wave][lane]; u += part[i][MT + wave][lane]; }
             const int r = 16 * wave + l16;
-            if (r < rows) {
+            if (r < rows && (WR == 16 || quad < 2)) {
                 typedef A vec4 __attribute__((ext_vector_type(4)));
                 vec4 o;
 #pragma unroll
@@ -65,7 +65,8 @@ __device__ __forceinline__ void few_rows_end(unsigned char* smem, const nvx_f32x
         nvx_f32x4 s = part[0][wave][lane];
 #pragma unroll
         for (int i = 1; i < FR_WAVES; ++i) s += part[i][wave][lane];
-        const int r = 16 * (wave % MT) + l16, o = n0 + 16 * (wave / MT) + 4 * quad;
+        const int r = 16 * (wave % MT) + l16, o = n0 + WR * (wave / MT) + 4 * quad;
+        if (WR == 8 && quad >= 2) return;
         if (bias)
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[i] += (float)bias[o + i];
@@ -77,21 +78,22 @@ __device__ __forceinline__ void few_rows_end(unsigned char* smem, const nvx_f32x
     }
 }
 
-// MT: tiles of 16 rows of x; DEPTH: pieces of 64 columns a wave has on their way.  k % 512 == 0, n % 16 == 0, rows <= 16 * MT.
-template <typename A, int MT, int NT, int DEPTH, int GLU>
+// MT: tiles of 16 rows of x; DEPTH: pieces of 64 columns a wave has on their way.  k % 512 == 0, n % 16 == 0, rows <= 16 * MT.  WR: rows of w in a tile; with
+// 8 the matrix instruction has each of them twice, and the second half of its results is left.
+template <typename A, int MT, int NT, int DEPTH, int GLU, int WR>
 __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __restrict__ x, int64_t x_stride, const A* __restrict__ w,
                                                                 const A* __restrict__ bias, void* __restrict__ y, int f32_out, int rows, int n, int k,
                                                                 float limit, float alpha, float shift) {
     static_assert(!GLU || NT == 2, "16 gate rows and the 16 up rows beside them");
-    constexpr int PIECE = (NT + MT) * 2048, LOADS = 2 * (NT + MT);         // [16 NT rows of w | 16 MT rows of x], 128 bytes each
+    constexpr int WL = NT * WR / 8, LOADS = WL + 2 * MT, PIECE = LOADS * 1024;      // [WR NT rows of w | 16 MT rows of x], 128 bytes each
     static_assert(DEPTH * PIECE >= MT * NT * 1024, "the sums meet in the pieces' memory");
     __shared__ __align__(16) unsigned char smem[FR_WAVES * DEPTH * PIECE];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, n0 = blockIdx.x * 16 * (GLU ? 1 : NT);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, n0 = blockIdx.x * WR * (GLU ? 1 : NT);
     const A* from[LOADS];                                                  // rows 8 i + lane / 8; the piece that belongs at place lane % 8
     const int r8 = lane >> 3, c = wave * 64 + ((lane & 7) ^ r8) * 8;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-        from[i] = i < 2 * NT ? w + (int64_t)(n0 + (GLU && i >= 2 ? n / 2 - 16 : 0) + 8 * i + r8) * k + c : x + (int64_t)min(8 * (i - 2 * NT) + r8, rows - 1) * x_stride + c;   // (rows past the last are not stored)
+        from[i] = i < WL ? w + (int64_t)(n0 + (GLU && i >= WL / 2 ? n / 2 - WR : 0) + 8 * i + r8) * k + c : x + (int64_t)min(8 * (i - WL) + r8, rows - 1) * x_stride + c;   // (rows past the last are not stored)
     const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)smem + wave * DEPTH * PIECE;
     typedef __attribute__((address_space(3))) const nvx_u32x4 lds_u4;
     auto ask = [&](int t) {
@@ -110,15 +112,15 @@ __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __rest
         // piece t has landed, up to DEPTH - 1 later ones need not have (only this wave reads what it asked for: no barrier)
         if (t + DEPTH <= turns) asm volatile("s_waitcnt vmcnt(%0)" : : "n"((DEPTH - 1) * LOADS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        const unsigned at = lds0 + (unsigned)(t % DEPTH) * PIECE + l16 * 128;
+        const unsigned at = lds0 + (unsigned)(t % DEPTH) * PIECE, w_at = at + (l16 & (WR - 1)) * 128, x_at = at + WL * 1024 + l16 * 128;
         nvx_u32x4 fw[2][NT], fx[2][MT];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const unsigned off = (unsigned)((4 * h + quad) ^ (l16 & 7)) * 16;
 #pragma unroll
-            for (int i = 0; i < NT; ++i) fw[h][i] = *reinterpret_cast<lds_u4*>((uintptr_t)(at + i * 2048 + off));
+            for (int i = 0; i < NT; ++i) fw[h][i] = *reinterpret_cast<lds_u4*>((uintptr_t)(w_at + i * (WR * 128) + off));
 #pragma unroll
-            for (int j = 0; j < MT; ++j) fx[h][j] = *reinterpret_cast<lds_u4*>((uintptr_t)(at + (NT + j) * 2048 + off));
+            for (int j = 0; j < MT; ++j) fx[h][j] = *reinterpret_cast<lds_u4*>((uintptr_t)(x_at + j * 2048 + off));
         }
         asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");               // read before the place is filled again
         if (t + DEPTH < turns) ask(t + DEPTH);
@@ -129,7 +131,7 @@ __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __rest
 #pragma unroll
                 for (int j = 0; j < MT; ++j) acc[i][j] = mfma_few(fw[h][i], fx[h][j], acc[i][j], A{});
     }
-    few_rows_end<A, MT, NT, GLU>(smem, acc, bias, y, f32_out, rows, n, n0, limit, alpha, shift);
+    few_rows_end<A, MT, NT, GLU, WR>(smem, acc, bias, y, f32_out, rows, n, n0, limit, alpha, shift);
 }
 
 // The same with what stands in front of it: x_out = x (+ y) (+ add) (+ x_bias), h = x_out / rms(x_out) * w_norm in the format, out = h W^T.  Every
@@ -233,19 +235,28 @@ __global__ __launch_bounds__(2 * FR_WAVES * 64) void few_rows_lead_kernel(const 
     few_rows_end<A, 1, NT, GLU>(smem, acc, bias, out, 0, rows, n, n0, 0.f, 0.f, 0.f);
 }
 
-// 16 rows of w a workgroup leave the most workgroups for the chip; where there are more than run at once, more of them share the reads of x.  us at
+// What a workgroup waits for is its rows of w and of x, at some 34 bytes a clock for a compute unit, and 16 rows of x are as much as 16 of w.  While twice the
+// workgroups still find a compute unit each, they take eight rows of w (the same sums in the same order).  us, tiles of 16 / of eight, 16 rows: 512 x 4096 5.3 / 4.7, 1024 x 2048 4.0 / 3.7,
+// 2048 x 2048 5.15 / 4.7, 1024 x 3072 6.0 / 5.3, 2048 x 6144 11.4 / 10.1, gated 2048 x 1024 4.0 / 3.8, 4096 x 2048 7.0 / 6.3; one row 2048 x 2048 4.5 / 4.3; 32 rows 6.2 / 5.6; past that line 16 rows 3072 x 2048 5.6 / 6.4,
+// gated 6144 x 1024 5.3 / 5.9.  (More pieces of K on their way instead, all loads of a workgroup at once: 2 to 4 % slower.)
+// Beyond, 16 rows of w a workgroup leave the most workgroups for the chip; where there are more than run at once, more of them share the reads of x.  us at
 // 16 rows, 16 against 64 rows of w: 9216 x 2048 11.7 / 11.9, 12288 x 2048 14.0 / 13.4, 32000 x 1024 18.2 / 14.6; at 32 rows, 16 against
 // 32: 4096 x 2048 7.4 / 8.1, 6144 x 1024 7.5 / 6.1, 8192 x 4096 21.0 / 18.0.
 template <typename A, int MT>
 static void launch_few_rows(const void* x, int64_t x_stride, const void* w, const void* bias, void* y, int f32_out, int rows, int n, int k, int glu,
                             float limit, float alpha, float shift, hipStream_t st) {
-#define NVX_FEW(N_, D_, G_) hipLaunchKernelGGL((few_rows_kernel<A, MT, N_, D_, G_>), dim3((unsigned)(n / (16 * N_))), dim3(FR_WAVES * 64), 0, st, (const A*)x, x_stride, \
+#define NVX_FEW(N_, D_, G_, W_) hipLaunchKernelGGL((few_rows_kernel<A, MT, N_, D_, G_, W_>), dim3((unsigned)(n / (W_ * N_))), dim3(FR_WAVES * 64), 0, st, (const A*)x, x_stride, \
                                            (const A*)w, (const A*)bias, y, f32_out, rows, n, k, limit, alpha, shift)
-    if (glu == 1) NVX_FEW(2, 2, 1);
-    else if (glu == 2) NVX_FEW(2, 2, 2);
-    else if (n >= 12288 && n % 64 == 0) NVX_FEW(4, 1, 0);
-    else if (MT == 2 && n > 4096 && n % 32 == 0) NVX_FEW(2, 2, 0);
-    else NVX_FEW(1, 2, 0);
+    constexpr int CUS = 256;
+    if (glu && n <= 16 * CUS) {
+        if (glu == 1) NVX_FEW(2, 2, 1, 8);
+        else NVX_FEW(2, 2, 2, 8);
+    } else if (glu == 1) NVX_FEW(2, 2, 1, 16);
+    else if (glu == 2) NVX_FEW(2, 2, 2, 16);
+    else if (n >= 12288 && n % 64 == 0) NVX_FEW(4, 1, 0, 16);
+    else if (MT == 2 && n > 4096 && n % 32 == 0) NVX_FEW(2, 2, 0, 16);
+    else if (n <= 8 * CUS) NVX_FEW(1, 2, 0, 8);
+    else NVX_FEW(1, 2, 0, 16);
 #undef NVX_FEW
 }
 

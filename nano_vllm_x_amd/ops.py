@@ -2109,7 +2109,8 @@ FEW_ROWS = 32       # rows that csrc/few_rows.hip holds
 
 
 def few_rows_faster(rows: int, n: int, k: int) -> bool:
-    """Whether csrc/few_rows.hip beats the library's product of `rows` rows with n outputs from k columns (weights coming from memory).  us, library / here:
+    """Whether csrc/few_rows.hip beats the library's product of `rows` rows with n outputs from k columns (weights coming from memory).  us, library / here
+    (products of up to 2048 outputs with their tiles of 16 rows of w; those of eight take a tenth less):
     up to 16 rows every width of k <= 4096 (16 rows, 32000 x 4096 58 / 48, 6144 x 4096 14.5 / 13.6); deeper ones while the workgroups are few (2048 x 8192
     12.7 / 12.0, 4096 x 6144 22.7 / 12.3, but 6144 x 5120 15.9 / 16.9, 4096 x 16384 30 / 33), or very many (12288 x 6144 34.1 / 33.4).  Beyond 16 rows a
     compute unit holds one workgroup: not where a second turn of them is a quarter full or less (9216 x 2560 15.2 / 17.8, 24576 x 3072 30.8 / 34.7; 8192 x
@@ -2121,7 +2122,8 @@ def few_rows_faster(rows: int, n: int, k: int) -> bool:
 
 def gated_rows_faster(rows: int, n: int, k: int) -> bool:
     """The same for a [gate | up] projection that ends in its activation (n: both halves), against the product and the activation's own launch: 17 rows,
-    6144 x 4096 17.6 / 14.9, 32 rows 12288 x 3072 21.0 / 21.8, 16 rows 2048 x 6144 14.3 / 14.4."""
+    6144 x 4096 17.6 / 14.9, 32 rows 12288 x 3072 21.0 / 21.8, 16 rows 2048 x 6144 14.3 / 14.4 (in tiles
+    of 16; up to 4096 outputs go by eight now, a tenth faster)."""
     return k <= 4096 and (rows <= 16 or (n <= 32768 and _turns_are_full(n // 32)))
 
 
