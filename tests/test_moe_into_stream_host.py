@@ -22,6 +22,6 @@ def test_the_call_is_made_where_something_hangs_on_it(what, monkeypatch):
     elif what == "weight":
         m.w_gu = type("P", (torch.nn.Parameter,), {})(m.w_gu.data)
     h = torch.zeros(3, 64)
-    with torch.overrides.TorchFunctionMode() if what == "mode" else torch.no_grad():
+    with torch.overrides.BaseTorchFunctionMode() if what == "mode" else torch.no_grad():
         got = m.into_stream(h, False, {"idx": None, "wts": None, "order": None}, h, torch.ones(1), 1e-5)
     assert (got == "made") if what == "nothing" else (got is None)
