@@ -245,7 +245,8 @@ class GibavikForCausalLM(nn.Module):
                 h = ops.postnorm_residual(x, y=layer.mixer(h, positions, md), w_post=layer.norm1, eps=eps, w_next=closing)
             if layer.mlp is not None:
                 closing = self.final_norm if last else None
-                done = layer.mlp.into_stream(h, decode_step, plans[i], x, layer.norm2, eps, closing) if layer.mlp_kind == "moe" else None
+                # (asked of the module that stands here: a wrapper that hands look-ups on to the one inside is called like any other module)
+                done = layer.mlp.into_stream(h, decode_step, plans[i], x, layer.norm2, eps, closing) if type(layer.mlp) is TableMoE else None
                 if done is None:
                     y = layer.mlp(h) if layer.mlp_kind == "dense" else layer.mlp(h, input_ids, decode_step, plan=plans[i])
                     done = ops.postnorm_residual(x, y=y, w_post=layer.norm2, eps=eps, w_next=closing)

@@ -138,6 +138,9 @@ class ExpertBank(nn.Module):
         return ops.moe_gather_rows(ys, dst, wts if weight_out else None)
 
 
+_RUN = ExpertBank.run      # as it is written here: TableMoE.into_stream passes it by
+
+
 class SigmoidInputMoE(ExpertBank):
     """scores = sigmoid(W_router h) (float32); every token takes the `top` experts with the largest scores, and a score
     scales its expert's INPUT (no renormalisation): out = sum_e expert_e(score_e * h).  Expert: g = min(W_gate x, limit),
@@ -208,8 +211,8 @@ class TableMoE(ExpertBank):
     def into_stream(self, h: torch.Tensor, decode_step: bool, plan: dict, x: torch.Tensor, w_post: torch.Tensor, eps: float, w_next=None):
         """ops.postnorm_residual of what calling this module gives, without the call; None where something else hangs on the call or the step is not
         one of ops.moe_expert_rows."""
-        if not (untouched(self, TableMoE) and as_written(TableMoE) and calls_are_plain() and type(self.w_gu) is type(self.w_d) is nn.Parameter
-                and self.by_rows(h.shape[0], decode_step, h)):
+        if not (untouched(self, TableMoE) and as_written(TableMoE) and calls_are_plain() and TableMoE.run is _RUN and "run" not in vars(self)
+                and type(self.w_gu) is type(self.w_d) is nn.Parameter and self.by_rows(h.shape[0], decode_step, h)):
             return None
         return ops.moe_expert_rows_postnorm(h, plan["idx"], plan["wts"], self.w_gu, self.w_d, self.limit, self.alpha, x, w_post, eps, self.shift, True,
                                             decode_step, w_next)
