@@ -75,6 +75,8 @@ class ModelRunner:
         self._stage_output, self._defer_stage_send = None, False
         self.decode_chain: Optional[ops.DecodeChain] = None      # decode steps whose layers are one launch, and their graphs
         self.chain_graph: Optional[HIPGraph] = None
+        self._chain_steps: list = []         # launched, ids not collected: such steps and those that read their ids, for computing them again
+        self._by_chain, self._chain_left, self._chain_lost, self._collected = False, 0, False, []
         self._last_done = 0.0
         self.stats = {"prefill_steps": 0, "decode_steps": 0, "graph_steps": 0, "eager_decode_steps": 0, "prefill_s": 0.0, "decode_s": 0.0}
         self.graph_sizes_dropped: list = []               # decode batch sizes whose graph was slower than a larger one's
@@ -275,11 +277,16 @@ class ModelRunner:
     @torch.inference_mode()
     def compute_hidden(self, batch: ForwardBatch, ids_on_device=None):
         """Forward pass of one scheduled batch -> the normed hidden state of each sequence's last token (num_seqs, hidden);
-        None on a pipeline stage other than the last."""
+        None on a pipeline stage other than the last.  Nothing is waited for: a decode step whose layers gave up waiting for each other (ops.DecodeChain)
+        gives NaN, and the next step asked for says so."""
         decode = batch.forward_mode == ForwardMode.DECODE
         tpd.check_peer_status()      # results leave through here too (tests, tools): never on top of a failed exchange
-        if self.decode_chain is not None:
-            self.decode_chain.check()
+        self._by_chain = False
+        self._settle_chain()
+        if self._chain_lost:
+            self._chain_lost = False
+            raise RuntimeError("a decode step gave up waiting for its own workgroups (the device was taken by other work) when its results had left already: they are "
+                               "NaN, and so may be the rows it wrote; steps go layer by layer from here on")
         if self.graph_step_possible(batch):
             hidden = self._execute_model_graph(batch, ids_on_device)
             self.stats["graph_steps"] += 1
@@ -310,7 +317,7 @@ class ModelRunner:
         step can be queued while the one before it is still running."""
         if batch.num_seqs == 0:
             return None
-        t0 = time.perf_counter()
+        t0, left = time.perf_counter(), self._chain_left
         temperatures, min_ps, top_ps, top_ks = self.prepare_sampling_params(batch)
         n = batch.num_seqs
         if (self._lmhead_packed is not None and self.pp_size == 1 and self._sp_unfiltered and n <= min(self.max_bs, LMHEAD_FUSED_MAX_ROWS)
@@ -326,10 +333,15 @@ class ModelRunner:
                                          self.sampler.calls, ws=self._lmhead_ws, keys=True)
                 ids = ops.sample_pick(tpd.tp_all_gather_rows(keys), out=self._sample_out[:n])
             else:
-                ids = ops.lmhead_sample(self._lmhead_packed, self._lmhead_rows, hidden, temperatures, start, vocab, self.sampler.seed,
-                                        self.sampler.calls, ws=self._lmhead_ws, out=self._sample_out[:n])
+                def draw(hidden, call):
+                    return ops.lmhead_sample(self._lmhead_packed, self._lmhead_rows, hidden, temperatures, start, vocab, self.sampler.seed, call,
+                                             ws=self._lmhead_ws, out=self._sample_out[:n])
+                ids = draw(hidden, self.sampler.calls)
             self.stats["fused_lm_head_steps"] = self.stats.get("fused_lm_head_steps", 0) + 1
-            return (batch, self._ids_to_host(ids, n), t0)
+            k = self._ids_to_host(ids, n)
+            if self.decode_chain is not None:
+                self._keep_chain_step(k, n, ids_on_device, draw, left)
+            return (batch, k, t0)
         if self.tp_size > 1 and self.pp_size == 1 and self._sp_unfiltered and n <= self.max_bs and self.shard_sampling:
             # every rank draws over its own shard of the vocabulary; the ranks exchange one 64-bit key per row and all
             # pick the same token: no gather of the logits (vocab_parallel_embedding.py:147-151), no broadcast of the ids
@@ -344,7 +356,48 @@ class ModelRunner:
         else:
             ids = self.sampler(logits, temperatures, min_ps, top_ps, top_ks, out=self._sample_out[:n] if n <= self.max_bs else None)
         tpd.broadcast_sampled_ids(ids)
-        return (batch, self._ids_to_host(ids, n), t0)
+        k = self._ids_to_host(ids, n)
+        if self.decode_chain is not None:
+            def draw(hidden, call):
+                self.sampler.calls, now = call - 1, self.sampler.calls
+                try:
+                    return self.sampler(self.model.compute_logits(hidden), temperatures, min_ps, top_ps, top_ks, out=self._sample_out[:n])
+                finally:
+                    self.sampler.calls = now
+            self._keep_chain_step(k, n, ids_on_device, draw, left)
+        return (batch, k, t0)
+
+    def _keep_chain_step(self, k: int, n: int, ids_on_device, draw, left: int):
+        """What a launched step would be computed again from: for those whose layers were one launch, and those that read the ids of such a step."""
+        by_chain, self._by_chain, self._chain_left = self._by_chain, False, left      # (its ids are collected: what it leaves is looked at)
+        if by_chain or (self._chain_steps and ids_on_device is not None):
+            self._chain_steps = self._chain_steps[-1:] + [(k, n, self.block_table.steps_staged, self.sampler.calls, draw)]
+
+    @torch.inference_mode()
+    def _settle_chain(self):
+        """Where a step of ops.DecodeChain has given up: no further step goes that way, and those whose ids were not collected are computed again layer by layer,
+        with the draws they had.  Results that left through compute_hidden or compute_logits cannot be (_chain_lost)."""
+        if self.decode_chain is None or not self.decode_chain.failed:
+            return
+        if any(self.block_table.steps_staged - staged > 1 for _, _, staged, _, _ in self._chain_steps):
+            raise RuntimeError("a decode step gave up waiting for its own workgroups with its ids not collected two steps later: it cannot be computed again")
+        torch.cuda.synchronize(self.device)
+        print(f"[nano_vllm_x_amd] rank {self.rank}: a decode step in one launch gave up waiting for its own workgroups (other work holds the device); decode steps go "
+              "layer by layer from here on", file=sys.stderr, flush=True)
+        self.chain_graph.clear()
+        self.decode_chain = self.chain_graph = None
+        steps, self._chain_steps = self._chain_steps, []
+        self._chain_lost, self._chain_left = self._chain_lost or self._chain_left > 0, 0
+        if steps and 0 < len(self._collected) <= self.max_bs:      # the ids that the first of them may read: its own draw has taken their place
+            self._sample_out[:len(self._collected)] = torch.tensor(self._collected, dtype=torch.int64, device=self.device)
+        for k, n, staged, call, draw in steps:
+            self.block_table.stage_again(staged)
+            size = self.graph.match_bs(n)
+            self.graph.replay(size)
+            ids = draw(self.graph.get_output_buffer(f"hidden_states {size}")[:n], call)
+            self._sample_hosts[k][:n].copy_(ids, non_blocking=True)
+            self._sample_events[k].record()
+        self.stats["chain_steps_again"] = len(steps)
 
     def _ids_to_host(self, ids: torch.Tensor, n: int):
         """Start the copy of a step's ids into the next pinned buffer; returns what finish_step needs."""
@@ -395,16 +448,23 @@ class ModelRunner:
         n = batch.num_seqs
         if isinstance(ids, int):     # index of the pinned buffer the ids land in
             self._sample_events[ids].synchronize()
+            if self.decode_chain is not None:
+                self._settle_chain()      # (it may have computed this step again)
+                self._sample_events[ids].synchronize()
+                at = next((i for i, step in enumerate(self._chain_steps) if step[0] == ids), None)
+                if at is not None:
+                    if self._chain_left < self._chain_steps[at][2]:
+                        self._chain_left = 0      # (what left ahead of a step that is whole is whole)
+                    del self._chain_steps[:at + 1]
             out = self._sample_hosts[ids][:n].tolist()
         else:
             out = ids.tolist()
+        self._collected = out
         key = "decode_s" if batch.forward_mode == ForwardMode.DECODE else "prefill_s"
         try:
             tpd.check_peer_status()      # a direct-peer exchange that gave up waiting must not pass as a result
         except RuntimeError as e:
             raise RuntimeError(f"{e} [rank {self.rank}, {key[:-2]} step of {n} sequences, steps so far {self.stats}]") from None
-        if self.decode_chain is not None:
-            self.decode_chain.check()
         # launch to completion; a step queued behind another is charged from the moment that one completed
         now = time.perf_counter()
         self.stats[key] = self.stats.get(key, 0.0) + (now - max(t0, self._last_done))
@@ -458,6 +518,7 @@ class ModelRunner:
             padded = chain.match_bs(bs)
             self.decode_chain.in_turn(lambda: chain.replay(padded))
             self.stats["chain_steps"] = self.stats.get("chain_steps", 0) + 1
+            self._by_chain, self._chain_left = True, self.block_table.steps_staged
             return chain.get_output_buffer(f"hidden_states {padded}")[:bs]
         self.graph.replay(padded)
         return self.graph.get_output_buffer(f"hidden_states {padded}")[:bs]
@@ -519,15 +580,21 @@ class ModelRunner:
             with self.graph.capture(bs):
                 self.graph.set_output_buffer(f"hidden_states {bs}", self._decode_forward(bs))
         if self.decode_chain is not None:
-            self.chain_graph = HIPGraph()
-            self.chain_graph.graph_pool = self.graph.graph_pool      # (steps of either follow each other on a stream)
-            for bs in reversed(sizes):
-                if bs <= ops.DecodeChain.ROWS:
-                    with self.chain_graph.capture(bs):
-                        self.chain_graph.set_output_buffer(f"hidden_states {bs}", self._decode_forward(bs, self.decode_chain))
+            if self.decode_chain.failed:      # (the warm-up found the device taken)
+                self.decode_chain = None
+            else:
+                self._capture_chain([bs for bs in sizes if bs <= ops.DecodeChain.ROWS])
         torch.cuda.synchronize()
         if os.environ.get("NVX_GRAPH_PRUNE", "1") != "0":
             self.prune_slow_graph_sizes()
+
+    @torch.inference_mode()
+    def _capture_chain(self, sizes):
+        self.chain_graph = HIPGraph()
+        self.chain_graph.graph_pool = self.graph.graph_pool      # (steps of either follow each other on a stream)
+        for bs in reversed(sizes):
+            with self.chain_graph.capture(bs):
+                self.chain_graph.set_output_buffer(f"hidden_states {bs}", self._decode_forward(bs, self.decode_chain))
 
     def prune_slow_graph_sizes(self, reps: int = 3, margin: float = 1.04):
         """A padded batch costs what its projections cost at that many rows, and a BLAS library's choice of kernel is not

@@ -19,9 +19,11 @@
 //   * Attention: workgroup g has head g % 8, so that a head's projections, chunks and read-outs stay within what is one XCD here, and chunk g / 8 of the step's rows;
 //     chunks are as short as 16 for all rows allow, so long rows get more of them.  The first 64 keys and values of a chunk are on their way before the queries exist.
 //
-// Every wait ends: a word that does not come within `ticks` of the wall clock makes the wave stop waiting for the rest of the launch and raises the status word
-// on the host, which the host looks at before it uses results.  What a wait is for is another workgroup of the same launch, so all 128 have to be on the chip at
-// once; the host asks the device for twice that room (nvx_internal_decode_chain_fits) and lets no more than two go side by side (ops.DecodeChain).
+// Every wait ends: a word that does not come within `ticks` of the wall clock makes the wave stop waiting for the rest of the launch.  Nothing that such a launch
+// leaves passes for a result: its workgroup ends with NaN for every row, marks the words as no longer good (launches queued behind this one find that and end the
+// same way), and raises the status word on the host, which computes the steps whose ids nobody has yet again, launch by launch (ModelRunner).
+// What a wait is for is another workgroup of the same launch, so all 128 have to be on the chip at
+// once; the host asks the device for twice that room (nvx_internal_decode_chain_fits) and lets no more than two of a process go side by side (ops.DecodeChain).
 #include "nvx_dev.h"
 #include "rope_dev.h"
 
@@ -43,7 +45,7 @@ struct DcArgs {
     const float* cos_sin;
     int64_t max_pos, n_slots;
     unsigned long long* words;
-    unsigned* epoch;
+    unsigned* epoch;                    // the first tag of the step, and whether a launch has given up (then every wait of a later one has run out as it starts)
     int* status;
     long long ticks;
     float eps, scale_log2;
@@ -293,8 +295,9 @@ __global__ __launch_bounds__(DC_WAVES * 64, 1) void decode_chain_kernel(const Dc
         const uint64_t p = layer[l][which];
         return reinterpret_cast<uint16_t*>((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32 | (unsigned)__builtin_amdgcn_readfirstlane((int)p));
     };
-    const unsigned epoch = __hip_atomic_load(a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    DcWait wait = {wall_clock64() + a.ticks, a.ticks <= 0};
+    const dc_word state = __hip_atomic_load(reinterpret_cast<dc_word*>(a.epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned epoch = (unsigned)state;
+    DcWait wait = {wall_clock64() + a.ticks, (state >> 32) != 0};
     // ---- the chunks: the shortest length, a multiple of 64, that leaves at most 16 of them ----------------------------------------------------------
     int chunk;
     {
@@ -592,8 +595,19 @@ __global__ __launch_bounds__(DC_WAVES * 64, 1) void decode_chain_kernel(const Dc
         dc_fetch<5, 8>(wg, w_gate_up, gate_rows, wave, lane);
     }
     if (wave == 0 && live && lane < 32) dc_put(dc_at(a.residual_out, dc_again(l16 * DC_H + col)), dc_u32x2{res.x, res.y});
-    if (wait.dead && lane == 0) __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    // every workgroup has left words that this one has read since, so every one has read the epoch
+    if (lane == 0) meet_l[0][wave] = wait.dead ? 1.f : 0.f;
+    __syncthreads();
+    float gave_up = 0.f;
+#pragma unroll
+    for (int w = 0; w < DC_WAVES; ++w) gave_up += meet_l[0][w];
+    if (gave_up != 0.f) {                                               // (24 columns of the last product's rows that are no numbers make none of every number behind it)
+        for (int i = threadIdx.x; i < rows * 24; i += DC_WAVES * 64) a.act[i / 24 * DC_FF + g * 24 + i % 24] = 0x7fc0;
+        if (threadIdx.x == 0) {
+            __hip_atomic_store(a.epoch + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    // every workgroup has left words that this one has read since, so every one has read the epoch (or this one has given up, and no later launch goes by it)
     if (g == 0 && threadIdx.x == 0) __hip_atomic_store(a.epoch, epoch + layers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -612,14 +626,16 @@ extern "C" int nvx_internal_decode_chain_fits(void) {
 }
 
 // layers: per layer o, post-attention norm, gate | up, down, the next layer's input norm and qkv (the last: none), q norm, k norm, k rows, v rows.  ws: `words`
-// of zeros, epoch: one int at 1 or more; both are the next call's as this one leaves them.  status: pinned host memory.
+// of zeros, epoch: two ints, 1 or more and 0; both are the next call's as this one leaves them.  status: pinned host memory.  workgroups: 128; with fewer the waits
+// for what the others would leave run out, `seconds` into the launch.
 extern "C" int nvx_internal_decode_chain(const int64_t* layers, int64_t n_layers, int64_t rows, const void* qkv, const void* residual, void* act, void* residual_out,
                                          const int64_t* positions, const int64_t* kv_start, const int32_t* kv_len, const int64_t* out_slots, const int32_t* kv_indices,
-                                         const float* cos_sin, int64_t max_pos, int64_t n_slots, void* ws, void* epoch, void* status, double seconds, float eps,
-                                         float sm_scale, nvx_stream_t stream) {
+                                         const float* cos_sin, int64_t max_pos, int64_t n_slots, void* ws, void* epoch, void* status, double seconds, int64_t workgroups,
+                                         float eps, float sm_scale, nvx_stream_t stream) {
     NVX_REQUIRE(layers && qkv && residual && act && residual_out && positions && kv_start && kv_len && out_slots && kv_indices && cos_sin && ws && epoch && status, NVX_EINVAL,
                 "nvx_internal_decode_chain: null pointer");
-    NVX_REQUIRE(n_layers > 0 && n_layers <= DC_LAYERS && rows > 0 && rows <= DC_ROWS && max_pos > 0 && n_slots > 0 && seconds > 0, NVX_EUNSUPPORTED,
+    NVX_REQUIRE(n_layers > 0 && n_layers <= DC_LAYERS && rows > 0 && rows <= DC_ROWS && max_pos > 0 && n_slots > 0 && seconds > 0 && seconds <= 60 && workgroups > 0 &&
+                    workgroups <= DC_WGS, NVX_EUNSUPPORTED,
                 "nvx_internal_decode_chain: sizes");
     DcArgs a = {};
     for (int64_t i = 0; i < n_layers; ++i) {
@@ -629,8 +645,8 @@ extern "C" int nvx_internal_decode_chain(const int64_t* layers, int64_t n_layers
             a.layer[i][j] = (uint64_t)p[j];
         }
     }
-    NVX_REQUIRE(nvx_aligned16(qkv) && nvx_aligned16(residual) && nvx_aligned16(act) && nvx_aligned16(residual_out) && nvx_aligned16(cos_sin) && nvx_aligned16(ws), NVX_EINVAL,
-                "nvx_internal_decode_chain: pointers must be 16-byte aligned");
+    NVX_REQUIRE(nvx_aligned16(qkv) && nvx_aligned16(residual) && nvx_aligned16(act) && nvx_aligned16(residual_out) && nvx_aligned16(cos_sin) && nvx_aligned16(ws) &&
+                    (reinterpret_cast<uintptr_t>(epoch) & 7) == 0, NVX_EINVAL, "nvx_internal_decode_chain: pointers must be 16-byte aligned");
     a.layers = (int)n_layers; a.rows = (int)rows;
     a.qkv = (const uint16_t*)qkv; a.residual = (const uint16_t*)residual; a.act = (uint16_t*)act; a.residual_out = (uint16_t*)residual_out;
     a.positions = positions; a.kv_start = kv_start; a.out_slots = out_slots; a.kv_len = kv_len; a.kv_indices = kv_indices;
@@ -639,9 +655,10 @@ extern "C" int nvx_internal_decode_chain(const int64_t* layers, int64_t n_layers
     a.ticks = (long long)(seconds * 1e8);                               // the wall clock counts at 100 MHz
     a.eps = eps; a.scale_log2 = sm_scale * 1.4426950408889634f;
     hipStream_t st = (hipStream_t)stream;
-    if (rows == 1) hipLaunchKernelGGL(decode_chain_kernel<1>, dim3(DC_WGS), dim3(DC_WAVES * 64), 0, st, a);
-    else if (rows == 2) hipLaunchKernelGGL(decode_chain_kernel<2>, dim3(DC_WGS), dim3(DC_WAVES * 64), 0, st, a);
-    else if (rows <= 4) hipLaunchKernelGGL(decode_chain_kernel<4>, dim3(DC_WGS), dim3(DC_WAVES * 64), 0, st, a);
-    else hipLaunchKernelGGL(decode_chain_kernel<8>, dim3(DC_WGS), dim3(DC_WAVES * 64), 0, st, a);
+    const dim3 grid((unsigned)workgroups);
+    if (rows == 1) hipLaunchKernelGGL(decode_chain_kernel<1>, grid, dim3(DC_WAVES * 64), 0, st, a);
+    else if (rows == 2) hipLaunchKernelGGL(decode_chain_kernel<2>, grid, dim3(DC_WAVES * 64), 0, st, a);
+    else if (rows <= 4) hipLaunchKernelGGL(decode_chain_kernel<4>, grid, dim3(DC_WAVES * 64), 0, st, a);
+    else hipLaunchKernelGGL(decode_chain_kernel<8>, grid, dim3(DC_WAVES * 64), 0, st, a);
     return nvx_check_launch("nvx_internal_decode_chain");
 }

@@ -241,6 +241,7 @@ class BlockTable:
         self._step_hosts = [torch.zeros(ints, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
         self._step_nps = [h.numpy() for h in self._step_hosts]
         self._step_turn = 0
+        self.steps_staged = 0
         self.clear_step()
 
     def clear_step(self):
@@ -289,6 +290,7 @@ class BlockTable:
         written as -1-j: the id that step sampled for its row j and that has not reached the host yet."""
         n, m = len(seqs), self.max_bs
         self._step_turn ^= 1
+        self.steps_staged += 1
         buf = self._step_nps[self._step_turn]
         buf[0] = n
         row_of = self.row_of
@@ -303,6 +305,11 @@ class BlockTable:
             buf[4 + 4 * m:4 + 4 * m + n] = [s.state_slot for s in seqs]
             buf[4 + 4 * m + n:] = -1          # no state is read or written for padding rows
         self.step_dev.copy_(self._step_hosts[self._step_turn], non_blocking=True)
+
+    def stage_again(self, which: int):
+        """The upload of a step that was staged before, by its number (steps_staged): the newest or the one in front of it, the others' integers are written over."""
+        assert 0 <= self.steps_staged - which < 2
+        self.step_dev.copy_(self._step_hosts[self._step_turn ^ (self.steps_staged - which)], non_blocking=True)
 
     def fits(self, seqs) -> bool:
         return all(s.seq_id in self.row_of and len(s.kv_indices) <= self.row_capacity for s in seqs)

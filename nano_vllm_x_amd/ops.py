@@ -280,17 +280,20 @@ def _decode_boundary(x, w, mode, squares, eps, residual, norm_weight):
 
 class DecodeChain:
     """What steps of csrc/decode_chain.hip keep from one to the next: the words that their workgroups leave each other, the number of layers computed so far (no
-    word is ever marked with a number twice) and, in host memory, whether a wait ran out.  Steps that share one follow each other on a stream.
+    word is ever marked with a number twice) and, there and in host memory, whether a wait ran out.  Steps that share one follow each other on a stream.
+
+    A step whose waits run out (SECONDS: other work held the device for as long, where a step is a millisecond) gives NaN for every number, and so does every
+    later one of this object: `failed` says so once such a step has ended, and the caller goes on without it.
 
     The workgroups of a step wait for each other, so all of them must find room on the device.  There is room for two steps; where a process keeps more than
     two of these on a device, its steps take turns (in_turn), whatever their streams."""
 
-    ROWS, LAYERS, SECONDS = 8, 32, 10.0
+    ROWS, LAYERS, SECONDS, WORKGROUPS = 8, 32, 1.0, 128
     _alive, _turn, _lock = _weakref.WeakSet(), {}, _threading.Lock()
 
     def __init__(self, device):
         self.words = torch.zeros(_lib.load().nvx_internal_decode_chain_words(), dtype=torch.int64, device=device)
-        self.epoch = torch.ones(1, dtype=torch.int32, device=device)
+        self.epoch = torch.tensor([1, 0], dtype=torch.int32, device=device)
         self.status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
         self._status = self.status.numpy()
         with self._lock:
@@ -332,9 +335,13 @@ class DecodeChain:
     def available() -> bool:
         return bool(_lib.load().nvx_internal_decode_chain_fits())
 
+    @property
+    def failed(self) -> bool:
+        return bool(self._status[0])
+
     def check(self):
-        if self._status[0]:
-            raise RuntimeError("a decode step gave up waiting for its own workgroups: the device was taken by other work, and the step's results are not whole")
+        if self.failed:
+            raise RuntimeError("a decode step gave up waiting for its own workgroups: the device was taken by other work, and the step's results are NaN")
 
 
 def decode_chain(chain, layers, qkv, residual, positions, kv_start, kv_len, out_slots, kv_indices, cos_sin_cache, eps, sm_scale):
@@ -361,7 +368,7 @@ def decode_chain(chain, layers, qkv, residual, positions, kv_start, kv_len, out_
     act, new = torch.empty((m, 3072), dtype=bf, device=qkv.device), torch.empty_like(residual)
     _lib.check(_lib.load().nvx_internal_decode_chain(table, len(layers), m, _ptr(qkv), _ptr(residual), _ptr(act), _ptr(new), _ptr(positions), _ptr(kv_start), _ptr(kv_len),
                                                      _ptr(out_slots), _ptr(kv_indices), _ptr(cos_sin_cache), cos_sin_cache.shape[0], n_slots, _ptr(chain.words),
-                                                     _ptr(chain.epoch), chain.status.data_ptr(), DecodeChain.SECONDS, float(eps), float(sm_scale), _stream()), "decode_chain")
+                                                     _ptr(chain.epoch), chain.status.data_ptr(), DecodeChain.SECONDS, DecodeChain.WORKGROUPS, float(eps), float(sm_scale), _stream()), "decode_chain")
     return act, new
 
 
