@@ -200,9 +200,9 @@ class ModelRunner:
         self.block_table = BlockTable(self.max_bs, n_rows, 2 * self.context_len, self.device)
         self.decode_ws = ops.DecodeWorkspace(self.max_bs, self.num_heads, self.num_kv_heads, self.device)
         cfg = self.hf_config
-        if self.tp_size * self.pp_size == 1 and not self.enforce_eager and ops.DecodeChain.available() \
+        if self.tp_size * self.pp_size == 1 and not self.enforce_eager and os.environ.get("NVX_DECODE_CHAIN", "1") != "0" and ops.DecodeChain.available() \
                 and ops.DecodeChain.fits(1, self.num_layers, cfg.hidden_size, self.num_heads, self.num_kv_heads, cfg.intermediate_size, self.dtype):
-            self.decode_chain = ops.DecodeChain(self.device)
+            self.decode_chain = ops.DecodeChain.on(self.device)
         if not self.enforce_eager:
             self.graph = HIPGraph()
             try:

@@ -23,7 +23,8 @@
 // leaves passes for a result: its workgroup ends with NaN for every row, marks the words as no longer good (launches queued behind this one find that and end the
 // same way), and raises the status word on the host, which computes the steps whose ids nobody has yet again, launch by launch (ModelRunner).
 // What a wait is for is another workgroup of the same launch, so all 128 have to be on the chip at
-// once; the host asks the device for twice that room (nvx_internal_decode_chain_fits) and lets no more than two of a process go side by side (ops.DecodeChain).
+// once; the host asks the device for twice that room (nvx_internal_decode_chain_fits) and lets no more than two go side by side, of all processes that share a network
+// namespace (ops.DecodeChain, core/device_places.py); others that hold the chip longer than `ticks` are what the clock is for.
 #include "nvx_dev.h"
 #include "rope_dev.h"
 

@@ -9,13 +9,12 @@ capturable into a hipGraph.  `nano_vllm_x_amd.torch_ops` registers the stateless
 from __future__ import annotations
 
 import ctypes as _ctypes
-import threading as _threading
-import weakref as _weakref
 from typing import Optional
 
 import torch
 
 from . import _lib
+from .core.device_places import Sharers as _Sharers
 from .layers.plain import operators_are_plain
 
 BF16 = torch.bfloat16
@@ -285,29 +284,33 @@ class DecodeChain:
     A step whose waits run out (SECONDS: other work held the device for as long, where a step is a millisecond) gives NaN for every number, and so does every
     later one of this object: `failed` says so once such a step has ended, and the caller goes on without it.
 
-    The workgroups of a step wait for each other, so all of them must find room on the device.  There is room for two steps; where a process keeps more than
-    two of these on a device, its steps take turns (in_turn), whatever their streams."""
+    The workgroups of a step wait for each other, so all of them must find room on the device.  There is room for two steps, and the processes of a machine share
+    these two places: `on` gives nothing where others hold both.  Where a process has more of these on a device than places, its steps take turns (in_turn),
+    whatever their streams."""
 
     ROWS, LAYERS, SECONDS, WORKGROUPS = 8, 32, 1.0, 128
-    _alive, _turn, _lock = _weakref.WeakSet(), {}, _threading.Lock()
+    _sharers, _turn = _Sharers("nvx-decode-chain", 2), {}
+
+    @classmethod
+    def on(cls, device):
+        return cls(device) if cls._sharers.room(torch.device(device)) else None
 
     def __init__(self, device):
         self.words = torch.zeros(_lib.load().nvx_internal_decode_chain_words(), dtype=torch.int64, device=device)
         self.epoch = torch.tensor([1, 0], dtype=torch.int32, device=device)
         self.status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
         self._status = self.status.numpy()
-        with self._lock:
-            self._alive.add(self)
-            if self._crowded():        # steps under way went without an event that the next ones could wait for
-                torch.cuda.synchronize(self.words.device)
-
-    def _crowded(self) -> bool:
-        return sum(c.words.device == self.words.device for c in self._alive) > 2
+        device = self.words.device
+        with self._sharers.lock:
+            self._sharers.add(self, device)
+            if self._sharers.crowded(device):        # steps under way went without an event that the next ones could wait for
+                torch.cuda.synchronize(device)
 
     def in_turn(self, launch):
-        """launch(), which queues a step of this chain on the current stream; behind every other chain's where more than two are kept on the device."""
-        with self._lock:
-            crowded, device = self._crowded(), self.words.device
+        """launch(), which queues a step of this chain on the current stream; behind every other chain's where there are more than places on the device."""
+        with self._sharers.lock:
+            device = self.words.device
+            crowded = self._sharers.crowded(device)
             if crowded:
                 stream, last = torch.cuda.current_stream(device), self._turn.get(device)
                 if last is not None and last[0] != stream:

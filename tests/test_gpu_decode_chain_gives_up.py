@@ -1,4 +1,6 @@
 """Decode steps in one launch whose workgroups wait in vain: the launch ends by its clock, nothing of it passes for a result, and the runner goes on layer by layer."""
+import os
+
 import pytest
 import torch
 
@@ -132,3 +134,22 @@ def test_a_warm_up_that_gives_up_leaves_the_layers(monkeypatch):
     assert r.decode_chain is None and r.chain_graph is None
     _prefill(r, seqs)
     assert _step(r, seqs).isfinite().all() and "chain_steps" not in r.stats and r.stats["graph_steps"] == 1
+
+
+def test_without_a_place_or_when_asked_the_layers_are_taken(monkeypatch):
+    """(Other processes of the machine hold both places of the GPU.)"""
+    from nano_vllm_x_amd import ops
+    from nano_vllm_x_amd.core.device_places import Sharers, device_name, take_place
+
+    sharers = Sharers(f"nvx-test-{os.getpid()}", 2)
+    monkeypatch.setattr(ops.DecodeChain, "_sharers", sharers)
+    taken = [take_place(f"{sharers.name}-{device_name(0)}", 2) for _ in range(2)]
+    assert all(taken)
+    for _ in range(2):
+        r, seqs = _runner(1, 100), _sequences((50,), 4)
+        r.initialize_kv_cache(64)
+        _prefill(r, seqs)
+        assert r.decode_chain is None and _step(r, seqs).isfinite().all() and "chain_steps" not in r.stats
+        for t in taken:
+            t.close()
+        monkeypatch.setenv("NVX_DECODE_CHAIN", "0")
