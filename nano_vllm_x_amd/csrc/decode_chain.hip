@@ -6,7 +6,7 @@
 // them where the weights stand still.  Qwen3-0.6B, us a step, layers of launches and now: 1 sequence of 40 / 333 / 1900 tokens 787 / 867 / 915 -> 531 / 552 / 590; 2 of 300-900 887
 // -> 613; 4 of 100-1024 902 -> 671; 8 of 20-40 837 -> 687, of 100-1024 954 -> 848.
 //
-//   * A hand-over is a word of 8 bytes, 4 of data and 4 of a tag that no earlier layer or step has used: data and the news of it travel together, the reader
+//   * A hand-over is a word of 8 bytes, 4 of data and 4 of a tag that no earlier layer or step has used since the words were zeros: data and the news of it travel together, the reader
 //     asks for the very words that it needs until all of them carry the tag.  No counter, no fence, no second trip: 1.2 us among all workgroups, 0.85 among those
 //     of an XCD, with nothing else going on; a launch boundary with the first trip of its loads is 4.5.  Both sides are relaxed atomics of device scope, which
 //     pass by the caches that the XCDs do not share.  A second question on its way behind the first made it slower (552 -> 622: the questions wait for each other).
@@ -627,7 +627,7 @@ extern "C" int nvx_internal_decode_chain_fits(void) {
 }
 
 // layers: per layer o, post-attention norm, gate | up, down, the next layer's input norm and qkv (the last: none), q norm, k norm, k rows, v rows.  ws: `words`
-// of zeros, epoch: two ints, 1 or more and 0; both are the next call's as this one leaves them.  status: pinned host memory.  workgroups: 128; with fewer the waits
+// of zeros, epoch: two ints, 1 or more and 0; both are the next call's as this one leaves them, for fewer than 2^32 / n_layers calls.  status: pinned host memory.  workgroups: 128; with fewer the waits
 // for what the others would leave run out, `seconds` into the launch.
 extern "C" int nvx_internal_decode_chain(const int64_t* layers, int64_t n_layers, int64_t rows, const void* qkv, const void* residual, void* act, void* residual_out,
                                          const int64_t* positions, const int64_t* kv_start, const int32_t* kv_len, const int64_t* out_slots, const int32_t* kv_indices,

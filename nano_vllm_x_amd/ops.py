@@ -278,8 +278,8 @@ def _decode_boundary(x, w, mode, squares, eps, residual, norm_weight):
 
 
 class DecodeChain:
-    """What steps of csrc/decode_chain.hip keep from one to the next: the words that their workgroups leave each other, the number of layers computed so far (no
-    word is ever marked with a number twice) and, there and in host memory, whether a wait ran out.  Steps that share one follow each other on a stream.
+    """What steps of csrc/decode_chain.hip keep from one to the next: the words that their workgroups leave each other, the number of layers computed so far (a word's
+    mark; of 32 bits: after STEPS steps, half of them at most, the words are cleared and it starts anew, so none is met twice) and, there and in host memory, whether a wait ran out.  Steps that share one follow each other on a stream.
 
     A step whose waits run out (SECONDS: other work held the device for as long, where a step is a millisecond) gives NaN for every number, and so does every
     later one of this object: `failed` says so once such a step has ended, and the caller goes on without it.
@@ -288,7 +288,7 @@ class DecodeChain:
     these two places: `on` gives nothing where others hold both.  Where a process has more of these on a device than places, its steps take turns (in_turn),
     whatever their streams."""
 
-    ROWS, LAYERS, SECONDS, WORKGROUPS = 8, 32, 1.0, 128
+    ROWS, LAYERS, SECONDS, WORKGROUPS, STEPS = 8, 32, 1.0, 128, 1 << 26
     _sharers, _turn = _Sharers("nvx-decode-chain", 2), {}
 
     @classmethod
@@ -299,7 +299,7 @@ class DecodeChain:
         self.words = torch.zeros(_lib.load().nvx_internal_decode_chain_words(), dtype=torch.int64, device=device)
         self.epoch = torch.tensor([1, 0], dtype=torch.int32, device=device)
         self.status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-        self._status = self.status.numpy()
+        self._status, self.steps = self.status.numpy(), 0
         device = self.words.device
         with self._sharers.lock:
             self._sharers.add(self, device)
@@ -315,6 +315,11 @@ class DecodeChain:
                 stream, last = torch.cuda.current_stream(device), self._turn.get(device)
                 if last is not None and last[0] != stream:
                     stream.wait_event(last[1])
+            if self.steps == self.STEPS:
+                self.words.zero_()
+                self.epoch[:1].fill_(1)
+                self.steps = 0
+            self.steps += 1
             out = launch()
             if crowded:
                 event = torch.cuda.Event()

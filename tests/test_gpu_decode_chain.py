@@ -124,3 +124,26 @@ def test_three_on_a_device_take_turns():
         r.decode_chain.check()
         assert r.stats["chain_steps"] == 4
     assert all(torch.equal(got[0], g) for g in got)
+
+
+def test_the_words_are_cleared_before_their_marks_come_round():
+    """Marks of 32 bits: the count starts anew long before, with words that carry none."""
+    from nano_vllm_x_amd import ops
+
+    assert ops.DecodeChain.STEPS * ops.DecodeChain.LAYERS <= 1 << 31
+    r = _runner(4, 300)
+    lengths = (100, 7, 250, 64)
+    r.initialize_kv_cache(sum(lengths) + len(lengths))
+    seqs, chain = _sequences(lengths, 1), r.decode_chain
+    _prefill(r, seqs)
+    want = {n: _step(r, seqs[:n]) for n in (1, 4)}
+    torch.cuda.synchronize()
+    # as after so many steps of one sequence: the other rows' words still carry what they were left with, here the marks of the steps to come
+    chain.steps = chain.STEPS - 1
+    chain.words.copy_((1 + torch.arange(chain.words.numel(), device="cuda") % (2 * LAYERS)) << 32)
+    chain.epoch[:1].fill_(1 << 20)
+    for n, epoch in ((1, (1 << 20) + LAYERS), (4, 1 + LAYERS), (1, 1 + 2 * LAYERS)):
+        assert torch.equal(_step(r, seqs[:n]), want[n])
+        torch.cuda.synchronize()
+        assert chain.epoch.tolist() == [epoch, 0]
+    assert chain.steps == 2
