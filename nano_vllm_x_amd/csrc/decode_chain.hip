@@ -163,7 +163,7 @@ __device__ __forceinline__ void dc_take(unsigned (*xs)[DC_XS], dc_word* words, i
             if (wave < rows && lane == 0) squares_of[wave] = ss;
         }
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);                                 // vmcnt(0): this wave's rows of the weights are there as well
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");                  // this wave's rows of the weights are there as well, in LDS behind the compiler's back
 }
 // a tile's sums of a wave, of MR rows of x: lane (quad, row)
 template <int MR>
