@@ -514,7 +514,8 @@ class ModelRunner:
         padded = self.graph.match_bs(bs)
         self.block_table.stage_decode_step(batch.seqs, ids_on_device)
         chain = self.chain_graph
-        if chain is not None and bs <= chain.max_bs and self.decode_chain.faster(bs, sum(len(s.kv_indices) for s in batch.seqs)):
+        lengths = [len(s.kv_indices) for s in batch.seqs] if chain is not None and bs <= chain.max_bs else None
+        if lengths and self.decode_chain.faster(bs, sum(lengths)) and self.decode_chain.pays(lengths, chain.match_bs(bs)):
             padded = chain.match_bs(bs)
             self.decode_chain.in_turn(lambda: chain.replay(padded))
             self.stats["chain_steps"] = self.stats.get("chain_steps", 0) + 1

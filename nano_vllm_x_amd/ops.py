@@ -340,6 +340,20 @@ class DecodeChain:
         return rows <= DecodeChain.ROWS and tokens <= (60000 if rows <= 2 else 32000 if rows <= 4 else 10000)
 
     @staticmethod
+    def pays(lengths, rows: int) -> bool:
+        """The same for sequences of these lengths in a graph of so many rows (the rest: padding, a chunk each), where 16 chunks for all of them come out too long: of five
+        to eight rows, and more than 6000 tokens.  The longest chunk sets the pace there: 662 us and 28.7 a tile of 64 keys of it, where the layers launch by launch take 878
+        and 12.4 for 1000 tokens and 28.7 for 1000 of the longest sequence; fitted to 56 draws (within 2 % and 3 %, the choice wrong by 1 % at most).  us, launches and chain:
+        5 sequences of 2000 1046 and 1114, 3 of 3000 and 5 of 100 1088 and 1111, 6 of 1600 1037 and 1033, one of 7000 and 7 of 10 1159 and 1029."""
+        total = sum(lengths)
+        if rows <= 4 or total <= 6000:
+            return True
+        least, most, padding = -(-total // 1024), -(-total // 512), rows - len(lengths)
+        step = (most - least + 62) // 63                    # (as the kernel finds it)
+        tiles = next(t for t in range(least, most + 64 * step, step or 1) if sum(max(1, -(-n // (64 * t))) for n in lengths) + padding <= 16)
+        return 662 + 28.7 * tiles <= 878 + 0.0124 * total + 0.0287 * max(lengths)
+
+    @staticmethod
     def available() -> bool:
         return bool(_lib.load().nvx_internal_decode_chain_fits())
 
