@@ -789,10 +789,13 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a, StepEnds e
             if (cont && r < dim) s[u] = *reinterpret_cast<const nvx_f32x4*>(Sp + (int64_t)r * vdim + e0);
         }
     };
-    if (grp < n_groups) {
-        load_rows(grp);
+    const auto load_val = [&] {
 #pragma unroll
         for (int i = 0; i < 4; ++i) val[i] = scan_act(ld_f(xr, a.v_off + hd * vdim + e0 + i), a.act);
+    };
+    if (ENDS && grp < n_groups) {
+        load_rows(grp);
+        load_val();
     }
     nvx_f32x4 w2[STEP_RANK / 4];
     float z[4], wn[4], w2_bias = 0.f;
@@ -862,8 +865,9 @@ __global__ __launch_bounds__(256) void memory_step_kernel(ScanArgs a, StepEnds e
     }
     __syncthreads();
     if (grp < n_groups) {
+        if (!ENDS) load_val();
         for (int r0 = grp; r0 < dim; r0 += n_groups * U) {
-            if (r0 != grp) load_rows(r0);
+            if (!ENDS || r0 != grp) load_rows(r0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int r = r0 + u * n_groups;
