@@ -2065,14 +2065,23 @@ def memory_step_fits(layout: StepLayout, h, mem, w1, w2=None) -> bool:
         return False
     if h.data_ptr() % item or any(t.data_ptr() % 16 for t in (mem, w1) + (() if w2 is None else (w2,))):
         return False
-    return w2 is None or (dim <= 256 and w1.shape[0] % 4 == 0 and 0 < w1.shape[0] <= 32 and w1.numel() <= 1 << 16 and gla_step_faster(layout.n_tok, heads, dim, vdim, w1.shape[0]))
+    if w2 is None:
+        return mlstm_step_faster(layout.n_tok, heads, dim, vdim)
+    return dim <= 256 and w1.shape[0] % 4 == 0 and 0 < w1.shape[0] <= 32 and w1.numel() <= 1 << 16 and gla_step_faster(layout.n_tok, heads, dim, vdim, w1.shape[0])
+
+
+def mlstm_step_faster(n_seq: int, heads: int, dim: int, vdim: int) -> bool:
+    """Whether mlstm's step with its gates, norm and output gate in the launch beats the three launches: up to eight workgroups a compute unit, and with memories that take
+    long beside the rest.  us, one launch and the three, 16 heads of 64 x 128, 2048 inputs: 64 sequences 15.9 and 22.1, 128 31.0 and 34.4, 192 45.0 and 44.4, 256 59.0 and
+    54.3; 16 of 64 x 64, 256 sequences 42.4 and 36.1; of 128 x 128, 256 sequences 95.6 and 98.9, of 128 x 256 216 and 228."""
+    return n_seq * heads <= 2048 or dim * vdim >= 16384
 
 
 def gla_step_faster(n_seq: int, heads: int, dim: int, vdim: int, rank: int) -> bool:
-    """Whether gla's step with its small projections in the launch beats the separate launches: up to three workgroups a compute unit, which run at once, always; up to six
+    """The same of gla's step with its decays' projections, against four launches: up to three workgroups a compute unit, which run at once, always; up to six
     while what each of them projects again is little beside its memory.  us, one launch and the four, heads of 64 x 128, rank 16 of 2048 inputs, 16 heads: 48 sequences
-    15.2 and 20.3, 64 26.5 and 25.2, 128 46 and 39, 256 87 and 63; rank 4 96 sequences 28.7 and 33.7, 128 39.1 and 38.5; 8 heads of 128 x 256, 128 sequences 53 and 56, 256 102 and 101.
-    (mlstm, whose heads project two numbers each, is ahead everywhere: 256 sequences of 16 heads 59 and 61.)"""
+    15.2 and 20.5, 64 26.4 and 25.2, 128 45.5 and 37.2, 256 86 and 57; rank 4 96 sequences 28.3 and 31.8, 128 39.8 and 36.9; 8 heads of 128 x 256, 128 sequences 53 and
+    55, 256 102 and 103."""
     return n_seq * heads <= 768 or (n_seq * heads <= 1536 and rank * 2048 <= dim * vdim)
 
 
