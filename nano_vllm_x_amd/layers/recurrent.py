@@ -62,7 +62,7 @@ class MLSTM(nn.Module):
         hd, he, n = self.heads * self.dim, self.heads * self.vdim, self.state_name if at is None else at
         x = self.qkvg_proj(h) if made is None else made
         S, norm, peak = (md.cache.state((n, which)) for which in ("S", "n", "m"))
-        if ops.memory_step_fits(md.layout, h, S, self.gate_w):
+        if ops.memory_step_fits(md.layout, h, S, self.gate_w, x=x):
             return self.o_proj(ops.mlstm_step(x, (0, hd, 2 * hd), 2 * hd + he, h, self.gate_w, self.gate_b, self.gate_cap, self.norm, self.eps, S, norm, peak,
                                               md.layout, self.heads, self.dim, self.vdim))
         gates = ops.skinny_proj(h, self.gate_w)
@@ -245,7 +245,7 @@ class GatedLinearAttention(nn.Module):
         """`made`: as at MLSTM."""
         hd, he, n = self.heads * self.dim, self.heads * self.vdim, self.state_name if at is None else at
         x, S = self.qkvg_proj(h) if made is None else made, md.cache.state((n, "S"))
-        if ops.memory_step_fits(md.layout, h, S, self.a1, self.a2):
+        if ops.memory_step_fits(md.layout, h, S, self.a1, self.a2, x=x):
             return self.o_proj(ops.gla_step(x, (0, hd, 2 * hd), 2 * hd + he, h, self.a1, self.a2, self.a2_b, 1.0 / self.tau, self.norm, self.eps, S, md.layout,
                                             self.heads, self.dim, self.vdim, q_mul=self.dim ** -0.5))
         alpha = ops.skinny_proj(ops.skinny_proj(h, self.a1), self.a2, bias=self.a2_b, out_act="sigmoid_pow", power=1.0 / self.tau)

@@ -2054,10 +2054,11 @@ def gla_scan(x, offsets, alpha, mem, layout: StepLayout, heads: int, dim: int, v
     return out
 
 
-def memory_step_fits(layout: StepLayout, h, mem, w1, w2=None) -> bool:
+def memory_step_fits(layout: StepLayout, h, mem, w1, w2=None, x=None) -> bool:
     """Whether mlstm_step (w1: its gates' weights) or gla_step (w1, w2: its decays') serves this step: one token per sequence, heads and rows that
-    their kernel is built for.  Every head of every sequence computes gla's `rank` numbers again, so they must be few."""
-    if layout.qo_indptr is not None:
+    their kernel is built for, the projections' rows `x` in h's format, inputs as many as skinny_proj takes.  Every head of every sequence computes gla's `rank` numbers
+    again, so they must be few."""
+    if layout.qo_indptr is not None or (x is not None and x.dtype != h.dtype) or h.shape[1] > 12288:
         return False
     heads, dim, vdim = mem.shape[1:]
     item = 4 * h.element_size()

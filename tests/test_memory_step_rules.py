@@ -1,7 +1,11 @@
 """Sizes at which the steps of one token of gla and mlstm keep their projections in launches of their own (no GPU: the rules)."""
+import types
+
 import pytest
+import torch
 
 from nano_vllm_x_amd import ops
+from nano_vllm_x_amd.layers import recurrent
 
 
 @pytest.mark.parametrize("n_seq,heads,dim,vdim,rank,one", [      # us of the one launch and of the four
@@ -32,3 +36,28 @@ def test_where_the_four_launches_are_the_faster(n_seq, heads, dim, vdim, rank, o
     (256, 16, 256, 256, True)])           # 419 and 435
 def test_where_the_three_launches_of_mlstm_are_the_faster(n_seq, heads, dim, vdim, one):
     assert ops.mlstm_step_faster(n_seq, heads, dim, vdim) is one
+
+
+def test_rows_of_another_format_and_inputs_that_no_projection_takes_keep_the_separate_launches():
+    """A replaced projection may give its rows in a format of its own, which the separate launches read; more than 12288 inputs they refuse."""
+    lay = types.SimpleNamespace(qo_indptr=None, n_tok=3)
+    mem, w = torch.zeros(3, 2, 64, 64), lambda r, k=64: torch.zeros(r, k)
+    h, x = torch.zeros(3, 64).bfloat16(), torch.zeros(3, 512)
+    for w1, w2 in ((w(4), None), (w(16), w(128, 16))):
+        assert ops.memory_step_fits(lay, h, mem, w1, w2, x=x.bfloat16()) and ops.memory_step_fits(lay, x[:, :64], mem, w1, w2, x=x)
+        assert not ops.memory_step_fits(lay, h, mem, w1, w2, x=x) and not ops.memory_step_fits(lay, h, mem, w1, w2, x=x.half())
+    assert ops.memory_step_fits(lay, torch.zeros(3, 12288), mem, w(4, 12288), x=x) and not ops.memory_step_fits(lay, torch.zeros(3, 12292), mem, w(4, 12292), x=x)
+
+
+def test_the_modules_ask_with_their_rows(monkeypatch):
+    asked = []
+    monkeypatch.setattr(ops, "memory_step_fits", lambda layout, h, *a, x=None: asked.append((h.dtype, x.dtype)) or False)
+    for name in ("skinny_proj", "mlstm_scan", "gla_scan"):
+        monkeypatch.setattr(ops, name, lambda *a, **k: None)
+    monkeypatch.setattr(ops, "head_norm_gate", lambda *a, gate, **k: gate)
+    md = types.SimpleNamespace(layout=None, cache=types.SimpleNamespace(state=lambda key: None))
+    for m in (recurrent.MLSTM(64, 1, 64, 64, 15.0, 1e-5, "s"), recurrent.GatedLinearAttention(64, 1, 64, 64, 16.0, 16, 1e-5, "s")):
+        m.qkvg_proj.forward = lambda h: torch.zeros(len(h), 256)
+        m.o_proj.forward = lambda y: y
+        assert m(torch.zeros(3, 64).bfloat16(), md).dtype == torch.float32
+    assert asked == [(torch.bfloat16, torch.float32)] * 2
