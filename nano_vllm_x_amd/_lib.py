@@ -210,6 +210,7 @@ INTERNAL["nvx_internal_decode_boundary"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64
 INTERNAL["nvx_internal_linear_decode_scaled"] = (_c_i32, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_vp, _c_f32, _c_vp])
 INTERNAL["nvx_internal_memory_step"] = (_c_i32, [ctypes.POINTER(MemoryStep), _c_vp])
 INTERNAL["nvx_internal_decode_chain_words"] = (_c_i64, [])
+INTERNAL["nvx_internal_prefill_planless"] = (_c_i64, [])
 INTERNAL["nvx_internal_decode_chain_fits"] = (_c_i32, [])
 INTERNAL["nvx_internal_decode_chain"] = (_c_i32, [_c_vp, _c_i64, _c_i64] + [_c_vp] * 10 + [_c_i64, _c_i64, _c_vp, _c_vp, _c_vp, ctypes.c_double, _c_i64, _c_f32, _c_f32, _c_vp])
 INTERNAL["nvx_internal_few_rows"] = (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_vp, _c_i32, _c_i32, _c_i64, _c_i64, _c_i64, _c_i32, _c_f32, _c_f32, _c_f32, _c_vp])

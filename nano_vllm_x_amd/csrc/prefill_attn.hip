@@ -24,6 +24,7 @@ namespace NVX_NS {
 
 #define PF_KVBLK 64
 #define PF_RING 3               // tiles of a workgroup with waves that only fetch
+#define PF_SORTED 64             // sequences (a lane each) whose blocks are found without a plan
 #define PF_IDS (2 * PF_RING)    // tiles whose slot ids such a wave keeps
 #define PF_LOG2E 1.4426950408889634f
 
@@ -34,6 +35,7 @@ typedef __attribute__((address_space(3))) pf_s16x4 pf_lds_s16x4;
 //   table t at ws + t*(batch+2): [0] = total blocks, [1 + b] = first block of sequence b, [1 + batch] = total
 #ifndef NVX_F16   // independent of the 16-bit format: defined by the bfloat16 build only
 extern "C" int64_t nvx_prefill_plan_ws_ints(int64_t batch) { return 3 * (batch + 2); }
+extern "C" int64_t nvx_internal_prefill_planless(void) { return PF_SORTED; }      // up to so many sequences nvx_paged_prefill reads no plan
 
 __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __restrict__ qo_indptr, int batch,
                                                             int32_t* __restrict__ ws) {
@@ -164,7 +166,6 @@ extern "C" int nvx_debug_pf_stamps(unsigned long long* host) { return (int)hipMe
 // sequences, whose neighbours share their keys in an XCD's L2.  No plan is read (two trips to memory less ahead of the first keys, and no launch of the plan).  Qwen3-0.6B, us a step by
 // the plan, in order of length throughout, and by this rule: 8 prompts of 200-900 tokens 7086 / 6938 / 6918, 32 of 100-1024 21620 / 21395 / 21427, 64 of 20-400 13597 / 13595 / 13488, 20 of
 // 100-400 behind 30-1000 cached ones 7739 / 7508 / 7498; with the waves for the copies (below) 9 of 100-400 behind 900-3000 6326 / - / 5330.
-#define PF_SORTED 64
 #define PF_SORT_BLOCKS 128
 #define PF_SORT_KEYS 704
 struct PfBlock { int qb, q0, lq, kv0, lkv; };       // qb < 0: there is none

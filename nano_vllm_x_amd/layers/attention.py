@@ -85,7 +85,7 @@ class PagedPrefillWrapper:
         b = qo_indptr.numel() - 1
         if self._plan_ws is None or self._plan_ws.numel() < 3 * (b + 2):
             self._plan_ws = ops.prefill_plan_ws(max(b, 256), qo_indptr.device)
-        if b > ops.PREFILL_PLANLESS:
+        if b > ops.prefill_planless():
             torch.ops.nvx.prefill_plan(qo_indptr, self._plan_ws)
         self._planned = (qo_indptr, paged_kv_indptr, paged_kv_indices, num_qo_heads, num_kv_heads)
 

@@ -549,7 +549,9 @@ def prefill_plan_ws(batch: int, device):
     return torch.zeros(lib.nvx_prefill_plan_ws_ints(batch), dtype=torch.int32, device=device)
 
 
-PREFILL_PLANLESS = 64      # sequences whose blocks the attention of prompts finds without a plan (PF_SORTED of csrc/prefill_attn.hip); the plan's launch is 8 us
+def prefill_planless() -> int:
+    """Sequences whose blocks the attention of prompts finds without a plan (as the kernel has it); the plan's launch is 8 us."""
+    return _lib.load().nvx_internal_prefill_planless()
 
 
 def prefill_plan(qo_indptr, plan_ws):

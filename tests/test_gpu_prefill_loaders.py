@@ -58,3 +58,25 @@ def test_blocks_in_order_of_length(n):
         if a:
             assert torch.equal(_run(q[at_q:at_q + a], k, v, [(a, b)], slots[at_k:at_k + b].clone(), 4, 2), got[at_q:at_q + a])
         at_q, at_k = at_q + a, at_k + b
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 300])
+def test_no_plan_is_read_where_none_is_made(n):
+    """Through the wrapper, which makes a plan only for more sequences than the kernel says: with its workspace empty every row is there, and right."""
+    from nano_vllm_x_amd import ops
+    from nano_vllm_x_amd.layers.attention import PagedPrefillWrapper
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    parts = [(i % 70, i % 70 + i % 11) for i in range(1, n + 1)]
+    ends = torch.tensor([(0, 0)] + parts).cumsum(0).to(torch.int32).cuda()
+    qo, kv = ends[:, 0].contiguous(), ends[:, 1].contiguous()
+    nq, nk = int(qo[-1]), int(kv[-1])
+    q = torch.randn(nq, 4 * 128, generator=gen, device="cuda").bfloat16()
+    k, v = (torch.randn(nk, 2, 128, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    slots = torch.randperm(nk, generator=gen, device="cuda").to(torch.int32)
+    w = PagedPrefillWrapper()
+    w._plan_ws = ops.prefill_plan_ws(n, "cuda")
+    w.plan(qo, kv, slots, None, 4, 2, 128)
+    assert bool((w._plan_ws != 0).any()) == (n > ops.prefill_planless())
+    out = torch.full((nq, 4 * 128), torch.nan, device="cuda", dtype=torch.bfloat16)
+    assert torch.equal(w.run(q, (k, v), out=out).reshape(nq, -1), _run(q, k, v, parts, slots, 4, 2))
