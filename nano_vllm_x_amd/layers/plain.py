@@ -20,7 +20,7 @@ def untouched(m, cls) -> bool:
     """Whether calling module `m` runs the forward that its class `cls` has, and nothing else: another class (a replaced, wrapped, quantised or
     parametrised module), a forward of the instance's own, and hooks all want the call.  (Looked up where nn.Module keeps them: a step asks this of
     every module.)  as_written says the same of the class."""
-    if m.__class__ is not cls:
+    if type(m) is not cls:      # (m.__class__ is what a proxy says of the module inside)
         return False
     d = m.__dict__
     return not d["_forward_hooks"] and not d["_forward_pre_hooks"] and "forward" not in d and "_compiled_call_impl" not in d
