@@ -236,8 +236,7 @@ __global__ __launch_bounds__(2 * FR_WAVES * 64) void few_rows_lead_kernel(const 
 }
 
 // What a workgroup waits for is its rows of w and of x, at some 34 bytes a clock for a compute unit, and 16 rows of x are as much as 16 of w.  While twice the
-// workgroups still find a compute unit each, they take eight rows of w (the same sums in the same order), from more than 1024 columns on or gated (a wave's one or two turns
-// of shorter rows are one trip either way: 2048 x 1024, one row 2.9 / 3.0, 16 rows 3.0 / 3.1, 256 x 512 2.1 / 2.2).  us, tiles of 16 / of eight, 16 rows: 512 x 4096 5.3 / 4.7, 1024 x 2048 4.0 / 3.7,
+// workgroups still find a compute unit each, they take eight rows of w (the same sums in the same order).  us, tiles of 16 / of eight, 16 rows: 512 x 4096 5.3 / 4.7, 1024 x 2048 4.0 / 3.7,
 // 2048 x 2048 5.15 / 4.7, 1024 x 3072 6.0 / 5.3, 2048 x 6144 11.4 / 10.1, gated 2048 x 1024 4.0 / 3.8, 4096 x 2048 7.0 / 6.3; one row 2048 x 2048 4.5 / 4.3; 32 rows 6.2 / 5.6; past that line 16 rows 3072 x 2048 5.6 / 6.4,
 // gated 6144 x 1024 5.3 / 5.9.  (More pieces of K on their way instead, all loads of a workgroup at once: 2 to 4 % slower.)
 // Beyond, 16 rows of w a workgroup leave the most workgroups for the chip; where there are more than run at once, more of them share the reads of x.  us at
@@ -256,7 +255,7 @@ static void launch_few_rows(const void* x, int64_t x_stride, const void* w, cons
     else if (glu == 2) NVX_FEW(2, 2, 2, 16);
     else if (n >= 12288 && n % 64 == 0) NVX_FEW(4, 1, 0, 16);
     else if (MT == 2 && n > 4096 && n % 32 == 0) NVX_FEW(2, 2, 0, 16);
-    else if (n <= 8 * CUS && k > 1024) NVX_FEW(1, 2, 0, 8);
+    else if (n <= 8 * CUS) NVX_FEW(1, 2, 0, 8);
     else NVX_FEW(1, 2, 0, 16);
 #undef NVX_FEW
 }
