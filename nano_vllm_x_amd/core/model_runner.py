@@ -282,7 +282,8 @@ class ModelRunner:
         decode = batch.forward_mode == ForwardMode.DECODE
         tpd.check_peer_status()      # results leave through here too (tests, tools): never on top of a failed exchange
         self._by_chain = False
-        self._settle_chain()
+        if self.decode_chain is not None and self.decode_chain.failed:
+            self._settle_chain()
         if self._chain_lost:
             self._chain_lost = False
             raise RuntimeError("a decode step gave up waiting for its own workgroups (the device was taken by other work) when its results had left already: they are "
@@ -377,8 +378,6 @@ class ModelRunner:
     def _settle_chain(self):
         """Where a step of ops.DecodeChain has given up: no further step goes that way, and those whose ids were not collected are computed again layer by layer,
         with the draws they had.  Results that left through compute_hidden or compute_logits cannot be (_chain_lost)."""
-        if self.decode_chain is None or not self.decode_chain.failed:
-            return
         if any(self.block_table.steps_staged - staged > 1 for _, _, staged, _, _ in self._chain_steps):
             raise RuntimeError("a decode step gave up waiting for its own workgroups with its ids not collected two steps later: it cannot be computed again")
         torch.cuda.synchronize(self.device)
@@ -448,9 +447,10 @@ class ModelRunner:
         n = batch.num_seqs
         if isinstance(ids, int):     # index of the pinned buffer the ids land in
             self._sample_events[ids].synchronize()
-            if self.decode_chain is not None:
+            if self.decode_chain is not None and self.decode_chain.failed:
                 self._settle_chain()      # (it may have computed this step again)
                 self._sample_events[ids].synchronize()
+            if self._chain_steps:
                 at = next((i for i, step in enumerate(self._chain_steps) if step[0] == ids), None)
                 if at is not None:
                     if self._chain_left < self._chain_steps[at][2]:
