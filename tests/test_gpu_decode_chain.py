@@ -74,7 +74,8 @@ def test_one_launch_against_many(lengths):
 
 
 def test_replays_among_other_work():
-    """Batches of several sizes in turn, each several times with eager work between: every replay gives what the first gave, and a padded batch what its own size gives."""
+    """Batches of several sizes in turn, each several times with eager work between: every replay gives what the first gave, and that, padded rows beside it or not (three
+    go as four, five as eight), is what the layers launch by launch give."""
     r = _runner(8, 300)
     lengths = (100, 7, 250, 64, 31, 128, 1, 199)
     r.initialize_kv_cache(sum(lengths) + len(lengths))
@@ -89,6 +90,11 @@ def test_replays_among_other_work():
             assert torch.equal(first[n], got), (turn, n)
     assert r.stats["chain_steps"] == 18 and r.stats["graph_steps"] == 18
     r.decode_chain.check()
+    r.chain_graph = None
+    bound = 2.0 ** -8 / 3 ** 0.5 * (2 * (ROUNDINGS * LAYERS + 1)) ** 0.5      # (as above)
+    for n, got in first.items():
+        want = _step(r, seqs[:n])
+        assert got.shape == want.shape and float((got - want).norm() / want.norm()) < bound, n
 
 
 def test_more_tokens_than_pay_take_the_launches():
