@@ -19,6 +19,8 @@
 //   * Attention: workgroup g has head g % 8, so that a head's projections, chunks and read-outs stay within what is one XCD here, and chunk g / 8 of the step's rows;
 //     chunks are as short as 16 for all rows allow, so long rows get more of them.  The first 64 keys and values of a chunk are on their way before the queries exist.
 //
+// Built for these sizes in bfloat16 alone (ops.DecodeChain.fits): which rows of which weight a workgroup keeps, in LDS or in registers, is laid out for them and fills both.
+//
 // Every wait ends: a word that does not come within `ticks` of the wall clock makes the wave stop waiting for the rest of the launch.  Nothing that such a launch
 // leaves passes for a result: its workgroup ends with NaN for every row, marks the words as no longer good (launches queued behind this one find that and end the
 // same way), and raises the status word on the host, which computes the steps whose ids nobody has yet again, launch by launch (ModelRunner).

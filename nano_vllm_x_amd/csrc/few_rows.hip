@@ -137,7 +137,8 @@ __global__ __launch_bounds__(FR_WAVES * 64) void few_rows_kernel(const A* __rest
 // The same with what stands in front of it: x_out = x (+ y) (+ add) (+ x_bias), h = x_out / rms(x_out) * w_norm in the format, out = h W^T.  Every
 // workgroup forms all rows of h from the float32 stream: eight waves take two rows each and leave them in LDS, while eight others have the workgroup's rows of W on
 // their way (loads of one wave come back in order: rows behind weights would wait for them).  Workgroup r writes row r of x_out and h (x_out is not x: others
-// still read that).  k = 1024, rows <= 16: wider rows would take twice as long to come, and longer than the boundary's own launch.  Bound: the stream's rows come to every compute unit at some 34 bytes a clock (16 rows of 1024 with a result to
+// still read that).  k = 1024, rows <= 16: rows of 2048 take 2.4 us to come, and the
+// form for them spilled; a form for narrower ones was not built.  Bound: the stream's rows come to every compute unit at some 34 bytes a clock (16 rows of 1024 with a result to
 // add: 96 KB, 1.2 us), beside the weights' latency.  us, against the boundary's
 // launch and the product's: 16 rows, 3072 x 1024 7.1 against 3.5 + 4.6; gated 6144 x 1024 6.8 against 3.5 + 4.8.  (With the rows loaded straight in operand order, 64
 // requests of 16 bytes an instruction, and ahead of them the weights by the same waves, it came out behind the two launches: a step of 292 us took 306, now 284.)
@@ -237,7 +238,8 @@ __global__ __launch_bounds__(2 * FR_WAVES * 64) void few_rows_lead_kernel(const 
 
 // What a workgroup waits for is its rows of w and of x, at some 34 bytes a clock for a compute unit, and 16 rows of x are as much as 16 of w.  While twice the
 // workgroups still find a compute unit each, they take eight rows of w (the same sums in the same order).  us, tiles of 16 / of eight, 16 rows: 512 x 4096 5.3 / 4.7, 1024 x 2048 4.0 / 3.7,
-// 2048 x 2048 5.15 / 4.7, 1024 x 3072 6.0 / 5.3, 2048 x 6144 11.4 / 10.1, gated 2048 x 1024 4.0 / 3.8, 4096 x 2048 7.0 / 6.3; one row 2048 x 2048 4.5 / 4.3; 32 rows 6.2 / 5.6; past that line 16 rows 3072 x 2048 5.6 / 6.4,
+// 2048 x 2048 5.15 / 4.7, 1024 x 3072 6.0 / 5.3, 2048 x 6144 11.4 / 10.1, gated 2048 x 1024 4.0 / 3.8, 4096 x 2048 7.0 / 6.3; one row 2048 x 2048 4.5 / 4.3; of 512 and 1024 columns nothing either way by themselves (2048 x 1024, one row 2.9 / 3.0), and a step of
+// Kabidra of 1024 363 / 360; 32 rows 6.2 / 5.6; past that line 16 rows 3072 x 2048 5.6 / 6.4,
 // gated 6144 x 1024 5.3 / 5.9.  (More pieces of K on their way instead, all loads of a workgroup at once: 2 to 4 % slower.)
 // Beyond, 16 rows of w a workgroup leave the most workgroups for the chip; where there are more than run at once, more of them share the reads of x.  us at
 // 16 rows, 16 against 64 rows of w: 9216 x 2048 11.7 / 11.9, 12288 x 2048 14.0 / 13.4, 32000 x 1024 18.2 / 14.6; at 32 rows, 16 against

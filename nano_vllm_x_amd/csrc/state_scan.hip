@@ -711,6 +711,8 @@ __global__ __launch_bounds__(256) void decay_step_kernel(const A* __restrict__ x
 // head) and the norm and gate of the read-out (as at decay_step_kernel) are part of the launch.  Everything that waits for nothing is asked
 // for first: the memory's first rows, the gate, the weights.  16 sequences, 8 heads of 64 x 128, rows of 1024, us of all launches (and the gaps between them
 // fall away): gla with 16 numbers 6.8 + 5.3 + 4.8 + 3.6 -> 11.9, mlstm 7.4 + 5.3 + 3.6 -> 9.6; bound: the chain projections, decays, memory, norm in one workgroup.
+// With very many sequences the launches are the faster (ops.gla_step_faster, mlstm_step_faster).  Without ENDS the rows are asked for behind queries and keys: ahead of them
+// cost up to a sixth at 4096 workgroups.
 constexpr int STEP_RANK = 32;              // most numbers that gla's decays pass through: a key channel's weights wait in a thread's registers
 struct StepEnds {
     const void* h;                         // rows the projections read
