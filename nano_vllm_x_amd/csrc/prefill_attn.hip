@@ -164,8 +164,9 @@ extern "C" int nvx_debug_pf_stamps(unsigned long long* host) { return (int)hipMe
 // QPOS) from its cached tokens on.  In the order of the sequences a launch of two workgroups a CU ended on whatever came last: 32 prompts of 100 to 1024 tokens, 2088
 // workgroups of 15 us in the mean, 512 at a time, took 82 us.  Many short blocks (more than PF_SORT_BLOCKS, none that sees PF_SORT_KEYS) stay in the order of the
 // sequences, whose neighbours share their keys in an XCD's L2.  No plan is read (two trips to memory less ahead of the first keys, and no launch of the plan).  Qwen3-0.6B, us a step by
-// the plan, in order of length throughout, and by this rule: 8 prompts of 200-900 tokens 7086 / 6938 / 6918, 32 of 100-1024 21620 / 21395 / 21427, 64 of 20-400 13597 / 13595 / 13488, 20 of
-// 100-400 behind 30-1000 cached ones 7739 / 7508 / 7498; with the waves for the copies (below) 9 of 100-400 behind 900-3000 6326 / - / 5330.
+// the plan, in order of length throughout, and by this rule (runs of one differ by 0.1-0.3 %): 8 prompts of 200-900 tokens 5590 / 5532 / 5537, 32 of 100-1024 22513 / 22240 / 22237 and
+// 24184 / 24018 / 24009, 64 of 20-400 15105 / 15116 / 15060, 20 of 100-400 behind 30-1000 cached ones 8310 / 8200 / 8204, 9 of 100-400 behind 900-3000 6420 / 5834 / 5796.  One
+// sequence has nothing to sort: 459 tokens by the plan, sorted, and without either 2006 / 2018 / 1995.
 #define PF_SORT_BLOCKS 128
 #define PF_SORT_KEYS 704
 struct PfBlock { int qb, q0, lq, kv0, lkv; };       // qb < 0: there is none
@@ -182,6 +183,10 @@ __device__ __forceinline__ int pf_wave_sum(int v) {
 }
 template <int QPOS>
 __device__ __forceinline__ PfBlock pf_block_of(const int32_t* __restrict__ qo_indptr, const int32_t* __restrict__ kv_indptr, int batch, int gblk, int lane) {
+    if (batch == 1) {                                // nothing to look for: last blocks first
+        const int a = qo_indptr[0], n = qo_indptr[1] - a, k = kv_indptr[0], blocks = n > 0 ? (n + QPOS - 1) / QPOS : 0;
+        return PfBlock{gblk < blocks ? blocks - 1 - gblk : -1, a, n, k, kv_indptr[1] - k};
+    }
     int q0 = 0, q1 = 0, k0 = 0, k1 = 0;
     if (lane < batch) { q0 = qo_indptr[lane]; q1 = qo_indptr[lane + 1]; k0 = kv_indptr[lane]; k1 = kv_indptr[lane + 1]; }
     const int lq = q1 - q0, lkv = k1 - k0, nb = lq > 0 ? (lq + QPOS - 1) / QPOS : 0, base = lkv > lq ? (lkv - lq) / QPOS : 0, end = nb ? base + nb : 0;
