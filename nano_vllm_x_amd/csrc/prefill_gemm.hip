@@ -167,7 +167,7 @@ static const PrefillTile PREFILL_TILES[] = {
 // The least of those.  us with cold weights, the rule before (the smallest tile whose workgroups all run at once, from some size on rounds times a round's cost) and
 // this one: SILU 6144 x 1024, 384 rows 14.9 and 12.9, 459 15.2 and 12.4, 512 16.2 and 13.0, 1100 25.6 and 22.1, 1200 25.5 and 24.7; 1024 x 3072, 1100 rows 20.2 and 15.9, 1500
 // 20.3 and 16.3, 2000 23.3 and 20.9; 1024 x 2048, 1500 rows 13.2 and 11.7, 2560 18.9 and 17.1; 4096 x 1024, 700 rows 11.1 and 10.6, 1100 17.6 and 16.6.
-// QKV: of 129 to 512 rows, by steps (figures at prefill_step.hip: with cold weights the product takes 14.9 us at 459 rows, the plain one 8.9 and the launch behind it some 5, and a step
+// QKV: of 129 to 512 rows, by steps (figures at prefill_step.hip: with cold weights the product takes 14.4 us at 459 rows, the plain one 8.9 and the launch behind it some 5, and a step
 // is 1.6 % the shorter; 1024 rows with warm weights 17.6 and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).  Its tiles of 64, 96 and 128 rows: 0.99 to 1.02 of a step of 300 to 1024 tokens.
 static int prefill_gemm_rule(int64_t m, int64_t n, bool silu, bool wide) {
     int best = NVX_PG_64_128;
