@@ -76,7 +76,9 @@ class ModelRunner:
         self.decode_chain: Optional[ops.DecodeChain] = None      # decode steps whose layers are one launch, and their graphs
         self.chain_graph: Optional[HIPGraph] = None
         self._chain_steps: list = []         # launched, ids not collected: such steps and those that read their ids, for computing them again
-        self._by_chain, self._chain_left, self._chain_lost, self._collected = False, 0, False, []
+        # whether the last step was one; the last (as BlockTable counts) whose results left uncollected, as it is and as the two launches under way found it; whether such a
+        # step gave up; the ids collected last
+        self._by_chain, self._chain_left, self._left_at_launch, self._chain_lost, self._collected = False, 0, [0, 0], False, []
         self._last_done = 0.0
         self.stats = {"prefill_steps": 0, "decode_steps": 0, "graph_steps": 0, "eager_decode_steps": 0, "prefill_s": 0.0, "decode_s": 0.0}
         self.graph_sizes_dropped: list = []               # decode batch sizes whose graph was slower than a larger one's
@@ -371,6 +373,8 @@ class ModelRunner:
     def _keep_chain_step(self, k: int, n: int, ids_on_device, draw, left: int):
         """What a launched step would be computed again from: for those whose layers were one launch, and those that read the ids of such a step."""
         by_chain, self._by_chain, self._chain_left = self._by_chain, False, left      # (its ids are collected: what it leaves is looked at)
+        if isinstance(k, int):
+            self._left_at_launch[k] = left
         if by_chain or (self._chain_steps and ids_on_device is not None):
             self._chain_steps = self._chain_steps[-1:] + [(k, n, self.block_table.steps_staged, self.sampler.calls, draw)]
 
@@ -450,12 +454,11 @@ class ModelRunner:
             if self.decode_chain is not None and self.decode_chain.failed:
                 self._settle_chain()      # (it may have computed this step again)
                 self._sample_events[ids].synchronize()
+            if self._chain_left == self._left_at_launch[ids]:
+                self._chain_left = 0              # (what left ahead of a step that has ended well is whole)
             if self._chain_steps:
-                at = next((i for i, step in enumerate(self._chain_steps) if step[0] == ids), None)
-                if at is not None:
-                    if self._chain_left < self._chain_steps[at][2]:
-                        self._chain_left = 0      # (what left ahead of a step that is whole is whole)
-                    del self._chain_steps[:at + 1]
+                at = next((i for i, step in enumerate(self._chain_steps) if step[0] == ids), -1)
+                del self._chain_steps[:at + 1]
             out = self._sample_hosts[ids][:n].tolist()
         else:
             out = ids.tolist()

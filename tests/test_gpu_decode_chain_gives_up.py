@@ -124,6 +124,23 @@ def test_a_step_left_uncollected_for_two_more_is_an_error(monkeypatch):
             r.finish_step(handle)
 
 
+@pytest.mark.parametrize("layers", [False, True])
+def test_what_left_ahead_of_a_step_that_ended_well_is_not_told_of_later(monkeypatch, layers):
+    """Whichever way that step went: a failure after it is that of another step."""
+    r, seqs = _runner_with((150, 7, 64))
+    _step(r, seqs)
+    assert r._chain_left > 0
+    graph = r.chain_graph
+    if layers:
+        r.chain_graph = None
+    r.finish_step(r.launch_step(_with_params(seqs)))
+    r.chain_graph = graph
+    assert r._chain_left == 0
+    _wait_in_vain(r, monkeypatch)
+    r.finish_step(r.launch_step(_batch(seqs)))
+    assert r.decode_chain is None and _step(r, seqs).isfinite().all()
+
+
 def test_a_warm_up_that_gives_up_leaves_the_layers(monkeypatch):
     from nano_vllm_x_amd import ops
 
