@@ -23,7 +23,7 @@ namespace NVX_NS {
 
 
 #define PF_KVBLK 64
-#define PF_RING 3               // tiles of a workgroup with waves that only fetch
+#define PF_RING 4               // tiles of a workgroup with waves that only fetch: one read for values, the next for keys, one landing, one asked for
 #define PF_SORTED 64             // sequences (a lane each) whose blocks are found without a plan
 #define PF_IDS (2 * PF_RING)    // tiles whose slot ids such a wave keeps
 #define PF_LOG2E 1.4426950408889634f
@@ -146,6 +146,12 @@ __device__ __forceinline__ void pf_gather(unsigned ids, int krow0, unsigned n_sl
     for (int p = 0; p < PASSES; ++p) pf_gather_one(id[p], n_slots, kbase, vbase, row_bytes, k_dst + p * STEP, v_dst + p * STEP);
 }
 
+// What a query's scores are taken relative to (log2 units): the largest so far, but one that is exceeded by less than 2^PF_SLACK stays.  Weights of up to 256 are as exact as
+// weights of up to 1 in either format, their sums are float32, and the accumulators need not be rescaled (64 multiplications a lane, between products) wherever any
+// of a wave's 32 queries finds a larger score: of 48 tiles of random scores that was every second.
+#define PF_SLACK 8.0f
+__device__ __forceinline__ float pf_reference(float was, float largest) { return largest > was + PF_SLACK ? largest : was; }
+
 #if defined(PF_STAMPS) && !defined(NVX_F16)
 // Build-time instrumentation (tools/build_variant.sh ... "-DPF_STAMPS"): shader-clock stamps of waves 0 and 3 of the
 // workgroups of blocks 8 and 9 (kv head 0; blocks of a sequence are taken last first, so these are query blocks 119 and
@@ -245,7 +251,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     constexpr int BUF_BYTES = 2 * PF_KVBLK * 256;
     constexpr int IDS_BYTES = 4 * PF_KVBLK;
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = LOADERS ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, lane = tid & 63;
     const int half = lane >> 5, l32 = lane & 31;
     const int unit = blockIdx.x;
     const int gblk = unit / hkv, head = unit % hkv;
@@ -306,23 +312,46 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
             const unsigned lds0 = pf_lds_addr(smem), rows = (unsigned)__builtin_amdgcn_readfirstlane(me * 4 * 256);
             const unsigned ids = lds0 + (unsigned)__builtin_amdgcn_readfirstlane(RING * BUF_BYTES + me * PF_IDS * IDS_BYTES);
             auto fetch_ids = [&](int t) { pf_fetch_slot_ids(seq_slots, t, lkv, lane, ids + (t % PF_IDS) * IDS_BYTES); };
-            auto fetch_rows = [&](int t) {
+            // where a tile's rows lie is found a turn before they are asked for: behind a barrier nothing is in front of the copies
+            unsigned long long from[PASSES];
+            auto find_rows = [&](int t) __attribute__((always_inline)) {
+                const unsigned at = ids + (t % PF_IDS) * IDS_BYTES;
+#pragma unroll
+                for (int p = 0; p < PASSES; ++p) {
+                    unsigned slot = (unsigned)*reinterpret_cast<pf_lds_i32*>((uintptr_t)(at + 4 * (krow0 + p * KEYS_PER_PASS)));
+                    slot = slot < n_slots_u ? slot : 0u;
+                    from[p] = (unsigned long long)slot * ((unsigned)hkv * 256u);
+                }
+            };
+            auto fetch_rows = [&](int t) __attribute__((always_inline)) {
                 const unsigned at = lds0 + (unsigned)(t % RING) * BUF_BYTES + rows;
-                pf_gather<PASSES, KEYS_PER_PASS>(ids + (t % PF_IDS) * IDS_BYTES, krow0, n_slots_u, kg, vg, (unsigned)hkv * 256u, at, at + PF_KVBLK * 256);
+#pragma unroll
+                for (int p = 0; p < PASSES; ++p) {
+                    pf_dma16(kg + from[p], at + p * (KEYS_PER_PASS * 256));
+                    pf_dma16(vg + from[p], at + PF_KVBLK * 256 + p * (KEYS_PER_PASS * 256));
+                }
             };
             for (int t = 0; t < n_tiles && t < 2 * RING - 1; ++t) fetch_ids(t);
             pf_wait_copies();
-            for (int t = 0; t < n_tiles && t < RING - 1; ++t) fetch_rows(t);
-            if (n_tiles > RING - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "n"((RING - 2) * 2 * PASSES) : "memory");
+            for (int t = 0; t < n_tiles && t < RING - 1; ++t) {
+                find_rows(t);
+                fetch_rows(t);
+            }
+            find_rows(RING - 1);                                                   // (whatever lies there if there is no such tile: not used)
+            // tile t's turn begins when tile t + 1 has landed
+            static_assert(RING == 4, "what may be on its way at a barrier: the rows of one tile");
+            if (n_tiles >= RING - 1) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
             else pf_wait_copies();
             __syncthreads();
             for (int t = 0; t < n_tiles; ++t) {
-                if (t + RING - 1 < n_tiles) fetch_rows(t + RING - 1);              // (to where tile t - 1 was)
-                if (t + 2 * RING - 1 < n_tiles) {
-                    fetch_ids(t + 2 * RING - 1);
-                    // since the rows of tile t + 1: the ids asked for behind them, RING - 2 tiles
-                    asm volatile("s_waitcnt vmcnt(%0)" : : "n"((RING - 2) * (2 * PASSES + 1)) : "memory");
-                } else pf_wait_copies();
+                const bool more_rows = t + RING - 1 < n_tiles, more_ids = t + 2 * RING - 1 < n_tiles;
+                if (more_rows) fetch_rows(t + RING - 1);                           // (to where tile t - 1 was)
+                if (more_ids) fetch_ids(t + 2 * RING - 1);
+                find_rows(t + RING);                                               // (its ids came with tile t - 3's turn)
+                // all but what this turn asked for: tile t + 2 has landed
+                if (more_ids) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES + 1) : "memory");
+                else if (more_rows) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
+                else pf_wait_copies();
                 __syncthreads();
             }
             return;
@@ -385,6 +414,184 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     }
     __syncthreads();
     { const unsigned t0 = ids0; ids0 = ids1; ids1 = t0; }
+    if constexpr (LOADERS > 0) {
+        // A turn: the sums of values of `tile` and the scores of the tile behind it.  A wave that has its SIMD to itself and makes a tile's scores, their probabilities and the sums
+        // of values one after the other lets the matrix pipe wait for the vector ALU and the other way round; here every group of products has exponentials or maxima beside
+        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  What a turn takes: figures at nvx_paged_prefill.
+        typedef __attribute__((ext_vector_type(8))) short s16x8;
+        const int vis = q_ok ? qi + offset : -1;                                          // last key this lane's query sees
+        // 32-key blocks of a tile that hold keys some query of the wave sees (wave-uniform)
+        const int tiles_u = __builtin_amdgcn_readfirstlane(n_tiles), last_u = __builtin_amdgcn_readfirstlane(wave_last_key), first_u = __builtin_amdgcn_readfirstlane(wave_first_vis);
+        auto blocks_of = [&](int t) { return t >= tiles_u || t * PF_KVBLK > last_u ? 0 : t * PF_KVBLK + 32 <= last_u ? 2 : 1; };
+        nvx_f32x16 st[2];                                                                 // scores of the next tile
+        float ex[2][16], mx[2], alpha = 0.f;                                              // what the exponentials of the present one are taken of; the largest; what becomes of the sums so far
+        nvx_u32x4 keys[8];                                                                // the next tile's first block
+        // half of the columns of a tile's keys: both blocks of 32, whose products take turns (0.88 us a tile where a block's eight in a row were 0.91)
+        auto read_keys = [&](nvx_u32x4 (&kf)[8], int t, int h) __attribute__((always_inline)) {
+            const unsigned at = lds0 + (unsigned)(t % RING) * BUF_BYTES + k_lane_off;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) kf[i] = pf_lds_read16((at ^ ((4 * h + (i >> 1)) << 5)) + (i & 1) * 32 * 256);
+        };
+        auto multiply_keys = [&](const nvx_u32x4 (&kf)[8], int h) __attribute__((always_inline)) {
+            if (h == 0) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) st[0][r] = st[1][r] = 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) st[i & 1] = mfma_32x32x16_h16(__builtin_bit_cast(nvx_h16x8, kf[i]), qf[4 * h + (i >> 1)], st[i & 1]);
+        };
+        auto mask = [&](int t) __attribute__((always_inline)) {
+            if (t * PF_KVBLK + PF_KVBLK - 1 <= first_u) return;                           // wave-uniform
+            const int upto = vis - t * PF_KVBLK - 4 * half;
+            asm volatile("" : : : "memory");
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) st[kb][r] = kb * 32 + (r & 3) + 8 * (r >> 2) <= upto ? st[kb][r] : -INFINITY;
+        };
+        auto maximum = [&](int kb) __attribute__((always_inline)) {
+            mx[kb] = st[kb][0];
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mx[kb] = fmaxf(mx[kb], st[kb][r]);
+        };
+        uint32_t pw[4][4];                                                                 // P^T, 16 keys a group
+        auto half_group = [&](int h) __attribute__((always_inline)) {                      // four exponentials per lane
+            const int gi = h >> 1, j0 = 2 * (h & 1);
+#pragma unroll
+            for (int j = j0; j < j0 + 2; ++j) {
+                const float p0 = __builtin_amdgcn_exp2f(ex[gi >> 1][8 * (gi & 1) + 2 * j]);
+                const float p1 = __builtin_amdgcn_exp2f(ex[gi >> 1][8 * (gi & 1) + 2 * j + 1]);
+                l_run = h == 0 && j == 0 ? fmaf(l_run, alpha, p0 + p1) : l_run + (p0 + p1);
+                pw[gi][j] = pack_h16x2(p0, p1);
+            }
+            asm volatile("" : "+v"(pw[gi][j0]), "+v"(pw[gi][j0 + 1]), "+v"(l_run));        // here, and not behind the next branch, where the products need them
+        };
+        float mref = 0.f;
+        auto begin = [&]() __attribute__((always_inline)) {
+            float m = fmaxf(mx[0], mx[1]);
+            m = fmaxf(m, xor32(m));
+            const float m_new = pf_reference(m_run, m * scale_log2);     // scale_log2 > 0
+            mref = m_new == -INFINITY ? 0.f : m_new;
+            alpha = __builtin_amdgcn_exp2f(m_run - mref);
+            m_run = m_new;
+        };
+        auto exponents = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ex[kb][r] = fmaf(st[kb][r], scale_log2, -mref);
+        };
+        // `tile`, begun, whose first NKB blocks are multiplied with values, and the scores of the tile behind it if NEXT (what that has beyond its last key is masked)
+        auto turn = [&](auto nkb_tag, auto next_tag, int tile) __attribute__((always_inline)) {
+            constexpr int NKB = decltype(nkb_tag)::value, NEXT = decltype(next_tag)::value ? 2 : 0, NGRP = 2 * NKB, STAGES = NEXT + NGRP;   // groups of 16 keys; of products
+            const unsigned vfrag0 = lds0 + (unsigned)(tile % RING) * BUF_BYTES + PF_KVBLK * 256 + v_lane_off;
+            nvx_u32x4 second[8];
+            s16x8 vf[NGRP][4];
+            auto read_group = [&](int gi) __attribute__((always_inline)) {                // V^T fragments, as below
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const unsigned pa = (vfrag0 ^ (d << 6)) + gi * 16 * 256;
+                    const pf_s16x4 va = pf_lds_read_tr(pa);
+                    const pf_s16x4 vb = pf_lds_read_tr(pa + 8 * 256);
+                    vf[gi][d] = s16x8{va[0], va[1], va[2], va[3], vb[0], vb[1], vb[2], vb[3]};
+                }
+            };
+            if (NEXT == 0) {
+                read_group(0);
+                half_group(0);
+                half_group(1);
+            }
+#pragma unroll
+            for (int i = 0; i < STAGES; ++i) {
+                if (NEXT > 0 && i == NEXT) mask(tile + 1);
+                if (i == NEXT && !__all(alpha == 1.0f)) {
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o_acc[d][r] *= alpha;
+                }
+                if (i == STAGES - 1) {                                                    // everything of this tile is in registers
+                    __syncthreads();                                                      // tile + 2 has landed, this one's place is free
+                    if (NEXT > 0) read_keys(keys, tile + 2, 0);                           // (whatever lies there if there is no such tile: not used)
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                // products: a block's scores, then a group's values
+                if (i < NEXT) {
+                    multiply_keys(i == 0 ? keys : second, i);
+                } else {
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const uint32_t* w = pw[i - NEXT];
+                        o_acc[d] = mfma_32x32x16_h16(__builtin_bit_cast(nvx_h16x8, vf[i - NEXT][d]), __builtin_bit_cast(nvx_h16x8, make_uint4(w[0], w[1], w[2], w[3])), o_acc[d]);
+                    }
+                }
+                // reads for what comes next
+                if (i + 1 < NEXT) read_keys(second, tile + 1, 1);
+                else if (i + 1 < STAGES) read_group(i + 1 - NEXT);
+                // beside them, dealt out by what they cost: a group's exponentials are as long as four to six of the products
+                if (NEXT == 0) {
+                    if (i + 1 < NGRP) {
+                        half_group(2 * i + 2);
+                        half_group(2 * i + 3);
+                    }
+                } else if (i < 2) {
+                    half_group(3 * i);
+                    half_group(3 * i + 1);
+                    half_group(3 * i + 2);
+                } else if (i == 2) {
+                    half_group(6);
+                    half_group(7);
+                } else if (i == 3) {
+                    maximum(0);
+                    maximum(1);
+                } else if (i == 4) {
+                    begin();
+                } else {
+                    exponents(0);
+                    exponents(1);
+                }
+                if (i < NEXT) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int tile = 0;
+        if (blocks_of(0) > 0) {
+            read_keys(keys, 0, 0);
+            multiply_keys(keys, 0);
+            read_keys(keys, 0, 1);
+            multiply_keys(keys, 1);
+            read_keys(keys, 1, 0);                                  // (whatever lies there if there is no such tile: not used)
+            mask(0);
+            maximum(0);
+            maximum(1);
+            begin();
+            exponents(0);
+            exponents(1);
+            for (; blocks_of(tile + 1) > 0; ++tile) turn(std::integral_constant<int, 2>{}, std::true_type{}, tile);
+            if (blocks_of(tile) == 2) turn(std::integral_constant<int, 2>{}, std::false_type{}, tile);
+            else turn(std::integral_constant<int, 1>{}, std::false_type{}, tile);
+            ++tile;
+        }
+        for (; tile < n_tiles; ++tile) __syncthreads();      // (nothing of these is visible to this wave)
+    } else {
     // at the top of tile t: ids0 holds the ids of tile t + 1, ids1 is free (its ids were used a tile ago)
 #ifdef PF_STAMPS
     const int stamp_blk = gblk;
@@ -394,7 +601,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         PF_STAMP(0);
         const unsigned k_lds = ring0;   // LDS byte addresses
         const unsigned v_lds = k_lds + PF_KVBLK * 256;
-        if (LOADERS == 0 && tile + 1 < n_tiles) {   // the other buffer held tile t - 1: every wave left it before the last barrier
+        if (tile + 1 < n_tiles) {   // the other buffer held tile t - 1: every wave left it before the last barrier
             if (tile > 0)           // (tile 1 came with tile 0)
                 pf_gather<PASSES, KEYS_PER_PASS>(ids0, krow0, n_slots_u, kg, vg, row_bytes, ring1 + wave_rows, ring1 + PF_KVBLK * 256 + wave_rows);
             if (tile + 2 < n_tiles && wave == 0) pf_fetch_slot_ids(seq_slots, tile + 2, lkv, lane, ids1);
@@ -457,11 +664,10 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         }
         float mx = NKB == 2 ? fmaxf(mxb[0], mxb[NKB - 1]) : mxb[0];
         mx = fmaxf(mx, xor32(mx));
-        const float m_new = fmaxf(m_run, mx * scale_log2);     // scale_log2 > 0
+        const float m_new = pf_reference(m_run, mx * scale_log2);     // scale_log2 > 0
         const float mref = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m_run - mref);
         m_run = m_new;
-        l_run *= alpha;
         if (!__all(alpha == 1.0f)) {
 #pragma unroll
             for (int d = 0; d < 4; ++d)
@@ -502,7 +708,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
             for (int j = 0; j < 4; ++j) {
                 const float p0 = __builtin_amdgcn_exp2f(fmaf(st[kb][8 * s2 + 2 * j], scale_log2, -mref));
                 const float p1 = __builtin_amdgcn_exp2f(fmaf(st[kb][8 * s2 + 2 * j + 1], scale_log2, -mref));
-                l_run += p0 + p1;
+                l_run = gi == 0 && j == 0 ? fmaf(l_run, alpha, p0 + p1) : l_run + (p0 + p1);
                 w[j] = pack_h16x2(p0, p1);
             }
             pf[gi] = __builtin_bit_cast(nvx_h16x8, make_uint4(w[0], w[1], w[2], w[3]));
@@ -532,13 +738,13 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         };
         if (key_base + 32 <= wave_last_key) tile_body(std::integral_constant<int, 2>{});        // wave-uniform
         else if (key_base <= wave_last_key) tile_body(std::integral_constant<int, 1>{});        // else: nothing visible
-        if (LOADERS == 0) pf_wait_copies();
+        pf_wait_copies();
         PF_STAMP(6);
         __syncthreads();   // tile + 1 and the ids of tile + 2 visible; this tile's buffer free
         PF_STAMP(7);
-        if (LOADERS) ring0 = ring0 == lds0 + (RING - 1) * BUF_BYTES ? lds0 : ring0 + BUF_BYTES;
-        else { const unsigned t0 = ring0; ring0 = ring1; ring1 = t0; }
+        { const unsigned t0 = ring0; ring0 = ring1; ring1 = t0; }
         { const unsigned t0 = ids0; ids0 = ids1; ids1 = t0; }
+    }
     }
 
     // ---- epilogue: O = O^T / l ----
@@ -607,11 +813,14 @@ extern "C" int NVX_ENTRY(nvx_paged_prefill)(const void* q, int64_t q_row_stride,
                            n_slots, qo_indptr, kv_indptr, kv_indices, plan_ws, (uint16_t*)out, (int)batch, n_kv_heads,  \
                            scale_log2);                                                                                 \
     } while (0)
-    // Few workgroups (of so many query positions, at most): waves of their own for the copies, and 32 positions of two heads as two waves, which read half as much LDS a tile.  us a
-    // step of Qwen3-0.6B before and now: 40 tokens 1378 and 1327, 459 2041 and 1970, 1024 2963 and 2843, 3000 6431 and 6068; 2160 tokens behind 900-3000 cached ones (320 workgroups)
-    // 5591 and 5382, 480 behind as many 3330 and 3057; 32 positions at 328 workgroups 3051 where 64 are 3031; 64 at 392 workgroups 5512 and 5338, at 488 5320 and 5330, at 592 7545 and 7734.
-    // Qwen3-8B, four layers: 459 tokens 1345 and 1324, 1500 2671 and 2634.
+    // Few workgroups (of so many query positions, at most): waves of their own for the copies, and 32 positions of two heads as two waves, which read half as much LDS a tile.  us a launch
+    // with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.4 (32 positions) and 13.5, 1024 18.7 and 24.4; 64 positions: 2500 tokens 43.1 and 57.3, six
+    // questions behind 900-3000 keys (272 workgroups) 56.7 and 74.4, ten (496) 76.7 and 84.3, twelve (560) 93.0 and 80.8, six prompts of 100-1024 (488) 26.3 and 29.6, eight (648) 35.6
+    // and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 459 tokens 12.0 and 13.1, 1500 29.0 and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
+    // Before a turn made the next tile's scores: 459 tokens 12.1, 1024 21.8, 64 queries of 3072 keys 54.3 (now 43.4: 0.79 us a tile, of 0.43 the matrix pipe needs).
     const auto groups = [&](int64_t positions) { return ((n_tokens + positions - 1) / positions + batch - 1) * n_kv_heads; };
+    // two rounds of a workgroup a CU, unless most blocks of a round and a half may be short ones
+    const auto few = [&](int64_t workgroups) { return workgroups <= (n_tokens >= 128 * batch ? 512 : 392); };
     switch (g) {
         case 1: NVX_PF(1, 4, 128, 0); break;
         // two 4-wave workgroups per CU (each in its own phase of the tile loop) measured faster than one
@@ -619,11 +828,11 @@ extern "C" int NVX_ENTRY(nvx_paged_prefill)(const void* q, int64_t q_row_stride,
         // copies two tiles ahead) changed neither
         case 2:
             if (groups(32) <= 256) NVX_PF(2, 2, 32, 4);
-            else if (groups(64) <= 392) NVX_PF(2, 4, 64, 4);
+            else if (few(groups(64))) NVX_PF(2, 4, 64, 4);
             else NVX_PF(2, 4, 64, 0);
             break;
         case 4:
-            if (groups(32) <= 392) NVX_PF(4, 4, 32, 4);
+            if (few(groups(32))) NVX_PF(4, 4, 32, 4);
             else NVX_PF(4, 4, 32, 0);
             break;   // 8 waves / 64 queries measured slower here too (1.77 vs 1.57 ms at 32 q heads)
         case 8: NVX_PF(8, 8, 32, 0); break;

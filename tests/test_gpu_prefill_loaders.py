@@ -31,8 +31,12 @@ def test_the_same_alone_and_among_others(dtype, hq, hkv, parts):
     alone = _run(q[:n], k, v, parts, slots, hq, hkv)
     among = _run(q, k, v, parts + filler, slots, hq, hkv)
     assert bool(torch.isfinite(alone).all()) and torch.equal(alone, among[:n])
-    # one sequence against float64
-    (a, b), heads = parts[0], hq // hkv
+    _against_float64(alone, q, k, v, slots, parts[0], hq, hkv, dtype)
+
+
+def _against_float64(got, q, k, v, slots, part, hq, hkv, dtype):
+    """The first sequence of a launch."""
+    (a, b), heads = part, hq // hkv
     rows = slots[:b].long()
     s = torch.einsum("ihd,jhd->hij", q[:a].view(a, hq, 128).double(), k[rows].double().repeat_interleave(heads, 1)) * 128 ** -0.5
     s = s.masked_fill(torch.arange(b, device="cuda")[None] > torch.arange(a, device="cuda")[:, None] + b - a, -torch.inf).softmax(2)
@@ -40,7 +44,26 @@ def test_the_same_alone_and_among_others(dtype, hq, hkv, parts):
     unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     size = torch.einsum("hij,jhd->ihd", s, v[rows].double().abs().repeat_interleave(heads, 1)).reshape(a, -1)
     # weights rounded to the format (half a unit each, the sum of them is not), the result once more; scores in float32
-    assert bool(((alone[:a].double() - want).abs() <= unit * size + unit * want.abs() + 2.0 ** -14 * size).all())
+    assert bool(((got[:a].double() - want).abs() <= unit * size + unit * want.abs() + 2.0 ** -14 * size).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("step", [0.25, 3.0, 5.5, 12.0, -3.0])
+def test_scores_that_climb(dtype, step):
+    """Scores that rise by `step` from tile to tile (and fall): the value that weights are taken relative to stays for rises of up to eight powers of two, and moves behind them."""
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    part, filler, hq, hkv = (150, 700), ((64, 64),) * 200, 4, 2
+    nq, nk = part[0] + 64 * 200, part[1] + 64 * 200
+    q = torch.zeros(nq, hq, 128, device="cuda")
+    q[:, :, 0] = 128 ** 0.5                                  # a score is a key's first element, and what the others add
+    q[:, :, 1:] = 0.1 * torch.randn(nq, hq, 127, generator=gen, device="cuda")
+    k = 0.5 * torch.randn(nk, hkv, 128, generator=gen, device="cuda")
+    k[:, :, 0] += (torch.arange(nk, device="cuda") % part[1] // 64 * step)[:, None]
+    q, k, v = q.view(nq, -1).to(dtype), k.to(dtype), torch.randn(nk, hkv, 128, generator=gen, device="cuda").to(dtype)
+    slots = torch.arange(nk, device="cuda", dtype=torch.int32)
+    alone = _run(q[:part[0]], k, v, (part,), slots, hq, hkv)
+    assert torch.equal(alone, _run(q, k, v, (part, *filler), slots, hq, hkv)[:part[0]])
+    _against_float64(alone, q, k, v, slots, part, hq, hkv, dtype)
 
 
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130])
