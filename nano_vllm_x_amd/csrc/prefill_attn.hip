@@ -509,6 +509,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
                         for (int r = 0; r < 16; ++r) o_acc[d][r] *= alpha;
                 }
                 if (i == STAGES - 1) {                                                    // everything of this tile is in registers
+                    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");                  // (a barrier alone does not wait for reads)
                     __syncthreads();                                                      // tile + 2 has landed, this one's place is free
                     if (NEXT > 0) read_keys(keys, tile + 2, 0);                           // (whatever lies there if there is no such tile: not used)
                 }

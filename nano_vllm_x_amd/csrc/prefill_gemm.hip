@@ -13,6 +13,8 @@
 //     11.2 / 9.7 / 13.6 and 4 / 12.5, 1536 rows 17.7 / 13.7 / 28.9 and 4 / 17.1).
 #include "prefill_gemm.h"
 
+#include <type_traits>
+
 namespace NVX_NS {
 
 // 64 lanes x 16 bytes from the lanes' addresses to 1 KB of LDS from a wave-uniform address on; the compiler does not count these loads, so every
@@ -35,6 +37,7 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
     static_assert(PIECES <= 16, "fragments of 16 rows share a swizzle");
     constexpr int ROWS = TM + TN, LOADS = ROWS / AT_ONCE / 4;              // copies of a wave a step
     constexpr int STAGE = ROWS * KS * 2;
+    static_assert(STAGES >= 2 && STAGES <= 4, "the last steps are written out");
     static_assert(ROWS % (4 * AT_ONCE) == 0 && (!SILU || FN % 2 == 0) && (MODE != NVX_PG_QKV || TN == 128) && (STAGES - 1) * LOADS < 64, "tile");
     constexpr int OUT = SILU ? TN / 2 : TN, LO = OUT + 8;                  // outputs of a row; elements of a row in LDS
     static_assert(TM * LO * 2 <= STAGES * STAGE, "the results turn around in the stages' memory");
@@ -56,10 +59,10 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
         from[i] = (r < TM ? x : w) + (int64_t)(r < TM ? rx : ww) * (r < TM ? x_stride : k) + c;
     }
     const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)smem;
-    auto ask = [&](int step) {
-        const unsigned at = lds0 + (unsigned)(step % STAGES) * STAGE + wave * LOADS * 1024;
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) piece_to_lds(from[i] + (int64_t)step * KS, at + i * 1024);
+    // one of a wave's copies of a step, then its next step's place
+    auto ask = [&](int i, unsigned slot) __attribute__((always_inline)) {
+        piece_to_lds(from[i], lds0 + slot + (wave * LOADS + i) * 1024);
+        from[i] += KS;
     };
     const int wm = wave / WN, wn = wave % WN;
     nvx_f32x4 acc[FN][FM];
@@ -70,42 +73,87 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
     typedef __attribute__((address_space(3))) const nvx_u32x4 lds_u4;
     const int steps = k / KS;
     struct Operands { nvx_u32x4 x[KS / 32][FM], w[KS / 32][FN]; };
-    auto read = [&](int step, Operands& f) {
-        const unsigned base = lds0 + (unsigned)(step % STAGES) * STAGE;
-        const unsigned xb = base + (wm * FM * 16 + l16) * (KS * 2), wb = base + (TM + wn * FN * 16 + l16) * (KS * 2);
+    constexpr int EACH = FM + FN, READS = KS / 32 * EACH, MULS = KS / 32 * FM * FN, EARLY = MULS >= 8 ? MULS * 5 / 8 : MULS;   // the reads are among the first EARLY products
+    const unsigned xl = lds0 + (wm * FM * 16 + l16) * (KS * 2), wl = lds0 + (TM + wn * FN * 16 + l16) * (KS * 2);
+    auto read = [&](int q, unsigned slot, Operands& f) __attribute__((always_inline)) {
+        const int kk = q / EACH, i = q % EACH;
+        const unsigned off = slot + (unsigned)((4 * kk + quad) ^ (l16 & (PIECES - 1))) * 16;
+        if (i < FM) f.x[kk][i] = *reinterpret_cast<lds_u4*>((uintptr_t)(xl + i * 16 * KS * 2 + off));
+        else f.w[kk][i - FM] = *reinterpret_cast<lds_u4*>((uintptr_t)(wl + (i - FM) * 16 * KS * 2 + off));
+    };
+    unsigned slot = 0;                                                              // of step s
+    // Step s is in registers; step s + 1 is read while it is multiplied, and its place in LDS is asked to be filled with step s + STAGES (ASKS).  Copies and reads are dealt
+    // out between the products: a wave that asks for all its copies at once waits for as long as the CU takes them in (64 bytes a clock), and multiplies nothing meanwhile.
+    // FLYING: copies of later steps than s + 1 that need not have landed; LAST: there is no step s + 1.
+    auto turn = [&](auto flying, auto asks, auto last, const Operands& now, Operands& next) __attribute__((always_inline)) {
+        constexpr bool ASKS = decltype(asks)::value, LAST = decltype(last)::value;
+        const unsigned free_slot = slot;
+        slot = slot == (STAGES - 1) * STAGE ? 0 : slot + STAGE;
+        if (!LAST) {
+            wait_for_all_but<decltype(flying)::value>();                            // step s + 1 has landed
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");                    // and this wave has read step s (a barrier alone does not wait for reads)
+            __syncthreads();                                                        // everybody's part of it has, and everybody has read step s
+        }
 #pragma unroll
-        for (int kk = 0; kk < KS / 32; ++kk) {
-            const unsigned off = (unsigned)((4 * kk + quad) ^ (l16 & (PIECES - 1))) * 16;
+        for (int u = 0; u < MULS; ++u) {
+            const int kk = u / (FM * FN), i = u / FM % FN, j = u % FM;
+            if (!LAST) {
 #pragma unroll
-            for (int j = 0; j < FM; ++j) f.x[kk][j] = *reinterpret_cast<lds_u4*>((uintptr_t)(xb + j * 16 * KS * 2 + off));
+                for (int q = 0; q < READS; ++q)
+                    if (q * EARLY / READS == u) read(q, slot, next);
+            }
+            if (ASKS) {
 #pragma unroll
-            for (int i = 0; i < FN; ++i) f.w[kk][i] = *reinterpret_cast<lds_u4*>((uintptr_t)(wb + i * 16 * KS * 2 + off));
+                for (int q = 0; q < LOADS; ++q)
+                    if (q * MULS / LOADS == u) ask(q, free_slot);
+            }
+            acc[i][j] = mfma_16x16x32_h16(now.w[kk][i], now.x[kk][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // step s is in registers; step s + 1 is read while it is multiplied, and its place in LDS is asked to be filled with step s + STAGES
-    auto turn = [&](int s, const Operands& now, Operands& next) {
-        if (s + STAGES <= steps) wait_for_all_but<(STAGES - 2) * LOADS>();          // step s + 1 has landed, STAGES - 2 later ones need not have
-        else wait_for_all_but<0>();
-        __syncthreads();                                                            // everybody's part of it has, and everybody has read step s
-        if (s + STAGES < steps) ask(s + STAGES);
-        read(s + 1, next);                                                          // (after the last step: whatever lies there, not used)
-        __builtin_amdgcn_sched_barrier(0);
+    const int begun = min(STAGES, steps);
+    for (int s = 0; s < begun; ++s)
 #pragma unroll
-        for (int kk = 0; kk < KS / 32; ++kk)
-#pragma unroll
-            for (int i = 0; i < FN; ++i)
-#pragma unroll
-                for (int j = 0; j < FM; ++j) acc[i][j] = mfma_16x16x32_h16(now.w[kk][i], now.x[kk][j], acc[i][j]);
-    };
-    for (int s = 0; s < STAGES && s < steps; ++s) ask(s);
+        for (int i = 0; i < LOADS; ++i) ask(i, s * STAGE);
+    std::true_type yes;
+    std::false_type no;
+    Operands even, odd;
     if (STAGES <= steps) wait_for_all_but<(STAGES - 1) * LOADS>();
     else wait_for_all_but<0>();
     __syncthreads();
-    Operands even, odd;
-    read(0, even);
-    for (int s = 0; s < steps; s += 2) {
-        turn(s, even, odd);
-        turn(s + 1, odd, even);
+#pragma unroll
+    for (int q = 0; q < READS; ++q) read(q, 0, even);
+    if (steps < STAGES) {                                                           // (k / KS is even)
+        std::integral_constant<int, 0> none;
+        for (int s = 0; s + 2 < steps; s += 2) {
+            turn(none, no, no, even, odd);
+            turn(none, no, no, odd, even);
+        }
+        turn(none, no, no, even, odd);
+        turn(none, no, yes, odd, even);
+    } else {
+        std::integral_constant<int, (STAGES - 2) * LOADS> most;
+        int left = steps - STAGES;
+        for (; left > 1; left -= 2) {
+            turn(most, yes, no, even, odd);
+            turn(most, yes, no, odd, even);
+        }
+        auto rest = [&](Operands& now, Operands& next) __attribute__((always_inline)) {     // the last STAGES steps, which have all been asked for
+            auto one = [&](auto j, Operands& a, Operands& b) __attribute__((always_inline)) {
+                constexpr int J = decltype(j)::value, F = STAGES - 2 - J;
+                if constexpr (J < STAGES) turn(std::integral_constant<int, (F > 0 ? F : 0) * LOADS>{}, no, std::integral_constant<bool, J == STAGES - 1>{}, a, b);
+            };
+            one(std::integral_constant<int, 0>{}, now, next);
+            one(std::integral_constant<int, 1>{}, next, now);
+            one(std::integral_constant<int, 2>{}, now, next);
+            one(std::integral_constant<int, 3>{}, next, now);
+        };
+        if constexpr (STAGES % 2) {
+            turn(most, yes, no, even, odd);
+            rest(odd, even);
+        } else {
+            rest(even, odd);
+        }
     }
     // a lane has row l16 of every 16 rows of x and four neighbouring outputs (4 * quad ..) of every 16
     __syncthreads();
@@ -153,30 +201,39 @@ static void launch_prefill_gemm(const void* x, int64_t x_stride, const void* w, 
 
 using namespace NVX_NS;
 
-// What a tile costs, us of 1024 columns of K with weights that no cache holds: the first `slots` workgroups, and every further as many (0: not built).  Fitted to
-// 100 to 2560 rows of 4096, 2048 and 1024 outputs and, with SILU, of 6144 (deeper K: the same order).  Up to one workgroup a CU a product costs what its tile brings
-// into a CU, 82 KB a us whatever the kernel (rows of w straight to registers in operand order: the same times), so the tile that just fills the CUs is the best.
-struct PrefillTile { int tile, m, n, slots, silu_slots; float us, more, us_silu, more_silu; bool wide; };
+// What a tile costs, us, with weights that no cache holds: us + k / 1024 * (us_k + (rounds - 1) * round + (workgroups / 256 - 1) * over), rounds of 256 workgroups and the last term from
+// the 257th on (us_k 0: not built).  Fitted to 40 to 4096 rows of 1024 to 4096 outputs of 512 to 6144 columns, 1 900 products: over these the tile it picks costs 0.6 % more than the best one
+// (17 % at worst), where the table for 1024 columns that was here before cost 4.8 % (39 %).  A step of a few KB is as long as its copies' way into a CU, its reads from LDS and two barriers'
+// skew, hardly any of which hides any other at one workgroup a CU, so the tile that just fills the CUs is the best; us a product before, with the copies of a step asked for at
+// once, and now: 2160 rows 1024 x 2048 18.9 (128 x 128) and 15.1 (160 x 64), 1024 x 3072 29.2 (128 x 128) and 21.1 (160 x 64); 1900 rows 16.0 and 13.2, 24.7 and 20.6 (128 x 64); 459 rows 7.9 and
+// 7.6, 11.1 and 10.9 (32 x 64), 4096 x 1024 10.4 (64 x 128) and 8.6 (128 x 64).  A deeper ring (all of LDS) was no faster; nor were rows of w a multiple of 128 bytes and 64 apart.
+struct PrefillCost { float us, us_k, round, over; };
+struct PrefillTile { int tile, m, n; PrefillCost plain, silu; bool wide; };
 static const PrefillTile PREFILL_TILES[] = {
-    {NVX_PG_32_32, 32, 32, 256, 0, 4.2f, 1.65f, 0.f, 0.f, false},       {NVX_PG_32_64, 32, 64, 256, 256, 5.3f, 3.6f, 6.0f, 4.6f, false},
-    {NVX_PG_64_64, 64, 64, 256, 256, 6.4f, 2.9f, 7.7f, 3.6f, false},    {NVX_PG_96_64, 96, 64, 256, 0, 7.5f, 4.0f, 0.f, 0.f, false},
-    {NVX_PG_64_128, 64, 128, 256, 768, 9.2f, 4.9f, 20.5f, 17.f, false}, {NVX_PG_128_128, 128, 128, 256, 256, 10.6f, 8.4f, 12.5f, 9.5f, true},
-    {NVX_PG_128_256, 128, 256, 256, 256, 16.8f, 17.f, 25.f, 15.5f, true}, {NVX_PG_192_256, 192, 256, 256, 256, 18.6f, 7.f, 27.5f, 19.f, true},
-    {NVX_PG_256_256, 256, 256, 256, 256, 22.7f, 12.f, 31.f, 18.f, true}};
+    {NVX_PG_32_32, 32, 32, {1.9f, 2.1f, 1.f, .5f}, {}, false},
+    {NVX_PG_32_64, 32, 64, {2.4f, 2.8f, 2.5f, .6f}, {2.7f, 3.1f, 5.f, -.6f}, false},
+    {NVX_PG_64_64, 64, 64, {1.7f, 4.3f, 2.f, 1.3f}, {1.5f, 6.f, 3.f, .8f}, false},
+    {NVX_PG_96_64, 96, 64, {2.2f, 4.7f, 2.8f, 1.6f}, {}, false},
+    {NVX_PG_128_64, 128, 64, {2.7f, 5.3f, 5.4f, 1.5f}, {}, false},
+    {NVX_PG_160_64, 160, 64, {3.f, 6.1f, 6.3f, 1.7f}, {}, false},
+    {NVX_PG_192_64, 192, 64, {3.4f, 6.8f, 7.5f, 2.f}, {}, false},
+    {NVX_PG_64_128, 64, 128, {1.4f, 6.8f, 2.1f, 3.4f}, {.2f, 14.3f, 1.f, 5.3f}, false},
+    {NVX_PG_128_128, 128, 128, {3.1f, 7.7f, 7.3f, 2.9f}, {4.2f, 8.3f, 10.f, -.2f}, true},
+    {NVX_PG_128_256, 128, 256, {-1.4f, 19.1f, 16.9f, 8.1f}, {1.4f, 22.4f, 16.4f, 1.f}, true},
+    {NVX_PG_192_256, 192, 256, {.1f, 20.1f, 21.6f, 1.2f}, {3.8f, 22.9f, 19.1f, 3.1f}, true},
+    {NVX_PG_256_256, 256, 256, {2.4f, 21.8f, 12.f, 10.f}, {5.8f, 25.f, 22.9f, 4.7f}, true}};
 
-// The least of those.  us with cold weights, the rule before (the smallest tile whose workgroups all run at once, from some size on rounds times a round's cost) and
-// this one: SILU 6144 x 1024, 384 rows 14.9 and 12.9, 459 15.2 and 12.4, 512 16.2 and 13.0, 1100 25.6 and 22.1, 1200 25.5 and 24.7; 1024 x 3072, 1100 rows 20.2 and 15.9, 1500
-// 20.3 and 16.3, 2000 23.3 and 20.9; 1024 x 2048, 1500 rows 13.2 and 11.7, 2560 18.9 and 17.1; 4096 x 1024, 700 rows 11.1 and 10.6, 1100 17.6 and 16.6.
+// The least of those.
 // QKV: of 129 to 512 rows, by steps (figures at prefill_step.hip: with cold weights the product takes 14.4 us at 459 rows, the plain one 8.9 and the launch behind it some 5, and a step
 // is 1.6 % the shorter; 1024 rows with warm weights 17.6 and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).  Its tiles of 64, 96 and 128 rows: 0.99 to 1.02 of a step of 300 to 1024 tokens.
-static int prefill_gemm_rule(int64_t m, int64_t n, bool silu, bool wide) {
-    int best = NVX_PG_64_128;
+static int prefill_gemm_rule(int64_t m, int64_t n, int64_t k, bool silu, bool wide) {
+    int best = NVX_PG_64_64;
     float least = 0.f;
     for (const PrefillTile& t : PREFILL_TILES) {
-        const int slots = silu ? t.silu_slots : t.slots;
-        if (!slots || n % t.n || (t.wide && !wide)) continue;
-        const int64_t rounds = ((m + t.m - 1) / t.m * (n / t.n) + slots - 1) / slots;
-        const float cost = (silu ? t.us_silu : t.us) + (float)(rounds - 1) * (silu ? t.more_silu : t.more);
+        const PrefillCost& c = silu ? t.silu : t.plain;
+        if (c.us_k == 0.f || n % t.n || (t.wide && !wide)) continue;
+        const int64_t workgroups = (m + t.m - 1) / t.m * (n / t.n), rounds = (workgroups + 255) / 256;
+        const float cost = c.us + (float)k / 1024.f * (c.us_k + (float)(rounds - 1) * c.round + (workgroups > 256 ? (float)workgroups / 256.f - 1.f : 0.f) * c.over);
         if (least == 0.f || cost < least) best = t.tile, least = cost;
     }
     return best;
@@ -192,7 +249,7 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
     NVX_REQUIRE((m + 31) / 32 * (n / 32) < (1ll << 30), NVX_EUNSUPPORTED, "nvx_prefill_gemm: too many tiles");
     const bool silu = mode == NVX_PG_SILU;
     if (mode == NVX_PG_QKV) tile = NVX_PG_32_128;
-    else if (tile == 0) tile = prefill_gemm_rule(m, n, silu, x_stride < (1 << 21) && n * k < (1ll << 30));       // (what the wide tiles' offsets hold)
+    else if (tile == 0) tile = prefill_gemm_rule(m, n, k, silu, x_stride < (1 << 21) && n * k < (1ll << 30));       // (what the wide tiles' offsets hold)
     if (tile >= NVX_PG_256_256 && tile < NVX_PG_64_128)
         return NVX_ENTRY(nvx_prefill_wide)(x, x_stride, w, y, m, n, k, silu, tile == NVX_PG_256_256 ? 256 : tile == NVX_PG_192_256 ? 192 : 128, tile == NVX_PG_128_128 ? 128 : 256, st);
 #define NVX_PG(TM, TN, KS, ST, MODE) launch_prefill_gemm<TM, TN, KS, ST, 2, MODE>(x, x_stride, w, y, m, n, k, qkv, st)
@@ -201,6 +258,9 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
         case NVX_PG_64_64: if (silu) NVX_PG(64, 64, 64, 4, NVX_PG_SILU); else NVX_PG(64, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_64: if (silu) NVX_PG(32, 64, 128, 4, NVX_PG_SILU); else NVX_PG(32, 64, 128, 4, NVX_PG_PLAIN); break;
         case NVX_PG_96_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(96, 64, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_128_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(128, 64, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_160_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(160, 64, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_192_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(192, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_32: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 32, 128, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_128: NVX_REQUIRE(mode == NVX_PG_QKV, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 128, 64, 4, NVX_PG_QKV); break;
         default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);

@@ -22,3 +22,23 @@ def test_one_order_of_summation(dtype, m, n, k):
     y = torch.empty((m, n // 2), dtype=dtype, device="cuda")
     with pytest.raises(RuntimeError):
         _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 1, 7, ops._stream()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 256), (127, 128, 512), (129, 256, 768), (159, 128, 1024), (161, 128, 256), (193, 1024, 512), (320, 128, 1280), (577, 4096, 256), (2100, 1024, 3072)])
+def test_tall_tiles_and_few_steps(dtype, m, n, k):
+    """Tiles of 128, 160 and 192 x 64, and those of 32 rows whose steps of 128 columns are fewer than a ring holds: the bits of 64 x 64, no row past the last written."""
+    from nano_vllm_x_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 64, generator=gen, device="cuda").to(dtype)[:, 32:32 + k]
+    w = (torch.randn(n, k, generator=gen, device="cuda") * k ** -0.5).to(dtype)
+    fn, first = getattr(_lib.load(), "nvx_internal_prefill_gemm" + ("_f16" if dtype == torch.float16 else "")), None
+    for tile in (6, 11, 12, 13, 5, 8, 9):
+        y = torch.full((m + 200, n), float("nan"), dtype=dtype, device="cuda")
+        _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 0, tile, ops._stream()))
+        first = y[:m] if first is None else first
+        assert bool(torch.isfinite(y[:m]).all()) and bool(torch.isnan(y[m:]).all()) and torch.equal(y[:m], first), tile
+    for tile in (9, 11, 12, 13):      # no SiluAndMul in these
+        with pytest.raises(RuntimeError):
+            _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 1, tile, ops._stream()))
