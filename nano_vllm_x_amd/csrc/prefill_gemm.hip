@@ -23,6 +23,11 @@ __device__ __forceinline__ void piece_to_lds(const void* g, unsigned lds) {
     const unsigned uni = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(uni) : "memory");
 }
+// 64 lanes x 4 bytes likewise
+__device__ __forceinline__ void words_to_lds(const void* g, unsigned lds) {
+    const unsigned uni = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(uni) : "memory");
+}
 template <int N>
 __device__ __forceinline__ void wait_for_all_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
@@ -111,6 +116,33 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    // QKV: where the tile's tokens stand and what their heads' ends read of memory.  Positions and slots come ahead of all copies, into LDS (a wave's wait for a step
+    // covers its older copies); what they lead to is on its way during the last steps.  459 tokens of Qwen3-0.6B, us a step: 1979 with tiles of 32 rows, two a CU, whose ends read one after
+    // the other; 1903 with one of 64.
+    constexpr bool HEADS = MODE == NVX_PG_QKV;
+    __shared__ int64_t where[HEADS ? 2 * TM : 1];
+    QkvHeadIn foreseen[HEADS ? TM / 16 : 1];
+    uint2 wa = {}, wb = {};
+    if constexpr (HEADS) {
+        static_assert(TM % 32 == 0, "a copy is 32 tokens");
+        for (int c = wave; c < TM / 16; c += 4) {
+            const bool first = c < TM / 32;
+            words_to_lds(reinterpret_cast<const int32_t*>(first ? qkv.positions : qkv.slots) + 2 * min(m0 + (first ? c : c - TM / 32) * 32 + (lane >> 1), m - 1) + (lane & 1),
+                         (unsigned)(uintptr_t)(const __attribute__((address_space(3))) int64_t*)where + c * 256);
+        }
+    }
+    auto foresee = [&]() __attribute__((always_inline)) {
+        if constexpr (HEADS) {
+            const uint16_t* const norm = tn < qkv.hq ? qkv.q_norm : qkv.k_norm;
+            wa = *reinterpret_cast<const uint2*>(norm + 4 * l16);
+            wb = *reinterpret_cast<const uint2*>(norm + 64 + 4 * l16);
+#pragma unroll
+            for (int i = 0; i < TM / 16; ++i) {
+                const int r = (int)(threadIdx.x >> 4) + 16 * i;
+                foreseen[i] = qkv_head_in(l16, tn, where[r], where[TM + r], qkv);
+            }
+        }
+    };
     const int begun = min(STAGES, steps);
     for (int s = 0; s < begun; ++s)
 #pragma unroll
@@ -124,6 +156,7 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
 #pragma unroll
     for (int q = 0; q < READS; ++q) read(q, 0, even);
     if (steps < STAGES) {                                                           // (k / KS is even)
+        foresee();
         std::integral_constant<int, 0> none;
         for (int s = 0; s + 2 < steps; s += 2) {
             turn(none, no, no, even, odd);
@@ -150,8 +183,10 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
         };
         if constexpr (STAGES % 2) {
             turn(most, yes, no, even, odd);
+            foresee();
             rest(odd, even);
         } else {
+            foresee();
             rest(even, odd);
         }
     }
@@ -177,9 +212,12 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
     }
     __syncthreads();
     if constexpr (MODE == NVX_PG_QKV) {
-        for (int r = threadIdx.x >> 4; r < TM && m0 + r < m; r += 16) {
+#pragma unroll
+        for (int i = 0; i < TM / 16; ++i) {
+            const int r = (int)(threadIdx.x >> 4) + 16 * i;
             const HalfQuad hq = load_half_quads(so + r * LO, l16);
-            qkv_head_out(hq, quarter_sum(qkv_lane_squares(hq)), l16, tn, m0 + r, qkv);
+            const float ss = quarter_sum(qkv_lane_squares(hq));
+            if (m0 + r < m) qkv_head_out(hq, ss, foreseen[i], wa, wb, l16, tn, m0 + r, qkv);
         }
         return;
     }
@@ -223,12 +261,29 @@ static const PrefillTile PREFILL_TILES[] = {
     {NVX_PG_192_256, 192, 256, {.1f, 20.1f, 21.6f, 1.2f}, {3.8f, 22.9f, 19.1f, 3.1f}, true},
     {NVX_PG_256_256, 256, 256, {2.4f, 21.8f, 12.f, 10.f}, {5.8f, 25.f, 22.9f, 4.7f}, true}};
 
-// The least of those.
-// QKV: of 129 to 512 rows, by steps (figures at prefill_step.hip: with cold weights the product takes 14.4 us at 459 rows, the plain one 8.9 and the launch behind it some 5, and a step
-// is 1.6 % the shorter; 1024 rows with warm weights 17.6 and 17; a 256 x 256 tile's take 15 us, in which its CU multiplies nothing).  Its tiles of 64, 96 and 128 rows: 0.99 to 1.02 of a step of 300 to 1024 tokens.
-static int prefill_gemm_rule(int64_t m, int64_t n, int64_t k, bool silu, bool wide) {
+// QKV, a tile as wide as a head: us + k / 1024 * (us_k + (rounds - 1) * round), less what the launch costs that norms and turns the heads behind a plain product (the two grow alike with
+// the rows).  Fitted to steps of 20 to 3000 tokens of layers of 512 to 2560: with one round of workgroups these costs, held against the plain tiles', were right wherever the two ways differ by more than
+// 1 us a layer.  us a layer of 1024 columns and 32 heads, plain and launch / here: 130 tokens 55.9 / 54.5, 256 61.3 / 59.8 (32 rows), 300 66.1 / 65.2, 459 73.4 / 71.3 (64 rows), 768 98.2 / 94.0 (96), 900
+// 98.5 / 96.8 (128); two rounds of 96 rows, 1500 129.2 / 123.8, but 1152 (384 workgroups of the 512) 110.8 / 112.8: two rounds must be 13/16 full.  2048 columns: 300 115.0 / 116.2, not taken, 400 117.3 / 116.0.
+// Two workgroups a CU or more rounds were never the better way, nor steps of 128 columns.  A 256 x 256 tile's heads take 15 us, in which its CU multiplies nothing.
+struct HeadsTile { int tile, m; float us, us_k, round; };
+static const HeadsTile HEADS_TILES[] = {
+    {NVX_PG_32_128, 32, -.9f, 5.3f, 0.f}, {NVX_PG_64_128, 64, -.3f, 6.3f, 0.f}, {NVX_PG_96_128, 96, .5f, 6.4f, 7.6f}, {NVX_PG_HEADS_128_128, 128, 1.5f, 7.7f, 0.f}};
+static int heads_tile(int64_t m, int64_t n, int64_t k, float& cost) {
+    int best = 0;
+    for (const HeadsTile& t : HEADS_TILES) {
+        const int64_t workgroups = (m + t.m - 1) / t.m * (n / 128);
+        if (workgroups > 256 && (t.round == 0.f || workgroups > 512 || workgroups < 416)) continue;
+        const float c = t.us + (float)k / 1024.f * (t.us_k + (workgroups > 256 ? t.round : 0.f));
+        if (!best || c < cost) best = t.tile, cost = c;
+    }
+    return best;
+}
+
+// The least of the first table's.
+static int prefill_gemm_rule(int64_t m, int64_t n, int64_t k, bool silu, bool wide, float& least) {
     int best = NVX_PG_64_64;
-    float least = 0.f;
+    least = 0.f;
     for (const PrefillTile& t : PREFILL_TILES) {
         const PrefillCost& c = silu ? t.silu : t.plain;
         if (c.us_k == 0.f || n % t.n || (t.wide && !wide)) continue;
@@ -237,6 +292,13 @@ static int prefill_gemm_rule(int64_t m, int64_t n, int64_t k, bool silu, bool wi
         if (least == 0.f || cost < least) best = t.tile, least = cost;
     }
     return best;
+}
+
+bool NVX_ENTRY(nvx_prefill_heads_ride)(int64_t m, int64_t n, int64_t k) {
+    float here = 0.f, plain;
+    if (!heads_tile(m, n, k, here)) return false;
+    prefill_gemm_rule(m, n, k, false, n * k < (1ll << 30), plain);
+    return here < plain;
 }
 
 // tile: one of NVX_PG_*, or 0 by the rule
@@ -248,12 +310,21 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
     if (m == 0) return NVX_OK;
     NVX_REQUIRE((m + 31) / 32 * (n / 32) < (1ll << 30), NVX_EUNSUPPORTED, "nvx_prefill_gemm: too many tiles");
     const bool silu = mode == NVX_PG_SILU;
-    if (mode == NVX_PG_QKV) tile = NVX_PG_32_128;
-    else if (tile == 0) tile = prefill_gemm_rule(m, n, k, silu, x_stride < (1 << 21) && n * k < (1ll << 30));       // (what the wide tiles' offsets hold)
-    if (tile >= NVX_PG_256_256 && tile < NVX_PG_64_128)
+    float cost;
+    if (tile == 0 && mode == NVX_PG_QKV) {
+        tile = heads_tile(m, n, k, cost);
+        if (!tile) tile = NVX_PG_32_128;
+    } else if (tile == 0) tile = prefill_gemm_rule(m, n, k, silu, x_stride < (1 << 21) && n * k < (1ll << 30), cost);       // (what the wide tiles' offsets hold)
+    if (mode != NVX_PG_QKV && tile >= NVX_PG_256_256 && tile < NVX_PG_64_128)
         return NVX_ENTRY(nvx_prefill_wide)(x, x_stride, w, y, m, n, k, silu, tile == NVX_PG_256_256 ? 256 : tile == NVX_PG_192_256 ? 192 : 128, tile == NVX_PG_128_128 ? 128 : 256, st);
 #define NVX_PG(TM, TN, KS, ST, MODE) launch_prefill_gemm<TM, TN, KS, ST, 2, MODE>(x, x_stride, w, y, m, n, k, qkv, st)
-    switch (tile) {
+    if (mode == NVX_PG_QKV) switch (tile) {
+        case NVX_PG_32_128: NVX_PG(32, 128, 64, 4, NVX_PG_QKV); break;
+        case NVX_PG_64_128: NVX_PG(64, 128, 64, 4, NVX_PG_QKV); break;
+        case NVX_PG_96_128: NVX_PG(96, 128, 64, 4, NVX_PG_QKV); break;
+        case NVX_PG_HEADS_128_128: NVX_PG(128, 128, 64, 4, NVX_PG_QKV); break;
+        default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);
+    } else switch (tile) {
         case NVX_PG_64_128: if (silu) NVX_PG(64, 128, 64, 2, NVX_PG_SILU); else NVX_PG(64, 128, 64, 3, NVX_PG_PLAIN); break;
         case NVX_PG_64_64: if (silu) NVX_PG(64, 64, 64, 4, NVX_PG_SILU); else NVX_PG(64, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_64: if (silu) NVX_PG(32, 64, 128, 4, NVX_PG_SILU); else NVX_PG(32, 64, 128, 4, NVX_PG_PLAIN); break;
@@ -262,7 +333,6 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
         case NVX_PG_160_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(160, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_192_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(192, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_32: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 32, 128, 4, NVX_PG_PLAIN); break;
-        case NVX_PG_32_128: NVX_REQUIRE(mode == NVX_PG_QKV, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(32, 128, 64, 4, NVX_PG_QKV); break;
         default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);
     }
 #undef NVX_PG
@@ -275,4 +345,11 @@ int NVX_ENTRY(nvx_prefill_gemm)(const void* x, int64_t x_stride, const void* w, 
 extern "C" int NVX_ENTRY(nvx_internal_prefill_gemm)(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, int silu, int tile,
                                                     nvx_stream_t stream) {
     return prefill_gemm(tile, x, x_stride, w, y, m, n, k, silu ? NVX_PG_SILU : NVX_PG_PLAIN, nullptr, (hipStream_t)stream);
+}
+// what becomes of one [q | k | v] projection, by a tile of the caller's choice (0: the rule's)
+extern "C" int NVX_ENTRY(nvx_internal_prefill_heads)(const void* x, int64_t x_stride, const void* w, int64_t m, int64_t k, int tile, const int64_t* positions, const int64_t* slots,
+                                                     const float* rope, int64_t rope_rows, int64_t n_slots, const void* q_norm, const void* k_norm, void* q, void* k_cache, void* v_cache,
+                                                     int hq, int hkv, float eps, nvx_stream_t stream) {
+    const NvxQkvOut out = {positions, slots, rope, rope_rows, n_slots, (const uint16_t*)q_norm, (const uint16_t*)k_norm, (uint16_t*)q, (uint16_t*)k_cache, (uint16_t*)v_cache, hq, hkv, eps};
+    return prefill_gemm(tile, x, x_stride, w, nullptr, m, (int64_t)(hq + 2 * hkv) * 128, k, NVX_PG_QKV, &out, (hipStream_t)stream);
 }

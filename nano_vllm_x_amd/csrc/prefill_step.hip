@@ -32,11 +32,7 @@ extern "C" int NVX_ENTRY(nvx_internal_prefill_step)(const NvxPrefillStep* s, nvx
     int turn = 0;
     for (int64_t l = 0; l < s->n_layers; ++l) {
         const int64_t* w = s->layers + 10 * l;
-        // a head's norm and rotation behind the product: us a step of Qwen3-0.6B, in a launch of their own / there, 129 tokens 1553 / 1533, 200 1610 / 1592, 256 1712 / 1684,
-        // 300 1877 / 1906, 350 1984 / 2015, 400 2028 / 1997, 459 2057 / 2024, 512 2142 / 2102 (the plain product's rule finds a better tile at 300 and 350; up to 128 the product has
-        // smaller tiles, which hold no head: 40 tokens 1557 / 1594, 128 1700 / 1718; beyond 512 see prefill_gemm_rule).  Other sizes, there as a part of
-        // its own launch's, 129 to 512 tokens: layers of 256 x 768 0.99-1.00, 512 x 1536 0.94-1.00, 768 x 2304 0.99-1.00, 1024 x 8192 0.99, 1536 x 4096 1.00, 2048 x 6144 0.98-1.00
-        if (t > 128 && t <= 512) {
+        if (NVX_ENTRY(nvx_prefill_heads_ride)(t, qw, hid)) {      // a head's norm and rotation at the end of the product (sizes and figures there)
             const NvxQkvOut out = {s->positions, s->slots, s->rope, s->rope_rows, s->n_slots, (const uint16_t*)w[2], (const uint16_t*)w[3], (uint16_t*)s->q,
                                    (uint16_t*)w[8], (uint16_t*)w[9], (int)s->hq, (int)s->hkv, eps};
             NVX_STEP(NVX_ENTRY(nvx_prefill_gemm)(s->h, hid, (const void*)w[1], nullptr, t, qw, hid, NVX_PG_QKV, &out, st));

@@ -23,9 +23,7 @@ __device__ __forceinline__ HalfQuad load_half_quads(const uint16_t* row, int l16
 }
 
 // Eager bf16 arithmetic: cos/sin rounded to bf16, every product and sum rounded to bf16.
-__device__ __forceinline__ uint4 rotate_interleave(const HalfQuad& x, const float* cs_row, int l16) {
-    const float4 c4 = *reinterpret_cast<const float4*>(cs_row + 4 * l16);
-    const float4 s4 = *reinterpret_cast<const float4*>(cs_row + 64 + 4 * l16);
+__device__ __forceinline__ uint4 rotate_interleave(const HalfQuad& x, const float4& c4, const float4& s4) {
     const float c[4] = {round_h16(c4.x), round_h16(c4.y), round_h16(c4.z), round_h16(c4.w)};
     const float s[4] = {round_h16(s4.x), round_h16(s4.y), round_h16(s4.z), round_h16(s4.w)};
     uint32_t o[4];
@@ -37,6 +35,9 @@ __device__ __forceinline__ uint4 rotate_interleave(const HalfQuad& x, const floa
     }
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
+__device__ __forceinline__ uint4 rotate_interleave(const HalfQuad& x, const float* cs_row, int l16) {
+    return rotate_interleave(x, *reinterpret_cast<const float4*>(cs_row + 4 * l16), *reinterpret_cast<const float4*>(cs_row + 64 + 4 * l16));
+}
 
 __device__ __forceinline__ int64_t clamp_pos(int64_t p, int64_t max_pos) {
     return p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
@@ -45,9 +46,9 @@ __device__ __forceinline__ int64_t clamp_pos(int64_t p, int64_t max_pos) {
 
 // RMSNorm over the 128 elements of a head (ss = their sum of squares, already reduced over the 16
 // lanes), rounded to bf16 as the unfused norm hands it to the rotary op, then rotated and interleaved.
-// (wa, wb: the norm's weights of the lane's elements)
+// (wa, wb: the norm's weights of the lane's elements; c4, s4: their cosines and sines)
 __device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float ss, const uint2& wa, const uint2& wb, float eps,
-                                                        const float* cs_row, int l16) {
+                                                        const float4& c4, const float4& s4) {
     const float wA[4] = {h16lo_to_f32(wa.x), h16hi_to_f32(wa.x), h16lo_to_f32(wa.y), h16hi_to_f32(wa.y)};
     const float wB[4] = {h16lo_to_f32(wb.x), h16hi_to_f32(wb.x), h16lo_to_f32(wb.y), h16hi_to_f32(wb.y)};
     const float inv = 1.0f / sqrtf(ss / 128.0f + eps);
@@ -57,7 +58,11 @@ __device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float
         n.a[j] = round_h16((x.a[j] * inv) * wA[j]);
         n.b[j] = round_h16((x.b[j] * inv) * wB[j]);
     }
-    return rotate_interleave(n, cs_row, l16);
+    return rotate_interleave(n, c4, s4);
+}
+__device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float ss, const uint2& wa, const uint2& wb, float eps,
+                                                        const float* cs_row, int l16) {
+    return norm_rotate_interleave(x, ss, wa, wb, eps, *reinterpret_cast<const float4*>(cs_row + 4 * l16), *reinterpret_cast<const float4*>(cs_row + 64 + 4 * l16));
 }
 __device__ __forceinline__ uint4 norm_rotate_interleave(const HalfQuad& x, float ss, const uint16_t* __restrict__ w, float eps,
                                                         const float* cs_row, int l16) {
