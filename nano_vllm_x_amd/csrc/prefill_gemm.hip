@@ -8,8 +8,8 @@
 // it multiplies), which splitting K over the waves would halve; but K is never split: a row's sum runs over K in order, in one chain of
 // v_mfma_f32_16x16x32, whatever the tile, so that a token's result does not depend on how many tokens share its step (and equals the library's
 // above some 200 rows, whose products take K in the same order).
-// The products of a layer of Qwen3-0.6B with weights that no cache holds, us, qkv / o / gate | up / down: 100 rows 5.4 / 5.7 / 7.8 / 7.1, 200 rows 6.4 / 5.8 / 10.4 / 7.5,
-//     459 rows 8.9 / 7.5 / 12.4 / 9.8, 1500 rows 18.8 / 11.7 / 28.7 / 16.4 (the library with weights in its caches: 64 rows 8.8 / 8.4 / 9.0 and SiluAndMul's 4 / 10.1, 459 rows
+// The products of a layer of Qwen3-0.6B with weights that no cache holds, us, qkv / o / gate | up / down: 100 rows 5.2 / 6.0 / 7.3 / 8.1, 200 rows 6.5 / 6.1 / 9.4 / 8.2,
+//     459 rows 8.5 / 8.0 / 12.2 / 11.0, 1500 rows 17.2 / 12.1 / 28.7 / 17.6 (the library with weights in its caches: 64 rows 8.8 / 8.4 / 9.0 and SiluAndMul's 4 / 10.1, 459 rows
 //     11.2 / 9.7 / 13.6 and 4 / 12.5, 1536 rows 17.7 / 13.7 / 28.9 and 4 / 17.1).
 #include "prefill_gemm.h"
 
@@ -240,41 +240,44 @@ static void launch_prefill_gemm(const void* x, int64_t x_stride, const void* w, 
 using namespace NVX_NS;
 
 // What a tile costs, us, with weights that no cache holds: us + k / 1024 * (us_k + (rounds - 1) * round + (workgroups / 256 - 1) * over), rounds of 256 workgroups and the last term from
-// the 257th on (us_k 0: not built).  Fitted to 40 to 4096 rows of 1024 to 4096 outputs of 512 to 6144 columns, 1 900 products: over these the tile it picks costs 0.6 % more than the best one
-// (17 % at worst), where the table for 1024 columns that was here before cost 4.8 % (39 %).  A step of a few KB is as long as its copies' way into a CU, its reads from LDS and two barriers'
-// skew, hardly any of which hides any other at one workgroup a CU, so the tile that just fills the CUs is the best; us a product before, with the copies of a step asked for at
-// once, and now: 2160 rows 1024 x 2048 18.9 (128 x 128) and 15.1 (160 x 64), 1024 x 3072 29.2 (128 x 128) and 21.1 (160 x 64); 1900 rows 16.0 and 13.2, 24.7 and 20.6 (128 x 64); 459 rows 7.9 and
-// 7.6, 11.1 and 10.9 (32 x 64), 4096 x 1024 10.4 (64 x 128) and 8.6 (128 x 64).  A deeper ring (all of LDS) was no faster; nor were rows of w a multiple of 128 bytes and 64 apart.
+// the 257th on (us_k 0: not built, or never the least: SiluAndMul by 128 x 256).  Fitted to 40 to 4000 rows of 1024 to 12288 outputs of 512 to 3072 columns, 6 200 times of 383 products: over these the tile it picks
+// costs 0.3 % more than the best one (8 % at worst), SiluAndMul's 0.6 % (11 %).  A step of a few KB is as long as its copies' way into a CU, its reads from LDS and two barriers'
+// skew, hardly any of which hides any other at one workgroup a CU, so the tile that just fills the CUs is the best, and there is one for most sizes: without the tiles of 96 to 224 x 128, and with
+// two and three steps of 64 x 128 in LDS, the choice was 6 % and 8 % off.  us a product without and with them: SiluAndMul's 6144 x 1024, 256 rows 11.1 and 10.2 (64 x 128), 768 22.5 and 16.0 (160 x 128), 900 21.6 and 17.9, 1024 22.7 and 19.1;
+// 4096 x 1024, 1280 rows 20.5 and 15.6, 1536 24.4 and 17.5; 2048 x 2048, 3072 rows 38.0 and 27.8; 6144 x 2560, 768 rows 44.7 and 32.3.  256 x 128 needs more registers than there are.  A deeper
+// ring (all of LDS) was no faster; nor were rows of w a multiple of 128 bytes and 64 apart.
 struct PrefillCost { float us, us_k, round, over; };
 struct PrefillTile { int tile, m, n; PrefillCost plain, silu; bool wide; };
 static const PrefillTile PREFILL_TILES[] = {
-    {NVX_PG_32_32, 32, 32, {1.9f, 2.1f, 1.f, .5f}, {}, false},
-    {NVX_PG_32_64, 32, 64, {2.4f, 2.8f, 2.5f, .6f}, {2.7f, 3.1f, 5.f, -.6f}, false},
-    {NVX_PG_64_64, 64, 64, {1.7f, 4.3f, 2.f, 1.3f}, {1.5f, 6.f, 3.f, .8f}, false},
-    {NVX_PG_96_64, 96, 64, {2.2f, 4.7f, 2.8f, 1.6f}, {}, false},
-    {NVX_PG_128_64, 128, 64, {2.7f, 5.3f, 5.4f, 1.5f}, {}, false},
-    {NVX_PG_160_64, 160, 64, {3.f, 6.1f, 6.3f, 1.7f}, {}, false},
-    {NVX_PG_192_64, 192, 64, {3.4f, 6.8f, 7.5f, 2.f}, {}, false},
-    {NVX_PG_64_128, 64, 128, {1.4f, 6.8f, 2.1f, 3.4f}, {.2f, 14.3f, 1.f, 5.3f}, false},
-    {NVX_PG_128_128, 128, 128, {3.1f, 7.7f, 7.3f, 2.9f}, {4.2f, 8.3f, 10.f, -.2f}, true},
-    {NVX_PG_128_256, 128, 256, {-1.4f, 19.1f, 16.9f, 8.1f}, {1.4f, 22.4f, 16.4f, 1.f}, true},
-    {NVX_PG_192_256, 192, 256, {.1f, 20.1f, 21.6f, 1.2f}, {3.8f, 22.9f, 19.1f, 3.1f}, true},
-    {NVX_PG_256_256, 256, 256, {2.4f, 21.8f, 12.f, 10.f}, {5.8f, 25.f, 22.9f, 4.7f}, true}};
+    {NVX_PG_32_32, 32, 32, {2.1f, 2.05f, 1.2f, .4f}, {}, false},
+    {NVX_PG_32_64, 32, 64, {2.3f, 2.9f, 2.35f, 1.1f}, {1.8f, 4.2f, 4.4f, -.7f}, false},
+    {NVX_PG_64_64, 64, 64, {2.2f, 4.2f, 2.f, 1.45f}, {2.3f, 4.2f, 2.95f, 1.f}, false},
+    {NVX_PG_96_64, 96, 64, {2.7f, 4.7f, 2.8f, 1.75f}, {}, false},
+    {NVX_PG_128_64, 128, 64, {3.1f, 5.2f, 5.5f, 1.5f}, {}, false},
+    {NVX_PG_160_64, 160, 64, {3.5f, 6.1f, 6.f, 2.6f}, {}, false},
+    {NVX_PG_192_64, 192, 64, {3.8f, 7.f, 7.1f, 2.4f}, {}, false},
+    {NVX_PG_64_128, 64, 128, {2.8f, 6.f, 5.55f, 1.3f}, {2.9f, 6.7f, 8.9f, -1.8f}, false},
+    {NVX_PG_96_128, 96, 128, {3.6f, 7.25f, 6.6f, 2.3f}, {4.f, 7.6f, 9.2f, 0.f}, false},
+    {NVX_PG_128_128, 128, 128, {4.f, 7.7f, 6.65f, 2.3f}, {4.7f, 7.6f, 9.f, .5f}, true},
+    {NVX_PG_160_128, 160, 128, {5.f, 9.4f, 10.3f, 1.9f}, {5.1f, 10.4f, 11.9f, 1.1f}, false},
+    {NVX_PG_192_128, 192, 128, {5.3f, 10.9f, 10.75f, 3.3f}, {6.1f, 11.1f, 12.2f, 3.3f}, false},
+    {NVX_PG_224_128, 224, 128, {5.35f, 11.9f, 11.15f, 6.8f}, {6.5f, 12.f, 14.7f, 2.6f}, false},
+    {NVX_PG_128_256, 128, 256, {.7f, 21.4f, 13.6f, 3.7f}, {}, true},
+    {NVX_PG_192_256, 192, 256, {1.7f, 23.2f, 14.3f, 8.6f}, {5.9f, 22.5f, 16.4f, 7.2f}, true},
+    {NVX_PG_256_256, 256, 256, {4.9f, 23.8f, 12.f, 10.f}, {8.3f, 24.f, 23.2f, 4.f}, true}};
 
-// QKV, a tile as wide as a head: us + k / 1024 * (us_k + (rounds - 1) * round), less what the launch costs that norms and turns the heads behind a plain product (the two grow alike with
-// the rows).  Fitted to steps of 20 to 3000 tokens of layers of 512 to 2560: with one round of workgroups these costs, held against the plain tiles', were right wherever the two ways differ by more than
+// QKV, a tile as wide as a head, in one round of workgroups: us + k / 1024 * us_k, less what the launch costs that norms and turns the heads behind a plain product (the two grow alike with
+// the rows).  Fitted to steps of 20 to 1024 tokens of layers of 512 to 2560: these costs, held against the plain tiles', were right wherever the two ways differ by more than
 // 1 us a layer.  us a layer of 1024 columns and 32 heads, plain and launch / here: 130 tokens 55.9 / 54.5, 256 61.3 / 59.8 (32 rows), 300 66.1 / 65.2, 459 73.4 / 71.3 (64 rows), 768 98.2 / 94.0 (96), 900
-// 98.5 / 96.8 (128); two rounds of 96 rows, 1500 129.2 / 123.8, but 1152 (384 workgroups of the 512) 110.8 / 112.8: two rounds must be 13/16 full.  2048 columns: 300 115.0 / 116.2, not taken, 400 117.3 / 116.0.
-// Two workgroups a CU or more rounds were never the better way, nor steps of 128 columns.  A 256 x 256 tile's heads take 15 us, in which its CU multiplies nothing.
-struct HeadsTile { int tile, m; float us, us_k, round; };
-static const HeadsTile HEADS_TILES[] = {
-    {NVX_PG_32_128, 32, -.9f, 5.3f, 0.f}, {NVX_PG_64_128, 64, -.3f, 6.3f, 0.f}, {NVX_PG_96_128, 96, .5f, 6.4f, 7.6f}, {NVX_PG_HEADS_128_128, 128, 1.5f, 7.7f, 0.f}};
+// 98.5 / 96.8 (128), 64 49.6 / 50.8, not taken; 2048 columns: 300 115.0 / 116.2, not taken, 400 117.3 / 116.0.  In two rounds the plain tiles lead (96 rows at 1500 tokens by some 1 us).
+// Two workgroups a CU were never the better way, nor steps of 128 columns.  A 256 x 256 tile's heads take 15 us, in which its CU multiplies nothing.
+struct HeadsTile { int tile, m; float us, us_k; };
+static const HeadsTile HEADS_TILES[] = {{NVX_PG_32_128, 32, -.4f, 5.3f}, {NVX_PG_64_128, 64, .1f, 6.3f}, {NVX_PG_96_128, 96, .9f, 6.4f}, {NVX_PG_HEADS_128_128, 128, 2.4f, 7.7f}};
 static int heads_tile(int64_t m, int64_t n, int64_t k, float& cost) {
     int best = 0;
     for (const HeadsTile& t : HEADS_TILES) {
-        const int64_t workgroups = (m + t.m - 1) / t.m * (n / 128);
-        if (workgroups > 256 && (t.round == 0.f || workgroups > 512 || workgroups < 416)) continue;
-        const float c = t.us + (float)k / 1024.f * (t.us_k + (workgroups > 256 ? t.round : 0.f));
+        if ((m + t.m - 1) / t.m * (n / 128) > 256) continue;
+        const float c = t.us + (float)k / 1024.f * t.us_k;
         if (!best || c < cost) best = t.tile, cost = c;
     }
     return best;
@@ -325,7 +328,11 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
         case NVX_PG_HEADS_128_128: NVX_PG(128, 128, 64, 4, NVX_PG_QKV); break;
         default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);
     } else switch (tile) {
-        case NVX_PG_64_128: if (silu) NVX_PG(64, 128, 64, 2, NVX_PG_SILU); else NVX_PG(64, 128, 64, 3, NVX_PG_PLAIN); break;
+        case NVX_PG_64_128: if (silu) NVX_PG(64, 128, 64, 4, NVX_PG_SILU); else NVX_PG(64, 128, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_96_128: if (silu) NVX_PG(96, 128, 64, 4, NVX_PG_SILU); else NVX_PG(96, 128, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_160_128: if (silu) NVX_PG(160, 128, 64, 4, NVX_PG_SILU); else NVX_PG(160, 128, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_192_128: if (silu) NVX_PG(192, 128, 64, 4, NVX_PG_SILU); else NVX_PG(192, 128, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_224_128: if (silu) NVX_PG(224, 128, 64, 3, NVX_PG_SILU); else NVX_PG(224, 128, 64, 3, NVX_PG_PLAIN); break;
         case NVX_PG_64_64: if (silu) NVX_PG(64, 64, 64, 4, NVX_PG_SILU); else NVX_PG(64, 64, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_32_64: if (silu) NVX_PG(32, 64, 128, 4, NVX_PG_SILU); else NVX_PG(32, 64, 128, 4, NVX_PG_PLAIN); break;
         case NVX_PG_96_64: NVX_REQUIRE(!silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(96, 64, 64, 4, NVX_PG_PLAIN); break;

@@ -42,3 +42,26 @@ def test_tall_tiles_and_few_steps(dtype, m, n, k):
     for tile in (9, 11, 12, 13):      # no SiluAndMul in these
         with pytest.raises(RuntimeError):
             _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 1, tile, ops._stream()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 256), (63, 256, 512), (65, 128, 768), (95, 128, 1024), (97, 256, 256), (159, 128, 1280), (161, 256, 512), (193, 384, 256), (223, 128, 512),
+                                   (225, 128, 256), (449, 1024, 1024), (768, 6144, 1024), (1024, 6144, 256)])
+def test_tiles_as_wide_as_128(dtype, m, n, k):
+    """Tiles of 64, 96, 160, 192 and 224 x 128, plain and with SiluAndMul: the bits of 64 x 64, no row past the last written."""
+    from nano_vllm_x_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 64, generator=gen, device="cuda").to(dtype)[:, 32:32 + k]
+    w = (torch.randn(n, k, generator=gen, device="cuda") * k ** -0.5).to(dtype)
+    fn = getattr(_lib.load(), "nvx_internal_prefill_gemm" + ("_f16" if dtype == torch.float16 else ""))
+    for silu in (0, 1):
+        first = None
+        for tile in (6, 5, 14, 16, 17, 18, 0):
+            y = torch.full((m + 230, n // (1 + silu)), float("nan"), dtype=dtype, device="cuda")
+            _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, silu, tile, ops._stream()))
+            first = y[:m] if first is None else first
+            assert bool(torch.isfinite(y[:m]).all()) and bool(torch.isnan(y[m:]).all()) and torch.equal(y[:m], first), (silu, tile)
+        for tile in (10, 15, 19):      # heads' tiles and none
+            with pytest.raises(RuntimeError):
+                _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, silu, tile, ops._stream()))
