@@ -820,7 +820,8 @@ extern "C" int NVX_ENTRY(nvx_paged_prefill)(const void* q, int64_t q_row_stride,
     // and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 459 tokens 12.0 and 13.1, 1500 29.0 and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
     // Before a turn made the next tile's scores: 459 tokens 12.1, 1024 21.8, 64 queries of 3072 keys 54.3 (now 43.4: 0.79 us a tile, of 0.43 the matrix pipe needs).
     const auto groups = [&](int64_t positions) { return ((n_tokens + positions - 1) / positions + batch - 1) * n_kv_heads; };
-    // two rounds of a workgroup a CU, unless most blocks of a round and a half may be short ones
+    // two rounds of a workgroup a CU, unless most blocks of a round and a half may be short ones.  us a step with the limit at 392 and at 512 workgroups: prompts of 0.3 to 1.7 of their mean length, 2948
+    // tokens (408) 4903 and 4814, 3187 (424) 5259 and 5168, 3727 (512) 5313 and 5296; prompts of one length, which the host does not look for, 3200 tokens (432) 5061 and 5096, 3600 (496) 5075 and 5153.
     const auto few = [&](int64_t workgroups) { return workgroups <= (n_tokens >= 128 * batch ? 512 : 392); };
     switch (g) {
         case 1: NVX_PF(1, 4, 128, 0); break;
