@@ -14,8 +14,8 @@ struct NvxQkvOut {
     float eps;
 };
 enum { NVX_PG_PLAIN = 0, NVX_PG_SILU = 1, NVX_PG_QKV = 2 };
-// tiles; 96_64, 128_64, 160_64, 192_64 and 32_32: not SILU; 32_128 and HEADS_128_128: QKV only
-enum { NVX_PG_256_256 = 1, NVX_PG_192_256, NVX_PG_128_256, NVX_PG_128_128, NVX_PG_64_128, NVX_PG_64_64, NVX_PG_96_64, NVX_PG_32_64, NVX_PG_32_32, NVX_PG_32_128, NVX_PG_128_64, NVX_PG_160_64, NVX_PG_192_64, NVX_PG_96_128, NVX_PG_HEADS_128_128, NVX_PG_160_128, NVX_PG_192_128, NVX_PG_224_128 };
+// tiles; 96_64, 128_64, 160_64, 192_64 and 32_32: not SILU; 32_128 and HEADS_128_128: QKV only; 64_128_THREE (of which a CU has three): SILU only
+enum { NVX_PG_256_256 = 1, NVX_PG_192_256, NVX_PG_128_256, NVX_PG_128_128, NVX_PG_64_128, NVX_PG_64_64, NVX_PG_96_64, NVX_PG_32_64, NVX_PG_32_32, NVX_PG_32_128, NVX_PG_128_64, NVX_PG_160_64, NVX_PG_192_64, NVX_PG_96_128, NVX_PG_HEADS_128_128, NVX_PG_160_128, NVX_PG_192_128, NVX_PG_224_128, NVX_PG_64_128_THREE = 20 };
 
 // mode PLAIN: y (m, n) = x (m, k) w (n, k)^T; SILU: y (m, n / 2) = SiluAndMul of it; QKV: the rows of `qkv`, y unused.  In the 16-bit format; rows of x
 // `x_stride` elements apart

@@ -34,7 +34,7 @@ __device__ __forceinline__ void wait_for_all_but() { asm volatile("s_waitcnt vmc
 // TM rows of x by TN rows of w a workgroup of four waves (WM of them along the rows of x), KS columns a step.  With SILU the TN rows of w are 16
 // gate and 16 up rows in turn, and the tile gives TN / 2 outputs; with QKV a tile is one head.  m: rows of x; k % (2 * KS) == 0, n (rows of w) % TN == 0.
 template <int TM, int TN, int KS, int STAGES, int WM, int MODE>
-__global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w,
+__global__ __launch_bounds__(256, STAGES == 2 ? 3 : 1) void prefill_gemm_kernel(const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w,
                                                           uint16_t* __restrict__ y, int m, int n, int k, const NvxQkvOut qkv) {
     constexpr bool SILU = MODE == NVX_PG_SILU;
     constexpr int WN = 4 / WM, FM = TM / WM / 16, FN = TN / WN / 16;       // fragments of a wave
@@ -155,7 +155,31 @@ __global__ __launch_bounds__(256) void prefill_gemm_kernel(const uint16_t* __res
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < READS; ++q) read(q, 0, even);
-    if (steps < STAGES) {                                                           // (k / KS is even)
+    if constexpr (STAGES == 2) {
+        // Three workgroups a CU, of which each multiplies while the others wait: all copies and reads of a step at once.  Dealt out they take 204 registers, and a SIMD with three waves has 168 for each.
+        auto plain_turn = [&](int s, const Operands& now, Operands& next) __attribute__((always_inline)) {
+            wait_for_all_but<0>();
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+            __syncthreads();                                                        // step s + 1 has landed, and everybody has read step s
+            if (s + 2 < steps) {
+#pragma unroll
+                for (int i = 0; i < LOADS; ++i) ask(i, slot);
+            }
+            slot ^= STAGE;
+#pragma unroll
+            for (int q = 0; q < READS; ++q) read(q, slot, next);                    // (behind the last step whatever lies there: not used)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < MULS; ++u) {
+                const int kk = u / (FM * FN), i = u / FM % FN, j = u % FM;
+                acc[i][j] = mfma_16x16x32_h16(now.w[kk][i], now.x[kk][j], acc[i][j]);
+            }
+        };
+        for (int s = 0; s < steps; s += 2) {                                        // (k / KS is even)
+            plain_turn(s, even, odd);
+            plain_turn(s + 1, odd, even);
+        }
+    } else if (steps < STAGES) {                                                    // (k / KS is even)
         foresee();
         std::integral_constant<int, 0> none;
         for (int s = 0; s + 2 < steps; s += 2) {
@@ -239,32 +263,36 @@ static void launch_prefill_gemm(const void* x, int64_t x_stride, const void* w, 
 
 using namespace NVX_NS;
 
-// What a tile costs, us, with weights that no cache holds: us + k / 1024 * (us_k + (rounds - 1) * round + (workgroups / 256 - 1) * over), rounds of 256 workgroups and the last term from
-// the 257th on (us_k 0: not built, or never the least: SiluAndMul by 128 x 256).  Fitted to 40 to 4000 rows of 1024 to 12288 outputs of 512 to 3072 columns, 6 200 times of 383 products: over these the tile it picks
-// costs 0.3 % more than the best one (8 % at worst), SiluAndMul's 0.6 % (11 %).  A step of a few KB is as long as its copies' way into a CU, its reads from LDS and two barriers'
+// What a tile costs, us, with weights that no cache holds: us + (rounds - 1) * again + k / 1024 * (us_k + (rounds - 1) * round + (workgroups / 256 - 1) * over), rounds of 256 workgroups and the last
+// term from the 257th on (us_k 0: not built).  Plain: fitted to 40 to 4000 rows of 1024 to 12288 outputs of 512 to 3072 columns, with `again` 0; of 813 products of 30 to 8000 rows of 256 to 8192 columns
+// the tile it picks costs 0.7 % more than the best one (the tiles and costs before 7 %).  SiluAndMul: fitted to 868 products of 30 to 8000 rows, 256 to 2048 columns, over which its choice is 0.4 % off the best; without `again`, what
+// a round costs however few its columns are (results, SiluAndMul, first copies), narrow layers got tiles 5 to 45 % off.  A step of a few KB is as long as its copies' way into a CU, its reads from LDS and two barriers'
 // skew, hardly any of which hides any other at one workgroup a CU, so the tile that just fills the CUs is the best, and there is one for most sizes: without the tiles of 96 to 224 x 128, and with
-// two and three steps of 64 x 128 in LDS, the choice was 6 % and 8 % off.  us a product without and with them: SiluAndMul's 6144 x 1024, 256 rows 11.1 and 10.2 (64 x 128), 768 22.5 and 16.0 (160 x 128), 900 21.6 and 17.9, 1024 22.7 and 19.1;
-// 4096 x 1024, 1280 rows 20.5 and 15.6, 1536 24.4 and 17.5; 2048 x 2048, 3072 rows 38.0 and 27.8; 6144 x 2560, 768 rows 44.7 and 32.3.  256 x 128 needs more registers than there are.  A deeper
+// two and three steps of 64 x 128 in LDS, the choice was 6 % and 8 % off.  us a product without and with them: SiluAndMul's 6144 x 1024, 256 rows 11.7 and 10.4 (64 x 128), 768 20.2 and 16.5 (160 x 128), 900 20.7 and 18.3, 1024 21.9 and 19.2;
+// 4096 x 1024, 1200 rows 23.0 and 15.7, 1500 23.9 and 17.6; 2048 x 2048, 3072 rows 42.7 and 27.9; 12288 x 2048, 300 rows 35.6 and 26.9.  256 x 128 needs more registers than there are.  A deeper
 // ring (all of LDS) was no faster; nor were rows of w a multiple of 128 bytes and 64 apart.
-struct PrefillCost { float us, us_k, round, over; };
+// 64_128_THREE: three workgroups a CU, where all of them run at once (768; `again` and `round` for every 256 past the first), which is the best for narrow layers: SiluAndMul's 1536 x 256, 4096 rows 8.1 and by the best
+// of the others 9.6; 3072 x 256, 1836 rows 8.0 and 9.0; 3072 x 512, 2048 rows 12.3 and 12.9; 1024 x 512, 5300 rows 11.0 and 11.5.
+struct PrefillCost { float us, again, us_k, round, over; };
 struct PrefillTile { int tile, m, n; PrefillCost plain, silu; bool wide; };
 static const PrefillTile PREFILL_TILES[] = {
-    {NVX_PG_32_32, 32, 32, {2.1f, 2.05f, 1.2f, .4f}, {}, false},
-    {NVX_PG_32_64, 32, 64, {2.3f, 2.9f, 2.35f, 1.1f}, {1.8f, 4.2f, 4.4f, -.7f}, false},
-    {NVX_PG_64_64, 64, 64, {2.2f, 4.2f, 2.f, 1.45f}, {2.3f, 4.2f, 2.95f, 1.f}, false},
-    {NVX_PG_96_64, 96, 64, {2.7f, 4.7f, 2.8f, 1.75f}, {}, false},
-    {NVX_PG_128_64, 128, 64, {3.1f, 5.2f, 5.5f, 1.5f}, {}, false},
-    {NVX_PG_160_64, 160, 64, {3.5f, 6.1f, 6.f, 2.6f}, {}, false},
-    {NVX_PG_192_64, 192, 64, {3.8f, 7.f, 7.1f, 2.4f}, {}, false},
-    {NVX_PG_64_128, 64, 128, {2.8f, 6.f, 5.55f, 1.3f}, {2.9f, 6.7f, 8.9f, -1.8f}, false},
-    {NVX_PG_96_128, 96, 128, {3.6f, 7.25f, 6.6f, 2.3f}, {4.f, 7.6f, 9.2f, 0.f}, false},
-    {NVX_PG_128_128, 128, 128, {4.f, 7.7f, 6.65f, 2.3f}, {4.7f, 7.6f, 9.f, .5f}, true},
-    {NVX_PG_160_128, 160, 128, {5.f, 9.4f, 10.3f, 1.9f}, {5.1f, 10.4f, 11.9f, 1.1f}, false},
-    {NVX_PG_192_128, 192, 128, {5.3f, 10.9f, 10.75f, 3.3f}, {6.1f, 11.1f, 12.2f, 3.3f}, false},
-    {NVX_PG_224_128, 224, 128, {5.35f, 11.9f, 11.15f, 6.8f}, {6.5f, 12.f, 14.7f, 2.6f}, false},
-    {NVX_PG_128_256, 128, 256, {.7f, 21.4f, 13.6f, 3.7f}, {}, true},
-    {NVX_PG_192_256, 192, 256, {1.7f, 23.2f, 14.3f, 8.6f}, {5.9f, 22.5f, 16.4f, 7.2f}, true},
-    {NVX_PG_256_256, 256, 256, {4.9f, 23.8f, 12.f, 10.f}, {8.3f, 24.f, 23.2f, 4.f}, true}};
+    {NVX_PG_32_32, 32, 32, {2.1f, 0.f, 2.05f, 1.2f, .4f}, {}, false},
+    {NVX_PG_32_64, 32, 64, {2.3f, 0.f, 2.9f, 2.35f, 1.1f}, {2.4f, 1.4f, 3.5f, 2.6f, .4f}, false},
+    {NVX_PG_64_64, 64, 64, {2.2f, 0.f, 4.2f, 2.f, 1.45f}, {2.1f, .4f, 5.25f, 2.f, 1.4f}, false},
+    {NVX_PG_96_64, 96, 64, {2.7f, 0.f, 4.7f, 2.8f, 1.75f}, {}, false},
+    {NVX_PG_128_64, 128, 64, {3.1f, 0.f, 5.2f, 5.5f, 1.5f}, {}, false},
+    {NVX_PG_160_64, 160, 64, {3.5f, 0.f, 6.1f, 6.f, 2.6f}, {}, false},
+    {NVX_PG_192_64, 192, 64, {3.8f, 0.f, 7.f, 7.1f, 2.4f}, {}, false},
+    {NVX_PG_64_128, 64, 128, {2.8f, 0.f, 6.f, 5.55f, 1.3f}, {2.9f, 2.35f, 7.35f, 4.4f, .65f}, false},
+    {NVX_PG_64_128_THREE, 64, 128, {}, {2.4f, .8f, 11.6f, 2.5f, 0.f}, false},
+    {NVX_PG_96_128, 96, 128, {3.6f, 0.f, 7.25f, 6.6f, 2.3f}, {3.9f, 3.05f, 7.7f, 5.4f, 1.4f}, false},
+    {NVX_PG_128_128, 128, 128, {4.f, 0.f, 7.7f, 6.65f, 2.3f}, {4.5f, 2.2f, 8.4f, 6.2f, 1.3f}, true},
+    {NVX_PG_160_128, 160, 128, {5.f, 0.f, 9.4f, 10.3f, 1.9f}, {5.3f, 4.f, 10.2f, 7.7f, 3.f}, false},
+    {NVX_PG_192_128, 192, 128, {5.3f, 0.f, 10.9f, 10.75f, 3.3f}, {5.8f, 5.9f, 11.4f, 5.3f, 4.2f}, false},
+    {NVX_PG_224_128, 224, 128, {5.35f, 0.f, 11.9f, 11.15f, 6.8f}, {6.3f, 5.7f, 12.3f, 7.9f, 3.f}, false},
+    {NVX_PG_128_256, 128, 256, {.7f, 0.f, 21.4f, 13.6f, 3.7f}, {4.3f, 3.9f, 21.1f, 10.6f, 3.5f}, true},
+    {NVX_PG_192_256, 192, 256, {1.7f, 0.f, 23.2f, 14.3f, 8.6f}, {6.6f, 5.9f, 22.f, 11.5f, 6.2f}, true},
+    {NVX_PG_256_256, 256, 256, {4.9f, 0.f, 23.8f, 12.f, 10.f}, {9.2f, 7.f, 23.35f, 15.8f, 5.3f}, true}};
 
 // QKV, a tile as wide as a head, in one round of workgroups: us + k / 1024 * us_k, less what the launch costs that norms and turns the heads behind a plain product (the two grow alike with
 // the rows).  Fitted to steps of 20 to 1024 tokens of layers of 512 to 2560: these costs, held against the plain tiles', were right wherever the two ways differ by more than
@@ -290,8 +318,10 @@ static int prefill_gemm_rule(int64_t m, int64_t n, int64_t k, bool silu, bool wi
     for (const PrefillTile& t : PREFILL_TILES) {
         const PrefillCost& c = silu ? t.silu : t.plain;
         if (c.us_k == 0.f || n % t.n || (t.wide && !wide)) continue;
-        const int64_t workgroups = (m + t.m - 1) / t.m * (n / t.n), rounds = (workgroups + 255) / 256;
-        const float cost = c.us + (float)k / 1024.f * (c.us_k + (float)(rounds - 1) * c.round + (workgroups > 256 ? (float)workgroups / 256.f - 1.f : 0.f) * c.over);
+        const int64_t workgroups = (m + t.m - 1) / t.m * (n / t.n);
+        if (t.tile == NVX_PG_64_128_THREE && workgroups > 768) continue;
+        const float past = workgroups > 256 ? (float)workgroups / 256.f - 1.f : 0.f, rounds = t.tile == NVX_PG_64_128_THREE ? past : (float)((workgroups + 255) / 256 - 1);      // past the first
+        const float cost = c.us + rounds * c.again + (float)k / 1024.f * (c.us_k + rounds * c.round + past * c.over);
         if (least == 0.f || cost < least) best = t.tile, least = cost;
     }
     return best;
@@ -329,6 +359,7 @@ static int prefill_gemm(int tile, const void* x, int64_t x_stride, const void* w
         default: return nvx_fail(NVX_EUNSUPPORTED, "nvx_prefill_gemm: no tile %d", tile);
     } else switch (tile) {
         case NVX_PG_64_128: if (silu) NVX_PG(64, 128, 64, 4, NVX_PG_SILU); else NVX_PG(64, 128, 64, 4, NVX_PG_PLAIN); break;
+        case NVX_PG_64_128_THREE: NVX_REQUIRE(silu, NVX_EUNSUPPORTED, "nvx_prefill_gemm: tile"); NVX_PG(64, 128, 64, 2, NVX_PG_SILU); break;
         case NVX_PG_96_128: if (silu) NVX_PG(96, 128, 64, 4, NVX_PG_SILU); else NVX_PG(96, 128, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_160_128: if (silu) NVX_PG(160, 128, 64, 4, NVX_PG_SILU); else NVX_PG(160, 128, 64, 4, NVX_PG_PLAIN); break;
         case NVX_PG_192_128: if (silu) NVX_PG(192, 128, 64, 4, NVX_PG_SILU); else NVX_PG(192, 128, 64, 4, NVX_PG_PLAIN); break;
@@ -352,6 +383,11 @@ int NVX_ENTRY(nvx_prefill_gemm)(const void* x, int64_t x_stride, const void* w, 
 extern "C" int NVX_ENTRY(nvx_internal_prefill_gemm)(const void* x, int64_t x_stride, const void* w, void* y, int64_t m, int64_t n, int64_t k, int silu, int tile,
                                                     nvx_stream_t stream) {
     return prefill_gemm(tile, x, x_stride, w, y, m, n, k, silu ? NVX_PG_SILU : NVX_PG_PLAIN, nullptr, (hipStream_t)stream);
+}
+// the rule's tile
+extern "C" int NVX_ENTRY(nvx_internal_prefill_tile)(int64_t m, int64_t n, int64_t k, int silu) {
+    float cost;
+    return prefill_gemm_rule(m, n, k, silu, n * k < (1ll << 30), cost);
 }
 // what becomes of one [q | k | v] projection, by a tile of the caller's choice (0: the rule's)
 extern "C" int NVX_ENTRY(nvx_internal_prefill_heads)(const void* x, int64_t x_stride, const void* w, int64_t m, int64_t k, int tile, const int64_t* positions, const int64_t* slots,

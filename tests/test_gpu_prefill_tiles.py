@@ -65,3 +65,23 @@ def test_tiles_as_wide_as_128(dtype, m, n, k):
         for tile in (10, 15, 19):      # heads' tiles and none
             with pytest.raises(RuntimeError):
                 _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, silu, tile, ops._stream()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 256), (63, 256, 512), (64, 128, 768), (65, 384, 1024), (129, 256, 1280), (1030, 6144, 256), (4096, 1536, 256), (2049, 3072, 512)])
+def test_three_workgroups_a_cu(dtype, m, n, k):
+    """SiluAndMul by 64 x 128 with two steps in LDS, and by the rule's tile: the bits of 64 x 64, no row past the last written; no plain product in it."""
+    from nano_vllm_x_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 64, generator=gen, device="cuda").to(dtype)[:, 32:32 + k]
+    w = (torch.randn(n, k, generator=gen, device="cuda") * k ** -0.5).to(dtype)
+    fn, first = getattr(_lib.load(), "nvx_internal_prefill_gemm" + ("_f16" if dtype == torch.float16 else "")), None
+    for tile in (6, 20, 0):
+        y = torch.full((m + 70, n // 2), float("nan"), dtype=dtype, device="cuda")
+        _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 1, tile, ops._stream()))
+        first = y[:m] if first is None else first
+        assert bool(torch.isfinite(y[:m]).all()) and bool(torch.isnan(y[m:]).all()) and torch.equal(y[:m], first), tile
+    y = torch.empty((m, n), dtype=dtype, device="cuda")
+    with pytest.raises(RuntimeError):
+        _lib.check(fn(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), m, n, k, 0, 20, ops._stream()))
