@@ -201,6 +201,7 @@ class MemoryStep(ctypes.Structure):
 INTERNAL = {name: (_c_i32, [ctypes.POINTER(PrefillStep), _c_vp]) for name in ("nvx_internal_prefill_step", "nvx_internal_prefill_step_f16")}
 INTERNAL.update({name: (_c_i32, [_c_vp, _c_i64, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_vp])
                  for name in ("nvx_internal_prefill_gemm", "nvx_internal_prefill_gemm_f16")})
+INTERNAL.update({name: (_c_i32, [_c_i64] * 2 + [_c_i32] * 2) for name in ("nvx_internal_prefill_loaders", "nvx_internal_prefill_loaders_f16")})
 INTERNAL.update({name: (_c_i32, [_c_i64] * 3 + [_c_i32]) for name in ("nvx_internal_prefill_tile", "nvx_internal_prefill_tile_f16")})
 INTERNAL.update({name: (_c_i32, [_c_vp, _c_i64, _c_vp, _c_i64, _c_i64, _c_i32, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64] + [_c_vp] * 5 + [_c_i32, _c_i32, _c_f32, _c_vp])
                  for name in ("nvx_internal_prefill_heads", "nvx_internal_prefill_heads_f16")})

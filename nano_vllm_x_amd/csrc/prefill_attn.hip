@@ -417,7 +417,8 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     if constexpr (LOADERS > 0) {
         // A turn: the sums of values of `tile` and the scores of the tile behind it.  A wave that has its SIMD to itself and makes a tile's scores, their probabilities and the sums
         // of values one after the other lets the matrix pipe wait for the vector ALU and the other way round; here every group of products has exponentials or maxima beside
-        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  What a turn takes: figures at nvx_paged_prefill.
+        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  Alone and with its keys in the caches a turn takes 0.79 us, of which the matrix
+        // pipe needs 0.43 (64 queries of 3072 keys 54.3 us before, 43.4 now).
         typedef __attribute__((ext_vector_type(8))) short s16x8;
         const int vis = q_ok ? qi + offset : -1;                                          // last key this lane's query sees
         // 32-key blocks of a tile that hold keys some query of the wave sees (wave-uniform)
@@ -783,6 +784,21 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     }
 }
 
+// Workgroups of so many query positions, at most
+static int64_t pf_groups(int64_t positions, int64_t n_tokens, int64_t batch, int64_t hkv) { return ((n_tokens + positions - 1) / positions + batch - 1) * hkv; }
+// Few workgroups: waves of their own for the copies, and where there are fewer still 32 positions of two heads as two waves, which read half as much LDS a tile.  us a launch
+// with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.4 (32 positions) and 13.5, 1024 18.7 and 24.4; 64 positions: 2500 tokens 43.1 and 57.3, six
+// questions behind 900-3000 keys (272 workgroups) 56.7 and 74.4, twelve (560) 93.0 and 80.8, eight prompts of 100-1024 (648) 35.6 and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 459 tokens
+// 12.0 and 13.1, 1500 29.0 and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
+// Between 392 and 512 workgroups what decides is how uneven the blocks are, of which the host knows the tokens and the sequences only: one or two sequences' blocks see more and more keys, and the longest are done
+// first.  us a step of Qwen3-0.6B with loader waves and without, 400 to 512 workgroups: one sequence 0.94 to 0.97 of the time (3168 tokens 6376 and 6800), one behind 300 to 6000 keys 0.94 to 0.975, two of one length
+// 0.97 to 1.00, two of 0.4 and 1.6 times their mean 0.94 to 0.98; three or more of one length up to 1.05 (eight of 452 tokens 5324 and 5215, ten of 272 behind 400 keys 5202 and 4953; as many uneven ones 0.93 to 1.04).  Four layers
+// of Qwen3-8B: one sequence 0.98 to 1.02, 0.995 in the mean; two 0.98 to 1.02, more 1.00 to 1.02.
+static bool pf_loaders(int g, int64_t n_tokens, int64_t batch, int64_t hkv) {
+    return (g == 2 || g == 4) && pf_groups(g == 2 ? 64 : 32, n_tokens, batch, hkv) <= (batch <= (g == 2 ? 2 : 1) ? 512 : 392);
+}
+extern "C" int NVX_ENTRY(nvx_internal_prefill_loaders)(int64_t n_tokens, int64_t batch, int n_q_heads, int n_kv_heads) { return pf_loaders(n_q_heads / n_kv_heads, n_tokens, batch, n_kv_heads); }
+
 extern "C" int NVX_ENTRY(nvx_paged_prefill)(const void* q, int64_t q_row_stride, const void* k_cache, const void* v_cache,
                                  int64_t n_slots, const int32_t* qo_indptr, const int32_t* kv_indptr,
                                  const int32_t* kv_indices, const int32_t* plan_ws, void* out, int64_t n_tokens,
@@ -814,27 +830,19 @@ extern "C" int NVX_ENTRY(nvx_paged_prefill)(const void* q, int64_t q_row_stride,
                            n_slots, qo_indptr, kv_indptr, kv_indices, plan_ws, (uint16_t*)out, (int)batch, n_kv_heads,  \
                            scale_log2);                                                                                 \
     } while (0)
-    // Few workgroups (of so many query positions, at most): waves of their own for the copies, and 32 positions of two heads as two waves, which read half as much LDS a tile.  us a launch
-    // with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.4 (32 positions) and 13.5, 1024 18.7 and 24.4; 64 positions: 2500 tokens 43.1 and 57.3, six
-    // questions behind 900-3000 keys (272 workgroups) 56.7 and 74.4, ten (496) 76.7 and 84.3, twelve (560) 93.0 and 80.8, six prompts of 100-1024 (488) 26.3 and 29.6, eight (648) 35.6
-    // and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 459 tokens 12.0 and 13.1, 1500 29.0 and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
-    // Before a turn made the next tile's scores: 459 tokens 12.1, 1024 21.8, 64 queries of 3072 keys 54.3 (now 43.4: 0.79 us a tile, of 0.43 the matrix pipe needs).
-    const auto groups = [&](int64_t positions) { return ((n_tokens + positions - 1) / positions + batch - 1) * n_kv_heads; };
-    // two rounds of a workgroup a CU, unless most blocks of a round and a half may be short ones.  us a step with the limit at 392 and at 512 workgroups: prompts of 0.3 to 1.7 of their mean length, 2948
-    // tokens (408) 4903 and 4814, 3187 (424) 5259 and 5168, 3727 (512) 5313 and 5296; prompts of one length, which the host does not look for, 3200 tokens (432) 5061 and 5096, 3600 (496) 5075 and 5153.
-    const auto few = [&](int64_t workgroups) { return workgroups <= (n_tokens >= 128 * batch ? 512 : 392); };
+    const bool loaders = pf_loaders(g, n_tokens, batch, n_kv_heads);
     switch (g) {
         case 1: NVX_PF(1, 4, 128, 0); break;
         // two 4-wave workgroups per CU (each in its own phase of the tile loop) measured faster than one
         // 8-wave workgroup of 128 queries (0.75 vs 0.86 ms on the bench prompts); a third tile buffer (row
         // copies two tiles ahead) changed neither
         case 2:
-            if (groups(32) <= 256) NVX_PF(2, 2, 32, 4);
-            else if (few(groups(64))) NVX_PF(2, 4, 64, 4);
+            if (pf_groups(32, n_tokens, batch, n_kv_heads) <= 256) NVX_PF(2, 2, 32, 4);
+            else if (loaders) NVX_PF(2, 4, 64, 4);
             else NVX_PF(2, 4, 64, 0);
             break;
         case 4:
-            if (few(groups(32))) NVX_PF(4, 4, 32, 4);
+            if (loaders) NVX_PF(4, 4, 32, 4);
             else NVX_PF(4, 4, 32, 0);
             break;   // 8 waves / 64 queries measured slower here too (1.77 vs 1.57 ms at 32 q heads)
         case 8: NVX_PF(8, 8, 32, 0); break;
