@@ -20,3 +20,10 @@ def test_order_is_a_stable_sort(experts, pairs):
         want[order] = torch.arange(order.numel())
         assert torch.equal(dst[real], want)
         assert torch.equal(counts.long(), torch.bincount(idx[real].long(), minlength=experts))
+
+
+@pytest.mark.parametrize("experts", [1, 4, 5, 6, 7])
+@pytest.mark.parametrize("pairs", [16384, 16385, 65536, 70001])
+def test_many_pairs_of_few_experts(experts, pairs):
+    """Several turns of every wave, on both sides of the line between a ballot an expert and a ballot a bit."""
+    test_order_is_a_stable_sort(experts, pairs)
