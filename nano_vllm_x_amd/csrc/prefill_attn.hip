@@ -26,6 +26,7 @@ namespace NVX_NS {
 #define PF_RING 4               // tiles of a workgroup with waves that only fetch: one read for values, the next for keys, one landing, one asked for
 #define PF_SORTED 64             // sequences (a lane each) whose blocks are found without a plan
 #define PF_IDS (2 * PF_RING)    // tiles whose slot ids such a wave keeps
+#define PF_SHORT 2              // tiles up to which such a workgroup makes them one after the other
 #define PF_LOG2E 1.4426950408889634f
 
 typedef __attribute__((ext_vector_type(4))) short pf_s16x4;
@@ -337,11 +338,28 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
                 find_rows(t);
                 fetch_rows(t);
             }
+            static_assert(RING == 4, "what may be on its way at a barrier: the rows of one tile, or of two");
+            // One or two tiles: a turn that makes the scores of the tile behind it has nothing to hide there, waits for a second tile ahead of the first, and makes scores of keys that nobody sees.  us
+            // a launch one tile after the other as in the loop, by turns, and by this: 20 tokens 4.30, 4.82, 4.31; 100 5.82, 6.12, 5.83; 200 7.48, 7.73, 7.43; 459 11.9, 11.3, 11.0 (between products
+            // 12.3, 12.4, 11.5); 1000 21.6, 18.8, 18.5; four of 100 6.51, 6.86, 6.52.  With three tiles as well 4 x 200 8.6 instead of 8.4, up to six 459 tokens 11.1 and six prompts of 300 12.1 instead of 11.0.
+            if (n_tiles <= PF_SHORT) {
+                // tile t's turn begins when tile t has landed; no ids are left to ask for
+                static_assert(PF_SHORT < 2 * PF_RING, "ids of a short run");
+                for (int t = -1; t < n_tiles; ++t) {
+                    if (t >= 0 && t + RING - 1 < n_tiles) {
+                        find_rows(t + RING - 1);
+                        fetch_rows(t + RING - 1);                                  // (to where tile t - 1 was)
+                    }
+                    if (t + 3 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(4 * PASSES) : "memory");
+                    else if (t + 2 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
+                    else pf_wait_copies();
+                    __syncthreads();
+                }
+                return;
+            }
             find_rows(RING - 1);                                                   // (whatever lies there if there is no such tile: not used)
             // tile t's turn begins when tile t + 1 has landed
-            static_assert(RING == 4, "what may be on its way at a barrier: the rows of one tile");
-            if (n_tiles >= RING - 1) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
-            else pf_wait_copies();
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
             __syncthreads();
             for (int t = 0; t < n_tiles; ++t) {
                 const bool more_rows = t + RING - 1 < n_tiles, more_ids = t + 2 * RING - 1 < n_tiles;
@@ -414,7 +432,8 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     }
     __syncthreads();
     { const unsigned t0 = ids0; ids0 = ids1; ids1 = t0; }
-    if constexpr (LOADERS > 0) {
+    bool made = false;
+    if constexpr (LOADERS > 0) if (n_tiles > PF_SHORT) {
         // A turn: the sums of values of `tile` and the scores of the tile behind it.  A wave that has its SIMD to itself and makes a tile's scores, their probabilities and the sums
         // of values one after the other lets the matrix pipe wait for the vector ALU and the other way round; here every group of products has exponentials or maxima beside
         // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  Alone and with its keys in the caches a turn takes 0.79 us, of which the matrix
@@ -593,7 +612,9 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
             ++tile;
         }
         for (; tile < n_tiles; ++tile) __syncthreads();      // (nothing of these is visible to this wave)
-    } else {
+        made = true;
+    }
+    if (!made) {
     // at the top of tile t: ids0 holds the ids of tile t + 1, ids1 is free (its ids were used a tile ago)
 #ifdef PF_STAMPS
     const int stamp_blk = gblk;
@@ -603,7 +624,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         PF_STAMP(0);
         const unsigned k_lds = ring0;   // LDS byte addresses
         const unsigned v_lds = k_lds + PF_KVBLK * 256;
-        if (tile + 1 < n_tiles) {   // the other buffer held tile t - 1: every wave left it before the last barrier
+        if (LOADERS == 0 && tile + 1 < n_tiles) {   // the other buffer held tile t - 1: every wave left it before the last barrier
             if (tile > 0)           // (tile 1 came with tile 0)
                 pf_gather<PASSES, KEYS_PER_PASS>(ids0, krow0, n_slots_u, kg, vg, row_bytes, ring1 + wave_rows, ring1 + PF_KVBLK * 256 + wave_rows);
             if (tile + 2 < n_tiles && wave == 0) pf_fetch_slot_ids(seq_slots, tile + 2, lkv, lane, ids1);
@@ -740,11 +761,12 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         };
         if (key_base + 32 <= wave_last_key) tile_body(std::integral_constant<int, 2>{});        // wave-uniform
         else if (key_base <= wave_last_key) tile_body(std::integral_constant<int, 1>{});        // else: nothing visible
-        pf_wait_copies();
+        if (LOADERS == 0) pf_wait_copies();
         PF_STAMP(6);
         __syncthreads();   // tile + 1 and the ids of tile + 2 visible; this tile's buffer free
         PF_STAMP(7);
-        { const unsigned t0 = ring0; ring0 = ring1; ring1 = t0; }
+        if (LOADERS) ring0 = ring0 == lds0 + (RING - 1) * BUF_BYTES ? lds0 : ring0 + BUF_BYTES;
+        else { const unsigned t0 = ring0; ring0 = ring1; ring1 = t0; }
         { const unsigned t0 = ids0; ids0 = ids1; ids1 = t0; }
     }
     }

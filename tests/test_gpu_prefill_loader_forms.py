@@ -55,6 +55,18 @@ def test_scores_that_climb(dtype, form, part, step):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("part", [(1, 1), (1, 32), (1, 33), (1, 64), (1, 65), (33, 97), (1, 128), (64, 128), (1, 129), (64, 192), (1, 193), (64, 257), (1, 449)])
+def test_few_tiles(dtype, form, part):
+    """One and two tiles are made one after the other, more by turns: edges of tiles and of their halves."""
+    hq, hkv, parts, q, k, v = _inputs(part, form, dtype, sum(part))
+    q, k, v = q.view(len(q), -1).to(dtype), k.to(dtype), v.to(dtype)
+    here, loop, slots = _both(q, k, v, parts, hq, hkv)
+    assert torch.equal(here, loop)
+    _against_float64(here, q, k, v, slots, part, hq, hkv, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
 @pytest.mark.parametrize("key", [0, 63, 64, 300, 699])
 def test_scores_that_are_no_numbers(dtype, form, value, key):
