@@ -265,7 +265,7 @@ using namespace NVX_NS;
 
 // What a tile costs, us, with weights that no cache holds: us + (rounds - 1) * again + k / 1024 * (us_k + (rounds - 1) * round + (workgroups / 256 - 1) * over), rounds of 256 workgroups and the last
 // term from the 257th on (us_k 0: not built).  Plain: fitted to 40 to 4000 rows of 1024 to 12288 outputs of 512 to 3072 columns, with `again` 0; of 813 products of 30 to 8000 rows of 256 to 8192 columns
-// the tile it picks costs 0.7 % more than the best one (the tiles and costs before 7 %).  SiluAndMul: fitted to 868 products of 30 to 8000 rows, 256 to 2048 columns, over which its choice is 0.4 % off the best; without `again`, what
+// the tile it picks costs 0.7 % more than the best one (the tiles and costs before 7 %).  SiluAndMul: fitted to 1 365 products of 30 to 18 000 rows, 256 to 2048 columns; over 1 358 others its choice is 0.2 % off the best (15 % at worst); without `again`, what
 // a round costs however few its columns are (results, SiluAndMul, first copies), narrow layers got tiles 5 to 45 % off.  A step of a few KB is as long as its copies' way into a CU, its reads from LDS and two barriers'
 // skew, hardly any of which hides any other at one workgroup a CU, so the tile that just fills the CUs is the best, and there is one for most sizes: without the tiles of 96 to 224 x 128, and with
 // two and three steps of 64 x 128 in LDS, the choice was 6 % and 8 % off.  us a product without and with them: SiluAndMul's 6144 x 1024, 256 rows 11.7 and 10.4 (64 x 128), 768 20.2 and 16.5 (160 x 128), 900 20.7 and 18.3, 1024 21.9 and 19.2;
@@ -277,22 +277,22 @@ struct PrefillCost { float us, again, us_k, round, over; };
 struct PrefillTile { int tile, m, n; PrefillCost plain, silu; bool wide; };
 static const PrefillTile PREFILL_TILES[] = {
     {NVX_PG_32_32, 32, 32, {2.1f, 0.f, 2.05f, 1.2f, .4f}, {}, false},
-    {NVX_PG_32_64, 32, 64, {2.3f, 0.f, 2.9f, 2.35f, 1.1f}, {2.4f, 1.4f, 3.5f, 2.6f, .4f}, false},
-    {NVX_PG_64_64, 64, 64, {2.2f, 0.f, 4.2f, 2.f, 1.45f}, {2.1f, .4f, 5.25f, 2.f, 1.4f}, false},
+    {NVX_PG_32_64, 32, 64, {2.3f, 0.f, 2.9f, 2.35f, 1.1f}, {2.49f, 1.4f, 3.51f, 3.3f, -.15f}, false},
+    {NVX_PG_64_64, 64, 64, {2.2f, 0.f, 4.2f, 2.f, 1.45f}, {2.07f, .51f, 5.51f, 1.97f, 1.01f}, false},
     {NVX_PG_96_64, 96, 64, {2.7f, 0.f, 4.7f, 2.8f, 1.75f}, {}, false},
     {NVX_PG_128_64, 128, 64, {3.1f, 0.f, 5.2f, 5.5f, 1.5f}, {}, false},
     {NVX_PG_160_64, 160, 64, {3.5f, 0.f, 6.1f, 6.f, 2.6f}, {}, false},
     {NVX_PG_192_64, 192, 64, {3.8f, 0.f, 7.f, 7.1f, 2.4f}, {}, false},
-    {NVX_PG_64_128, 64, 128, {2.8f, 0.f, 6.f, 5.55f, 1.3f}, {2.9f, 2.35f, 7.35f, 4.4f, .65f}, false},
-    {NVX_PG_64_128_THREE, 64, 128, {}, {2.4f, .8f, 11.6f, 2.5f, 0.f}, false},
-    {NVX_PG_96_128, 96, 128, {3.6f, 0.f, 7.25f, 6.6f, 2.3f}, {3.9f, 3.05f, 7.7f, 5.4f, 1.4f}, false},
-    {NVX_PG_128_128, 128, 128, {4.f, 0.f, 7.7f, 6.65f, 2.3f}, {4.5f, 2.2f, 8.4f, 6.2f, 1.3f}, true},
-    {NVX_PG_160_128, 160, 128, {5.f, 0.f, 9.4f, 10.3f, 1.9f}, {5.3f, 4.f, 10.2f, 7.7f, 3.f}, false},
-    {NVX_PG_192_128, 192, 128, {5.3f, 0.f, 10.9f, 10.75f, 3.3f}, {5.8f, 5.9f, 11.4f, 5.3f, 4.2f}, false},
-    {NVX_PG_224_128, 224, 128, {5.35f, 0.f, 11.9f, 11.15f, 6.8f}, {6.3f, 5.7f, 12.3f, 7.9f, 3.f}, false},
-    {NVX_PG_128_256, 128, 256, {.7f, 0.f, 21.4f, 13.6f, 3.7f}, {4.3f, 3.9f, 21.1f, 10.6f, 3.5f}, true},
-    {NVX_PG_192_256, 192, 256, {1.7f, 0.f, 23.2f, 14.3f, 8.6f}, {6.6f, 5.9f, 22.f, 11.5f, 6.2f}, true},
-    {NVX_PG_256_256, 256, 256, {4.9f, 0.f, 23.8f, 12.f, 10.f}, {9.2f, 7.f, 23.35f, 15.8f, 5.3f}, true}};
+    {NVX_PG_64_128, 64, 128, {2.8f, 0.f, 6.f, 5.55f, 1.3f}, {3.06f, 2.24f, 7.24f, 5.09f, .26f}, false},
+    {NVX_PG_64_128_THREE, 64, 128, {}, {2.33f, .88f, 13.23f, 1.54f, 0.f}, false},
+    {NVX_PG_96_128, 96, 128, {3.6f, 0.f, 7.25f, 6.6f, 2.3f}, {3.82f, 3.12f, 7.55f, 5.31f, 1.09f}, false},
+    {NVX_PG_128_128, 128, 128, {4.f, 0.f, 7.7f, 6.65f, 2.3f}, {4.37f, 2.08f, 8.85f, 6.12f, 1.54f}, true},
+    {NVX_PG_160_128, 160, 128, {5.f, 0.f, 9.4f, 10.3f, 1.9f}, {5.52f, 4.14f, 10.18f, 8.66f, 1.27f}, false},
+    {NVX_PG_192_128, 192, 128, {5.3f, 0.f, 10.9f, 10.75f, 3.3f}, {6.08f, 4.79f, 10.69f, 8.47f, 2.44f}, false},
+    {NVX_PG_224_128, 224, 128, {5.35f, 0.f, 11.9f, 11.15f, 6.8f}, {6.48f, 5.05f, 12.48f, 9.56f, 2.79f}, false},
+    {NVX_PG_128_256, 128, 256, {.7f, 0.f, 21.4f, 13.6f, 3.7f}, {4.41f, 3.44f, 21.14f, 10.54f, 3.89f}, true},
+    {NVX_PG_192_256, 192, 256, {1.7f, 0.f, 23.2f, 14.3f, 8.6f}, {6.68f, 5.94f, 22.64f, 10.51f, 6.78f}, true},
+    {NVX_PG_256_256, 256, 256, {4.9f, 0.f, 23.8f, 12.f, 10.f}, {8.95f, 7.72f, 23.45f, 12.06f, 9.64f}, true}};
 
 // QKV, a tile as wide as a head, in one round of workgroups: us + k / 1024 * us_k, less what the launch costs that norms and turns the heads behind a plain product (the two grow alike with
 // the rows).  Fitted to steps of 20 to 1024 tokens of layers of 512 to 2560: these costs, held against the plain tiles', were right wherever the two ways differ by more than
