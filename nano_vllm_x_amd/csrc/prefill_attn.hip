@@ -147,12 +147,6 @@ __device__ __forceinline__ void pf_gather(unsigned ids, int krow0, unsigned n_sl
     for (int p = 0; p < PASSES; ++p) pf_gather_one(id[p], n_slots, kbase, vbase, row_bytes, k_dst + p * STEP, v_dst + p * STEP);
 }
 
-// What a query's scores are taken relative to (log2 units): the largest so far, but one that is exceeded by less than 2^PF_SLACK stays.  Weights of up to 256 are as exact as
-// weights of up to 1 in either format, their sums are float32, and the accumulators need not be rescaled (64 multiplications a lane, between products) wherever any
-// of a wave's 32 queries finds a larger score: of 48 tiles of random scores that was every second.
-#define PF_SLACK 8.0f
-__device__ __forceinline__ float pf_reference(float was, float largest) { return largest > was + PF_SLACK ? largest : was; }
-
 #if defined(PF_STAMPS) && !defined(NVX_F16)
 // Build-time instrumentation (tools/build_variant.sh ... "-DPF_STAMPS"): shader-clock stamps of waves 0 and 3 of the
 // workgroups of blocks 8 and 9 (kv head 0; blocks of a sequence are taken last first, so these are query blocks 119 and
@@ -436,8 +430,9 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     if constexpr (LOADERS > 0) if (n_tiles > PF_SHORT) {
         // A turn: the sums of values of `tile` and the scores of the tile behind it.  A wave that has its SIMD to itself and makes a tile's scores, their probabilities and the sums
         // of values one after the other lets the matrix pipe wait for the vector ALU and the other way round; here every group of products has exponentials or maxima beside
-        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  Alone and with its keys in the caches a turn takes 0.79 us, of which the matrix
-        // pipe needs 0.43 (64 queries of 3072 keys 54.3 us before, 43.4 now).
+        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  Alone and with its keys in the caches a turn takes 0.88 us, of which the matrix
+        // pipe needs 0.43 (64 queries of 3072 keys 54.2 us before, 48.1 now; 43.6 if weights were relative to a score that later ones may exceed by 2^8, which spares most of the accumulators' multiplications
+        // but rounds the largest weight, and so results: 1.00 to 1.24 of the error against 64 bits).
         typedef __attribute__((ext_vector_type(8))) short s16x8;
         const int vis = q_ok ? qi + offset : -1;                                          // last key this lane's query sees
         // 32-key blocks of a tile that hold keys some query of the wave sees (wave-uniform)
@@ -490,7 +485,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         auto begin = [&]() __attribute__((always_inline)) {
             float m = fmaxf(mx[0], mx[1]);
             m = fmaxf(m, xor32(m));
-            const float m_new = pf_reference(m_run, m * scale_log2);     // scale_log2 > 0
+            const float m_new = fmaxf(m_run, m * scale_log2);     // scale_log2 > 0
             mref = m_new == -INFINITY ? 0.f : m_new;
             alpha = __builtin_amdgcn_exp2f(m_run - mref);
             m_run = m_new;
@@ -687,7 +682,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         }
         float mx = NKB == 2 ? fmaxf(mxb[0], mxb[NKB - 1]) : mxb[0];
         mx = fmaxf(mx, xor32(mx));
-        const float m_new = pf_reference(m_run, mx * scale_log2);     // scale_log2 > 0
+        const float m_new = fmaxf(m_run, mx * scale_log2);     // scale_log2 > 0
         const float mref = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m_run - mref);
         m_run = m_new;

@@ -1,5 +1,5 @@
-"""Attention of prompts by each form of the kernel whose tiles are fetched by waves of their own (32 positions of two heads as two waves, 64 of two, 32 of four): scores that climb past
-what a query's weights are taken relative to, scores that are infinite or no numbers, and tiles that a wave sees nothing of, against the loop without such waves and against float64."""
+"""Attention of prompts by each form of the kernel whose tiles are fetched by waves of their own (32 positions of two heads as two waves, 64 of two, 32 of four): scores that climb
+from tile to tile, scores that are infinite or no numbers, and tiles that a wave sees nothing of, against the loop without such waves and against float64."""
 import pytest
 import torch
 
@@ -51,6 +51,26 @@ def test_scores_that_climb(dtype, form, part, step):
     here, loop, slots = _both(q, k, v, parts, hq, hkv)
     assert torch.equal(here, loop)
     _against_float64(here, q, k, v, slots, part, hq, hkv, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form", FORMS)
+def test_the_largest_weight_is_exact(dtype, form):
+    """Weights are taken relative to the largest score so far, whose weight is 1 in any format: where one key has nearly all of it and the rows of values are alike, a query gets that row, with no
+    rounding of its weight in it (relative to an earlier, smaller score the weight itself is rounded, by up to half a unit, and so is the result)."""
+    part = (64, 448)
+    hq, hkv, parts, q, k, v = _inputs(part, form, dtype, 3)
+    q.zero_()
+    q[:, :, 0] = 128 ** 0.5 * torch.linspace(0.5, 1.0, len(q), device="cuda")[torch.randperm(len(q), generator=torch.Generator().manual_seed(1)).cuda()][:, None]
+    k.zero_()
+    k[:part[1], :, 0] = -40.0
+    k[0, :, 0] = 0.0                                         # the largest of the first tile; the one behind exceeds it by 2^3.9 to 2^7.8
+    k[330, :, 0] = 5.4
+    unit = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    v[:] = 2.0 - unit                                        # (an error of half a unit of a weight is a whole one here)
+    q, k, v = q.view(len(q), -1).to(dtype), k.to(dtype), v.to(dtype)
+    here, loop, _ = _both(q, k, v, parts, hq, hkv)
+    assert bool((here[:part[0]] == 2.0 - unit).all()) and bool((loop[:part[0]] == 2.0 - unit).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

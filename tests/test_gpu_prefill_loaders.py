@@ -50,7 +50,7 @@ def _against_float64(got, q, k, v, slots, part, hq, hkv, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("step", [0.25, 3.0, 5.5, 12.0, -3.0])
 def test_scores_that_climb(dtype, step):
-    """Scores that rise by `step` from tile to tile (and fall): the value that weights are taken relative to stays for rises of up to eight powers of two, and moves behind them."""
+    """Scores that rise by `step` from tile to tile (and fall): what weights are taken relative to moves with every tile, or stays."""
     gen = torch.Generator(device="cuda").manual_seed(7)
     part, filler, hq, hkv = (150, 700), ((64, 64),) * 200, 4, 2
     nq, nk = part[0] + 64 * 200, part[1] + 64 * 200
