@@ -26,7 +26,7 @@ namespace NVX_NS {
 #define PF_RING 4               // tiles of a workgroup with waves that only fetch: one read for values, the next for keys, one landing, one asked for
 #define PF_SORTED 64             // sequences (a lane each) whose blocks are found without a plan
 #define PF_IDS (2 * PF_RING)    // tiles whose slot ids such a wave keeps
-#define PF_SHORT 2              // tiles up to which such a workgroup makes them one after the other
+#define PF_SHORT 4              // tiles up to which such a workgroup makes them one after the other
 #define PF_LOG2E 1.4426950408889634f
 
 typedef __attribute__((ext_vector_type(4))) short pf_s16x4;
@@ -293,7 +293,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     kmax = kmax > lkv ? lkv : kmax;
     const int wave_last_key = qb * QPOS + pb * 32 + 31 + offset;  // last key any query of this wave sees
     const int wave_first_vis = qb * QPOS + pb * 32 + offset;      // last key the wave's FIRST query sees
-    const int n_tiles = (kmax + PF_KVBLK - 1) / PF_KVBLK;
+    const int n_tiles = (max(kmax, 0) + PF_KVBLK - 1) / PF_KVBLK;
 
     if constexpr (LOADERS > 0) {
         if (wave >= NWAVES) {
@@ -328,29 +328,29 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
             };
             for (int t = 0; t < n_tiles && t < 2 * RING - 1; ++t) fetch_ids(t);
             pf_wait_copies();
-            for (int t = 0; t < n_tiles && t < RING - 1; ++t) {
-                find_rows(t);
-                fetch_rows(t);
-            }
-            static_assert(RING == 4, "what may be on its way at a barrier: the rows of one tile, or of two");
-            // One or two tiles: a turn that makes the scores of the tile behind it has nothing to hide there, waits for a second tile ahead of the first, and makes scores of keys that nobody sees.  us
-            // a launch one tile after the other as in the loop, by turns, and by this: 20 tokens 4.30, 4.82, 4.31; 100 5.82, 6.12, 5.83; 200 7.48, 7.73, 7.43; 459 11.9, 11.3, 11.0 (between products
-            // 12.3, 12.4, 11.5); 1000 21.6, 18.8, 18.5; four of 100 6.51, 6.86, 6.52.  With three tiles as well 4 x 200 8.6 instead of 8.4, up to six 459 tokens 11.1 and six prompts of 300 12.1 instead of 11.0.
+            // Few tiles: a turn that makes the scores of the tile behind it has little to hide there, waits for a second tile ahead of the first, and makes scores of keys that nobody sees.  us a launch, the
+            // loop with such waves alone (before there were turns), turns alone, and this: 20 tokens 4.31, 4.82, 4.23; 100 5.82, 6.12, 5.65; 200 7.48, 7.75, 7.12; 459 11.9, 11.7, 11.2 (between
+            // products 12.6, 12.5, 11.1); 1000 21.4, 19.9, 19.2; four of 100 6.50, 6.86, 6.31.  Turns from the third tile on: 200 tokens 7.46, four of 200 8.43 instead of 8.09; from the sixth: the same as from the fifth.
             if (n_tiles <= PF_SHORT) {
-                // tile t's turn begins when tile t has landed; no ids are left to ask for
+                // tile t's turn begins when tile t has landed; two are on their way, and no ids are left to ask for
                 static_assert(PF_SHORT < 2 * PF_RING, "ids of a short run");
-                for (int t = -1; t < n_tiles; ++t) {
-                    if (t >= 0 && t + RING - 1 < n_tiles) {
-                        find_rows(t + RING - 1);
-                        fetch_rows(t + RING - 1);                                  // (to where tile t - 1 was)
+                for (int t = -2; t < n_tiles; ++t) {
+                    if (t + 2 < n_tiles) {
+                        find_rows(t + 2);
+                        fetch_rows(t + 2);                                         // (to where tile t - 2 was)
                     }
-                    if (t + 3 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(4 * PASSES) : "memory");
-                    else if (t + 2 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
+                    if (t == -2) continue;
+                    if (t + 2 < n_tiles) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
                     else pf_wait_copies();
                     __syncthreads();
                 }
                 return;
             }
+            for (int t = 0; t < RING - 1; ++t) {
+                find_rows(t);
+                fetch_rows(t);
+            }
+            static_assert(RING == 4 && PF_SHORT >= RING - 2, "what may be on its way at a barrier: the rows of one tile");
             find_rows(RING - 1);                                                   // (whatever lies there if there is no such tile: not used)
             // tile t's turn begins when tile t + 1 has landed
             asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * PASSES) : "memory");
@@ -430,8 +430,8 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     if constexpr (LOADERS > 0) if (n_tiles > PF_SHORT) {
         // A turn: the sums of values of `tile` and the scores of the tile behind it.  A wave that has its SIMD to itself and makes a tile's scores, their probabilities and the sums
         // of values one after the other lets the matrix pipe wait for the vector ALU and the other way round; here every group of products has exponentials or maxima beside
-        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  Alone and with its keys in the caches a turn takes 0.88 us, of which the matrix
-        // pipe needs 0.43 (64 queries of 3072 keys 54.2 us before, 48.1 now; 43.6 if weights were relative to a score that later ones may exceed by 2^8, which spares most of the accumulators' multiplications
+        // it, and a turn begins under the last products of the one before.  All chains of sums run as in the loop below.  Alone and with its keys in the caches a turn takes 0.86 us, of which the matrix
+        // pipe needs 0.43 (64 queries of 3072 keys 54.2 us before, 46.8 now; 43.6 if weights were relative to a score that later ones may exceed by 2^8, which spares most of the accumulators' multiplications
         // but rounds the largest weight, and so results: 1.00 to 1.24 of the error against 64 bits).
         typedef __attribute__((ext_vector_type(8))) short s16x8;
         const int vis = q_ok ? qi + offset : -1;                                          // last key this lane's query sees
@@ -615,6 +615,8 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     const int stamp_blk = gblk;
     const bool stamp_on = (gblk == 8 || gblk == 9) && head == 0 && (wave == 0 || wave == 3);
 #endif
+    int last_key = wave_last_key;
+    if (LOADERS) asm volatile("" : "+v"(last_key));
     for (int tile = 0; tile < n_tiles; ++tile) {
         PF_STAMP(0);
         const unsigned k_lds = ring0;   // LDS byte addresses
@@ -754,8 +756,8 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
         }
         PF_STAMP(5);
         };
-        if (key_base + 32 <= wave_last_key) tile_body(std::integral_constant<int, 2>{});        // wave-uniform
-        else if (key_base <= wave_last_key) tile_body(std::integral_constant<int, 1>{});        // else: nothing visible
+        if (key_base + 32 <= last_key) tile_body(std::integral_constant<int, 2>{});        // wave-uniform
+        else if (key_base <= last_key) tile_body(std::integral_constant<int, 1>{});        // else: nothing visible
         if (LOADERS == 0) pf_wait_copies();
         PF_STAMP(6);
         __syncthreads();   // tile + 1 and the ids of tile + 2 visible; this tile's buffer free
@@ -804,13 +806,13 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
 // Workgroups of so many query positions, at most
 static int64_t pf_groups(int64_t positions, int64_t n_tokens, int64_t batch, int64_t hkv) { return ((n_tokens + positions - 1) / positions + batch - 1) * hkv; }
 // Few workgroups: waves of their own for the copies, and where there are fewer still 32 positions of two heads as two waves, which read half as much LDS a tile.  us a launch
-// with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.4 (32 positions) and 13.5, 1024 18.7 and 24.4; 64 positions: 2500 tokens 43.1 and 57.3, six
-// questions behind 900-3000 keys (272 workgroups) 56.7 and 74.4, twelve (560) 93.0 and 80.8, eight prompts of 100-1024 (648) 35.6 and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 459 tokens
-// 12.0 and 13.1, 1500 29.0 and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
+// with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.2 (32 positions) and 13.5, 1024 19.6 and 24.4.  Figures of turns that took 0.79 us (see there): 64 positions: 2500 tokens 43.1 and 57.3, six
+// questions behind 900-3000 keys (272 workgroups) 56.7 and 74.4, twelve (560) 93.0 and 80.8, eight prompts of 100-1024 (648) 35.6 and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 1500 tokens 29.0
+// and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
 // Between 392 and 512 workgroups what decides is how uneven the blocks are, of which the host knows the tokens and the sequences only: one or two sequences' blocks see more and more keys, and the longest are done
-// first.  us a step of Qwen3-0.6B with loader waves and without, 400 to 512 workgroups: one sequence 0.94 to 0.97 of the time (3168 tokens 6376 and 6800), one behind 300 to 6000 keys 0.94 to 0.975, two of one length
-// 0.97 to 1.00, two of 0.4 and 1.6 times their mean 0.94 to 0.98; three or more of one length up to 1.05 (eight of 452 tokens 5324 and 5215, ten of 272 behind 400 keys 5202 and 4953; as many uneven ones 0.93 to 1.04).  Four layers
-// of Qwen3-8B: one sequence 0.98 to 1.02, 0.995 in the mean; two 0.98 to 1.02, more 1.00 to 1.02.
+// first.  us a step of Qwen3-0.6B with loader waves and without, 400 to 512 workgroups: one sequence 0.94 to 0.97 of the time (3168 tokens 6445 and 6830), also behind 700 and 2500 keys; two of one length
+// 0.97 to 1.00, two of 0.4 and 1.6 times their mean 0.93 to 0.97; three or more of one length up to 1.05 (eight of 452 tokens 5324 and 5215, ten of 272 behind 400 keys 5202 and 4953; as many uneven ones 0.93 to 1.04).  Four layers
+// of Qwen3-8B: one sequence 0.985 to 1.01; two 0.99 to 1.01, more 1.00 to 1.02.
 static bool pf_loaders(int g, int64_t n_tokens, int64_t batch, int64_t hkv) {
     return (g == 2 || g == 4) && pf_groups(g == 2 ? 64 : 32, n_tokens, batch, hkv) <= (batch <= (g == 2 ? 2 : 1) ? 512 : 392);
 }

@@ -75,9 +75,9 @@ def test_the_largest_weight_is_exact(dtype, form):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("form", FORMS)
-@pytest.mark.parametrize("part", [(1, 1), (1, 32), (1, 33), (1, 64), (1, 65), (33, 97), (1, 128), (64, 128), (1, 129), (64, 192), (1, 193), (64, 257), (1, 449)])
+@pytest.mark.parametrize("part", [(1, 1), (1, 32), (1, 33), (1, 64), (1, 65), (33, 97), (1, 128), (64, 128), (1, 129), (64, 192), (1, 193), (64, 256), (1, 257), (64, 320), (64, 321), (1, 449)])
 def test_few_tiles(dtype, form, part):
-    """One and two tiles are made one after the other, more by turns: edges of tiles and of their halves."""
+    """Up to four tiles are made one after the other, more by turns: edges of tiles and of their halves."""
     hq, hkv, parts, q, k, v = _inputs(part, form, dtype, sum(part))
     q, k, v = q.view(len(q), -1).to(dtype), k.to(dtype), v.to(dtype)
     here, loop, slots = _both(q, k, v, parts, hq, hkv)
