@@ -8,9 +8,10 @@
 // it multiplies), which splitting K over the waves would halve; but K is never split: a row's sum runs over K in order, in one chain of
 // v_mfma_f32_16x16x32, whatever the tile, so that a token's result does not depend on how many tokens share its step (and equals the library's
 // above some 200 rows, whose products take K in the same order).
-// The products of a layer of Qwen3-0.6B with weights that no cache holds, us, qkv / o / gate | up / down: 100 rows 5.2 / 6.0 / 7.3 / 8.1, 200 rows 6.5 / 6.1 / 9.4 / 8.2,
-//     459 rows 8.5 / 8.0 / 12.2 / 11.0, 1500 rows 17.2 / 12.1 / 28.7 / 17.6 (the library with weights in its caches: 64 rows 8.8 / 8.4 / 9.0 and SiluAndMul's 4 / 10.1, 459 rows
-//     11.2 / 9.7 / 13.6 and 4 / 12.5, 1536 rows 17.7 / 13.7 / 28.9 and 4 / 17.1).
+// The products of a layer of Qwen3-0.6B with weights that no cache holds, one kind of product behind another of its kind, us, qkv / o / gate | up / down: 100 rows 5.6 / 6.2 / 7.4 / 8.2, 200 rows 7.0 / 6.3 / 9.5 / 8.3,
+//     459 rows 9.1 / 8.2 / 12.1 / 11.2, 1500 rows 18.0 / 12.6 / 29.2 / 18.0 (by the same measure before copies and reads were dealt out and there were tiles of 96 to 224 x 128: 100 rows 5.9 / 6.5 / 7.6 / 8.4, 200 7.2 / 6.6 / 10.5 /
+//     8.5, 459 10.6 / 8.5 / 12.9 / 11.4, 1500 24.0 / 13.0 / 29.2 / 18.3; the library with weights in its caches: 64 rows 8.8 / 8.4 / 9.0 and SiluAndMul's 4 / 10.1, 459 rows
+//     11.2 / 9.7 / 13.6 and 4 / 12.5, 1536 rows 17.7 / 13.7 / 28.9 and 4 / 17.1).  Within a step 459 rows take 12.5 with the heads' norms and rotations, 13.4 for gate | up, 9.95 in the mean of o and down.
 #include "prefill_gemm.h"
 
 #include <type_traits>

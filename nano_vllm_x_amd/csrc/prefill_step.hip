@@ -3,8 +3,8 @@
 //
 // Up to some thousand tokens the device needs less than 150 us for a layer and the host, through Python, 160 to queue it (220 where it calls
 // modules): four library products at 19 us each, shape look-up included, and six kernels at 10.  From here a kernel is 2-4 us, and the products are
-// those of prefill_gemm.hip.  Qwen3-0.6B, us a step through Python and from here: 20 tokens 4540 and 1380, 459 tokens 4560 and 1880 (6200
-// through the modules); 2160 tokens behind cached ones, float16, 6270 and 4960.
+// those of prefill_gemm.hip.  Qwen3-0.6B, us a step through Python and from here: 20 tokens 4540 and 1270, 459 tokens 4560 and 1850 (6200
+// through the modules); 2160 tokens behind cached ones, float16, 6270 and 4980.
 #include "prefill_gemm.h"
 
 // layers: ten addresses a layer: input norm, qkv, q norm, k norm, o, post-attention norm, gate | up, down (weights), k rows, v rows (caches).

@@ -186,9 +186,10 @@ def prefill_step_fits(hidden: int, n_q_heads: int, n_kv_heads: int, inter: int) 
 
 def gated_product_faster(rows: int, n: int, k: int) -> bool:
     """Whether SiluAndMul of a product of csrc/prefill_gemm.hip, n rows of weights of k columns, beats the library's product and silu_mul.  Up to 1536 columns it
-    does (us, 15754 rows: 6144 x 1024 182, library 159 and 50; 500 to 30 000 rows of 3072 x 512 to 16384 x 1024 and 8192 x 1536: 0.32 to 0.95 of the two, but for 1.03 and
-    1.01 at one size each); with more, where SiluAndMul is the smaller part, up to 2048 where four rounds of 256 x 256 tiles or more make an idle part of the last a small one: 12288 x
-    2048, 600 rows 47 and 40, 1300 97 and 82, 2048 132 and 106, 5500 rows 0.86 of the two, up to 30 000 0.85 to 0.99; 9728 x 1792, 4096 rows 193 and 163, from 7000 0.73 to 0.95."""
+    does (us, 15754 rows: 6144 x 1024 182, library 159 and 50; 500 to 30 000 rows of 3072 x 512 to 16384 x 1024 and 8192 x 1536: 0.32 to 0.95 of the two, but for 1.05 at 3000 rows of 8192 x 1536
+    and 1.01 at 1300 of 6144 x 1024); with more, where SiluAndMul is the smaller part, up to 2048 where four rounds of 256 x 256 tiles or more make an idle part of the last a small one (us here / both):
+    12288 x 2048, 600 rows 41.2 / 40.3, 1300 88.2 / 83.7, 2048 114 / 105, 4096 180 / 176, 5500 268 / 299, 8000 369 / 364.  Narrower weights of so many columns meet the two further down than the rule
+    takes them: 9728 x 1792, 600 rows 30.7 / 35.0, 900 52.1 / 50.2, 4096 157 / 167, 8000 268 / 352; 4096 x 2048, 600 rows 19.1 / 26.4, 8000 125 / 129."""
     return k <= 1536 or (k <= 2048 and rows * n >= 4 * 256 * 256 * 256)
 
 

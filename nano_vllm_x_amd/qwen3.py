@@ -97,10 +97,11 @@ DECODE_LINEAR_MAX_WEIGHT_BYTES = 16 << 20
 # Multiply-adds of a layer's projections up to which a prefill step is queued by one native call with the products of csrc/prefill_gemm.hip
 # (ops.prefill_step) in any case: there the host is the slower from Python.  Up to the second figure it is with layers of up to 1024 whose two products back to the
 # layer's size are one round of 128 x 128 tiles (rows of 128 times columns of 128 up to the CUs).  That is 4096 tokens of Qwen3-0.6B, 476 of Qwen3-1.7B, 124 of
-# Qwen3-8B.  us of 14 layers, native / library with SiluAndMul's product from here / library and silu_mul: layers of 1024 x 3072, 2600 tokens 2438 / 2524 / 2686, 4000
-# 2864 / 2970 / 3280, 4200 (two rounds) 3902 / 3536 / 3678, 4440 3961 / 3523 / 3671; 768 x 2304, 5000 tokens 2314 / 2477 / 2681, 6000 (two rounds) 2995 / 2724 / 2874;
-# 2048 x 6144, 600 tokens 2399 / 2243 / 2340, 1390 3612 / 3353 / 3401; 2048 x 2048, 2100 tokens 3267 / 2603 / 2591; 512 x 1536, 7000 tokens 2103 / 2429 / 2784.
-# 8B, a layer's products, 64 tokens 115 and the library's 120, 216 tokens 184 and 169.
+# Qwen3-8B.  us of 14 layers, native / library with SiluAndMul's product from here / library and silu_mul: layers of 1024 x 3072, 2600 tokens 2414 / 2509 / 2574, 4000
+# 2849 / 2948 / 3162; 768 x 2304, 5000 tokens 2197 / 2278 / 2431; 2048 x 6144, 476 tokens 1700 / 1786 / 1757; 512 x 1536, 8000 tokens 2140 / 2245 / 2584; 8B, four layers, 124 tokens 667 / 679 / 694.
+# The limits are of tiles that took longer; with those of now the two ways meet further up, and in between the library's costs up to 10 %: 1024 x 3072, 4200 tokens 3361 / 3517 / 3648, 4440 3435 /
+# 3427 / 3567, 6000 4275 / 4192 / 4528; 768 x 2304, 6000 tokens 2517 / 2617 / 2791, 8000 3071 / 3083 / 3574; 2048 x 6144, 600 tokens 1867 / 2057 / 2055, 1390 3460 / 3450 / 3523; 2048 x 2048, 1500 tokens
+# 2037 / 2157 / 2199, 2100 2665 / 2665 / 2591; 1536 x 4096, 1500 tokens 2234 / 2471 / 2503; 8B, 140 tokens 727 / 792 / 808, 216 810 / 813 / 828.
 PREFILL_STEP_MAX_WORK, PREFILL_STEP_MAX_WORK_NARROW = int(24e9), int(70e9)
 
 
