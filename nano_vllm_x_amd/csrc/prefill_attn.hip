@@ -615,6 +615,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
     const int stamp_blk = gblk;
     const bool stamp_on = (gblk == 8 || gblk == 9) && head == 0 && (wave == 0 || wave == 3);
 #endif
+    // (a branch of lanes: behind a uniform one the accumulators move between two sets of registers three times a tile, 0.2 us of it)
     int last_key = wave_last_key;
     if (LOADERS) asm volatile("" : "+v"(last_key));
     for (int tile = 0; tile < n_tiles; ++tile) {
@@ -806,7 +807,7 @@ __global__ __launch_bounds__((NWAVES + LOADERS) * 64, LOADERS ? 1 : 2) void page
 // Workgroups of so many query positions, at most
 static int64_t pf_groups(int64_t positions, int64_t n_tokens, int64_t batch, int64_t hkv) { return ((n_tokens + positions - 1) / positions + batch - 1) * hkv; }
 // Few workgroups: waves of their own for the copies, and where there are fewer still 32 positions of two heads as two waves, which read half as much LDS a tile.  us a launch
-// with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.2 (32 positions) and 13.5, 1024 19.6 and 24.4.  Figures of turns that took 0.79 us (see there): 64 positions: 2500 tokens 43.1 and 57.3, six
+// with loader waves and the loop without them, 16 query heads: one sequence of 459 tokens 11.2 (32 positions) and 13.5.  Figures of turns that took 0.79 us (see there): 64 positions: 2500 tokens 43.1 and 57.3, six
 // questions behind 900-3000 keys (272 workgroups) 56.7 and 74.4, twelve (560) 93.0 and 80.8, eight prompts of 100-1024 (648) 35.6 and 31.3, 32 of 20-60 (416) 7.1 and 6.5.  32 heads: 1500 tokens 29.0
 // and 38.1, 2000 (504) 44.2 and 51.2, 20 of 30-100 behind 900 (488) 46.5 and 39.2, 632 70 and 67.
 // Between 392 and 512 workgroups what decides is how uneven the blocks are, of which the host knows the tokens and the sequences only: one or two sequences' blocks see more and more keys, and the longest are done
